@@ -29,6 +29,8 @@
 namespace kfac {
 namespace mma {
 
+constexpr int kRowStride = KT + 1;   // floats from row to row of the first operand's LDS panel
+
 // First operand of a group of products: rows = channels, k = (sample, p), p < L
 // running over the group's domain (a whole image, one image row, one border column
 // or one pixel):
@@ -75,11 +77,11 @@ struct LoaderDomain {
   }
 
   __device__ __forceinline__ void store(const Regs &r, float *lds) const {
-    float *p = lds + (team_tid() >> 5) * Panel<ROWS>::kRowKStride + (team_tid() & 31);
+    float *p = lds + (team_tid() >> 5) * kRowStride + (team_tid() & 31);
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
       const int row = first_row + 8 * i;
-      p[8 * i * Panel<ROWS>::kRowKStride] = (r.kvalid && row < rows_valid) ? r.v[i] : 0.f;
+      p[8 * i * kRowStride] = (r.kvalid && row < rows_valid) ? r.v[i] : 0.f;
     }
   }
 };
@@ -185,7 +187,7 @@ __device__ __forceinline__ void corr_shifts_body(const Plan &pl, const ShiftGrou
                                                  float *__restrict__ partial) {
   static_assert(!STACKED || WM == 1, "stacked groups use 64-row tiles");
   constexpr int BMA = 64 * WM;
-  float *ldsA = lds, *ldsB = lds + Panel<BMA>::kFloats;
+  float *ldsA = lds, *ldsB = lds + BMA * kRowStride;
   const int ntile = pl.tiles_a * pl.tiles_b;
   const int split = q / ntile, tile = q - split * ntile;
   const int I = tile / pl.tiles_b, J = tile - I * pl.tiles_b;
@@ -275,7 +277,7 @@ __device__ __forceinline__ void corr_shifts_body(const Plan &pl, const ShiftGrou
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i)
-      ldsA[(rm + 8 * i) * Panel<BMA>::kRowKStride + jm] = (ra.kvalid && ((rm + 8 * i) & 31) < pl.C) ? ra.v[i] : 0.f;
+      ldsA[(rm + 8 * i) * kRowStride + jm] = (ra.kvalid && ((rm + 8 * i) & 31) < pl.C) ? ra.v[i] : 0.f;
   };
   if (kbeg < kend) {
     load_a(kbeg);
@@ -308,14 +310,14 @@ __device__ __forceinline__ void corr_shifts_body(const Plan &pl, const ShiftGrou
             (unsigned)__ballot(row_in && (unsigned)((int)b + dj_first + s) < vline));
     }
     const bool active = !STACKED || wm < g.stacked;
-    const float *pa = ldsA + (wm * WM * 32 + lrow) * Panel<BMA>::kRowKStride + lk;
+    const float *pa = ldsA + (wm * WM * 32 + lrow) * kRowStride + lk;
     const float *pb = ldsB + (wn * 32 + lrow) * kShiftStride + lk + 2 + g.dj0;
     // operands of step kk + 1 are read from LDS before the matrix instructions of
     // step kk issue (the scheduling barriers keep the compiler from sinking the
     // reads to their first use, which would expose the LDS latency in every step)
     float a[2][WM], b[2][NS];
 #pragma unroll
-    for (int im = 0; im < WM; ++im) a[0][im] = pa[im * 32 * Panel<BMA>::kRowKStride];
+    for (int im = 0; im < WM; ++im) a[0][im] = pa[im * 32 * kRowStride];
 #pragma unroll
     for (int s = 0; s < NS; ++s) b[0][s] = pb[s];
     if (active) {
@@ -324,7 +326,7 @@ __device__ __forceinline__ void corr_shifts_body(const Plan &pl, const ShiftGrou
       const int cur = kk & 1, nxt = cur ^ 1;
       if (kk + 1 < KT / 2) {
 #pragma unroll
-        for (int im = 0; im < WM; ++im) a[nxt][im] = pa[im * 32 * Panel<BMA>::kRowKStride + 2 * kk + 2];
+        for (int im = 0; im < WM; ++im) a[nxt][im] = pa[im * 32 * kRowStride + 2 * kk + 2];
 #pragma unroll
         for (int s = 0; s < NS; ++s) b[nxt][s] = pb[2 * kk + 2 + s];
       }
@@ -361,7 +363,7 @@ __device__ __forceinline__ void corr_shifts_body(const Plan &pl, const ShiftGrou
 // run beside the rest), then the whole-image groups.
 template <int WM>
 __global__ __launch_bounds__(THREADS, 2) void corr_kernel(Plan pl, float *__restrict__ partial) {
-  __shared__ float lds[Panel<64 * WM>::kFloats + 64 * kShiftStride];
+  __shared__ float lds[64 * WM * kRowStride + 64 * kShiftStride];
   int w = blockIdx.x;
   if (w >= pl.nsmall) w = pl.nsmall + item_of_block(w - pl.nsmall, pl.total - pl.nsmall);
   int gi = 0;

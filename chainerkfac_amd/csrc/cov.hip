@@ -237,6 +237,29 @@ __device__ __forceinline__ void write_rowsums(float (&rs)[WM], int I, int dt, in
   }
 }
 
+// The same from the sums that mainloop_rowsum leaves in the threads: `sum` of row threadIdx.x.
+template <int WM>
+__device__ __forceinline__ void write_rowsum(float sum, int I, int dt, int d, int direct, float count,
+                                             float alpha, float beta, float *__restrict__ vec,
+                                             float *__restrict__ C) {
+  constexpr int BM = 64 * WM;
+  if (team_tid() >= BM) return;
+  const int row = I * BM + team_tid();
+  if (!direct) {
+    vec[row] = sum;
+  } else if (row < dt) {
+    float v = alpha * sum;
+    if (beta != 0.f) v += beta * C[(long long)(d - 1) * d + row];
+    C[(long long)(d - 1) * d + row] = v;
+    C[(long long)row * d + d - 1] = v;
+  }
+  if (direct && row == 0) {
+    float v = alpha * count;
+    if (beta != 0.f) v += beta * C[(long long)(d - 1) * d + d - 1];
+    C[(long long)(d - 1) * d + d - 1] = v;
+  }
+}
+
 // With a single k-slice (direct != 0) the tile is scaled and written straight
 // from registers; otherwise the raw partial tile goes to the workspace.
 // Workgroup -> (tile, k-slice).  Hardware deals consecutive workgroup ids
@@ -286,7 +309,7 @@ __global__ __launch_bounds__(THREADS, 3) void syrk_kernel(Loader ld, long long K
                                                           float *__restrict__ partial,
                                                           float *__restrict__ C) {
   constexpr int BM = 64 * WM;
-  __shared__ float lds[2 * Panel<BM>::kFloats];
+  __shared__ __align__(16) float lds[2 * Panel<BM>::kFloats];
   __shared__ int2 tabA[BM];
   __shared__ int2 tabB[BM];
   float *ldsA = lds, *ldsB = lds + Panel<BM>::kFloats;
@@ -304,9 +327,7 @@ __global__ __launch_bounds__(THREADS, 3) void syrk_kernel(Loader ld, long long K
   if (kend > K) kend = K;
   floatx16 acc[WM][WM];
   zero_acc<WM, WM>(acc);
-  float rs[WM];
-#pragma unroll
-  for (int im = 0; im < WM; ++im) rs[im] = 0.f;
+  float rs = 0.f;
   const int wave = threadIdx.x >> 6;
   const bool active = syrk_wave_active<WM>(I * BM, J * BM, dt, wave);
   if (I == J)
@@ -317,8 +338,7 @@ __global__ __launch_bounds__(THREADS, 3) void syrk_kernel(Loader ld, long long K
   const long long slot = (long long)ntile * (BM * BM) + (long long)tiles * BM;
   float *mine = partial + split * slot;
   if (ones && I == J)
-    write_rowsums<WM>(rs, I, dt, d, direct, (float)K, alpha, beta, mine + (long long)ntile * (BM * BM), C,
-                      wave);
+    write_rowsum<WM>(rs, I, dt, d, direct, (float)K, alpha, beta, mine + (long long)ntile * (BM * BM), C);
   if (direct) {
     write_tile<WM>(acc, lds, I, J, dt, d, alpha, beta, C, wave);
     return;
@@ -1319,7 +1339,7 @@ __global__ __launch_bounds__(THREADS, 3) void syrk_group_kernel(const GroupItemS
                                                                 const int2 *__restrict__ tasks,
                                                                 float *__restrict__ ws) {
   constexpr int BM = 64 * WM;
-  __shared__ float lds[2 * Panel<BM>::kFloats];
+  __shared__ __align__(16) float lds[2 * Panel<BM>::kFloats];
   static_assert(2 * Panel<BM>::kFloats >= 64 * 65, "LDS too small for the epilogue transpose");
   float *ldsA = lds, *ldsB = lds + Panel<BM>::kFloats;
   const int2 task = tasks[blockIdx.x];
@@ -1340,12 +1360,10 @@ __global__ __launch_bounds__(THREADS, 3) void syrk_group_kernel(const GroupItemS
   if (kend > s.K) kend = s.K;
   floatx16 acc[WM][WM];
   zero_acc<WM, WM>(acc);
-  float rs[WM];
-#pragma unroll
-  for (int im = 0; im < WM; ++im) rs[im] = 0.f;
+  float rs = 0.f;
   int wave = threadIdx.x >> 6;
   const bool active = syrk_wave_active<WM>(I * BM, J * BM, dt, wave);
-  unsigned store = 0xfu, rowmask = 0x3u;
+  unsigned store = 0xfu;
   if (I != J) {
     mainloop<WM, WM, false>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, active, wave);
   } else if (WM == 2 && (I + 1) * BM <= dt) {
@@ -1353,16 +1371,15 @@ __global__ __launch_bounds__(THREADS, 3) void syrk_group_kernel(const GroupItemS
     const DiagRole role = diag_tile_role(wave);
     wave = role.role;
     store = role.compute == 0xdu ? 0xfu : role.store;
-    rowmask = role.compute == 0xdu ? 0x3u : (role.compute == 0x3u ? 0x1u : 0x2u);
     if (role.compute == 0xdu)
       mainloop_impl<WM, WM, true, true, Loader, Loader, 0xdu>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB,
-                                                             acc, rs, true, wave);
+                                                             acc, &rs, true, wave);
     else if (role.compute == 0x3u)
       mainloop_impl<WM, WM, true, true, Loader, Loader, 0x3u>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB,
-                                                             acc, rs, true, wave);
+                                                             acc, &rs, true, wave);
     else
       mainloop_impl<WM, WM, true, true, Loader, Loader, 0xcu>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB,
-                                                             acc, rs, true, wave);
+                                                             acc, &rs, true, wave);
   } else {
     mainloop_rowsum<WM, WM, true>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, rs, active,
                                   wave);
@@ -1370,8 +1387,8 @@ __global__ __launch_bounds__(THREADS, 3) void syrk_group_kernel(const GroupItemS
   const long long slot = (long long)s.ntile * (BM * BM) + (long long)s.tiles * BM;
   float *mine = ws + s.part_off + split * slot;
   if (s.ones && I == J)
-    write_rowsums<WM>(rs, I, dt, s.d, s.direct, s.count, v.alpha, v.beta,
-                      mine + (long long)s.ntile * (BM * BM), v.out, wave, rowmask);
+    write_rowsum<WM>(rs, I, dt, s.d, s.direct, s.count, v.alpha, v.beta,
+                     mine + (long long)s.ntile * (BM * BM), v.out);
   if (s.direct) {
     write_tile<WM>(acc, lds, I, J, dt, s.d, v.alpha, v.beta, v.out, wave, store);
     return;
@@ -1407,7 +1424,6 @@ __global__ __launch_bounds__(kMacroThreads, 1) void syrk_macro_kernel(
   const int team = threadIdx.x >> 8;
   const int ta = team >> 1, tb = team & 1;
   const int wave = (threadIdx.x >> 6) & 3;
-  const int lane = threadIdx.x & 63;
   const int2 task = tasks[blockIdx.x];
   if (task.x < 0) return;   // padding of a shorter XCD run
   const GroupItemStatic s = st[task.x];
@@ -1435,46 +1451,30 @@ __global__ __launch_bounds__(kMacroThreads, 1) void syrk_macro_kernel(
   if (kend > s.K) kend = s.K;
   floatx16 acc[WM][WM];
   zero_acc<WM, WM>(acc);
-  float rs[WM] = {0.f, 0.f};
   const bool active = has_tile && syrk_wave_active<WM>(I * BM, J * BM, dt, wave);
-  const bool sums = active && I == J;   // diagonal tile: also the row sums (the ones column)
   const int wm = wave >> 1, wn = wave & 1;
-  const int lrow = lane & 31, lk = lane >> 5;
   typename Loader::Regs r;
+  float sum[Loader::kSumSlots];   // the row sums (the ones column) of the panel this team stages
+#pragma unroll
+  for (int i = 0; i < Loader::kSumSlots; ++i) sum[i] = 0.f;
   if (stages && kbeg < kend) ld.load(r, prow * BM, kbeg, kend);
   for (long long k0 = kbeg; k0 < kend; k0 += KT) {
-    if (stages) ld.store(r, mine_panel);
+    if (stages) ld.template store<true>(r, mine_panel, sum);
     __syncthreads();
     if (stages && k0 + KT < kend) ld.load(r, prow * BM, k0 + KT, kend);
-    if (active) {
-#pragma unroll
-      for (int kk = 0; kk < KT / 2; ++kk) {
-        float a[WM], b[WM];
-#pragma unroll
-        for (int im = 0; im < WM; ++im)
-          a[im] = fetch<BM, Loader::kKRow>(pa, (wm * WM + im) * 32 + lrow, 2 * kk + lk);
-        if (sums) {
-#pragma unroll
-          for (int im = 0; im < WM; ++im) rs[im] += a[im];
-        }
-#pragma unroll
-        for (int in = 0; in < WM; ++in)
-          b[in] = fetch<BM, Loader::kKRow>(pb, (wn * WM + in) * 32 + lrow, 2 * kk + lk);
-#pragma unroll
-        for (int im = 0; im < WM; ++im)
-#pragma unroll
-          for (int in = 0; in < WM; ++in)
-            acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[im], b[in], acc[im][in], 0, 0, 0);
-      }
-    }
+    if (active) mma_panel<WM, WM>(pa, pb, wm, wn, acc);
     __syncthreads();
   }
-  if (!has_tile) return;
   const long long slot = (long long)s.ntile * (BM * BM) + (long long)s.tiles * BM;
   float *mine = ws + s.part_off + split * slot;
-  if (s.ones && I == J)
-    write_rowsums<WM>(rs, I, dt, s.d, 0, s.count, v.alpha, v.beta, mine + (long long)s.ntile * (BM * BM),
-                      v.out, wave);
+  if (on_diag && s.ones) {
+    // teams 0 and 1 stage the panels of the diagonal tiles
+    const float rs = add_row_sums<BM, Loader>(sum, mine_panel);
+    if (team < 2 && stages)
+      write_rowsum<WM>(rs, prow, dt, s.d, 0, s.count, v.alpha, v.beta, mine + (long long)s.ntile * (BM * BM),
+                       v.out);
+  }
+  if (!has_tile) return;
   float *out = mine + (long long)(I * (I + 1) / 2 + J) * (BM * BM);
   for_each_acc<WM, WM>(acc, [&](int rr, int cc, float val) { out[rr * BM + cc] = val; }, wave);
 }

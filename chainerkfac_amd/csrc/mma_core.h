@@ -1,11 +1,11 @@
-// FP32 MFMA tile engine shared by the covariance (SYRK), preconditioning (GEMM)
-// and inverse kernels.
+// Float32 tile engine on the matrix cores, shared by the covariance (SYRK),
+// preconditioning (GEMM) and inverse kernels.
 //
 // A workgroup of 256 threads (4 waves, 2 x 2) computes a (64*WM) x (64*WN)
-// tile of  D[i][j] = sum_k Aop(i, k) * Bop(j, k)  with v_mfma_f32_32x32x2_f32;
-// each wave owns WM x WN accumulator blocks of 32 x 32.  Operand panels
-// (rows x 32 k-values) are staged through LDS by "loaders" that know how an
-// operand is laid out in memory:
+// tile of  D[i][j] = sum_k Aop(i, k) * Bop(j, k);  each wave owns WM x WN
+// accumulator blocks of 32 x 32.  Operand panels (rows x 32 k-values) are
+// staged through LDS by "loaders" that know how an operand is laid out in
+// memory:
 //
 //   LoaderKC  k is the contiguous index:  (sample, row, l) tensors such as an
 //             NCHW activation viewed as rows = channel, k = (sample, pixel),
@@ -17,10 +17,34 @@
 //   LoaderIM  implicit im2col: row = (c, kh, kw) [+ ones], k = (sample, y, x);
 //             the patch matrix is gathered straight from the NCHW tensor.
 //
-// LDS panel layouts: "RowK" (row-major, stride 33, used by KC/IM) and "KRow"
-// (k-major, stride rows+4, used by KS); both give conflict-free MFMA operand
-// reads.  The main loop keeps one LDS buffer and prefetches the next panel
-// into registers while the current one feeds the matrix cores.
+// The float32 product.  The matrix cores multiply float32 at 256 flop per cycle
+// and CU and bfloat16 at 4096.  A float32 number is the exact sum of three
+// bfloat16 numbers (8 significand bits each: 24 in all), x = hi + mid + lo, each
+// the rounded rest of the one before, so a product of two float32 numbers is nine
+// products of bfloat16 numbers, every one exact in float32.  The three smallest
+// (mid*lo, lo*mid, lo*lo: at most 2^-23 of the product together and 2^-26 in the
+// root mean square, of either sign) are left out; the other six are accumulated in
+// float32, small ones first.  What is lost that way is less than what float32
+// accumulation loses by itself, and the accumulator is rounded less often (an
+// instruction adds sixteen k-values instead of two): against float64, products of
+// 4608 x 4608 x 4608 have
+// 0.63 to 0.85 times the error of the v_mfma_f32_32x32x2_f32 kernel this replaced
+// (root mean square relative to sum |a||b|: 6.4e-7 against 1.03e-6 for positive
+// operands, 2.35e-8 against 2.76e-8 for signed ones, 6.2e-8 against 8.0e-8 for
+// magnitudes spread over e^6).  The split is the published one of Henry, Tang and
+// Heinecke (2019).  Six products of bfloat16 at the rate a large library product
+// reaches here (1370 TFLOP/s at the clock the power budget leaves) are 228 TFLOP/s
+// of float32, against 157 that the float32 instructions could reach at best;
+// 128 x 128 tiles of this engine run at 165 .. 190 (the float32 kernel: 108 .. 127).
+//
+// An LDS panel holds one row of the operand after the other: 32 k-values of hi
+// (64 bytes), of mid, of lo, and 16 bytes that spread the rows over the banks.  A
+// lane's operand of v_mfma_f32_32x32x16_bf16 is eight consecutive k-values of a
+// plane, one 16-byte chunk; the chunks of a row are stored at their index xor
+// (row / 16) mod 4, so that the writes of every loader below (rows four apart in
+// LoaderKS) and the 16-byte reads all spread over the 64 banks.  One LDS buffer:
+// the next panel is prefetched into registers while the current one feeds the
+// matrix cores, and split when it is stored.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -31,6 +55,11 @@ namespace mma {
 constexpr int KT = 32;        // k-values per LDS panel
 constexpr int THREADS = 256;  // 4 waves
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
 // Loads from global memory at a wave-uniform base plus a 32-bit byte offset per
 // lane: the form of the load instruction that takes the base from scalar
@@ -51,13 +80,50 @@ __device__ __forceinline__ float gload1(const float *base, unsigned byte_off) {
 // four teams each stage and multiply like one such workgroup.
 __device__ __forceinline__ int team_tid() { return (int)(threadIdx.x & (THREADS - 1)); }
 
+// Two float32 numbers as three packed pairs of bfloat16 numbers (first number in the low
+// half), a = hi + mid + lo exactly.  11 vector instructions: three v_cvt_pk_bf16_f32 (round
+// to nearest even) and the two rests of either number.
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+  const floatx2 t = {a, b};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(t, bf16x2));
+}
+__device__ __forceinline__ void split_pair(float a, float b, unsigned &hi, unsigned &mid, unsigned &lo) {
+  hi = pack_bf16(a, b);
+  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
+  mid = pack_bf16(a1, b1);
+  const float a2 = a1 - __uint_as_float(mid << 16), b2 = b1 - __uint_as_float(mid & 0xffff0000u);
+  lo = pack_bf16(a2, b2);
+}
+// The six plane pairs of a product, smallest first (0 = hi, 1 = mid, 2 = lo).
+constexpr int kSplitTerms = 6;
+constexpr int kSplitA[kSplitTerms] = {2, 0, 1, 1, 0, 0};
+constexpr int kSplitB[kSplitTerms] = {0, 2, 1, 0, 1, 0};
+
 template <int ROWS>
 struct Panel {
-  static constexpr int kRowKStride = KT + 1;
-  static constexpr int kKRowStride = ROWS + 4;
-  static constexpr int kFloats =
-      (ROWS * kRowKStride > KT * kKRowStride) ? ROWS * kRowKStride : KT * kKRowStride;
+  static constexpr int kPlaneBytes = KT * 2;
+  static constexpr int kRowBytes = 3 * kPlaneBytes + 16;
+  static constexpr int kFloats = ROWS * kRowBytes / 4;
 };
+// Byte offset of 16-byte chunk `chunk` (k-values 8 chunk ..) of a row inside a plane of the row.
+__device__ __forceinline__ int panel_chunk(int row, int chunk) { return ((chunk ^ (row >> 4)) & 3) * 16; }
+
+// Store the planes of two or four consecutive k-values at their place in a row.
+__device__ __forceinline__ void panel_store2(char *p, float a, float b) {
+  unsigned h, m, l;
+  split_pair(a, b, h, m, l);
+  *reinterpret_cast<unsigned *>(p) = h;
+  *reinterpret_cast<unsigned *>(p + KT * 2) = m;
+  *reinterpret_cast<unsigned *>(p + KT * 4) = l;
+}
+__device__ __forceinline__ void panel_store4(char *p, float a, float b, float c, float d) {
+  unsigned h0, m0, l0, h1, m1, l1;
+  split_pair(a, b, h0, m0, l0);
+  split_pair(c, d, h1, m1, l1);
+  *reinterpret_cast<uintx2 *>(p) = uintx2{h0, h1};
+  *reinterpret_cast<uintx2 *>(p + KT * 2) = uintx2{m0, m1};
+  *reinterpret_cast<uintx2 *>(p + KT * 4) = uintx2{l0, l1};
+}
 
 // Loader protocol: init() fixes the panel (first row) and precomputes what
 // does not change along k (row offsets, row validity); load() issues the
@@ -68,6 +134,9 @@ struct Panel {
 // touches the loaded registers, so the loads stay in flight while the matrix
 // cores work on the previous panel.  Offsets are 32-bit element offsets from
 // the tensor base (tensors hold fewer than 2^30 elements, 4 GiB; checked on the host).
+// With SUM, store() also adds what it stores to the thread's row sums: slot i of `sum` belongs
+// to panel row sum_row(i), and the kSumParts threads with sum_part() = 0 .. kSumParts - 1 hold
+// the parts of a row (add_row_sums below).
 
 // ---------------------------------------------------------------------------
 // LoaderKC: element (row, kg) at base + (kg / L) * sample_stride
@@ -85,7 +154,6 @@ struct Panel {
 template <int ROWS, bool VEC>
 struct LoaderKC {
   static_assert(VEC, "the scalar variant is the specialisation below");
-  static constexpr bool kKRow = false;
   static constexpr int NV = ROWS / 32;
   struct Regs {
     float4 v[NV];
@@ -149,43 +217,38 @@ struct LoaderKC {
     }
   }
 
-  __device__ __forceinline__ void store(const Regs &r, float *lds) const {
-    const int kq = (team_tid() & 7) * 4;
+  static constexpr int kSumSlots = NV, kSumParts = 8;
+  __device__ __forceinline__ static int sum_row(int i) { return (team_tid() >> 3) + 32 * i; }
+  __device__ __forceinline__ static int sum_part() { return team_tid() & 7; }
+
+  template <bool SUM>
+  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
     const int rr = team_tid() >> 3;
-    if (r.fast) {
+    char *p = reinterpret_cast<char *>(lds) + rr * Panel<ROWS>::kRowBytes + (team_tid() & 1) * 8;
+    const int chunk = panel_chunk(rr, (team_tid() & 7) >> 1);
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        float *p = lds + (rr + 32 * i) * Panel<ROWS>::kRowKStride + kq;
-        p[0] = r.v[i].x;
-        p[1] = r.v[i].y;
-        p[2] = r.v[i].z;
-        p[3] = r.v[i].w;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        float *p = lds + (rr + 32 * i) * Panel<ROWS>::kRowKStride + kq;
-        const float t[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
+    for (int i = 0; i < NV; ++i) {
+      float t[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
+      if (!r.fast) {
         const bool rv = (rowvalid >> i) & 1u;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const bool kv = (r.kmask >> e) & 1u;
-          p[e] = (kv && rv) ? t[e] : 0.f;
-        }
+        for (int e = 0; e < 4; ++e) t[e] = (rv && ((r.kmask >> e) & 1u)) ? t[e] : 0.f;
       }
+      if (SUM) sum[i] += (t[0] + t[1]) + (t[2] + t[3]);
+      // rows 32 apart: the chunk index differs in bit 1
+      panel_store4(p + 32 * i * Panel<ROWS>::kRowBytes + ((i & 1) ? chunk ^ 32 : chunk), t[0], t[1], t[2], t[3]);
     }
   }
 };
 
-// Scalar variant: dword loads with the 32 lanes of a half-wave on 32 consecutive
-// k-values of one row.  It is the one that can subsample (line_len > 0).
+// Scalar variant: dword loads, a thread takes two consecutive k-values of a row and
+// 16 lanes the 32 of a panel.  It is the one that can subsample (line_len > 0).
 template <int ROWS>
 struct LoaderKC<ROWS, false> {
-  static constexpr bool kKRow = false;
-  static constexpr int NR = ROWS / 8;   // rows per thread
+  static constexpr int NR = ROWS / 16;   // rows per thread
   struct Regs {
-    float v[NR];
-    bool kvalid;   // this thread's k-value is inside the range
+    float v[NR][2];
+    unsigned kvalid;   // bit e: k-value e of this thread's pair is inside the range
   };
   const float *base;
   unsigned sample_stride;
@@ -197,29 +260,34 @@ struct LoaderKC<ROWS, false> {
   // line_stride + (p % line_len) * px_stride of the row.  line_len = 0: k-values
   // are consecutive elements.
   unsigned line_len = 0, line_stride = 0, px_stride = 1;
-  // per-thread panel state: row i of the thread is first_row + 8 i; rows past
+  // per-thread panel state: row i of the thread is first_row + 16 i; rows past
   // the end load from the last data row (masked when stored)
   int first_row;
   unsigned last_off;
 
   __device__ __forceinline__ void init(float *, int row0) {
-    first_row = row0 + (team_tid() >> 5);
+    first_row = row0 + (team_tid() >> 4);
     last_off = (unsigned)(rows_valid > 0 ? rows_valid - 1 : 0) * row_stride;
   }
 
   __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
-    const long long kg = k0 + (team_tid() & 31);
-    r.kvalid = kg < k_end;
-    const unsigned kc = r.kvalid ? (unsigned)kg : 0u;
-    unsigned koff = kc;
-    if (L < (unsigned)k_end || line_len) {  // more than one sample, or subsampled rows
-      const unsigned s = kc / L;
-      unsigned pix = kc - s * L;
-      if (line_len) {
-        const unsigned line = pix / line_len;
-        pix = line * line_stride + (pix - line * line_len) * px_stride;
+    const long long kg = k0 + (team_tid() & 15) * 2;
+    const long long left = k_end - kg;
+    r.kvalid = left >= 2 ? 3u : (left == 1 ? 1u : 0u);
+    unsigned koff[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const unsigned kc = ((r.kvalid >> e) & 1u) ? (unsigned)kg + e : 0u;
+      koff[e] = kc;
+      if (L < (unsigned)k_end || line_len) {  // more than one sample, or subsampled rows
+        const unsigned s = kc / L;
+        unsigned pix = kc - s * L;
+        if (line_len) {
+          const unsigned line = pix / line_len;
+          pix = line * line_stride + (pix - line * line_len) * px_stride;
+        }
+        koff[e] = s * sample_stride + pix;
       }
-      koff = s * sample_stride + pix;
     }
     // The row offsets are cheap to recompute and expensive to keep: hide the
     // row from the optimiser so that it does not hoist NR offsets per operand
@@ -229,17 +297,28 @@ struct LoaderKC<ROWS, false> {
     const unsigned off0 = (unsigned)fr * row_stride;
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-      const unsigned off = off0 + (unsigned)(8 * i) * row_stride;
-      r.v[i] = gload1(base, (koff + (off < last_off ? off : last_off)) * 4u);
+      const unsigned off = off0 + (unsigned)(16 * i) * row_stride;
+      const unsigned ro = off < last_off ? off : last_off;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) r.v[i][e] = gload1(base, (koff[e] + ro) * 4u);
     }
   }
 
-  __device__ __forceinline__ void store(const Regs &r, float *lds) const {
-    float *p = lds + (team_tid() >> 5) * Panel<ROWS>::kRowKStride + (team_tid() & 31);
+  static constexpr int kSumSlots = NR, kSumParts = 16;
+  __device__ __forceinline__ static int sum_row(int i) { return (team_tid() >> 4) + 16 * i; }
+  __device__ __forceinline__ static int sum_part() { return team_tid() & 15; }
+
+  template <bool SUM>
+  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
+    const int pr = team_tid() & 15;
+    char *p = reinterpret_cast<char *>(lds) + (team_tid() >> 4) * Panel<ROWS>::kRowBytes + (pr & 3) * 4;
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-      const int row = first_row + 8 * i;
-      p[8 * i * Panel<ROWS>::kRowKStride] = (r.kvalid && row < rows_valid) ? r.v[i] : 0.f;
+      const bool rv = first_row + 16 * i < rows_valid;
+      const float a = (rv && (r.kvalid & 1u)) ? r.v[i][0] : 0.f;
+      const float b = (rv && (r.kvalid & 2u)) ? r.v[i][1] : 0.f;
+      if (SUM) sum[i] += a + b;
+      panel_store2(p + 16 * i * Panel<ROWS>::kRowBytes + panel_chunk(16 * i, pr >> 2), a, b);
     }
   }
 };
@@ -250,13 +329,12 @@ struct LoaderKC<ROWS, false> {
 // ---------------------------------------------------------------------------
 template <int ROWS, bool VEC>
 struct LoaderKS {
-  static constexpr bool kKRow = true;
   static constexpr int RQ = ROWS / 4;          // row quads per k
-  static constexpr int KPP = THREADS / RQ;     // k-values per pass
-  static constexpr int NV = KT / KPP;
+  static constexpr int KPP = THREADS / RQ;     // threads per row quad
+  static constexpr int NV = KT / KPP;          // consecutive k-values of a thread: 4 or 2
   struct Regs {
     float4 v[NV];
-    unsigned kmask;  // bit i: k-value of pass i is inside the range
+    unsigned kmask;  // bit i: k-value i of this thread is inside the range
     bool fast;
   };
   const float *base;
@@ -276,14 +354,14 @@ struct LoaderKS {
   }
 
   __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
-    const int kk = team_tid() / RQ;
+    const int kk = team_tid() / RQ * NV;
     const bool full_k = k0 + KT <= k_end;
     r.fast = full_rows && full_k;
     r.kmask = 0;
     if (quad_ok) {
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        const long long kg = k0 + kk + KPP * i;
+        const long long kg = k0 + kk + i;
         const bool kok = full_k || kg < k_end;
         if (kok) r.kmask |= 1u << i;
         r.v[i] = gload4(base, ((unsigned)(kok ? kg : 0) * ld + (unsigned)row) * 4u);
@@ -291,7 +369,7 @@ struct LoaderKS {
     } else {
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        const long long kg = k0 + kk + KPP * i;
+        const long long kg = k0 + kk + i;
         const bool kok = kg < k_end;
         if (kok) r.kmask |= 1u << i;
         const unsigned kc = (unsigned)(kok ? kg : 0);
@@ -308,32 +386,36 @@ struct LoaderKS {
     }
   }
 
-  __device__ __forceinline__ void store(const Regs &r, float *lds) const {
-    const int rq = (team_tid() % RQ) * 4;
-    const int kk = team_tid() / RQ;
-    if (r.fast) {
+  static constexpr int kSumSlots = 4, kSumParts = KPP;
+  __device__ __forceinline__ static int sum_row(int i) { return (team_tid() % RQ) * 4 + i; }
+  __device__ __forceinline__ static int sum_part() { return team_tid() / RQ; }
+
+  template <bool SUM>
+  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
+    const int rq = team_tid() % RQ, kk = team_tid() / RQ * NV;
+    char *p = reinterpret_cast<char *>(lds) + rq * 4 * Panel<ROWS>::kRowBytes +
+              panel_chunk(rq * 4, kk >> 3) + (kk & 7) * 2;
 #pragma unroll
-      for (int i = 0; i < NV; ++i)
-        *reinterpret_cast<float4 *>(lds + (kk + KPP * i) * Panel<ROWS>::kKRowStride + rq) = r.v[i];
-    } else {
+    for (int e = 0; e < 4; ++e) {
+      const int re = row + e;
+      float t[NV];
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        const float t[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
-        const bool kv = (r.kmask >> i) & 1u;
-        float o[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int re = row + e;
+        t[i] = e == 0 ? r.v[i].x : e == 1 ? r.v[i].y : e == 2 ? r.v[i].z : r.v[i].w;
+        if (!r.fast) {
           float val = 0.f;
           if (re < rows_valid)
-            val = t[e];
+            val = t[i];
           else if (re == rows_valid && has_extra)
-            val = extra ? t[e] : 1.f;
-          o[e] = kv ? val : 0.f;
+            val = extra ? t[i] : 1.f;
+          t[i] = ((r.kmask >> i) & 1u) ? val : 0.f;
         }
-        *reinterpret_cast<float4 *>(lds + (kk + KPP * i) * Panel<ROWS>::kKRowStride + rq) =
-            make_float4(o[0], o[1], o[2], o[3]);
+        if (SUM) sum[e] += t[i];
       }
+      if (NV == 4)
+        panel_store4(p + e * Panel<ROWS>::kRowBytes, t[0], t[1], t[NV - 2], t[NV - 1]);
+      else
+        panel_store2(p + e * Panel<ROWS>::kRowBytes, t[0], t[1]);
     }
   }
 };
@@ -345,11 +427,10 @@ struct LoaderKS {
 // ---------------------------------------------------------------------------
 template <int ROWS>
 struct LoaderIM {
-  static constexpr bool kKRow = false;
-  static constexpr int NV = ROWS / 8;
+  static constexpr int NV = ROWS / 16;
   struct Regs {
-    float v[NV];
-    unsigned use;
+    float v[NV][2];
+    unsigned use;   // bit 2 i + e: value e of row i lies inside the image
   };
   const float *base;
   int C, H, W, kh, kw, sy, sx, ph, pw, ho, wo;
@@ -378,115 +459,156 @@ struct LoaderIM {
   }
 
   __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
-    const int k = team_tid() & 31;
-    const int rr = team_tid() >> 5;
-    const long long kg = k0 + k;
-    const bool kok = kg < k_end;
-    const unsigned kc = kok ? (unsigned)kg : 0u;
     const unsigned howo = (unsigned)(ho * wo);
-    const unsigned s = kc / howo;
-    const unsigned rem = kc - s * howo;
-    const int oy = (int)(rem / (unsigned)wo);
-    const int ox = (int)rem - oy * wo;
-    const int iy0 = oy * sy - ph;
-    const int ix0 = ox * sx - pw;
-    const long long idx0 = ((long long)s * C * H + iy0) * (long long)W + ix0;
+    bool kok[2];
+    int iy0[2], ix0[2];
+    long long idx0[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const long long kg = k0 + (team_tid() & 15) * 2 + e;
+      kok[e] = kg < k_end;
+      const unsigned kc = kok[e] ? (unsigned)kg : 0u;
+      const unsigned s = kc / howo;
+      const unsigned rem = kc - s * howo;
+      const int oy = (int)(rem / (unsigned)wo);
+      const int ox = (int)rem - oy * wo;
+      iy0[e] = oy * sy - ph;
+      ix0[e] = ox * sx - pw;
+      idx0[e] = ((long long)s * C * H + iy0[e]) * (long long)W + ix0[e];
+    }
     r.use = 0;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int2 e = table[rr + 8 * i];
-      const int iy = iy0 + (e.y >> 16);
-      const int ix = ix0 + (e.y & 0xffff);
-      const bool ok = kok && e.y >= 0 && (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W;
-      r.v[i] = base[ok ? idx0 + e.x : 0];
-      if (ok) r.use |= 1u << i;
+      const int2 t = table[(team_tid() >> 4) + 16 * i];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int iy = iy0[e] + (t.y >> 16);
+        const int ix = ix0[e] + (t.y & 0xffff);
+        const bool ok = kok[e] && t.y >= 0 && (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W;
+        r.v[i][e] = base[ok ? idx0[e] + t.x : 0];
+        if (ok) r.use |= 1u << (2 * i + e);
+      }
     }
   }
 
-  __device__ __forceinline__ void store(const Regs &r, float *lds) const {
-    const int k = team_tid() & 31;
-    const int rr = team_tid() >> 5;
+  static constexpr int kSumSlots = NV, kSumParts = 16;
+  __device__ __forceinline__ static int sum_row(int i) { return (team_tid() >> 4) + 16 * i; }
+  __device__ __forceinline__ static int sum_part() { return team_tid() & 15; }
+
+  template <bool SUM>
+  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
+    const int pr = team_tid() & 15;
+    char *p = reinterpret_cast<char *>(lds) + (team_tid() >> 4) * Panel<ROWS>::kRowBytes + (pr & 3) * 4;
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
-      lds[(rr + 8 * i) * Panel<ROWS>::kRowKStride + k] = ((r.use >> i) & 1u) ? r.v[i] : 0.f;
+    for (int i = 0; i < NV; ++i) {
+      const float a = ((r.use >> (2 * i)) & 1u) ? r.v[i][0] : 0.f;
+      const float b = ((r.use >> (2 * i + 1)) & 1u) ? r.v[i][1] : 0.f;
+      if (SUM) sum[i] += a + b;
+      panel_store2(p + 16 * i * Panel<ROWS>::kRowBytes + panel_chunk(16 * i, pr >> 2), a, b);
+    }
   }
 };
 
-// Operand fetch for one MFMA: lane l supplies element (row = l % 32, k = l / 32).
-template <int ROWS, bool KROW>
-__device__ __forceinline__ float fetch(const float *lds, int row, int k) {
-  if (KROW)
-    return lds[k * Panel<ROWS>::kKRowStride + row];
-  else
-    return lds[row * Panel<ROWS>::kRowKStride + k];
+// The MFMAs of one panel: this wave's WM x WN blocks from the LDS panels pa and pb (the same
+// array for the diagonal tile of a SYRK), 6 per block and 16 k-values.  Lane l supplies row
+// l % 32 and k-values 8 (l / 32) .. + 7 of a 16-k step.
+// MASK: bit im * WN + in set = this wave computes block (im, in) (compile time, so that a wave
+// that owns fewer blocks carries no test per MFMA).
+template <int WM, int WN, unsigned MASK = 0xffffffffu>
+__device__ __forceinline__ void mma_panel(const float *pa, const float *pb, int wm, int wn,
+                                          floatx16 (&acc)[WM][WN]) {
+  constexpr int RB = Panel<64>::kRowBytes;
+  const int lane = threadIdx.x & 63;
+  const int lrow = lane & 31, lk = lane >> 5;
+  // 32-row block b keeps chunk c of its lower / upper 16 rows at c ^ (2 b) / c ^ (2 b + 1) (mod 4)
+  const int lane_off = lrow * RB + ((lk ^ (lrow >> 4)) & 1) * 16;
+  const char *a0 = reinterpret_cast<const char *>(pa) + wm * WM * 32 * RB + lane_off;
+  const char *b0 = reinterpret_cast<const char *>(pb) + wn * WN * 32 * RB + lane_off;
+  const int pm = WM == 1 ? (wm & 1) * 32 : 0, pn = WN == 1 ? (wn & 1) * 32 : 0;
+#pragma unroll
+  for (int s = 0; s < KT / 16; ++s) {
+    bf16x8 fa[WM][3], fb[WN][3];
+#pragma unroll
+    for (int im = 0; im < WM; ++im) {
+      const char *p = a0 + im * 32 * RB + ((((s ^ im) & 1) * 32) ^ pm);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) fa[im][q] = *reinterpret_cast<const bf16x8 *>(p + q * (KT * 2));
+    }
+#pragma unroll
+    for (int in = 0; in < WN; ++in) {
+      const char *p = b0 + in * 32 * RB + ((((s ^ in) & 1) * 32) ^ pn);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) fb[in][q] = *reinterpret_cast<const bf16x8 *>(p + q * (KT * 2));
+    }
+#pragma unroll
+    for (int t = 0; t < kSplitTerms; ++t)
+#pragma unroll
+      for (int im = 0; im < WM; ++im)
+#pragma unroll
+        for (int in = 0; in < WN; ++in)
+          if (MASK & (1u << (im * WN + in)))
+            acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[im][kSplitA[t]], fb[in][kSplitB[t]],
+                                                                  acc[im][in], 0, 0, 0);
+  }
+}
+
+// The row sums of a panel from the parts that its threads added up while storing it (SUM in the
+// loaders), in a fixed order: the sum of panel row t in the team's thread t < ROWS.  `lds`: a
+// panel's memory of this team, free to overwrite.  Every thread of the workgroup calls it.
+template <int ROWS, class Loader>
+__device__ __forceinline__ float add_row_sums(const float *sum, float *lds) {
+  static_assert(Loader::kSumParts * ROWS <= Panel<ROWS>::kFloats, "the parts must fit a panel");
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < Loader::kSumSlots; ++i) lds[Loader::sum_part() * ROWS + Loader::sum_row(i)] = sum[i];
+  __syncthreads();
+  float total = 0.f;
+  if (team_tid() < ROWS) {
+#pragma unroll
+    for (int p = 0; p < Loader::kSumParts; ++p) total += lds[p * ROWS + team_tid()];
+  }
+  __syncthreads();
+  return total;
 }
 
 // Main loop.  acc[im][in] accumulates the 32x32 block at rows
 // (wave_m * WM + im) * 32 of the A panel and (wave_n * WN + in) * 32 of the B
 // panel.  With SAME the B operand is read from the A panel (diagonal tile of a
 // SYRK) and lb is not used.  ldsA / ldsB hold Panel<64*WM> / Panel<64*WN>
-// floats.  Operands of step kk+1 are fetched from LDS before the MFMAs of step
-// kk issue, so LDS latency hides behind the matrix pipeline.
-// With RS the lane also sums the A operand values it feeds to the matrix cores:
-// rs[im] ends as the sum over this lane's k-values (k = lane / 32 mod 2) of row
-// (wave_m * WM + im) * 32 + lane % 32, i.e. half of that row's sum.
+// floats.
+// With RS the sums over k of the A operand's rows are formed on the side:
+// *rowsum is that of row threadIdx.x of the tile (threads below 64*WM).
 // A wave with `active` false stages panels like the others but feeds nothing to
 // the matrix cores (its block of the tile is not needed: above the diagonal of a
 // symmetric product, or past the end of the matrix); its accumulators stay as
 // they are.
-// MASK: bit im * WN + in set = this wave computes block (im, in) of its 2 x 2
-// (compile time, so that a wave that owns fewer blocks carries no test per MFMA).
 template <int WM, int WN, bool SAME, bool RS, class LA, class LB, unsigned MASK = 0xffffffffu>
 __device__ __forceinline__ void mainloop_impl(const LA &la, const LB &lb, int rowA0, int rowB0,
                                               long long kbeg, long long kend, float *ldsA,
-                                              float *ldsB, floatx16 (&acc)[WM][WN], float *rs,
+                                              float *ldsB, floatx16 (&acc)[WM][WN], float *rowsum,
                                               bool active = true, int wave = threadIdx.x >> 6) {
-  constexpr int RA = 64 * WM, RB = 64 * WN;
-  const int lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
-  const int lrow = lane & 31, lk = lane >> 5;
   typename LA::Regs ra;
   typename LB::Regs rb;
+  float sum[LA::kSumSlots];
+#pragma unroll
+  for (int i = 0; i < LA::kSumSlots; ++i) sum[i] = 0.f;
   if (kbeg < kend) {
     la.load(ra, rowA0, kbeg, kend);
     if (!SAME) lb.load(rb, rowB0, kbeg, kend);
   }
   for (long long k0 = kbeg; k0 < kend; k0 += KT) {
-    la.store(ra, ldsA);
-    if (!SAME) lb.store(rb, ldsB);
+    la.template store<RS>(ra, ldsA, sum);
+    if (!SAME) lb.template store<false>(rb, ldsB, nullptr);
     __syncthreads();
     if (k0 + KT < kend) {
       la.load(ra, rowA0, k0 + KT, kend);
       if (!SAME) lb.load(rb, rowB0, k0 + KT, kend);
     }
-    if (active) {
-#pragma unroll
-    for (int kk = 0; kk < KT / 2; ++kk) {
-      float a[WM], b[WN];
-#pragma unroll
-      for (int im = 0; im < WM; ++im)
-        a[im] = fetch<RA, LA::kKRow>(ldsA, (wm * WM + im) * 32 + lrow, 2 * kk + lk);
-      if (RS) {
-#pragma unroll
-        for (int im = 0; im < WM; ++im) rs[im] += a[im];
-      }
-#pragma unroll
-      for (int in = 0; in < WN; ++in) {
-        if (SAME)
-          b[in] = fetch<RA, LA::kKRow>(ldsA, (wn * WN + in) * 32 + lrow, 2 * kk + lk);
-        else
-          b[in] = fetch<RB, LB::kKRow>(ldsB, (wn * WN + in) * 32 + lrow, 2 * kk + lk);
-      }
-#pragma unroll
-      for (int im = 0; im < WM; ++im)
-#pragma unroll
-        for (int in = 0; in < WN; ++in)
-          if (MASK & (1u << (im * WN + in)))
-            acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[im], b[in], acc[im][in], 0, 0, 0);
-    }
-    }
+    if (active) mma_panel<WM, WN, MASK>(ldsA, SAME ? ldsA : ldsB, wm, wn, acc);
     __syncthreads();
   }
+  if (RS) *rowsum = add_row_sums<64 * WM, LA>(sum, ldsA);
 }
 
 template <int WM, int WN, bool SAME, class LA, class LB>
@@ -502,9 +624,9 @@ template <int WM, int WN, bool SAME, class LA, class LB>
 __device__ __forceinline__ void mainloop_rowsum(const LA &la, const LB &lb, int rowA0, int rowB0,
                                                 long long kbeg, long long kend, float *ldsA,
                                                 float *ldsB, floatx16 (&acc)[WM][WN],
-                                                float (&rs)[WM], bool active = true,
+                                                float &rowsum, bool active = true,
                                                 int wave = threadIdx.x >> 6) {
-  mainloop_impl<WM, WN, SAME, true>(la, lb, rowA0, rowB0, kbeg, kend, ldsA, ldsB, acc, rs, active,
+  mainloop_impl<WM, WN, SAME, true>(la, lb, rowA0, rowB0, kbeg, kend, ldsA, ldsB, acc, &rowsum, active,
                                     wave);
 }
 

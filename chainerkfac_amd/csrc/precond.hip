@@ -31,8 +31,8 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_kernel(LA la_in, LB lb_in, in
                                                           float *__restrict__ C0, long long ld0,
                                                           int n_main, float *__restrict__ C1) {
   constexpr int BM = 64 * W;
-  __shared__ float ldsA[Panel<BM>::kFloats];
-  __shared__ float ldsB[Panel<BM>::kFloats];
+  __shared__ __align__(16) float ldsA[Panel<BM>::kFloats];
+  __shared__ __align__(16) float ldsB[Panel<BM>::kFloats];
   // Workgroup i of a launch runs on XCD i % 8 (each XCD has its own L2): every XCD gets a
   // contiguous run of the work list, which walks the tile rows of one tile column and
   // k-slice first, so that the workgroups that read the same B panels share an L2.
@@ -541,8 +541,8 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_group_kernel(const PreStatic 
                                                                 const int2 *__restrict__ tasks,
                                                                 float *__restrict__ ws) {
   constexpr int BM = 64 * W;
-  __shared__ float ldsA[Panel<BM>::kFloats];
-  __shared__ float ldsB[Panel<BM>::kFloats];
+  __shared__ __align__(16) float ldsA[Panel<BM>::kFloats];
+  __shared__ __align__(16) float ldsB[Panel<BM>::kFloats];
   const int2 task = tasks[blockIdx.x];
   const PreStatic s = st[task.x];
   const PreDyn v = dy[task.x];
