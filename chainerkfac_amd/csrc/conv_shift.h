@@ -40,7 +40,6 @@ constexpr int kRowStride = KT + 1;   // floats from row to row of the first oper
 // scalar variant).
 template <int ROWS>
 struct LoaderDomain {
-  static constexpr bool kKRow = false;
   static constexpr int NR = ROWS / 8;   // rows per thread
   struct Regs {
     float v[NR];

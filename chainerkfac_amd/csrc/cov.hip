@@ -301,19 +301,25 @@ __device__ __forceinline__ void work_decode(int bid, int total, int ntile, int t
   tile = I * (I + 1) / 2 + J;
 }
 
+// Workgroups per CU that the register budget of a product kernel is for: a 128-tile of split
+// products holds 128 accumulator values per lane and does not fit a third of the registers.  Two
+// against three per CU cost it 2 .. 7 % (2048 rows of 4096: 253 -> 269 us; with the float32
+// instruction 364).
+constexpr int product_groups_per_cu(int wm) { return wm == 2 ? 2 : 3; }
+
 template <int WM, class Loader>
-__global__ __launch_bounds__(THREADS, 3) void syrk_kernel(Loader ld, long long K,
+__global__ __launch_bounds__(THREADS, product_groups_per_cu(WM)) void syrk_kernel(Loader ld, long long K,
                                                           long long klen, int ntile, int nsplit,
                                                           int direct, int d, int ones,
                                                           float alpha, float beta,
                                                           float *__restrict__ partial,
                                                           float *__restrict__ C) {
   constexpr int BM = 64 * WM;
-  __shared__ __align__(16) float lds[2 * Panel<BM>::kFloats];
+  __shared__ __align__(16) float lds[2 * Panel<BM, kSplit>::kFloats];
   __shared__ int2 tabA[BM];
   __shared__ int2 tabB[BM];
-  float *ldsA = lds, *ldsB = lds + Panel<BM>::kFloats;
-  static_assert(2 * Panel<BM>::kFloats >= 64 * 65, "LDS too small for the epilogue transpose");
+  float *ldsA = lds, *ldsB = lds + Panel<BM, kSplit>::kFloats;
+  static_assert(2 * Panel<BM, kSplit>::kFloats >= 64 * 65, "LDS too small for the epilogue transpose");
   const int dt = d - ones;   // rows of the tile grid
   const int tiles = (dt + BM - 1) / BM;
   int split, tile, I, J;
@@ -1085,9 +1091,9 @@ bool kc_vec_ok(const float *base, long long sample_stride, long long row_stride,
 }
 
 template <int ROWS, bool VEC>
-LoaderKC<ROWS, VEC> make_kc(const float *base, long long sample_stride, long long row_stride, int L,
+LoaderKC<ROWS, VEC, kSplit> make_kc(const float *base, long long sample_stride, long long row_stride, int L,
                             int rows_valid) {
-  LoaderKC<ROWS, VEC> l;
+  LoaderKC<ROWS, VEC, kSplit> l;
   l.base = base;
   l.sample_stride = (unsigned)sample_stride;
   l.row_stride = (unsigned)row_stride;
@@ -1101,9 +1107,9 @@ bool ks_vec_ok(const float *base, long long ld) {
 }
 
 template <int ROWS, bool VEC>
-LoaderKS<ROWS, VEC> make_ks(const float *base, long long ld, int rows_valid, int has_extra,
+LoaderKS<ROWS, VEC, kSplit> make_ks(const float *base, long long ld, int rows_valid, int has_extra,
                             const float *extra) {
-  LoaderKS<ROWS, VEC> l;
+  LoaderKS<ROWS, VEC, kSplit> l;
   l.base = base;
   l.extra = extra;
   l.ld = (unsigned)ld;
@@ -1113,9 +1119,9 @@ LoaderKS<ROWS, VEC> make_ks(const float *base, long long ld, int rows_valid, int
 }
 
 template <int ROWS>
-LoaderIM<ROWS> make_im(const float *x, int c, int h, int w, int kh, int kw, int sy, int sx,
+LoaderIM<ROWS, kSplit> make_im(const float *x, int c, int h, int w, int kh, int kw, int sy, int sx,
                        int ph, int pw, int ho, int wo) {
-  LoaderIM<ROWS> l;
+  LoaderIM<ROWS, kSplit> l;
   l.base = x;
   l.C = c;
   l.H = h;
@@ -1301,10 +1307,10 @@ struct GroupItemDyn {
 template <class Loader>
 struct GroupLoader;
 
-template <int ROWS, bool VEC>
-struct GroupLoader<LoaderKC<ROWS, VEC>> {
-  static __device__ __forceinline__ LoaderKC<ROWS, VEC> make(const GroupItemStatic &s, const float *in) {
-    LoaderKC<ROWS, VEC> l;
+template <int ROWS, bool VEC, Format F>
+struct GroupLoader<LoaderKC<ROWS, VEC, F>> {
+  static __device__ __forceinline__ LoaderKC<ROWS, VEC, F> make(const GroupItemStatic &s, const float *in) {
+    LoaderKC<ROWS, VEC, F> l;
     l.base = in;
     l.sample_stride = s.sample_stride;
     l.row_stride = s.row_stride;
@@ -1319,10 +1325,10 @@ struct GroupLoader<LoaderKC<ROWS, VEC>> {
   }
 };
 
-template <int ROWS, bool VEC>
-struct GroupLoader<LoaderKS<ROWS, VEC>> {
-  static __device__ __forceinline__ LoaderKS<ROWS, VEC> make(const GroupItemStatic &s, const float *in) {
-    LoaderKS<ROWS, VEC> l;
+template <int ROWS, bool VEC, Format F>
+struct GroupLoader<LoaderKS<ROWS, VEC, F>> {
+  static __device__ __forceinline__ LoaderKS<ROWS, VEC, F> make(const GroupItemStatic &s, const float *in) {
+    LoaderKS<ROWS, VEC, F> l;
     l.base = in;
     l.extra = nullptr;
     l.ld = s.ld;
@@ -1334,14 +1340,14 @@ struct GroupLoader<LoaderKS<ROWS, VEC>> {
 
 // task = (item, tile + ntile * k-slice); WM = 1: items with 64-tiles, 2: 128-tiles
 template <int WM, class Loader>
-__global__ __launch_bounds__(THREADS, 3) void syrk_group_kernel(const GroupItemStatic *__restrict__ st,
+__global__ __launch_bounds__(THREADS, product_groups_per_cu(WM)) void syrk_group_kernel(const GroupItemStatic *__restrict__ st,
                                                                 const GroupItemDyn *__restrict__ dy,
                                                                 const int2 *__restrict__ tasks,
                                                                 float *__restrict__ ws) {
   constexpr int BM = 64 * WM;
-  __shared__ __align__(16) float lds[2 * Panel<BM>::kFloats];
-  static_assert(2 * Panel<BM>::kFloats >= 64 * 65, "LDS too small for the epilogue transpose");
-  float *ldsA = lds, *ldsB = lds + Panel<BM>::kFloats;
+  __shared__ __align__(16) float lds[2 * Panel<BM, kSplit>::kFloats];
+  static_assert(2 * Panel<BM, kSplit>::kFloats >= 64 * 65, "LDS too small for the epilogue transpose");
+  float *ldsA = lds, *ldsB = lds + Panel<BM, kSplit>::kFloats;
   const int2 task = tasks[blockIdx.x];
   if (task.x < 0) return;   // padding of a shorter XCD run
   const GroupItemStatic s = st[task.x];
@@ -1411,15 +1417,17 @@ __global__ __launch_bounds__(THREADS, 3) void syrk_group_kernel(const GroupItemS
 // the diagonal, past a ragged end) skips the work, never the barrier.
 // task = (item, macro-tile + nmacro * k-slice); partial tiles go to the same
 // slots as syrk_group_kernel's, so the finish launch is shared.
+// Float32 instructions: 1024 threads leave 128 registers per lane, less than the two
+// accumulators of a split product (which spilled, and ran eight times as long).
 constexpr int kMacroThreads = 4 * THREADS;
-constexpr size_t kMacroLdsBytes = 4 * Panel<128>::kFloats * sizeof(float);
+constexpr size_t kMacroLdsBytes = 4 * Panel<128, kF32>::kFloats * sizeof(float);
 
 template <class Loader>
 __global__ __launch_bounds__(kMacroThreads, 1) void syrk_macro_kernel(
     const GroupItemStatic *__restrict__ st, const GroupItemDyn *__restrict__ dy,
     const int2 *__restrict__ tasks, float *__restrict__ ws) {
   constexpr int BM = 128, WM = 2;
-  constexpr int PF = Panel<BM>::kFloats;
+  constexpr int PF = Panel<BM, kF32>::kFloats;
   extern __shared__ float lds[];
   const int team = threadIdx.x >> 8;
   const int ta = team >> 1, tb = team & 1;
@@ -1452,29 +1460,24 @@ __global__ __launch_bounds__(kMacroThreads, 1) void syrk_macro_kernel(
   floatx16 acc[WM][WM];
   zero_acc<WM, WM>(acc);
   const bool active = has_tile && syrk_wave_active<WM>(I * BM, J * BM, dt, wave);
+  const bool sums = active && I == J;   // diagonal tile: also the row sums (the ones column)
   const int wm = wave >> 1, wn = wave & 1;
+  float rs[WM] = {0.f, 0.f};
   typename Loader::Regs r;
-  float sum[Loader::kSumSlots];   // the row sums (the ones column) of the panel this team stages
-#pragma unroll
-  for (int i = 0; i < Loader::kSumSlots; ++i) sum[i] = 0.f;
   if (stages && kbeg < kend) ld.load(r, prow * BM, kbeg, kend);
   for (long long k0 = kbeg; k0 < kend; k0 += KT) {
-    if (stages) ld.template store<true>(r, mine_panel, sum);
+    if (stages) ld.template store<kF32, false>(r, mine_panel, nullptr);
     __syncthreads();
     if (stages && k0 + KT < kend) ld.load(r, prow * BM, k0 + KT, kend);
-    if (active) mma_panel<WM, WM>(pa, pb, wm, wn, acc);
+    if (active) mma_panel_f32<WM, WM, Loader::kKRow, Loader::kKRow>(pa, pb, wm, wn, acc, sums, rs);
     __syncthreads();
   }
+  if (!has_tile) return;
   const long long slot = (long long)s.ntile * (BM * BM) + (long long)s.tiles * BM;
   float *mine = ws + s.part_off + split * slot;
-  if (on_diag && s.ones) {
-    // teams 0 and 1 stage the panels of the diagonal tiles
-    const float rs = add_row_sums<BM, Loader>(sum, mine_panel);
-    if (team < 2 && stages)
-      write_rowsum<WM>(rs, prow, dt, s.d, 0, s.count, v.alpha, v.beta, mine + (long long)s.ntile * (BM * BM),
-                       v.out);
-  }
-  if (!has_tile) return;
+  if (s.ones && I == J)
+    write_rowsums<WM>(rs, I, dt, s.d, 0, s.count, v.alpha, v.beta, mine + (long long)s.ntile * (BM * BM),
+                      v.out, wave);
   float *out = mine + (long long)(I * (I + 1) / 2 + J) * (BM * BM);
   for_each_acc<WM, WM>(acc, [&](int rr, int cc, float val) { out[rr * BM + cc] = val; }, wave);
 }
@@ -1867,10 +1870,10 @@ extern "C" int kfac_cov_group_run_f32(kfac_cov_group_t group, const float *const
   const int2 *tasks = group->d_tasks.as<const int2>();
   using Kern = void (*)(const GroupItemStatic *, const GroupItemDyn *, const int2 *, float *);
   static const Kern kerns[kMacroKind0] = {
-      syrk_group_kernel<1, LoaderKC<64, true>>,   syrk_group_kernel<1, LoaderKC<64, false>>,
-      syrk_group_kernel<1, LoaderKS<64, true>>,   syrk_group_kernel<1, LoaderKS<64, false>>,
-      syrk_group_kernel<2, LoaderKC<128, true>>,  syrk_group_kernel<2, LoaderKC<128, false>>,
-      syrk_group_kernel<2, LoaderKS<128, true>>,  syrk_group_kernel<2, LoaderKS<128, false>>};
+      syrk_group_kernel<1, LoaderKC<64, true, kSplit>>,   syrk_group_kernel<1, LoaderKC<64, false, kSplit>>,
+      syrk_group_kernel<1, LoaderKS<64, true, kSplit>>,   syrk_group_kernel<1, LoaderKS<64, false, kSplit>>,
+      syrk_group_kernel<2, LoaderKC<128, true, kSplit>>,  syrk_group_kernel<2, LoaderKC<128, false, kSplit>>,
+      syrk_group_kernel<2, LoaderKS<128, true, kSplit>>,  syrk_group_kernel<2, LoaderKS<128, false, kSplit>>};
   // The launch with the most work stays on `s`, the others go to the group's side stream
   // (not while launches are being timed one by one, not in host-only mode, and under stream
   // capture only when the caller has declared `s` the capture's origin: a fork of a forked
@@ -1914,8 +1917,8 @@ extern "C" int kfac_cov_group_run_f32(kfac_cov_group_t group, const float *const
     KFAC_LAUNCH(kerns[k], dim3(group->ntask[k]), dim3(THREADS), 0, stream_of(k), st, dy,
                        tasks + group->task0[k], base);
   }
-  static const Kern macro_kerns[2] = {syrk_macro_kernel<LoaderKC<128, true>>,
-                                      syrk_macro_kernel<LoaderKC<128, false>>};
+  static const Kern macro_kerns[2] = {syrk_macro_kernel<LoaderKC<128, true, kF32>>,
+                                      syrk_macro_kernel<LoaderKC<128, false, kF32>>};
   static std::once_flag macro_attr;
   static hipError_t macro_attr_rc = hipSuccess;
   std::call_once(macro_attr, [&] {

@@ -22,20 +22,21 @@
 // bfloat16 numbers (8 significand bits each: 24 in all), x = hi + mid + lo, each
 // the rounded rest of the one before, so a product of two float32 numbers is nine
 // products of bfloat16 numbers, every one exact in float32.  The three smallest
-// (mid*lo, lo*mid, lo*lo: at most 2^-23 of the product together and 2^-26 in the
-// root mean square, of either sign) are left out; the other six are accumulated in
-// float32, small ones first.  What is lost that way is less than what float32
-// accumulation loses by itself, and the accumulator is rounded less often (an
-// instruction adds sixteen k-values instead of two): against float64, products of
-// 4608 x 4608 x 4608 have
-// 0.63 to 0.85 times the error of the v_mfma_f32_32x32x2_f32 kernel this replaced
-// (root mean square relative to sum |a||b|: 6.4e-7 against 1.03e-6 for positive
-// operands, 2.35e-8 against 2.76e-8 for signed ones, 6.2e-8 against 8.0e-8 for
-// magnitudes spread over e^6).  The split is the published one of Henry, Tang and
+// (mid*lo, lo*mid, lo*lo: at most 2^-23 of the product together, of either sign) are
+// left out; the other six are accumulated in float32.  hi*hi has an accumulator of its
+// own: it is rounded once per instruction, every sixteen k-values, where the float32
+// instruction is rounded every two; the five small products add up in a second one,
+// whose roundings are 2^-8 as large, and the two are added at the end.  (All six in one
+// accumulator round it six times per sixteen k-values, also where half of the operands
+// are zeros and the float32 sum is not rounded at all: 1.05 to 1.8 times the float32
+// instruction's error for rectified operands.)  The error against float64, root mean
+// square relative to sum |a||b|, over that of the float32 instruction: signed operands
+// 0.68 at 4 k-values, 0.43 at 16, 0.32 at 128, 0.5 at 8192; rectified ones 0.96, 0.73,
+// 0.51, 0.96 (one in six nonzero: 1.02, 0.99, 0.78, 0.99); magnitudes spread over e^6
+// 0.84, 0.63, 0.41, 0.49.  The split is the published one of Henry, Tang and
 // Heinecke (2019).  Six products of bfloat16 at the rate a large library product
 // reaches here (1370 TFLOP/s at the clock the power budget leaves) are 228 TFLOP/s
-// of float32, against 157 that the float32 instructions could reach at best;
-// 128 x 128 tiles of this engine run at 165 .. 190 (the float32 kernel: 108 .. 127).
+// of float32, against 157 that the float32 instructions could reach at best.
 //
 // An LDS panel holds one row of the operand after the other: 32 k-values of hi
 // (64 bytes), of mid, of lo, and 16 bytes that spread the rows over the banks.  A
@@ -59,7 +60,6 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned uintx2 __attribute__((ext_vector_type(2)));
-typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
 // Loads from global memory at a wave-uniform base plus a 32-bit byte offset per
 // lane: the form of the load instruction that takes the base from scalar
@@ -94,16 +94,28 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned &hi, unsig
   const float a2 = a1 - __uint_as_float(mid << 16), b2 = b1 - __uint_as_float(mid & 0xffff0000u);
   lo = pack_bf16(a2, b2);
 }
-// The six plane pairs of a product, smallest first (0 = hi, 1 = mid, 2 = lo).
+// The six plane pairs of a product (0 = hi, 1 = mid, 2 = lo), the leading one last.
 constexpr int kSplitTerms = 6;
 constexpr int kSplitA[kSplitTerms] = {2, 0, 1, 1, 0, 0};
 constexpr int kSplitB[kSplitTerms] = {0, 2, 1, 0, 1, 0};
 
-template <int ROWS>
+// How a product is formed: kSplit as six bfloat16 products of split operands, kF32 by the
+// float32 instruction.  A kF32 panel is row-major with a stride of 33 floats (loaders with k
+// contiguous) or k-major with a stride of rows + 4 (LoaderKS); either gives operand reads
+// without bank conflicts.  It fits the memory of a kSplit panel of as many rows.
+enum Format { kF32, kSplit };
+
+template <int ROWS, Format F>
 struct Panel {
   static constexpr int kPlaneBytes = KT * 2;
   static constexpr int kRowBytes = 3 * kPlaneBytes + 16;
   static constexpr int kFloats = ROWS * kRowBytes / 4;
+};
+template <int ROWS>
+struct Panel<ROWS, kF32> {
+  static constexpr int kRowKStride = KT + 1;
+  static constexpr int kKRowStride = ROWS + 4;
+  static constexpr int kFloats = ROWS * kRowKStride > KT * kKRowStride ? ROWS * kRowKStride : KT * kKRowStride;
 };
 // Byte offset of 16-byte chunk `chunk` (k-values 8 chunk ..) of a row inside a plane of the row.
 __device__ __forceinline__ int panel_chunk(int row, int chunk) { return ((chunk ^ (row >> 4)) & 3) * 16; }
@@ -125,6 +137,22 @@ __device__ __forceinline__ void panel_store4(char *p, float a, float b, float c,
   *reinterpret_cast<uintx2 *>(p + KT * 4) = uintx2{l0, l1};
 }
 
+// E consecutive k-values t of panel row r0 + RPP i, the lane's part `pr` of the row's 32
+// (the scalar loaders with k contiguous).
+template <int ROWS, Format FMT, bool SUM, int RPP, int E>
+__device__ __forceinline__ void store_row(float *lds, int r0, int pr, int i, const float (&t)[E], float *sum) {
+  if constexpr (FMT == kF32) {
+    float *p = lds + (r0 + RPP * i) * Panel<ROWS, kF32>::kRowKStride + pr * E;
+#pragma unroll
+    for (int e = 0; e < E; ++e) p[e] = t[e];
+  } else {
+    static_assert(E == 2 && RPP == 16, "pairs of k-values, sixteen rows per pass");
+    if (SUM) sum[i] += t[0] + t[1];
+    char *p = reinterpret_cast<char *>(lds) + r0 * Panel<ROWS, kSplit>::kRowBytes + (pr & 3) * 4;
+    panel_store2(p + 16 * i * Panel<ROWS, kSplit>::kRowBytes + panel_chunk(16 * i, pr >> 2), t[0], t[1]);
+  }
+}
+
 // Loader protocol: init() fixes the panel (first row) and precomputes what
 // does not change along k (row offsets, row validity); load() issues the
 // global loads of one panel; store() writes it to LDS.  Interior panels (all
@@ -134,7 +162,10 @@ __device__ __forceinline__ void panel_store4(char *p, float a, float b, float c,
 // touches the loaded registers, so the loads stay in flight while the matrix
 // cores work on the previous panel.  Offsets are 32-bit element offsets from
 // the tensor base (tensors hold fewer than 2^30 elements, 4 GiB; checked on the host).
-// With SUM, store() also adds what it stores to the thread's row sums: slot i of `sum` belongs
+// F is the format that a loader's thread layout is made for (two consecutive k-values per thread
+// and row where the planes are written in pairs, one where float32 is written), FMT the one that
+// store() writes: F, or kF32 from the layout of kSplit.
+// With SUM (kSplit), store() also adds what it stores to the thread's row sums: slot i of `sum` belongs
 // to panel row sum_row(i), and the kSumParts threads with sum_part() = 0 .. kSumParts - 1 hold
 // the parts of a row (add_row_sums below).
 
@@ -151,9 +182,11 @@ __device__ __forceinline__ void panel_store4(char *p, float a, float b, float c,
 // lanes concerned, so the reduction length is free.  A compile-time choice so
 // that this common case carries no code or registers of the scalar variant.
 // The primary template is this one.
-template <int ROWS, bool VEC>
+template <int ROWS, bool VEC, Format F>
 struct LoaderKC {
   static_assert(VEC, "the scalar variant is the specialisation below");
+  static constexpr Format kFormat = F;
+  static constexpr bool kKRow = false;
   static constexpr int NV = ROWS / 32;
   struct Regs {
     float4 v[NV];
@@ -221,10 +254,10 @@ struct LoaderKC {
   __device__ __forceinline__ static int sum_row(int i) { return (team_tid() >> 3) + 32 * i; }
   __device__ __forceinline__ static int sum_part() { return team_tid() & 7; }
 
-  template <bool SUM>
+  template <Format FMT, bool SUM>
   __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
     const int rr = team_tid() >> 3;
-    char *p = reinterpret_cast<char *>(lds) + rr * Panel<ROWS>::kRowBytes + (team_tid() & 1) * 8;
+    char *p = reinterpret_cast<char *>(lds) + rr * Panel<ROWS, kSplit>::kRowBytes + (team_tid() & 1) * 8;
     const int chunk = panel_chunk(rr, (team_tid() & 7) >> 1);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
@@ -234,21 +267,32 @@ struct LoaderKC {
 #pragma unroll
         for (int e = 0; e < 4; ++e) t[e] = (rv && ((r.kmask >> e) & 1u)) ? t[e] : 0.f;
       }
+      if constexpr (FMT == kF32) {
+        float *q = lds + (rr + 32 * i) * Panel<ROWS, kF32>::kRowKStride + (team_tid() & 7) * 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[e] = t[e];
+        continue;
+      }
       if (SUM) sum[i] += (t[0] + t[1]) + (t[2] + t[3]);
       // rows 32 apart: the chunk index differs in bit 1
-      panel_store4(p + 32 * i * Panel<ROWS>::kRowBytes + ((i & 1) ? chunk ^ 32 : chunk), t[0], t[1], t[2], t[3]);
+      panel_store4(p + 32 * i * Panel<ROWS, kSplit>::kRowBytes + ((i & 1) ? chunk ^ 32 : chunk), t[0], t[1], t[2], t[3]);
     }
   }
 };
 
-// Scalar variant: dword loads, a thread takes two consecutive k-values of a row and
-// 16 lanes the 32 of a panel.  It is the one that can subsample (line_len > 0).
-template <int ROWS>
-struct LoaderKC<ROWS, false> {
-  static constexpr int NR = ROWS / 16;   // rows per thread
+// Scalar variant: dword loads, a thread takes E consecutive k-values of a row and
+// KT / E lanes the 32 of a panel.  It is the one that can subsample (line_len > 0).
+template <int ROWS, Format F>
+struct LoaderKC<ROWS, false, F> {
+  static constexpr Format kFormat = F;
+  static constexpr bool kKRow = false;
+  static constexpr int E = F == kSplit ? 2 : 1;
+  static constexpr int LPR = KT / E;          // lanes per row
+  static constexpr int RPP = THREADS / LPR;   // rows per pass
+  static constexpr int NR = ROWS / RPP;       // rows per thread
   struct Regs {
-    float v[NR][2];
-    unsigned kvalid;   // bit e: k-value e of this thread's pair is inside the range
+    float v[NR][E];
+    unsigned kvalid;   // bit e: k-value e of this thread is inside the range
   };
   const float *base;
   unsigned sample_stride;
@@ -260,23 +304,23 @@ struct LoaderKC<ROWS, false> {
   // line_stride + (p % line_len) * px_stride of the row.  line_len = 0: k-values
   // are consecutive elements.
   unsigned line_len = 0, line_stride = 0, px_stride = 1;
-  // per-thread panel state: row i of the thread is first_row + 16 i; rows past
+  // per-thread panel state: row i of the thread is first_row + RPP i; rows past
   // the end load from the last data row (masked when stored)
   int first_row;
   unsigned last_off;
 
   __device__ __forceinline__ void init(float *, int row0) {
-    first_row = row0 + (team_tid() >> 4);
+    first_row = row0 + team_tid() / LPR;
     last_off = (unsigned)(rows_valid > 0 ? rows_valid - 1 : 0) * row_stride;
   }
 
   __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
-    const long long kg = k0 + (team_tid() & 15) * 2;
+    const long long kg = k0 + team_tid() % LPR * E;
     const long long left = k_end - kg;
-    r.kvalid = left >= 2 ? 3u : (left == 1 ? 1u : 0u);
-    unsigned koff[2];
+    r.kvalid = left >= E ? (1u << E) - 1u : (left == 1 ? 1u : 0u);
+    unsigned koff[E];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
+    for (int e = 0; e < E; ++e) {
       const unsigned kc = ((r.kvalid >> e) & 1u) ? (unsigned)kg + e : 0u;
       koff[e] = kc;
       if (L < (unsigned)k_end || line_len) {  // more than one sample, or subsampled rows
@@ -297,28 +341,27 @@ struct LoaderKC<ROWS, false> {
     const unsigned off0 = (unsigned)fr * row_stride;
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-      const unsigned off = off0 + (unsigned)(16 * i) * row_stride;
+      const unsigned off = off0 + (unsigned)(RPP * i) * row_stride;
       const unsigned ro = off < last_off ? off : last_off;
 #pragma unroll
-      for (int e = 0; e < 2; ++e) r.v[i][e] = gload1(base, (koff[e] + ro) * 4u);
+      for (int e = 0; e < E; ++e) r.v[i][e] = gload1(base, (koff[e] + ro) * 4u);
     }
   }
 
-  static constexpr int kSumSlots = NR, kSumParts = 16;
-  __device__ __forceinline__ static int sum_row(int i) { return (team_tid() >> 4) + 16 * i; }
-  __device__ __forceinline__ static int sum_part() { return team_tid() & 15; }
+  static constexpr int kSumSlots = NR, kSumParts = LPR;
+  __device__ __forceinline__ static int sum_row(int i) { return team_tid() / LPR + RPP * i; }
+  __device__ __forceinline__ static int sum_part() { return team_tid() % LPR; }
 
-  template <bool SUM>
+  template <Format FMT, bool SUM>
   __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
-    const int pr = team_tid() & 15;
-    char *p = reinterpret_cast<char *>(lds) + (team_tid() >> 4) * Panel<ROWS>::kRowBytes + (pr & 3) * 4;
+    const int pr = team_tid() % LPR;
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-      const bool rv = first_row + 16 * i < rows_valid;
-      const float a = (rv && (r.kvalid & 1u)) ? r.v[i][0] : 0.f;
-      const float b = (rv && (r.kvalid & 2u)) ? r.v[i][1] : 0.f;
-      if (SUM) sum[i] += a + b;
-      panel_store2(p + 16 * i * Panel<ROWS>::kRowBytes + panel_chunk(16 * i, pr >> 2), a, b);
+      const bool rv = first_row + RPP * i < rows_valid;
+      float t[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) t[e] = (rv && ((r.kvalid >> e) & 1u)) ? r.v[i][e] : 0.f;
+      store_row<ROWS, FMT, SUM, RPP>(lds, team_tid() / LPR, pr, i, t, sum);
     }
   }
 };
@@ -327,11 +370,13 @@ struct LoaderKC<ROWS, false> {
 // LoaderKS: element (row, kg) at base + kg * ld + row for row < rows_valid;
 // row == rows_valid reads extra[kg] (or 1 when extra is null) if has_extra.
 // ---------------------------------------------------------------------------
-template <int ROWS, bool VEC>
+template <int ROWS, bool VEC, Format F>
 struct LoaderKS {
+  static constexpr Format kFormat = F;
+  static constexpr bool kKRow = true;
   static constexpr int RQ = ROWS / 4;          // row quads per k
   static constexpr int KPP = THREADS / RQ;     // threads per row quad
-  static constexpr int NV = KT / KPP;          // consecutive k-values of a thread: 4 or 2
+  static constexpr int NV = KT / KPP;          // k-values of a thread: 4 or 2
   struct Regs {
     float4 v[NV];
     unsigned kmask;  // bit i: k-value i of this thread is inside the range
@@ -353,15 +398,19 @@ struct LoaderKS {
     full_rows = VEC && row0 + ROWS <= rows_valid;
   }
 
+  // k-value i of this thread in a panel: consecutive ones, or KPP apart where rows are stored whole
+  __device__ __forceinline__ static int k_of(int i) {
+    return F == kSplit ? team_tid() / RQ * NV + i : team_tid() / RQ + KPP * i;
+  }
+
   __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
-    const int kk = team_tid() / RQ * NV;
     const bool full_k = k0 + KT <= k_end;
     r.fast = full_rows && full_k;
     r.kmask = 0;
     if (quad_ok) {
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        const long long kg = k0 + kk + i;
+        const long long kg = k0 + k_of(i);
         const bool kok = full_k || kg < k_end;
         if (kok) r.kmask |= 1u << i;
         r.v[i] = gload4(base, ((unsigned)(kok ? kg : 0) * ld + (unsigned)row) * 4u);
@@ -369,7 +418,7 @@ struct LoaderKS {
     } else {
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        const long long kg = k0 + kk + i;
+        const long long kg = k0 + k_of(i);
         const bool kok = kg < k_end;
         if (kok) r.kmask |= 1u << i;
         const unsigned kc = (unsigned)(kok ? kg : 0);
@@ -390,10 +439,33 @@ struct LoaderKS {
   __device__ __forceinline__ static int sum_row(int i) { return (team_tid() % RQ) * 4 + i; }
   __device__ __forceinline__ static int sum_part() { return team_tid() / RQ; }
 
-  template <bool SUM>
+  template <Format FMT, bool SUM>
   __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
-    const int rq = team_tid() % RQ, kk = team_tid() / RQ * NV;
-    char *p = reinterpret_cast<char *>(lds) + rq * 4 * Panel<ROWS>::kRowBytes +
+    const int rq = team_tid() % RQ;
+    if constexpr (FMT == kF32) {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        float t[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
+        if (!r.fast) {
+          const bool kv = (r.kmask >> i) & 1u;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int re = row + e;
+            float val = 0.f;
+            if (re < rows_valid)
+              val = t[e];
+            else if (re == rows_valid && has_extra)
+              val = extra ? t[e] : 1.f;
+            t[e] = kv ? val : 0.f;
+          }
+        }
+        *reinterpret_cast<float4 *>(lds + k_of(i) * Panel<ROWS, kF32>::kKRowStride + rq * 4) =
+            make_float4(t[0], t[1], t[2], t[3]);
+      }
+      return;
+    }
+    const int kk = k_of(0);
+    char *p = reinterpret_cast<char *>(lds) + rq * 4 * Panel<ROWS, kSplit>::kRowBytes +
               panel_chunk(rq * 4, kk >> 3) + (kk & 7) * 2;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -413,9 +485,9 @@ struct LoaderKS {
         if (SUM) sum[e] += t[i];
       }
       if (NV == 4)
-        panel_store4(p + e * Panel<ROWS>::kRowBytes, t[0], t[1], t[NV - 2], t[NV - 1]);
+        panel_store4(p + e * Panel<ROWS, kSplit>::kRowBytes, t[0], t[1], t[NV - 2], t[NV - 1]);
       else
-        panel_store2(p + e * Panel<ROWS>::kRowBytes, t[0], t[1]);
+        panel_store2(p + e * Panel<ROWS, kSplit>::kRowBytes, t[0], t[1]);
     }
   }
 };
@@ -425,12 +497,17 @@ struct LoaderKS {
 //   row = (c * kh + i) * kw + j  for row < d_patch (rows past it read as 0);
 //   kg = (sample * ho + oy) * wo + ox.
 // ---------------------------------------------------------------------------
-template <int ROWS>
+template <int ROWS, Format F>
 struct LoaderIM {
-  static constexpr int NV = ROWS / 16;
+  static constexpr Format kFormat = F;
+  static constexpr bool kKRow = false;
+  static constexpr int E = F == kSplit ? 2 : 1;   // consecutive k-values of a thread
+  static constexpr int LPR = KT / E;              // lanes per row
+  static constexpr int RPP = THREADS / LPR;       // rows per pass
+  static constexpr int NV = ROWS / RPP;
   struct Regs {
-    float v[NV][2];
-    unsigned use;   // bit 2 i + e: value e of row i lies inside the image
+    float v[NV][E];
+    unsigned use;   // bit E i + e: value e of row i lies inside the image
   };
   const float *base;
   int C, H, W, kh, kw, sy, sx, ph, pw, ho, wo;
@@ -460,12 +537,12 @@ struct LoaderIM {
 
   __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
     const unsigned howo = (unsigned)(ho * wo);
-    bool kok[2];
-    int iy0[2], ix0[2];
-    long long idx0[2];
+    bool kok[E];
+    int iy0[E], ix0[E];
+    long long idx0[E];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const long long kg = k0 + (team_tid() & 15) * 2 + e;
+    for (int e = 0; e < E; ++e) {
+      const long long kg = k0 + team_tid() % LPR * E + e;
       kok[e] = kg < k_end;
       const unsigned kc = kok[e] ? (unsigned)kg : 0u;
       const unsigned s = kc / howo;
@@ -479,45 +556,88 @@ struct LoaderIM {
     r.use = 0;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int2 t = table[(team_tid() >> 4) + 16 * i];
+      const int2 t = table[team_tid() / LPR + RPP * i];
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
+      for (int e = 0; e < E; ++e) {
         const int iy = iy0[e] + (t.y >> 16);
         const int ix = ix0[e] + (t.y & 0xffff);
         const bool ok = kok[e] && t.y >= 0 && (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W;
         r.v[i][e] = base[ok ? idx0[e] + t.x : 0];
-        if (ok) r.use |= 1u << (2 * i + e);
+        if (ok) r.use |= 1u << (E * i + e);
       }
     }
   }
 
-  static constexpr int kSumSlots = NV, kSumParts = 16;
-  __device__ __forceinline__ static int sum_row(int i) { return (team_tid() >> 4) + 16 * i; }
-  __device__ __forceinline__ static int sum_part() { return team_tid() & 15; }
+  static constexpr int kSumSlots = NV, kSumParts = LPR;
+  __device__ __forceinline__ static int sum_row(int i) { return team_tid() / LPR + RPP * i; }
+  __device__ __forceinline__ static int sum_part() { return team_tid() % LPR; }
 
-  template <bool SUM>
+  template <Format FMT, bool SUM>
   __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
-    const int pr = team_tid() & 15;
-    char *p = reinterpret_cast<char *>(lds) + (team_tid() >> 4) * Panel<ROWS>::kRowBytes + (pr & 3) * 4;
+    const int pr = team_tid() % LPR;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const float a = ((r.use >> (2 * i)) & 1u) ? r.v[i][0] : 0.f;
-      const float b = ((r.use >> (2 * i + 1)) & 1u) ? r.v[i][1] : 0.f;
-      if (SUM) sum[i] += a + b;
-      panel_store2(p + 16 * i * Panel<ROWS>::kRowBytes + panel_chunk(16 * i, pr >> 2), a, b);
+      float t[E];
+#pragma unroll
+      for (int e = 0; e < E; ++e) t[e] = ((r.use >> (E * i + e)) & 1u) ? r.v[i][e] : 0.f;
+      store_row<ROWS, FMT, SUM, RPP>(lds, team_tid() / LPR, pr, i, t, sum);
     }
   }
 };
 
-// The MFMAs of one panel: this wave's WM x WN blocks from the LDS panels pa and pb (the same
+template <int WM, int WN>
+__device__ __forceinline__ void zero_acc(floatx16 (&acc)[WM][WN]) {
+#pragma unroll
+  for (int im = 0; im < WM; ++im)
+#pragma unroll
+    for (int in = 0; in < WN; ++in)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[im][in][v] = 0.f;
+}
+
+// Operand of v_mfma_f32_32x32x2_f32 from a kF32 panel: lane l supplies element (row = l % 32, k = l / 32).
+template <int ROWS, bool KROW>
+__device__ __forceinline__ float fetch(const float *lds, int row, int k) {
+  return KROW ? lds[k * Panel<ROWS, kF32>::kKRowStride + row] : lds[row * Panel<ROWS, kF32>::kRowKStride + k];
+}
+
+// The MFMAs of one kF32 panel.  With RS the lane also sums the A operand values it feeds to the
+// matrix cores: rs[im] ends as the sum over this lane's k-values (k = lane / 32 mod 2) of row
+// (wave_m * WM + im) * 32 + lane % 32, i.e. half of that row's sum.
+template <int WM, int WN, bool KROWA, bool KROWB, unsigned MASK = 0xffffffffu>
+__device__ __forceinline__ void mma_panel_f32(const float *pa, const float *pb, int wm, int wn,
+                                              floatx16 (&acc)[WM][WN], bool RS, float *rs) {
+  const int lane = threadIdx.x & 63;
+  const int lrow = lane & 31, lk = lane >> 5;
+#pragma unroll
+  for (int kk = 0; kk < KT / 2; ++kk) {
+    float a[WM], b[WN];
+#pragma unroll
+    for (int im = 0; im < WM; ++im) a[im] = fetch<64 * WM, KROWA>(pa, (wm * WM + im) * 32 + lrow, 2 * kk + lk);
+    if (RS) {
+#pragma unroll
+      for (int im = 0; im < WM; ++im) rs[im] += a[im];
+    }
+#pragma unroll
+    for (int in = 0; in < WN; ++in) b[in] = fetch<64 * WN, KROWB>(pb, (wn * WN + in) * 32 + lrow, 2 * kk + lk);
+#pragma unroll
+    for (int im = 0; im < WM; ++im)
+#pragma unroll
+      for (int in = 0; in < WN; ++in)
+        if (MASK & (1u << (im * WN + in)))
+          acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[im], b[in], acc[im][in], 0, 0, 0);
+  }
+}
+
+// The MFMAs of one kSplit panel: this wave's WM x WN blocks from the LDS panels pa and pb (the same
 // array for the diagonal tile of a SYRK), 6 per block and 16 k-values.  Lane l supplies row
-// l % 32 and k-values 8 (l / 32) .. + 7 of a 16-k step.
+// l % 32 and k-values 8 (l / 32) .. + 7 of a 16-k step.  hi * hi goes to acc, the other five to low.
 // MASK: bit im * WN + in set = this wave computes block (im, in) (compile time, so that a wave
 // that owns fewer blocks carries no test per MFMA).
 template <int WM, int WN, unsigned MASK = 0xffffffffu>
 __device__ __forceinline__ void mma_panel(const float *pa, const float *pb, int wm, int wn,
-                                          floatx16 (&acc)[WM][WN]) {
-  constexpr int RB = Panel<64>::kRowBytes;
+                                          floatx16 (&acc)[WM][WN], floatx16 (&low)[WM][WN]) {
+  constexpr int RB = Panel<64, kSplit>::kRowBytes;
   const int lane = threadIdx.x & 63;
   const int lrow = lane & 31, lk = lane >> 5;
   // 32-row block b keeps chunk c of its lower / upper 16 rows at c ^ (2 b) / c ^ (2 b + 1) (mod 4)
@@ -546,9 +666,10 @@ __device__ __forceinline__ void mma_panel(const float *pa, const float *pb, int 
       for (int im = 0; im < WM; ++im)
 #pragma unroll
         for (int in = 0; in < WN; ++in)
-          if (MASK & (1u << (im * WN + in)))
-            acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[im][kSplitA[t]], fb[in][kSplitB[t]],
-                                                                  acc[im][in], 0, 0, 0);
+          if (MASK & (1u << (im * WN + in))) {
+            floatx16 &sum = t == kSplitTerms - 1 ? acc[im][in] : low[im][in];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[im][kSplitA[t]], fb[in][kSplitB[t]], sum, 0, 0, 0);
+          }
   }
 }
 
@@ -557,7 +678,7 @@ __device__ __forceinline__ void mma_panel(const float *pa, const float *pb, int 
 // panel's memory of this team, free to overwrite.  Every thread of the workgroup calls it.
 template <int ROWS, class Loader>
 __device__ __forceinline__ float add_row_sums(const float *sum, float *lds) {
-  static_assert(Loader::kSumParts * ROWS <= Panel<ROWS>::kFloats, "the parts must fit a panel");
+  static_assert(Loader::kSumParts * ROWS <= Panel<ROWS, kSplit>::kFloats, "the parts must fit a panel");
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < Loader::kSumSlots; ++i) lds[Loader::sum_part() * ROWS + Loader::sum_row(i)] = sum[i];
@@ -593,21 +714,27 @@ __device__ __forceinline__ void mainloop_impl(const LA &la, const LB &lb, int ro
   float sum[LA::kSumSlots];
 #pragma unroll
   for (int i = 0; i < LA::kSumSlots; ++i) sum[i] = 0.f;
+  floatx16 low[WM][WN];
+  zero_acc<WM, WN>(low);
   if (kbeg < kend) {
     la.load(ra, rowA0, kbeg, kend);
     if (!SAME) lb.load(rb, rowB0, kbeg, kend);
   }
   for (long long k0 = kbeg; k0 < kend; k0 += KT) {
-    la.template store<RS>(ra, ldsA, sum);
-    if (!SAME) lb.template store<false>(rb, ldsB, nullptr);
+    la.template store<kSplit, RS>(ra, ldsA, sum);
+    if (!SAME) lb.template store<kSplit, false>(rb, ldsB, nullptr);
     __syncthreads();
     if (k0 + KT < kend) {
       la.load(ra, rowA0, k0 + KT, kend);
       if (!SAME) lb.load(rb, rowB0, k0 + KT, kend);
     }
-    if (active) mma_panel<WM, WN, MASK>(ldsA, SAME ? ldsA : ldsB, wm, wn, acc);
+    if (active) mma_panel<WM, WN, MASK>(ldsA, SAME ? ldsA : ldsB, wm, wn, acc, low);
     __syncthreads();
   }
+#pragma unroll
+  for (int im = 0; im < WM; ++im)
+#pragma unroll
+    for (int in = 0; in < WN; ++in) acc[im][in] += low[im][in];
   if (RS) *rowsum = add_row_sums<64 * WM, LA>(sum, ldsA);
 }
 
@@ -718,16 +845,6 @@ __device__ __forceinline__ void for_each_acc_masked(floatx16 (&acc)[WM][WN], uns
         f(row, col, acc[im][in][v]);
       }
     }
-}
-
-template <int WM, int WN>
-__device__ __forceinline__ void zero_acc(floatx16 (&acc)[WM][WN]) {
-#pragma unroll
-  for (int im = 0; im < WM; ++im)
-#pragma unroll
-    for (int in = 0; in < WN; ++in)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[im][in][v] = 0.f;
 }
 
 // Writes the finished tile: C[I,J] = alpha*acc + beta*C[I,J] and its mirror

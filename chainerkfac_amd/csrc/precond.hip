@@ -31,8 +31,8 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_kernel(LA la_in, LB lb_in, in
                                                           float *__restrict__ C0, long long ld0,
                                                           int n_main, float *__restrict__ C1) {
   constexpr int BM = 64 * W;
-  __shared__ __align__(16) float ldsA[Panel<BM>::kFloats];
-  __shared__ __align__(16) float ldsB[Panel<BM>::kFloats];
+  __shared__ __align__(16) float ldsA[Panel<BM, kSplit>::kFloats];
+  __shared__ __align__(16) float ldsB[Panel<BM, kSplit>::kFloats];
   // Workgroup i of a launch runs on XCD i % 8 (each XCD has its own L2): every XCD gets a
   // contiguous run of the work list, which walks the tile rows of one tile column and
   // k-slice first, so that the workgroups that read the same B panels share an L2.
@@ -138,8 +138,8 @@ bool ks_aligned(const float *base, long long ld) {
 }
 
 template <int ROWS, bool VEC>
-LoaderKC<ROWS, VEC> rowmajor_kc(const float *base, int rows, int K, long long ld) {
-  LoaderKC<ROWS, VEC> l;
+LoaderKC<ROWS, VEC, kSplit> rowmajor_kc(const float *base, int rows, int K, long long ld) {
+  LoaderKC<ROWS, VEC, kSplit> l;
   l.base = base;
   l.sample_stride = 0;
   l.row_stride = (unsigned)ld;
@@ -149,8 +149,8 @@ LoaderKC<ROWS, VEC> rowmajor_kc(const float *base, int rows, int K, long long ld
 }
 
 template <int ROWS, bool VEC>
-LoaderKS<ROWS, VEC> colop_ks(const float *base, long long ld, int rows_valid, const float *extra) {
-  LoaderKS<ROWS, VEC> l;
+LoaderKS<ROWS, VEC, kSplit> colop_ks(const float *base, long long ld, int rows_valid, const float *extra) {
+  LoaderKS<ROWS, VEC, kSplit> l;
   l.base = base;
   l.extra = extra;
   l.ld = (unsigned)ld;
@@ -541,8 +541,8 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_group_kernel(const PreStatic 
                                                                 const int2 *__restrict__ tasks,
                                                                 float *__restrict__ ws) {
   constexpr int BM = 64 * W;
-  __shared__ __align__(16) float ldsA[Panel<BM>::kFloats];
-  __shared__ __align__(16) float ldsB[Panel<BM>::kFloats];
+  __shared__ __align__(16) float ldsA[Panel<BM, kSplit>::kFloats];
+  __shared__ __align__(16) float ldsB[Panel<BM, kSplit>::kFloats];
   const int2 task = tasks[blockIdx.x];
   const PreStatic s = st[task.x];
   const PreDyn v = dy[task.x];
@@ -561,13 +561,13 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_group_kernel(const PreStatic 
   zero_acc<W, W>(acc);
   if (PHASE == 0) {
     // T = Ginv . [gradW | gradb]
-    LoaderKC<BM, VA> la;
+    LoaderKC<BM, VA, kSplit> la;
     la.base = v.Ginv;
     la.sample_stride = 0;
     la.row_stride = (unsigned)s.dG;
     la.L = (unsigned)s.dG;
     la.rows_valid = s.dG;
-    LoaderKS<BM, VB> lb;
+    LoaderKS<BM, VB, kSplit> lb;
     lb.base = v.gradW;
     lb.extra = v.gradb;
     lb.ld = (unsigned)s.dW;
@@ -578,13 +578,13 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_group_kernel(const PreStatic 
     mainloop<W, W, false>(la, lb, ti * BM, tj * BM, kbeg, kend, ldsA, ldsB, acc);
   } else {
     // kf = T . Ainv
-    LoaderKC<BM, VA> la;
+    LoaderKC<BM, VA, kSplit> la;
     la.base = T;
     la.sample_stride = 0;
     la.row_stride = (unsigned)s.ldT;
     la.L = (unsigned)s.dA;
     la.rows_valid = s.dG;
-    LoaderKC<BM, VB> lb;
+    LoaderKC<BM, VB, kSplit> lb;
     lb.base = v.Ainv;
     lb.sample_stride = 0;
     lb.row_stride = (unsigned)s.dA;

@@ -1,0 +1,38 @@
+"""What the compiler reports for the kernels of the tile engine: none of them may keep registers in memory."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+import __graft_entry__ as G
+
+KERNELS = re.compile('syrk_(macro_|group_)?kernel|gemm_(group_)?kernel')
+
+
+def _resources(source, tmp_path):
+    """{kernel: {resource: value}} from the compiler's resource remarks for one source file."""
+    flags = [f for f in G.HIPCC_FLAGS if f not in ('-shared', '-fPIC')]
+    run = subprocess.run([G._hipcc()] + flags + ['--offload-device-only', '-Rpass-analysis=kernel-resource-usage', '-c',
+                         os.path.join(G.CSRC, source), '-o', str(tmp_path / 'device.o')],
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT)
+    assert run.returncode == 0, run.stdout.decode()[-2000:]
+    found, name = {}, None
+    for line in run.stdout.decode().splitlines():
+        m = re.search(r'remark: .*?([A-Za-z][\w /\[\]]*): (\S+) \[-Rpass-analysis', line)
+        if m and m.group(1).endswith('Function Name'):
+            name = m.group(2)
+            found[name] = {}
+        elif m and name:
+            found[name][m.group(1).strip()] = m.group(2)
+    return found
+
+
+@pytest.mark.skipif(shutil.which(G._hipcc()) is None, reason='no hipcc')
+@pytest.mark.parametrize('source', ['cov.hip', 'precond.hip'])
+def test_no_kernel_spills_registers(source, tmp_path):
+    kernels = {k: v for k, v in _resources(source, tmp_path).items() if KERNELS.search(k)}
+    assert kernels
+    for name, use in kernels.items():
+        assert use['VGPRs Spill'] == '0' and use['ScratchSize [bytes/lane]'] == '0', (name, use)
