@@ -26,6 +26,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -49,6 +50,13 @@ struct SyrkPlan {
 
 constexpr int kFinishSplits = 8;
 
+// Reductions of at most this many panels take the float32 instruction.  Below 16 k-values a split
+// product is no more exact than it (1.02 times its error where most operands are zeros, 1.03 for a
+// single k-value: three of the nine plane products are left out); and a launch that short is output
+// traffic, which split products do not shorten (128 rows of 1000: 10.1 us either way, 64 of 4096: 24.3
+// with the float32 instruction, 24.5 with split products, 32 of 4096: 19.4 and 20.5).
+constexpr long long kShortPanels = 4;
+
 // No plan uses more k-slices than this (every planner clamps to it, and the
 // workspace bound of kfac_cov_workspace_bytes is computed from it): about
 // kMaxWorkgroups workgroups per launch.
@@ -65,7 +73,7 @@ SyrkPlan plan_syrk_panels(int d, long long nk, int panel_len) {
   p.bm = d <= bm64_max ? 64 : 128;
   // A short reduction (batch-norm blocks: K = batch size) is all output traffic:
   // 64-tiles spread the stores over four times as many workgroups.
-  if (panel_len == KT && nk <= 4 && kfac::ceil_div(d, 128) <= 32) p.bm = 64;
+  if (panel_len == KT && nk <= kShortPanels && kfac::ceil_div(d, 128) <= 32) p.bm = 64;
   p.tiles = kfac::ceil_div(d, p.bm);
   p.ntile = p.tiles * (p.tiles + 1) / 2;
   if (nk < 1) nk = 1;
@@ -305,21 +313,21 @@ __device__ __forceinline__ void work_decode(int bid, int total, int ntile, int t
 // products holds 128 accumulator values per lane and does not fit a third of the registers.  Two
 // against three per CU cost it 2 .. 7 % (2048 rows of 4096: 253 -> 269 us; with the float32
 // instruction 364).
-constexpr int product_groups_per_cu(int wm) { return wm == 2 ? 2 : 3; }
+constexpr int product_groups_per_cu(int wm, Format f) { return wm == 2 && f == kSplit ? 2 : 3; }
 
 template <int WM, class Loader>
-__global__ __launch_bounds__(THREADS, product_groups_per_cu(WM)) void syrk_kernel(Loader ld, long long K,
+__global__ __launch_bounds__(THREADS, product_groups_per_cu(WM, Loader::kFormat)) void syrk_kernel(Loader ld, long long K,
                                                           long long klen, int ntile, int nsplit,
                                                           int direct, int d, int ones,
                                                           float alpha, float beta,
                                                           float *__restrict__ partial,
                                                           float *__restrict__ C) {
   constexpr int BM = 64 * WM;
-  __shared__ __align__(16) float lds[2 * Panel<BM, kSplit>::kFloats];
+  __shared__ __align__(16) float lds[2 * Panel<BM, Loader::kFormat>::kFloats];
   __shared__ int2 tabA[BM];
   __shared__ int2 tabB[BM];
-  float *ldsA = lds, *ldsB = lds + Panel<BM, kSplit>::kFloats;
-  static_assert(2 * Panel<BM, kSplit>::kFloats >= 64 * 65, "LDS too small for the epilogue transpose");
+  float *ldsA = lds, *ldsB = lds + Panel<BM, Loader::kFormat>::kFloats;
+  static_assert(2 * Panel<BM, Loader::kFormat>::kFloats >= 64 * 65, "LDS too small for the epilogue transpose");
   const int dt = d - ones;   // rows of the tile grid
   const int tiles = (dt + BM - 1) / BM;
   int split, tile, I, J;
@@ -333,18 +341,26 @@ __global__ __launch_bounds__(THREADS, product_groups_per_cu(WM)) void syrk_kerne
   if (kend > K) kend = K;
   floatx16 acc[WM][WM];
   zero_acc<WM, WM>(acc);
-  float rs = 0.f;
   const int wave = threadIdx.x >> 6;
   const bool active = syrk_wave_active<WM>(I * BM, J * BM, dt, wave);
-  if (I == J)
-    mainloop_rowsum<WM, WM, true>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, rs, active,
-                                  wave);
-  else
-    mainloop<WM, WM, false>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, active, wave);
   const long long slot = (long long)ntile * (BM * BM) + (long long)tiles * BM;
   float *mine = partial + split * slot;
-  if (ones && I == J)
-    write_rowsum<WM>(rs, I, dt, d, direct, (float)K, alpha, beta, mine + (long long)ntile * (BM * BM), C);
+  float *sums = mine + (long long)ntile * (BM * BM);
+  if constexpr (Loader::kFormat == kF32) {
+    float rs[WM] = {};
+    if (I == J)
+      mainloop_f32<WM, WM, true, true>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, rs, active, wave);
+    else
+      mainloop_f32<WM, WM, false, false>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, nullptr, active, wave);
+    if (ones && I == J) write_rowsums<WM>(rs, I, dt, d, direct, (float)K, alpha, beta, sums, C, wave);
+  } else {
+    float rs = 0.f;
+    if (I == J)
+      mainloop_rowsum<WM, WM, true>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, rs, active, wave);
+    else
+      mainloop<WM, WM, false>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, active, wave);
+    if (ones && I == J) write_rowsum<WM>(rs, I, dt, d, direct, (float)K, alpha, beta, sums, C);
+  }
   if (direct) {
     write_tile<WM>(acc, lds, I, J, dt, d, alpha, beta, C, wave);
     return;
@@ -568,24 +584,32 @@ int check_ws(const SyrkPlan &p, void *ws, size_t ws_bytes) {
 
 // d: dimension of C; ones = 1 if its last row/column is a ones column, which
 // the loaders must then not supply (their rows end at d - 1).
-template <class L64, class L128>
-int run_syrk(const L64 &l64, const L128 &l128, int d, int ones, long long K, float alpha,
-             float beta, float *C, void *ws, size_t ws_bytes, hipStream_t stream) {
+// make(rows, format): the operand's loader for panels of that many rows in that format, both
+// given as integral constants.
+template <class Make>
+int run_syrk(const Make &make, int d, int ones, long long K, float alpha, float beta, float *C, void *ws,
+             size_t ws_bytes, hipStream_t stream) {
   if (d - ones == 0) return kfac::fail(KFAC_EINVAL, "empty factor");
   const SyrkPlan p = plan_syrk(d - ones, K);
   if (int rc = check_ws(p, ws, ws_bytes)) return rc;
   float *partial = static_cast<float *>(ws);
   const int grid = p.ntile * p.nsplit;
   const int direct = p.nsplit == 1 ? 1 : 0;
-  {
+  const bool float32 = kfac::ceil_div<long long>(K, KT) <= kShortPanels;
+  auto launch = [&](auto rows, auto format) {
+    const auto ld = make(rows, format);
     kfac::TimedLaunch timed(KFAC_TIMED_SYRK, stream);
-    if (p.bm == 64)
-      KFAC_LAUNCH((syrk_kernel<1, L64>), dim3(grid), dim3(THREADS), 0, stream, l64, K,
-                         p.klen, p.ntile, p.nsplit, direct, d, ones, alpha, beta, partial, C);
-    else
-      KFAC_LAUNCH((syrk_kernel<2, L128>), dim3(grid), dim3(THREADS), 0, stream, l128, K,
-                         p.klen, p.ntile, p.nsplit, direct, d, ones, alpha, beta, partial, C);
-  }
+    KFAC_LAUNCH((syrk_kernel<decltype(rows)::value / 64, std::decay_t<decltype(ld)>>), dim3(grid), dim3(THREADS), 0,
+                stream, ld, K, p.klen, p.ntile, p.nsplit, direct, d, ones, alpha, beta, partial, C);
+  };
+  using Rows64 = std::integral_constant<int, 64>;
+  using Rows128 = std::integral_constant<int, 128>;
+  using F32 = std::integral_constant<Format, kF32>;
+  using Split = std::integral_constant<Format, kSplit>;
+  if (p.bm == 64)
+    float32 ? launch(Rows64(), F32()) : launch(Rows64(), Split());
+  else
+    float32 ? launch(Rows128(), F32()) : launch(Rows128(), Split());
   KFAC_HIP_CHECK(hipGetLastError());
   if (direct) return KFAC_OK;
   return finish_partials(p, d, ones, (float)K, alpha, beta, C, partial, stream);
@@ -1090,10 +1114,10 @@ bool kc_vec_ok(const float *base, long long sample_stride, long long row_stride,
          (reinterpret_cast<uintptr_t>(base) % 16 == 0);
 }
 
-template <int ROWS, bool VEC>
-LoaderKC<ROWS, VEC, kSplit> make_kc(const float *base, long long sample_stride, long long row_stride, int L,
+template <int ROWS, bool VEC, Format F>
+LoaderKC<ROWS, VEC, F> make_kc(const float *base, long long sample_stride, long long row_stride, int L,
                             int rows_valid) {
-  LoaderKC<ROWS, VEC, kSplit> l;
+  LoaderKC<ROWS, VEC, F> l;
   l.base = base;
   l.sample_stride = (unsigned)sample_stride;
   l.row_stride = (unsigned)row_stride;
@@ -1106,10 +1130,10 @@ bool ks_vec_ok(const float *base, long long ld) {
   return (ld % 4 == 0) && (reinterpret_cast<uintptr_t>(base) % 16 == 0);
 }
 
-template <int ROWS, bool VEC>
-LoaderKS<ROWS, VEC, kSplit> make_ks(const float *base, long long ld, int rows_valid, int has_extra,
+template <int ROWS, bool VEC, Format F>
+LoaderKS<ROWS, VEC, F> make_ks(const float *base, long long ld, int rows_valid, int has_extra,
                             const float *extra) {
-  LoaderKS<ROWS, VEC, kSplit> l;
+  LoaderKS<ROWS, VEC, F> l;
   l.base = base;
   l.extra = extra;
   l.ld = (unsigned)ld;
@@ -1118,10 +1142,10 @@ LoaderKS<ROWS, VEC, kSplit> make_ks(const float *base, long long ld, int rows_va
   return l;
 }
 
-template <int ROWS>
-LoaderIM<ROWS, kSplit> make_im(const float *x, int c, int h, int w, int kh, int kw, int sy, int sx,
+template <int ROWS, Format F>
+LoaderIM<ROWS, F> make_im(const float *x, int c, int h, int w, int kh, int kw, int sy, int sx,
                        int ph, int pw, int ho, int wo) {
-  LoaderIM<ROWS, kSplit> l;
+  LoaderIM<ROWS, F> l;
   l.base = x;
   l.C = c;
   l.H = h;
@@ -1173,11 +1197,17 @@ extern "C" int kfac_cov_linear_f32(const float *x, int n, int d_in, int append_o
   const int ones = append_ones ? 1 : 0;
   const int d = d_in + ones;
   if (ks_vec_ok(x, d_in))
-    return run_syrk(make_ks<64, true>(x, d_in, d_in, 0, nullptr),
-                    make_ks<128, true>(x, d_in, d_in, 0, nullptr), d, ones, n, alpha, beta, C, ws,
+    return run_syrk(
+      [&](auto rows, auto format) {
+        return make_ks<decltype(rows)::value, true, decltype(format)::value>(x, d_in, d_in, 0, nullptr);
+      },
+       d, ones, n, alpha, beta, C, ws,
                     ws_bytes, kfac::as_stream(stream));
-  return run_syrk(make_ks<64, false>(x, d_in, d_in, 0, nullptr),
-                  make_ks<128, false>(x, d_in, d_in, 0, nullptr), d, ones, n, alpha, beta, C, ws,
+  return run_syrk(
+      [&](auto rows, auto format) {
+        return make_ks<decltype(rows)::value, false, decltype(format)::value>(x, d_in, d_in, 0, nullptr);
+      },
+       d, ones, n, alpha, beta, C, ws,
                   ws_bytes, kfac::as_stream(stream));
 }
 
@@ -1189,11 +1219,17 @@ extern "C" int kfac_cov_conv_g_f32(const float *gy, int n, int c, int howo, floa
   KFAC_REQUIRE(gy && C, "null pointer");
   const long long K = (long long)n * howo;
   if (kc_vec_ok(gy, (long long)c * howo, howo, howo))
-    return run_syrk(make_kc<64, true>(gy, (long long)c * howo, howo, howo, c),
-                    make_kc<128, true>(gy, (long long)c * howo, howo, howo, c), c, 0, K, alpha,
+    return run_syrk(
+      [&](auto rows, auto format) {
+        return make_kc<decltype(rows)::value, true, decltype(format)::value>(gy, (long long)c * howo, howo, howo, c);
+      },
+       c, 0, K, alpha,
                     beta, C, ws, ws_bytes, kfac::as_stream(stream));
-  return run_syrk(make_kc<64, false>(gy, (long long)c * howo, howo, howo, c),
-                  make_kc<128, false>(gy, (long long)c * howo, howo, howo, c), c, 0, K, alpha,
+  return run_syrk(
+      [&](auto rows, auto format) {
+        return make_kc<decltype(rows)::value, false, decltype(format)::value>(gy, (long long)c * howo, howo, howo, c);
+      },
+       c, 0, K, alpha,
                   beta, C, ws, ws_bytes, kfac::as_stream(stream));
 }
 
@@ -1226,21 +1262,30 @@ extern "C" int kfac_cov_conv_a_f32(const float *x, int n, int c, int h, int w, i
     // 1x1 convolution: the patch matrix is the NCHW tensor itself
     const int hw = h * w;
     if (kc_vec_ok(x, (long long)c * hw, hw, hw))
-      return run_syrk(make_kc<64, true>(x, (long long)c * hw, hw, hw, c),
-                      make_kc<128, true>(x, (long long)c * hw, hw, hw, c), d, ones, K, alpha,
+      return run_syrk(
+      [&](auto rows, auto format) {
+        return make_kc<decltype(rows)::value, true, decltype(format)::value>(x, (long long)c * hw, hw, hw, c);
+      },
+       d, ones, K, alpha,
                       beta, C, ws, ws_bytes, s);
-    return run_syrk(make_kc<64, false>(x, (long long)c * hw, hw, hw, c),
-                    make_kc<128, false>(x, (long long)c * hw, hw, hw, c), d, ones, K, alpha,
+    return run_syrk(
+      [&](auto rows, auto format) {
+        return make_kc<decltype(rows)::value, false, decltype(format)::value>(x, (long long)c * hw, hw, hw, c);
+      },
+       d, ones, K, alpha,
                     beta, C, ws, ws_bytes, s);
   }
   if (kh == 1 && kw == 1 && ph == 0 && pw == 0) {
     // strided 1x1 convolution: the same slab, every sx-th pixel of every sy-th line
-    auto l64 = make_kc<64, false>(x, (long long)c * h * w, (long long)h * w, ho * wo, c);
-    auto l128 = make_kc<128, false>(x, (long long)c * h * w, (long long)h * w, ho * wo, c);
-    l64.line_len = l128.line_len = (unsigned)wo;
-    l64.line_stride = l128.line_stride = (unsigned)(sy * w);
-    l64.px_stride = l128.px_stride = (unsigned)sx;
-    return run_syrk(l64, l128, d, ones, K, alpha, beta, C, ws, ws_bytes, s);
+    const auto subsampled = [&](auto rows, auto format) {
+      auto l = make_kc<decltype(rows)::value, false, decltype(format)::value>(x, (long long)c * h * w, (long long)h * w,
+                                                                              ho * wo, c);
+      l.line_len = (unsigned)wo;
+      l.line_stride = (unsigned)(sy * w);
+      l.px_stride = (unsigned)sx;
+      return l;
+    };
+    return run_syrk(subsampled, d, ones, K, alpha, beta, C, ws, ws_bytes, s);
   }
   {
     last_conv_route = KFAC_CONV_ROUTE_SHIFT;
@@ -1261,8 +1306,11 @@ extern "C" int kfac_cov_conv_a_f32(const float *x, int n, int c, int h, int w, i
     if (rc <= 0) return rc;   // 1 = shape left to the generic kernel
   }
   last_conv_route = KFAC_CONV_ROUTE_GATHER;
-  return run_syrk(make_im<64>(x, c, h, w, kh, kw, sy, sx, ph, pw, ho, wo),
-                  make_im<128>(x, c, h, w, kh, kw, sy, sx, ph, pw, ho, wo), d, ones, K, alpha,
+  return run_syrk(
+      [&](auto rows, auto format) {
+        return make_im<decltype(rows)::value, decltype(format)::value>(x, c, h, w, kh, kw, sy, sx, ph, pw, ho, wo);
+      },
+       d, ones, K, alpha,
                   beta, C, ws, ws_bytes, s);
 }
 
@@ -1296,6 +1344,7 @@ struct GroupItemStatic {
   unsigned line_len, line_stride, px_stride;
   unsigned ld;            // linear: leading dimension
   int rows_valid;
+  int float32;            // products by the float32 instruction (a short reduction; 64-tiles)
 };
 
 struct GroupItemDyn {
@@ -1340,7 +1389,7 @@ struct GroupLoader<LoaderKS<ROWS, VEC, F>> {
 
 // task = (item, tile + ntile * k-slice); WM = 1: items with 64-tiles, 2: 128-tiles
 template <int WM, class Loader>
-__global__ __launch_bounds__(THREADS, product_groups_per_cu(WM)) void syrk_group_kernel(const GroupItemStatic *__restrict__ st,
+__global__ __launch_bounds__(THREADS, product_groups_per_cu(WM, Loader::kFormat)) void syrk_group_kernel(const GroupItemStatic *__restrict__ st,
                                                                 const GroupItemDyn *__restrict__ dy,
                                                                 const int2 *__restrict__ tasks,
                                                                 float *__restrict__ ws) {
@@ -1366,11 +1415,16 @@ __global__ __launch_bounds__(THREADS, product_groups_per_cu(WM)) void syrk_group
   if (kend > s.K) kend = s.K;
   floatx16 acc[WM][WM];
   zero_acc<WM, WM>(acc);
-  float rs = 0.f;
+  float rs = 0.f, rs_half[WM] = {};
   int wave = threadIdx.x >> 6;
   const bool active = syrk_wave_active<WM>(I * BM, J * BM, dt, wave);
   unsigned store = 0xfu;
-  if (I != J) {
+  if (WM == 1 && s.float32) {
+    if (I == J)
+      mainloop_f32<WM, WM, true, true>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, rs_half, active, wave);
+    else
+      mainloop_f32<WM, WM, false, false>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, nullptr, active, wave);
+  } else if (I != J) {
     mainloop<WM, WM, false>(la, lb, I * BM, J * BM, kbeg, kend, ldsA, ldsB, acc, active, wave);
   } else if (WM == 2 && (I + 1) * BM <= dt) {
     // a whole diagonal 128-tile: all four waves share its ten blocks
@@ -1392,9 +1446,13 @@ __global__ __launch_bounds__(THREADS, product_groups_per_cu(WM)) void syrk_group
   }
   const long long slot = (long long)s.ntile * (BM * BM) + (long long)s.tiles * BM;
   float *mine = ws + s.part_off + split * slot;
-  if (s.ones && I == J)
-    write_rowsum<WM>(rs, I, dt, s.d, s.direct, s.count, v.alpha, v.beta,
-                     mine + (long long)s.ntile * (BM * BM), v.out);
+  if (s.ones && I == J) {
+    float *sums = mine + (long long)s.ntile * (BM * BM);
+    if (WM == 1 && s.float32)
+      write_rowsums<WM>(rs_half, I, dt, s.d, s.direct, s.count, v.alpha, v.beta, sums, v.out, wave);
+    else
+      write_rowsum<WM>(rs, I, dt, s.d, s.direct, s.count, v.alpha, v.beta, sums, v.out);
+  }
   if (s.direct) {
     write_tile<WM>(acc, lds, I, J, dt, s.d, v.alpha, v.beta, v.out, wave, store);
     return;
@@ -1694,7 +1752,8 @@ extern "C" int kfac_cov_group_create(int count, const kfac_cov_item *items, kfac
     // traffic: smaller tiles spread the stores over more workgroups).
     // Option group_bm64_max is a tuning override.
     const int bm64_max = kfac::option_int(kfac::kOptGroupBm64Max, 160);
-    s.bm = (it.c <= bm64_max || nk[i] <= 4) ? 64 : 128;
+    s.bm = (it.c <= bm64_max || nk[i] <= kShortPanels) ? 64 : 128;
+    s.float32 = nk[i] <= kShortPanels ? 1 : 0;
     s.tiles = kfac::ceil_div(it.c, s.bm);
     s.ntile = s.tiles * (s.tiles + 1) / 2;
     kind_of[i] = (s.bm == 64 ? 0 : 4) + (s.kind == KFAC_COV_SLAB ? 0 : 2) + (s.vec ? 0 : 1);

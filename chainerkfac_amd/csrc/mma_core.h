@@ -738,6 +738,33 @@ __device__ __forceinline__ void mainloop_impl(const LA &la, const LB &lb, int ro
   if (RS) *rowsum = add_row_sums<64 * WM, LA>(sum, ldsA);
 }
 
+// The same with the float32 instruction.  With RS rs[im] ends as half of a row's sum (mma_panel_f32).
+template <int WM, int WN, bool SAME, bool RS, class LA, class LB>
+__device__ __forceinline__ void mainloop_f32(const LA &la, const LB &lb, int rowA0, int rowB0,
+                                             long long kbeg, long long kend, float *ldsA, float *ldsB,
+                                             floatx16 (&acc)[WM][WN], float *rs, bool active,
+                                             int wave = threadIdx.x >> 6) {
+  const int wm = wave >> 1, wn = wave & 1;
+  typename LA::Regs ra;
+  typename LB::Regs rb;
+  if (kbeg < kend) {
+    la.load(ra, rowA0, kbeg, kend);
+    if (!SAME) lb.load(rb, rowB0, kbeg, kend);
+  }
+  for (long long k0 = kbeg; k0 < kend; k0 += KT) {
+    la.template store<kF32, false>(ra, ldsA, nullptr);
+    if (!SAME) lb.template store<kF32, false>(rb, ldsB, nullptr);
+    __syncthreads();
+    if (k0 + KT < kend) {
+      la.load(ra, rowA0, k0 + KT, kend);
+      if (!SAME) lb.load(rb, rowB0, k0 + KT, kend);
+    }
+    if (active)
+      mma_panel_f32<WM, WN, LA::kKRow, SAME ? LA::kKRow : LB::kKRow>(ldsA, SAME ? ldsA : ldsB, wm, wn, acc, RS, rs);
+    __syncthreads();
+  }
+}
+
 template <int WM, int WN, bool SAME, class LA, class LB>
 __device__ __forceinline__ void mainloop(const LA &la, const LB &lb, int rowA0, int rowB0,
                                          long long kbeg, long long kend, float *ldsA,

@@ -89,3 +89,22 @@ def test_covariance_of_rectified_values_as_exact_as_float32_sums(route, d, shift
             ops.CovGroup([(ops.COV_SLAB, n // 16, d, 4, 4, 1, 1, 0, 1)]).run([slab], [out], [1.0], [0.0])
     want = x.double().t() @ x.double()
     assert _rms(out, want, want) <= 1.1 * _rms(_float32_chain(x, slices), want, want)
+
+
+@pytest.mark.parametrize('route', ['linear', 'slab', 'group'])
+@pytest.mark.parametrize('n, d', [(1, 31), (1, 700), (5, 65), (31, 129), (128, 300), (33, 4200)])
+def test_short_covariances_round_a_product_once(route, n, d):
+    # One k-value with anything in it: every entry is one product, and a float32 sum rounds it once.
+    gen = torch.Generator(device='cuda').manual_seed(n * 10007 + d)
+    x = torch.zeros((n, d), device='cuda')
+    x[n // 2] = torch.randn(d, device='cuda', generator=gen)
+    out = torch.empty((d + 1, d + 1), device='cuda')
+    if route == 'linear':
+        ops.cov_linear(x, True, 1.0, out=out)
+    elif route == 'slab':
+        ops.cov_conv_a(x.view(n, d, 1, 1), 1, 1, 0, True, 1.0, out=out)
+    else:
+        ops.CovGroup([(ops.COV_LINEAR, n, d, 1, 1, 1, 1, 1, 1)]).run([x], [out], [1.0], [0.0])
+    row = x[n // 2].double()
+    assert torch.equal(out[:d, :d], (row[:, None] * row[None, :]).float())
+    assert torch.equal(out[d, :d], x[n // 2]) and torch.equal(out[:d, d], x[n // 2]) and float(out[d, d]) == n
