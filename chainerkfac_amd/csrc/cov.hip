@@ -313,10 +313,18 @@ __device__ __forceinline__ void work_decode(int bid, int total, int ntile, int t
 // products holds 128 accumulator values per lane and does not fit a third of the registers.  Two
 // against three per CU cost it 2 .. 7 % (2048 rows of 4096: 253 -> 269 us; with the float32
 // instruction 364).
-constexpr int product_groups_per_cu(int wm, Format f) { return wm == 2 && f == kSplit ? 2 : 3; }
+template <int WM, class Loader>
+struct GroupsPerCu {
+  static constexpr int value = WM == 2 && Loader::kFormat == kSplit ? 2 : 3;
+};
+// 98 and 107 registers otherwise: four workgroups instead of five
+template <>
+struct GroupsPerCu<1, LoaderKC<64, false, kSplit>> {
+  static constexpr int value = 5;
+};
 
 template <int WM, class Loader>
-__global__ __launch_bounds__(THREADS, product_groups_per_cu(WM, Loader::kFormat)) void syrk_kernel(Loader ld, long long K,
+__global__ __launch_bounds__(THREADS, (GroupsPerCu<WM, Loader>::value)) void syrk_kernel(Loader ld, long long K,
                                                           long long klen, int ntile, int nsplit,
                                                           int direct, int d, int ones,
                                                           float alpha, float beta,
@@ -582,6 +590,41 @@ int check_ws(const SyrkPlan &p, void *ws, size_t ws_bytes) {
   return KFAC_OK;
 }
 
+// Whether the 64-tiles of a launch take the float32 instruction although the reduction is long: a
+// split panel costs 11 vector instructions per pair of values and three times the LDS writes, which a
+// workgroup that has its CU to itself waits for, panel after panel; with several per CU the shorter
+// matrix work pays for it.  By what stages the operand, in microseconds with the float32 instruction and
+// with split products (dt rows, K k-values):
+//   rows contiguous, 16-byte loads, or k contiguous, 16-byte loads: up to one workgroup per CU, unless
+//     the launch is one tile, whose panel is both operands (320 x 2048, 150 workgroups: 18.0 and 18.6;
+//     512 x 1024, 180: 15.6 and 16.2; 512 x 2048, 360: 24.3 and 23.1; 64 x 2048, one tile: 16.1 and 15.2)
+struct SyrkLaunch {
+  int dt, ntile, workgroups;
+  long long panels;   // staged by all tiles together
+};
+bool float32_pays(const SyrkLaunch &l) { return l.ntile > 1 && l.workgroups <= 256; }
+template <Format F>
+bool float32_pays(const LoaderKS<64, true, F> &, const SyrkLaunch &l) { return float32_pays(l); }
+template <Format F>
+bool float32_pays(const LoaderKC<64, true, F> &, const SyrkLaunch &l) { return float32_pays(l); }
+//   rows contiguous, scalar loads: never (333 x 256, 21 workgroups: 16.0 and 14.9; 511 x 32768: 167 and 154)
+template <Format F>
+bool float32_pays(const LoaderKS<64, false, F> &, const SyrkLaunch &) { return false; }
+//   k contiguous, scalar loads: up to one workgroup per CU (200 x 1568, 70 workgroups: 17.6 and 20.0) and
+//     where one wave of four has rows to multiply (24 x 96800: 24.1 and 25.0; 64 x 96800: 27.2 and 25.9);
+//     subsampled, where the loads are most of the work, always (512 x 25088: 106 and 118)
+template <Format F>
+bool float32_pays(const LoaderKC<64, false, F> &ld, const SyrkLaunch &l) {
+  return ld.line_len != 0 || l.workgroups <= 256 || l.dt <= 32;
+}
+//   gathered patches (the float32 gather is the slower one): long reductions with little to multiply per
+//     panel, one wave's rows (27 x 802816: 79.7 and 83.5; 27 x 67600: 27.1 and 26.5) or a second tile row
+//     of one wave's rows (75 x 802816: 239 and 252; 75 x 150544: 68.3 and 66.0)
+template <Format F>
+bool float32_pays(const LoaderIM<64, F> &, const SyrkLaunch &l) {
+  return l.dt <= 32 ? l.panels > 4096 : l.dt > 64 && l.dt <= 96 && l.panels > 16384;
+}
+
 // d: dimension of C; ones = 1 if its last row/column is a ones column, which
 // the loaders must then not supply (their rows end at d - 1).
 // make(rows, format): the operand's loader for panels of that many rows in that format, both
@@ -595,7 +638,8 @@ int run_syrk(const Make &make, int d, int ones, long long K, float alpha, float 
   float *partial = static_cast<float *>(ws);
   const int grid = p.ntile * p.nsplit;
   const int direct = p.nsplit == 1 ? 1 : 0;
-  const bool float32 = kfac::ceil_div<long long>(K, KT) <= kShortPanels;
+  const long long nk = kfac::ceil_div<long long>(K, KT);
+  const SyrkLaunch shape{d - ones, p.ntile, grid, p.ntile * nk};
   auto launch = [&](auto rows, auto format) {
     const auto ld = make(rows, format);
     kfac::TimedLaunch timed(KFAC_TIMED_SYRK, stream);
@@ -606,10 +650,14 @@ int run_syrk(const Make &make, int d, int ones, long long K, float alpha, float 
   using Rows128 = std::integral_constant<int, 128>;
   using F32 = std::integral_constant<Format, kF32>;
   using Split = std::integral_constant<Format, kSplit>;
-  if (p.bm == 64)
-    float32 ? launch(Rows64(), F32()) : launch(Rows64(), Split());
+  if (p.bm == 64 && (nk <= kShortPanels || float32_pays(make(Rows64(), F32()), shape)))
+    launch(Rows64(), F32());
+  else if (p.bm == 64)
+    launch(Rows64(), Split());
+  else if (nk <= kShortPanels)
+    launch(Rows128(), F32());
   else
-    float32 ? launch(Rows128(), F32()) : launch(Rows128(), Split());
+    launch(Rows128(), Split());
   KFAC_HIP_CHECK(hipGetLastError());
   if (direct) return KFAC_OK;
   return finish_partials(p, d, ones, (float)K, alpha, beta, C, partial, stream);
@@ -1389,7 +1437,7 @@ struct GroupLoader<LoaderKS<ROWS, VEC, F>> {
 
 // task = (item, tile + ntile * k-slice); WM = 1: items with 64-tiles, 2: 128-tiles
 template <int WM, class Loader>
-__global__ __launch_bounds__(THREADS, product_groups_per_cu(WM, Loader::kFormat)) void syrk_group_kernel(const GroupItemStatic *__restrict__ st,
+__global__ __launch_bounds__(THREADS, (GroupsPerCu<WM, Loader>::value)) void syrk_group_kernel(const GroupItemStatic *__restrict__ st,
                                                                 const GroupItemDyn *__restrict__ dy,
                                                                 const int2 *__restrict__ tasks,
                                                                 float *__restrict__ ws) {

@@ -11,6 +11,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -31,8 +32,8 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_kernel(LA la_in, LB lb_in, in
                                                           float *__restrict__ C0, long long ld0,
                                                           int n_main, float *__restrict__ C1) {
   constexpr int BM = 64 * W;
-  __shared__ __align__(16) float ldsA[Panel<BM, kSplit>::kFloats];
-  __shared__ __align__(16) float ldsB[Panel<BM, kSplit>::kFloats];
+  __shared__ __align__(16) float ldsA[Panel<BM, LA::kFormat>::kFloats];
+  __shared__ __align__(16) float ldsB[Panel<BM, LA::kFormat>::kFloats];
   // Workgroup i of a launch runs on XCD i % 8 (each XCD has its own L2): every XCD gets a
   // contiguous run of the work list, which walks the tile rows of one tile column and
   // k-slice first, so that the workgroups that read the same B panels share an L2.
@@ -54,7 +55,10 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_kernel(LA la_in, LB lb_in, in
   if (kend > K) kend = K;
   floatx16 acc[W][W];
   zero_acc<W, W>(acc);
-  mainloop<W, W, false>(la, lb, ti * BM, tj * BM, kbeg, kend, ldsA, ldsB, acc);
+  if constexpr (LA::kFormat == kF32)
+    mainloop_f32<W, W, false, false>(la, lb, ti * BM, tj * BM, kbeg, kend, ldsA, ldsB, acc, nullptr, true);
+  else
+    mainloop<W, W, false>(la, lb, ti * BM, tj * BM, kbeg, kend, ldsA, ldsB, acc);
   if (partial) {
     float *out = partial + ((long long)split * ntiles + tile) * (BM * BM);
     for_each_acc<W, W>(acc, [&](int r, int c, float v) { out[r * BM + c] = v; });
@@ -100,6 +104,13 @@ struct GemmPlan {
   }
 };
 
+// A launch of 64-tiles with at most one workgroup per CU takes the float32 instruction: what a split panel
+// costs (11 vector instructions per pair of values, three times the LDS writes) a workgroup alone on its CU
+// waits for, panel after panel.  Both products of a layer of dG x dA, in microseconds with the float32
+// instruction and with split products: 64 x 577 18.8 and 20.4, 256 x 257 24.7 and 27.5, 512 x 577 (160 and 240
+// workgroups) 30.1 and 32.6; 768 x 577 (480 and 360) 40.2 and 36.8, 512 x 1025 (272 and 680) 47.8 and 43.4.
+constexpr int kIdleWorkgroups = 256;
+
 // 128x128 tiles with enough k-slices to put ~1000 workgroups in flight; 64x64
 // tiles when even that leaves most CUs idle (small products).
 GemmPlan plan_gemm(int M, int N, int K) {
@@ -137,9 +148,9 @@ bool ks_aligned(const float *base, long long ld) {
   return (ld % 4 == 0) && (reinterpret_cast<uintptr_t>(base) % 16 == 0);
 }
 
-template <int ROWS, bool VEC>
-LoaderKC<ROWS, VEC, kSplit> rowmajor_kc(const float *base, int rows, int K, long long ld) {
-  LoaderKC<ROWS, VEC, kSplit> l;
+template <int ROWS, bool VEC, Format F>
+LoaderKC<ROWS, VEC, F> rowmajor_kc(const float *base, int rows, int K, long long ld) {
+  LoaderKC<ROWS, VEC, F> l;
   l.base = base;
   l.sample_stride = 0;
   l.row_stride = (unsigned)ld;
@@ -148,9 +159,9 @@ LoaderKC<ROWS, VEC, kSplit> rowmajor_kc(const float *base, int rows, int K, long
   return l;
 }
 
-template <int ROWS, bool VEC>
-LoaderKS<ROWS, VEC, kSplit> colop_ks(const float *base, long long ld, int rows_valid, const float *extra) {
-  LoaderKS<ROWS, VEC, kSplit> l;
+template <int ROWS, bool VEC, Format F>
+LoaderKS<ROWS, VEC, F> colop_ks(const float *base, long long ld, int rows_valid, const float *extra) {
+  LoaderKS<ROWS, VEC, F> l;
   l.base = base;
   l.extra = extra;
   l.ld = (unsigned)ld;
@@ -263,23 +274,30 @@ __global__ __launch_bounds__(1024) void bn_select_batched_kernel(const BnPreItem
   bn_select(ws + it.y_off, it.d, it.g0, it.n0, it.g1, it.k0, it.k1, it.flag);
 }
 
-template <class LA64, class LB64, class LA128, class LB128>
-int launch_gemm(const LA64 &a64, const LB64 &b64, const LA128 &a128, const LB128 &b128, int M,
-                int N, int K, float *partial, float *C0, long long ld0, int n_main, float *C1,
-                hipStream_t stream) {
+// make_a / make_b(rows, format): the operands' loaders for panels of that many rows in that format,
+// both given as integral constants.
+template <class MakeA, class MakeB>
+int launch_gemm(const MakeA &make_a, const MakeB &make_b, int M, int N, int K, float *partial, float *C0,
+                long long ld0, int n_main, float *C1, hipStream_t stream) {
   const GemmPlan p = plan_gemm(M, N, K);
   const int ntiles = p.tm * p.tn;
   float *part = p.nsplit > 1 ? partial : nullptr;
-  {
+  auto launch = [&](auto rows, auto format) {
+    const auto a = make_a(rows, format);
+    const auto b = make_b(rows, format);
     kfac::TimedLaunch timed(KFAC_TIMED_GEMM, stream);
-    if (p.w == 2)
-      KFAC_LAUNCH((gemm_kernel<2, LA128, LB128>), dim3(ntiles * p.nsplit), dim3(THREADS), 0,
-                         stream, a128, b128, M, N, K, p.klen, p.tn, ntiles, part, C0, ld0, n_main,
-                         C1);
-    else
-      KFAC_LAUNCH((gemm_kernel<1, LA64, LB64>), dim3(ntiles * p.nsplit), dim3(THREADS), 0,
-                         stream, a64, b64, M, N, K, p.klen, p.tn, ntiles, part, C0, ld0, n_main, C1);
-  }
+    KFAC_LAUNCH((gemm_kernel<decltype(rows)::value / 64, std::decay_t<decltype(a)>, std::decay_t<decltype(b)>>),
+                dim3(ntiles * p.nsplit), dim3(THREADS), 0, stream, a, b, M, N, K, p.klen, p.tn, ntiles, part, C0, ld0,
+                n_main, C1);
+  };
+  using Rows64 = std::integral_constant<int, 64>;
+  using Rows128 = std::integral_constant<int, 128>;
+  using F32 = std::integral_constant<Format, kF32>;
+  using Split = std::integral_constant<Format, kSplit>;
+  if (p.w == 2)
+    launch(Rows128(), Split());
+  else
+    ntiles * p.nsplit <= kIdleWorkgroups ? launch(Rows64(), F32()) : launch(Rows64(), Split());
   KFAC_HIP_CHECK(hipGetLastError());
   if (part) {
     const long long total = (long long)M * N;
@@ -330,29 +348,34 @@ extern "C" int kfac_precond_conn_f32(const float *Ginv, int dG, const float *Ain
   // T (dG x dA) = Ginv (dG x dG) . [gradW | gradb] (dG x dA); float4 loads when
   // both operands are aligned, scalar loads otherwise
   int rc;
+  const auto first = [&](auto vec) {
+    return launch_gemm(
+        [&](auto rows, auto format) {
+          return rowmajor_kc<decltype(rows)::value, decltype(vec)::value, decltype(format)::value>(Ginv, dG, dG, dG);
+        },
+        [&](auto rows, auto format) {
+          return colop_ks<decltype(rows)::value, decltype(vec)::value, decltype(format)::value>(gradW, dW, dW, gradb);
+        },
+        dG, dA, dG, partial, T, ldT, dA, nullptr, s);
+  };
   if (kc_aligned(Ginv, dG) && ks_aligned(gradW, dW))
-    rc = launch_gemm(rowmajor_kc<64, true>(Ginv, dG, dG, dG), colop_ks<64, true>(gradW, dW, dW, gradb),
-                     rowmajor_kc<128, true>(Ginv, dG, dG, dG),
-                     colop_ks<128, true>(gradW, dW, dW, gradb), dG, dA, dG, partial, T, ldT, dA,
-                     nullptr, s);
+    rc = first(std::true_type());
   else
-    rc = launch_gemm(rowmajor_kc<64, false>(Ginv, dG, dG, dG),
-                     colop_ks<64, false>(gradW, dW, dW, gradb),
-                     rowmajor_kc<128, false>(Ginv, dG, dG, dG),
-                     colop_ks<128, false>(gradW, dW, dW, gradb), dG, dA, dG, partial, T, ldT, dA,
-                     nullptr, s);
+    rc = first(std::false_type());
   if (rc != KFAC_OK) return rc;
   // kf (dG x dA) = T . Ainv (symmetric: column j of Ainv is its row j); T is read with
   // 16-byte loads, Ainv too when its rows are aligned (dA a multiple of 4)
-  if (kc_aligned(Ainv, dA))
-    return launch_gemm(rowmajor_kc<64, true>(T, dG, dA, ldT), rowmajor_kc<64, true>(Ainv, dA, dA, dA),
-                       rowmajor_kc<128, true>(T, dG, dA, ldT),
-                       rowmajor_kc<128, true>(Ainv, dA, dA, dA), dG, dA, dA, partial, kfW, dW, dW,
-                       kfb, s);
-  return launch_gemm(rowmajor_kc<64, true>(T, dG, dA, ldT), rowmajor_kc<64, false>(Ainv, dA, dA, dA),
-                     rowmajor_kc<128, true>(T, dG, dA, ldT),
-                     rowmajor_kc<128, false>(Ainv, dA, dA, dA), dG, dA, dA, partial, kfW, dW, dW,
-                     kfb, s);
+  const auto second = [&](auto vec) {
+    return launch_gemm(
+        [&](auto rows, auto format) {
+          return rowmajor_kc<decltype(rows)::value, true, decltype(format)::value>(T, dG, dA, ldT);
+        },
+        [&](auto rows, auto format) {
+          return rowmajor_kc<decltype(rows)::value, decltype(vec)::value, decltype(format)::value>(Ainv, dA, dA, dA);
+        },
+        dG, dA, dA, partial, kfW, dW, dW, kfb, s);
+  };
+  return kc_aligned(Ainv, dA) ? second(std::true_type()) : second(std::false_type());
 }
 
 // ---------------------------------------------------------------------------

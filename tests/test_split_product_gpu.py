@@ -55,6 +55,29 @@ def test_inverse_within_the_float32_bound(d):
     assert float((out.cpu().double() - want).norm() / want.norm()) <= bound
 
 
+def _twelve_bits(shape, gen):
+    """Numbers of 12 significand bits (two bfloat16 numbers each): a product of two is a float32 number."""
+    sign = torch.randint(0, 2, shape, device='cuda', generator=gen) * 2 - 1
+    return (torch.randint(2048, 4096, shape, device='cuda', generator=gen) * sign).float() / 2048
+
+
+# launches of 64-tiles with the float32 instruction, of 64-tiles with split products and of 128-tiles, in both
+# products of a layer; loads of one and of four values; several k-slices
+@pytest.mark.parametrize('dG, dA', [(10, 101), (256, 257), (768, 577), (513, 1025), (1000, 785), (1100, 1100), (515, 2049)])
+@pytest.mark.parametrize('twelve', ['G', 'A'])
+def test_products_of_two_planes_are_exact(dG, dA, twelve):
+    # One operand pair of every output has mid planes on both sides (mid * mid is 2^-16 of the product), the other
+    # factor is a power of two: the result is a float32 number.
+    gen = torch.Generator(device='cuda').manual_seed(dG * 10007 + dA)
+    G, A = _signed_permutation(dG, gen), _signed_permutation(dA, gen)
+    F = G if twelve == 'G' else A
+    m = _twelve_bits(F.shape, gen)
+    F *= torch.tril(m) + torch.tril(m, -1).t()
+    g = _twelve_bits((dG, dA), gen)
+    kf, _ = ops.precond_conn(G, A, g)
+    assert torch.equal(kf, (G.double() @ g.double() @ A.double()).float())
+
+
 def _float32_chain(x, slices):
     """x^T x as float32 sums in the order of the k-values, one rounding each, slice by slice."""
     total = None
@@ -108,3 +131,28 @@ def test_short_covariances_round_a_product_once(route, n, d):
     row = x[n // 2].double()
     assert torch.equal(out[:d, :d], (row[:, None] * row[None, :]).float())
     assert torch.equal(out[d, :d], x[n // 2]) and torch.equal(out[:d, d], x[n // 2]) and float(out[d, d]) == n
+
+
+@pytest.mark.parametrize('dG, dA', [(1, 2), (10, 101), (64, 577), (256, 257), (512, 513)])
+def test_small_layers_round_a_product_once(dG, dA):
+    # Products with a workgroup per CU or less take the float32 instruction, which rounds a single product once.
+    gen = torch.Generator(device='cuda').manual_seed(dG * 10007 + dA)
+    G, A = _signed_permutation(dG, gen), _signed_permutation(dA, gen)
+    m = torch.rand(G.shape, device='cuda', generator=gen) + 0.5
+    G *= torch.tril(m) + torch.tril(m, -1).t()
+    g = torch.randn((dG, dA), device='cuda', generator=gen)
+    kf, _ = ops.precond_conn(G, A, g)
+    assert torch.equal(kf, ((G.double() @ g.double()).float().double() @ A.double()).float())
+
+
+@pytest.mark.parametrize('shape', [(2, 128, 14, 14), (4, 65, 13, 13), (3, 300, 9, 9)])
+@pytest.mark.parametrize('stride', [1, 2])
+def test_covariances_of_few_workgroups_round_a_product_once(shape, stride):
+    # Several tiles, a workgroup per CU or less, more than 128 k-values; subsampled slabs at any size.
+    gen = torch.Generator(device='cuda').manual_seed(shape[1])
+    shape = shape[:2] + (shape[2] * stride, shape[3] * stride)
+    x = torch.zeros(shape, device='cuda')
+    v = torch.randn(shape[1], device='cuda', generator=gen)
+    x[1, :, 2 * stride, 5 * stride] = v
+    out = ops.cov_conv_a(x, 1, stride, 0, False, 1.0)
+    assert torch.equal(out, (v.double()[:, None] * v.double()[None, :]).float())
