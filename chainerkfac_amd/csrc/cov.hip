@@ -1179,14 +1179,12 @@ bool ks_vec_ok(const float *base, long long ld) {
 }
 
 template <int ROWS, bool VEC, Format F>
-LoaderKS<ROWS, VEC, F> make_ks(const float *base, long long ld, int rows_valid, int has_extra,
-                            const float *extra) {
+LoaderKS<ROWS, VEC, F> make_ks(const float *base, long long ld, int rows_valid) {
   LoaderKS<ROWS, VEC, F> l;
   l.base = base;
-  l.extra = extra;
+  l.extra = nullptr;
   l.ld = (unsigned)ld;
   l.rows_valid = rows_valid;
-  l.has_extra = has_extra;
   return l;
 }
 
@@ -1247,13 +1245,13 @@ extern "C" int kfac_cov_linear_f32(const float *x, int n, int d_in, int append_o
   if (ks_vec_ok(x, d_in))
     return run_syrk(
       [&](auto rows, auto format) {
-        return make_ks<decltype(rows)::value, true, decltype(format)::value>(x, d_in, d_in, 0, nullptr);
+        return make_ks<decltype(rows)::value, true, decltype(format)::value>(x, d_in, d_in);
       },
        d, ones, n, alpha, beta, C, ws,
                     ws_bytes, kfac::as_stream(stream));
   return run_syrk(
       [&](auto rows, auto format) {
-        return make_ks<decltype(rows)::value, false, decltype(format)::value>(x, d_in, d_in, 0, nullptr);
+        return make_ks<decltype(rows)::value, false, decltype(format)::value>(x, d_in, d_in);
       },
        d, ones, n, alpha, beta, C, ws,
                   ws_bytes, kfac::as_stream(stream));
@@ -1430,7 +1428,6 @@ struct GroupLoader<LoaderKS<ROWS, VEC, F>> {
     l.extra = nullptr;
     l.ld = s.ld;
     l.rows_valid = s.rows_valid;
-    l.has_extra = 0;
     return l;
   }
 };
@@ -1569,10 +1566,11 @@ __global__ __launch_bounds__(kMacroThreads, 1) void syrk_macro_kernel(
   const bool sums = active && I == J;   // diagonal tile: also the row sums (the ones column)
   const int wm = wave >> 1, wn = wave & 1;
   float rs[WM] = {0.f, 0.f};
+  unsigned unused = kNothingSplit;
   typename Loader::Regs r;
   if (stages && kbeg < kend) ld.load(r, prow * BM, kbeg, kend);
   for (long long k0 = kbeg; k0 < kend; k0 += KT) {
-    if (stages) ld.template store<kF32, false>(r, mine_panel, nullptr);
+    if (stages) ld.template store<kF32, false>(r, mine_panel, nullptr, unused);
     __syncthreads();
     if (stages && k0 + KT < kend) ld.load(r, prow * BM, k0 + KT, kend);
     if (active) mma_panel_f32<WM, WM, Loader::kKRow, Loader::kKRow>(pa, pb, wm, wn, acc, sums, rs);

@@ -120,16 +120,32 @@ struct Panel<ROWS, kF32> {
 // Byte offset of 16-byte chunk `chunk` (k-values 8 chunk ..) of a row inside a plane of the row.
 __device__ __forceinline__ int panel_chunk(int row, int chunk) { return ((chunk ^ (row >> 4)) & 3) * 16; }
 
+// Range of the split.  Below 2^-110 the lowest bit of a float32 number is less than the least
+// bfloat16 number, and the planes hold fewer than 24 bits; from 0x1.ffp127 on hi rounds to infinity,
+// and the rests of an infinity are NaN.  Threads note the least nonzero magnitude that they split
+// (twice the bits without the sign, minus one: zero becomes the largest), and the main loop repeats a
+// tile with the float32 instruction if that is below 2^-110 or a sum came out as infinity or NaN, as
+// it does wherever an operand above the range takes part.
+constexpr unsigned kNothingSplit = 0xffffffffu;
+constexpr unsigned kLeastSplit = (17u << 24) - 1u;   // of 2^-110
+__device__ __forceinline__ void note_least(float a, float b, unsigned &least) {
+  const unsigned ka = (__float_as_uint(a) << 1) - 1u, kb = (__float_as_uint(b) << 1) - 1u;
+  least = min(least, min(ka, kb));
+}
+
 // Store the planes of two or four consecutive k-values at their place in a row.
-__device__ __forceinline__ void panel_store2(char *p, float a, float b) {
+__device__ __forceinline__ void panel_store2(char *p, float a, float b, unsigned &least) {
   unsigned h, m, l;
+  note_least(a, b, least);
   split_pair(a, b, h, m, l);
   *reinterpret_cast<unsigned *>(p) = h;
   *reinterpret_cast<unsigned *>(p + KT * 2) = m;
   *reinterpret_cast<unsigned *>(p + KT * 4) = l;
 }
-__device__ __forceinline__ void panel_store4(char *p, float a, float b, float c, float d) {
+__device__ __forceinline__ void panel_store4(char *p, float a, float b, float c, float d, unsigned &least) {
   unsigned h0, m0, l0, h1, m1, l1;
+  note_least(a, b, least);
+  note_least(c, d, least);
   split_pair(a, b, h0, m0, l0);
   split_pair(c, d, h1, m1, l1);
   *reinterpret_cast<uintx2 *>(p) = uintx2{h0, h1};
@@ -140,7 +156,8 @@ __device__ __forceinline__ void panel_store4(char *p, float a, float b, float c,
 // E consecutive k-values t of panel row r0 + RPP i, the lane's part `pr` of the row's 32
 // (the scalar loaders with k contiguous).
 template <int ROWS, Format FMT, bool SUM, int RPP, int E>
-__device__ __forceinline__ void store_row(float *lds, int r0, int pr, int i, const float (&t)[E], float *sum) {
+__device__ __forceinline__ void store_row(float *lds, int r0, int pr, int i, const float (&t)[E], float *sum,
+                                          unsigned &least) {
   if constexpr (FMT == kF32) {
     float *p = lds + (r0 + RPP * i) * Panel<ROWS, kF32>::kRowKStride + pr * E;
 #pragma unroll
@@ -149,7 +166,7 @@ __device__ __forceinline__ void store_row(float *lds, int r0, int pr, int i, con
     static_assert(E == 2 && RPP == 16, "pairs of k-values, sixteen rows per pass");
     if (SUM) sum[i] += t[0] + t[1];
     char *p = reinterpret_cast<char *>(lds) + r0 * Panel<ROWS, kSplit>::kRowBytes + (pr & 3) * 4;
-    panel_store2(p + 16 * i * Panel<ROWS, kSplit>::kRowBytes + panel_chunk(16 * i, pr >> 2), t[0], t[1]);
+    panel_store2(p + 16 * i * Panel<ROWS, kSplit>::kRowBytes + panel_chunk(16 * i, pr >> 2), t[0], t[1], least);
   }
 }
 
@@ -165,7 +182,7 @@ __device__ __forceinline__ void store_row(float *lds, int r0, int pr, int i, con
 // F is the format that a loader's thread layout is made for (two consecutive k-values per thread
 // and row where the planes are written in pairs, one where float32 is written), FMT the one that
 // store() writes: F, or kF32 from the layout of kSplit.
-// With SUM (kSplit), store() also adds what it stores to the thread's row sums: slot i of `sum` belongs
+// With kSplit, store() notes the least magnitude it split; with SUM it also adds what it stores to the thread's row sums: slot i of `sum` belongs
 // to panel row sum_row(i), and the kSumParts threads with sum_part() = 0 .. kSumParts - 1 hold
 // the parts of a row (add_row_sums below).
 
@@ -255,7 +272,7 @@ struct LoaderKC {
   __device__ __forceinline__ static int sum_part() { return team_tid() & 7; }
 
   template <Format FMT, bool SUM>
-  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
+  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum, unsigned &least) const {
     const int rr = team_tid() >> 3;
     char *p = reinterpret_cast<char *>(lds) + rr * Panel<ROWS, kSplit>::kRowBytes + (team_tid() & 1) * 8;
     const int chunk = panel_chunk(rr, (team_tid() & 7) >> 1);
@@ -275,7 +292,8 @@ struct LoaderKC {
       }
       if (SUM) sum[i] += (t[0] + t[1]) + (t[2] + t[3]);
       // rows 32 apart: the chunk index differs in bit 1
-      panel_store4(p + 32 * i * Panel<ROWS, kSplit>::kRowBytes + ((i & 1) ? chunk ^ 32 : chunk), t[0], t[1], t[2], t[3]);
+      panel_store4(p + 32 * i * Panel<ROWS, kSplit>::kRowBytes + ((i & 1) ? chunk ^ 32 : chunk), t[0], t[1], t[2], t[3],
+                   least);
     }
   }
 };
@@ -317,7 +335,8 @@ struct LoaderKC<ROWS, false, F> {
   __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
     const long long kg = k0 + team_tid() % LPR * E;
     const long long left = k_end - kg;
-    r.kvalid = left >= E ? (1u << E) - 1u : (left == 1 ? 1u : 0u);
+    r.kvalid = left > 0 ? 1u : 0u;
+    if (E == 2 && left > 1) r.kvalid = 3u;
     unsigned koff[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -353,7 +372,7 @@ struct LoaderKC<ROWS, false, F> {
   __device__ __forceinline__ static int sum_part() { return team_tid() % LPR; }
 
   template <Format FMT, bool SUM>
-  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
+  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum, unsigned &least) const {
     const int pr = team_tid() % LPR;
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
@@ -361,16 +380,16 @@ struct LoaderKC<ROWS, false, F> {
       float t[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) t[e] = (rv && ((r.kvalid >> e) & 1u)) ? r.v[i][e] : 0.f;
-      store_row<ROWS, FMT, SUM, RPP>(lds, team_tid() / LPR, pr, i, t, sum);
+      store_row<ROWS, FMT, SUM, RPP>(lds, team_tid() / LPR, pr, i, t, sum, least);
     }
   }
 };
 
 // ---------------------------------------------------------------------------
 // LoaderKS: element (row, kg) at base + kg * ld + row for row < rows_valid;
-// row == rows_valid reads extra[kg] (or 1 when extra is null) if has_extra.
+// with EXTRA row == rows_valid reads extra[kg], unless that is null.
 // ---------------------------------------------------------------------------
-template <int ROWS, bool VEC, Format F>
+template <int ROWS, bool VEC, Format F, bool EXTRA = false>
 struct LoaderKS {
   static constexpr Format kFormat = F;
   static constexpr bool kKRow = true;
@@ -386,7 +405,6 @@ struct LoaderKS {
   const float *extra;
   unsigned ld;
   int rows_valid;
-  int has_extra;
   // per-thread panel state
   int row;          // first of this thread's four rows
   bool quad_ok;     // all four rows are data rows and float4 loads are allowed
@@ -397,6 +415,8 @@ struct LoaderKS {
     quad_ok = VEC && row + 3 < rows_valid;
     full_rows = VEC && row0 + ROWS <= rows_valid;
   }
+
+  __device__ __forceinline__ bool is_row(int r) const { return r < rows_valid || (EXTRA && r == rows_valid && extra); }
 
   // k-value i of this thread in a panel: consecutive ones, or KPP apart where rows are stored whole
   __device__ __forceinline__ static int k_of(int i) {
@@ -426,9 +446,11 @@ struct LoaderKS {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int re = row + e;
-          const float *q = base + kc * ld + (unsigned)(re < rows_valid ? re : 0);
-          if (re == rows_valid && has_extra && extra) q = extra + kc;
-          t[e] = *q;
+          const unsigned at = kc * ld + (unsigned)(re < rows_valid ? re : 0);
+          if constexpr (EXTRA)
+            t[e] = *(re == rows_valid && extra ? extra + kc : base + at);
+          else
+            t[e] = gload1(base, at * 4u);
         }
         r.v[i] = make_float4(t[0], t[1], t[2], t[3]);
       }
@@ -440,7 +462,7 @@ struct LoaderKS {
   __device__ __forceinline__ static int sum_part() { return team_tid() / RQ; }
 
   template <Format FMT, bool SUM>
-  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
+  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum, unsigned &least) const {
     const int rq = team_tid() % RQ;
     if constexpr (FMT == kF32) {
 #pragma unroll
@@ -451,12 +473,7 @@ struct LoaderKS {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int re = row + e;
-            float val = 0.f;
-            if (re < rows_valid)
-              val = t[e];
-            else if (re == rows_valid && has_extra)
-              val = extra ? t[e] : 1.f;
-            t[e] = kv ? val : 0.f;
+            t[e] = kv && is_row(re) ? t[e] : 0.f;
           }
         }
         *reinterpret_cast<float4 *>(lds + k_of(i) * Panel<ROWS, kF32>::kKRowStride + rq * 4) =
@@ -475,19 +492,14 @@ struct LoaderKS {
       for (int i = 0; i < NV; ++i) {
         t[i] = e == 0 ? r.v[i].x : e == 1 ? r.v[i].y : e == 2 ? r.v[i].z : r.v[i].w;
         if (!r.fast) {
-          float val = 0.f;
-          if (re < rows_valid)
-            val = t[i];
-          else if (re == rows_valid && has_extra)
-            val = extra ? t[i] : 1.f;
-          t[i] = ((r.kmask >> i) & 1u) ? val : 0.f;
+          t[i] = ((r.kmask >> i) & 1u) && is_row(re) ? t[i] : 0.f;
         }
         if (SUM) sum[e] += t[i];
       }
       if (NV == 4)
-        panel_store4(p + e * Panel<ROWS, kSplit>::kRowBytes, t[0], t[1], t[NV - 2], t[NV - 1]);
+        panel_store4(p + e * Panel<ROWS, kSplit>::kRowBytes, t[0], t[1], t[NV - 2], t[NV - 1], least);
       else
-        panel_store2(p + e * Panel<ROWS, kSplit>::kRowBytes, t[0], t[1]);
+        panel_store2(p + e * Panel<ROWS, kSplit>::kRowBytes, t[0], t[1], least);
     }
   }
 };
@@ -573,14 +585,14 @@ struct LoaderIM {
   __device__ __forceinline__ static int sum_part() { return team_tid() % LPR; }
 
   template <Format FMT, bool SUM>
-  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum) const {
+  __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum, unsigned &least) const {
     const int pr = team_tid() % LPR;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       float t[E];
 #pragma unroll
       for (int e = 0; e < E; ++e) t[e] = ((r.use >> (E * i + e)) & 1u) ? r.v[i][e] : 0.f;
-      store_row<ROWS, FMT, SUM, RPP>(lds, team_tid() / LPR, pr, i, t, sum);
+      store_row<ROWS, FMT, SUM, RPP>(lds, team_tid() / LPR, pr, i, t, sum, least);
     }
   }
 };
@@ -692,17 +704,56 @@ __device__ __forceinline__ float add_row_sums(const float *sum, float *lds) {
   return total;
 }
 
-// Main loop.  acc[im][in] accumulates the 32x32 block at rows
+// Whether `mine` holds in any thread of the workgroup (of THREADS threads, all of which call it, once).
+__device__ __forceinline__ bool any_in_workgroup(bool mine) {
+  __shared__ int flag[THREADS / 64];
+  const bool any = __any(mine);
+  if ((threadIdx.x & 63) == 0) flag[threadIdx.x >> 6] = any;
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(flag[0] | flag[1] | flag[2] | flag[3]) != 0;
+}
+
+// Main loop of the float32 instruction.  acc[im][in] accumulates the 32x32 block at rows
 // (wave_m * WM + im) * 32 of the A panel and (wave_n * WN + in) * 32 of the B
 // panel.  With SAME the B operand is read from the A panel (diagonal tile of a
 // SYRK) and lb is not used.  ldsA / ldsB hold Panel<64*WM> / Panel<64*WN>
 // floats.
-// With RS the sums over k of the A operand's rows are formed on the side:
-// *rowsum is that of row threadIdx.x of the tile (threads below 64*WM).
+// With RS rs[im] ends as half of a row's sum (mma_panel_f32).
 // A wave with `active` false stages panels like the others but feeds nothing to
 // the matrix cores (its block of the tile is not needed: above the diagonal of a
 // symmetric product, or past the end of the matrix); its accumulators stay as
 // they are.
+template <int WM, int WN, bool SAME, bool RS, class LA, class LB, unsigned MASK = 0xffffffffu>
+__device__ __forceinline__ void mainloop_f32(const LA &la, const LB &lb, int rowA0, int rowB0,
+                                             long long kbeg, long long kend, float *ldsA, float *ldsB,
+                                             floatx16 (&acc)[WM][WN], float *rs, bool active,
+                                             int wave = threadIdx.x >> 6) {
+  const int wm = wave >> 1, wn = wave & 1;
+  unsigned unused = kNothingSplit;
+  typename LA::Regs ra;
+  typename LB::Regs rb;
+  if (kbeg < kend) {
+    la.load(ra, rowA0, kbeg, kend);
+    if (!SAME) lb.load(rb, rowB0, kbeg, kend);
+  }
+  for (long long k0 = kbeg; k0 < kend; k0 += KT) {
+    la.template store<kF32, false>(ra, ldsA, nullptr, unused);
+    if (!SAME) lb.template store<kF32, false>(rb, ldsB, nullptr, unused);
+    __syncthreads();
+    if (k0 + KT < kend) {
+      la.load(ra, rowA0, k0 + KT, kend);
+      if (!SAME) lb.load(rb, rowB0, k0 + KT, kend);
+    }
+    if (active)
+      mma_panel_f32<WM, WN, LA::kKRow, SAME ? LA::kKRow : LB::kKRow, MASK>(ldsA, SAME ? ldsA : ldsB, wm, wn, acc, RS,
+                                                                          rs);
+    __syncthreads();
+  }
+}
+
+// Main loop of split products, arguments as above; acc comes as zeros.  With RS the sums over k of the
+// A operand's rows are formed on the side, from the float32 values: *rowsum is that of row threadIdx.x
+// of the tile (threads below 64*WM).
 template <int WM, int WN, bool SAME, bool RS, class LA, class LB, unsigned MASK = 0xffffffffu>
 __device__ __forceinline__ void mainloop_impl(const LA &la, const LB &lb, int rowA0, int rowB0,
                                               long long kbeg, long long kend, float *ldsA,
@@ -714,6 +765,7 @@ __device__ __forceinline__ void mainloop_impl(const LA &la, const LB &lb, int ro
   float sum[LA::kSumSlots];
 #pragma unroll
   for (int i = 0; i < LA::kSumSlots; ++i) sum[i] = 0.f;
+  unsigned least = kNothingSplit;
   floatx16 low[WM][WN];
   zero_acc<WM, WN>(low);
   if (kbeg < kend) {
@@ -721,8 +773,8 @@ __device__ __forceinline__ void mainloop_impl(const LA &la, const LB &lb, int ro
     if (!SAME) lb.load(rb, rowB0, kbeg, kend);
   }
   for (long long k0 = kbeg; k0 < kend; k0 += KT) {
-    la.template store<kSplit, RS>(ra, ldsA, sum);
-    if (!SAME) lb.template store<kSplit, false>(rb, ldsB, nullptr);
+    la.template store<kSplit, RS>(ra, ldsA, sum, least);
+    if (!SAME) lb.template store<kSplit, false>(rb, ldsB, nullptr, least);
     __syncthreads();
     if (k0 + KT < kend) {
       la.load(ra, rowA0, k0 + KT, kend);
@@ -731,37 +783,20 @@ __device__ __forceinline__ void mainloop_impl(const LA &la, const LB &lb, int ro
     if (active) mma_panel<WM, WN, MASK>(ldsA, SAME ? ldsA : ldsB, wm, wn, acc, low);
     __syncthreads();
   }
+  float nonfinite = 0.f;   // NaN as soon as a sum is infinite or NaN
 #pragma unroll
   for (int im = 0; im < WM; ++im)
 #pragma unroll
-    for (int in = 0; in < WN; ++in) acc[im][in] += low[im][in];
-  if (RS) *rowsum = add_row_sums<64 * WM, LA>(sum, ldsA);
-}
-
-// The same with the float32 instruction.  With RS rs[im] ends as half of a row's sum (mma_panel_f32).
-template <int WM, int WN, bool SAME, bool RS, class LA, class LB>
-__device__ __forceinline__ void mainloop_f32(const LA &la, const LB &lb, int rowA0, int rowB0,
-                                             long long kbeg, long long kend, float *ldsA, float *ldsB,
-                                             floatx16 (&acc)[WM][WN], float *rs, bool active,
-                                             int wave = threadIdx.x >> 6) {
-  const int wm = wave >> 1, wn = wave & 1;
-  typename LA::Regs ra;
-  typename LB::Regs rb;
-  if (kbeg < kend) {
-    la.load(ra, rowA0, kbeg, kend);
-    if (!SAME) lb.load(rb, rowB0, kbeg, kend);
-  }
-  for (long long k0 = kbeg; k0 < kend; k0 += KT) {
-    la.template store<kF32, false>(ra, ldsA, nullptr);
-    if (!SAME) lb.template store<kF32, false>(rb, ldsB, nullptr);
-    __syncthreads();
-    if (k0 + KT < kend) {
-      la.load(ra, rowA0, k0 + KT, kend);
-      if (!SAME) lb.load(rb, rowB0, k0 + KT, kend);
+    for (int in = 0; in < WN; ++in) {
+      acc[im][in] += low[im][in];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) nonfinite = __builtin_fmaf(acc[im][in][v], 0.f, nonfinite);
     }
-    if (active)
-      mma_panel_f32<WM, WN, LA::kKRow, SAME ? LA::kKRow : LB::kKRow>(ldsA, SAME ? ldsA : ldsB, wm, wn, acc, RS, rs);
-    __syncthreads();
+  if (RS) *rowsum = add_row_sums<64 * WM, LA>(sum, ldsA);
+  if (__builtin_expect(any_in_workgroup(least < kLeastSplit || nonfinite != 0.f), 0)) {
+    zero_acc<WM, WN>(acc);
+    mainloop_f32<WM, WN, SAME, false, LA, LB, MASK>(la, lb, rowA0, rowB0, kbeg, kend, ldsA, ldsB, acc, nullptr, active,
+                                                    wave);
   }
 }
 

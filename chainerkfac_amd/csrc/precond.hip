@@ -160,13 +160,12 @@ LoaderKC<ROWS, VEC, F> rowmajor_kc(const float *base, int rows, int K, long long
 }
 
 template <int ROWS, bool VEC, Format F>
-LoaderKS<ROWS, VEC, F> colop_ks(const float *base, long long ld, int rows_valid, const float *extra) {
-  LoaderKS<ROWS, VEC, F> l;
+LoaderKS<ROWS, VEC, F, true> colop_ks(const float *base, long long ld, int rows_valid, const float *extra) {
+  LoaderKS<ROWS, VEC, F, true> l;
   l.base = base;
   l.extra = extra;
   l.ld = (unsigned)ld;
   l.rows_valid = rows_valid;
-  l.has_extra = extra != nullptr;
   return l;
 }
 
@@ -590,12 +589,11 @@ __global__ __launch_bounds__(THREADS, 2) void gemm_group_kernel(const PreStatic 
     la.row_stride = (unsigned)s.dG;
     la.L = (unsigned)s.dG;
     la.rows_valid = s.dG;
-    LoaderKS<BM, VB, kSplit> lb;
+    LoaderKS<BM, VB, kSplit, true> lb;
     lb.base = v.gradW;
     lb.extra = v.gradb;
     lb.ld = (unsigned)s.dW;
     lb.rows_valid = s.dW;
-    lb.has_extra = s.hb;
     la.init(nullptr, ti * BM);
     lb.init(nullptr, tj * BM);
     mainloop<W, W, false>(la, lb, ti * BM, tj * BM, kbeg, kend, ldsA, ldsB, acc);

@@ -156,3 +156,106 @@ def test_covariances_of_few_workgroups_round_a_product_once(shape, stride):
     x[1, :, 2 * stride, 5 * stride] = v
     out = ops.cov_conv_a(x, 1, stride, 0, False, 1.0)
     assert torch.equal(out, (v.double()[:, None] * v.double()[None, :]).float())
+
+
+# one shape per way that operands reach split products: 64- and 128-tiles, whole and ragged, every loader
+_COVARIANCES = {
+    'linear64': (8192, 320), 'linear64_scalar': (2048, 511), 'linear128': (300, 700), 'linear128_scalar': (300, 701),
+    'slab64': (32, 512, 14, 14), 'slab64_scalar': (32, 320, 13, 13), 'slab128': (4, 700, 10, 10),
+    'slab128_scalar': (4, 700, 9, 9), 'strided128': (4, 600, 18, 18), 'gather64': (16, 8, 31, 31),
+    'gather128': (4, 70, 11, 11), 'group64': (8, 100, 6, 6), 'group64_scalar': (8, 100, 5, 5),
+    'group128': (8, 300, 6, 6), 'group128_scalar': (8, 300, 5, 5), 'group_linear64': (200, 100),
+    'group_linear128': (200, 300), 'group_linear128_scalar': (200, 301),
+}
+
+
+def _covariance(route, make):
+    """(P^T P with a ones column, the patch matrix P) of an input ``make(shape)``; P in float64 on the GPU."""
+    shape = _COVARIANCES[route]
+    x = make(shape)
+    stride = 2 if route.startswith('strided') else 1
+    if len(shape) == 2:
+        P = x
+    elif route.startswith('gather'):
+        P = torch.nn.functional.unfold(x, 5).transpose(1, 2).reshape(-1, shape[1] * 25)
+    else:
+        P = x[:, :, ::stride, ::stride].permute(0, 2, 3, 1).reshape(-1, shape[1])
+    d = P.shape[1]
+    out = torch.empty((d + 1, d + 1), device='cuda')
+    if route.startswith('group'):
+        kind, hw = (ops.COV_LINEAR, (1, 1)) if len(shape) == 2 else (ops.COV_SLAB, shape[2:])
+        ops.CovGroup([(kind, shape[0], shape[1]) + hw + (1, 1, 1, 1)]).run([x], [out], [1.0], [0.0])
+    elif len(shape) == 2:
+        ops.cov_linear(x, True, 1.0, out=out)
+    else:
+        ops.cov_conv_a(x, 5 if route.startswith('gather') else 1, stride, 0, True, 1.0, out=out)
+    P = torch.cat([P, torch.ones((P.shape[0], 1), device='cuda')], 1).double()
+    return out, P
+
+
+def _assert_close_where_finite(got, want, scale, tol):
+    """Infinities and NaN as in ``want`` (float64, rounded to float32); elsewhere |difference| <= tol * scale."""
+    want32 = want.float()
+    assert torch.equal(torch.isnan(got), torch.isnan(want32))
+    assert torch.equal(got[torch.isinf(want32)], want32[torch.isinf(want32)])
+    fine = torch.isfinite(want32)
+    assert bool(torch.isfinite(got[fine]).all())
+    error = (got.double() - want).abs()
+    assert bool((error <= tol * scale)[fine].all()), float((error / scale)[fine].max())
+
+
+def _operands(shape, column, kind, gen):
+    x = torch.randn(shape, device='cuda', generator=gen)
+    if kind == 'inf':
+        x[0, column].view(-1)[-1:] = float('inf')
+    elif kind == 'nan':
+        x[0, column].view(-1)[-1:] = float('nan')
+    elif kind == 'huge':      # the last float32 numbers round to infinity as bfloat16
+        x *= 2.0 ** -20
+        x[0, column].view(-1)[-1:] = -torch.finfo(torch.float32).max
+    elif kind == 'both small':
+        x *= 2.0 ** -58
+    else:                     # a power of two; below 2^-110 a bfloat16 number cannot hold the last bits
+        x[:, column] *= 2.0 ** kind
+    return x
+
+
+@pytest.mark.parametrize('kind', ['inf', 'nan', 'huge', 'both small', -105, -109, -112, -120, -135])
+@pytest.mark.parametrize('route', list(_COVARIANCES))
+def test_covariances_over_the_range_of_float32(route, kind):
+    gen = torch.Generator(device='cuda').manual_seed(5)
+    column = _COVARIANCES[route][1] * 2 // 3
+    out, P = _covariance(route, lambda shape: _operands(shape, column, kind, gen))
+    # float32 sums of n products of either sign, to a part of n u (u = 2^-24) of the sum of their magnitudes; results
+    # under 2^-126 are held to multiples of 2^-149, once per sum of sixteen k-values or two
+    n = P.shape[0]
+    scale = P.abs().t() @ P.abs()
+    scale = torch.where(torch.isfinite(scale), scale, torch.ones_like(scale)) + n * 2.0 ** -149 / (64 * 2.0 ** -24)
+    _assert_close_where_finite(out, P.t() @ P, scale, 64 * 2.0 ** -24)
+
+
+@pytest.mark.parametrize('kind', ['inf', 'nan', 'huge', 'both small', -105, -109, -112, -120, -135])
+@pytest.mark.parametrize('dG, dA, group', [(768, 577, False), (1100, 1100, False), (513, 1025, False), (60, 70, True),
+                                           (200, 300, True), (201, 301, True)])
+def test_preconditioning_over_the_range_of_float32(dG, dA, group, kind):
+    gen = torch.Generator(device='cuda').manual_seed(6)
+    G = torch.eye(dG, device='cuda')
+    A = torch.randn((dA, dA), device='cuda', generator=gen)
+    A = torch.tril(A) + torch.tril(A, -1).t()
+    g = _operands((dA, dG), dG // 3, kind, gen).t().contiguous()
+    if kind == 'both small':
+        A *= 2.0 ** -58
+    if kind == 'huge':
+        A *= 2.0 ** -20
+    if kind in ('inf', 'nan'):
+        # the identity's zeros times an infinity are NaN in the whole column of the first product
+        G = torch.full((dG, dG), 0.5, device='cuda')
+    if group:
+        kf = torch.empty_like(g)
+        ops.PrecondGroup([(dG, dA, 0)]).run([G], [A], [g], [None], [kf], [None])
+    else:
+        kf, _ = ops.precond_conn(G, A, g)
+    T = G.double() @ g.double()
+    scale = (G.double().abs() @ g.double().abs()) @ A.double().abs()
+    scale = torch.where(torch.isfinite(scale), scale, torch.ones_like(scale)) + (dG + dA) * 2.0 ** -149 / (64 * 2.0 ** -24)
+    _assert_close_where_finite(kf, T @ A.double(), scale, 64 * 2.0 ** -24)
