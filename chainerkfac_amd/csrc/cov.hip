@@ -610,19 +610,21 @@ bool float32_pays(const LoaderKC<64, true, F> &, const SyrkLaunch &l) { return f
 //   rows contiguous, scalar loads: never (333 x 256, 21 workgroups: 16.0 and 14.9; 511 x 32768: 167 and 154)
 template <Format F>
 bool float32_pays(const LoaderKS<64, false, F> &, const SyrkLaunch &) { return false; }
-//   k contiguous, scalar loads: up to one workgroup per CU (200 x 1568, 70 workgroups: 17.6 and 20.0) and
-//     where one wave of four has rows to multiply (24 x 96800: 24.1 and 25.0; 64 x 96800: 27.2 and 25.9);
-//     subsampled, where the loads are most of the work, always (512 x 25088: 106 and 118)
+//   k contiguous, scalar loads: up to one workgroup per CU, two with several tiles (64 x 5408, 25 workgroups: 15.8
+//     and 16.8; 128 x 24200, 327: 24.4 and 25.2; 128 x 39200, 525: 30.2 and 28.9), and where a tile row has
+//     rows for half of the waves (32 x 394272: 43.9 and 46.7; 96 x 180000: 50.0 and 55.5; 64 x 394272:
+//     55.3 and 51.6); subsampled, where the loads are most of the work, always (512 x 25088: 106 and 118)
 template <Format F>
 bool float32_pays(const LoaderKC<64, false, F> &ld, const SyrkLaunch &l) {
-  return ld.line_len != 0 || l.workgroups <= 256 || l.dt <= 32;
+  return ld.line_len != 0 || l.workgroups <= (l.ntile == 1 ? 256 : 512) || (l.dt - 1) % 64 < 32;
 }
 //   gathered patches (the float32 gather is the slower one): long reductions with little to multiply per
-//     panel, one wave's rows (27 x 802816: 79.7 and 83.5; 27 x 67600: 27.1 and 26.5) or a second tile row
-//     of one wave's rows (75 x 802816: 239 and 252; 75 x 150544: 68.3 and 66.0)
+//     panel, one wave's rows (27 x 64800: 26.2 and 26.6; 27 x 819200: 79.1 and 86.3; 27 x 33800: 23.8 and
+//     23.2) or a second tile row of one wave's rows (75 x 135200: 62.9 and 64.3; 75 x 819200: 237 and 268;
+//     75 x 75272: 46.2 and 44.4)
 template <Format F>
 bool float32_pays(const LoaderIM<64, F> &, const SyrkLaunch &l) {
-  return l.dt <= 32 ? l.panels > 4096 : l.dt > 64 && l.dt <= 96 && l.panels > 16384;
+  return l.dt <= 32 ? l.panels > 1536 : l.dt > 64 && l.dt <= 96 && l.panels > 9000;
 }
 
 // d: dimension of C; ones = 1 if its last row/column is a ones column, which

@@ -547,34 +547,56 @@ struct LoaderIM {
     }
   }
 
-  __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
+  // k-value kg of the reduction: its patch's corner in the image, and the corner's offset from base
+  struct Corner {
+    bool kok;
+    int iy, ix;
+    long long idx;
+  };
+  __device__ __forceinline__ Corner corner(long long kg, long long k_end) const {
+    Corner o;
+    o.kok = kg < k_end;
+    const unsigned kc = o.kok ? (unsigned)kg : 0u;
     const unsigned howo = (unsigned)(ho * wo);
-    bool kok[E];
-    int iy0[E], ix0[E];
-    long long idx0[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const long long kg = k0 + team_tid() % LPR * E + e;
-      kok[e] = kg < k_end;
-      const unsigned kc = kok[e] ? (unsigned)kg : 0u;
-      const unsigned s = kc / howo;
-      const unsigned rem = kc - s * howo;
-      const int oy = (int)(rem / (unsigned)wo);
-      const int ox = (int)rem - oy * wo;
-      iy0[e] = oy * sy - ph;
-      ix0[e] = ox * sx - pw;
-      idx0[e] = ((long long)s * C * H + iy0[e]) * (long long)W + ix0[e];
-    }
+    const unsigned s = kc / howo;
+    const unsigned rem = kc - s * howo;
+    const int oy = (int)(rem / (unsigned)wo);
+    const int ox = (int)rem - oy * wo;
+    o.iy = oy * sy - ph;
+    o.ix = ox * sx - pw;
+    o.idx = ((long long)s * C * H + o.iy) * (long long)W + o.ix;
+    return o;
+  }
+
+  __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
+    const long long kg = k0 + team_tid() % LPR * E;
     r.use = 0;
+    if constexpr (E == 1) {
+      // (without the arrays of the pair below, which cost this variant 2 .. 8 %)
+      const Corner o = corner(kg, k_end);
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int2 t = table[team_tid() / LPR + RPP * i];
+        const int iy = o.iy + (t.y >> 16);
+        const int ix = o.ix + (t.y & 0xffff);
+        const bool ok = o.kok && t.y >= 0 && (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W;
+        r.v[i][0] = base[ok ? o.idx + t.x : 0];
+        if (ok) r.use |= 1u << i;
+      }
+      return;
+    }
+    Corner o[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) o[e] = corner(kg + e, k_end);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int2 t = table[team_tid() / LPR + RPP * i];
 #pragma unroll
       for (int e = 0; e < E; ++e) {
-        const int iy = iy0[e] + (t.y >> 16);
-        const int ix = ix0[e] + (t.y & 0xffff);
-        const bool ok = kok[e] && t.y >= 0 && (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W;
-        r.v[i][e] = base[ok ? idx0[e] + t.x : 0];
+        const int iy = o[e].iy + (t.y >> 16);
+        const int ix = o[e].ix + (t.y & 0xffff);
+        const bool ok = o[e].kok && t.y >= 0 && (unsigned)iy < (unsigned)H && (unsigned)ix < (unsigned)W;
+        r.v[i][e] = base[ok ? o[e].idx + t.x : 0];
         if (ok) r.use |= 1u << (E * i + e);
       }
     }
