@@ -274,6 +274,27 @@ struct LoaderKC {
   template <Format FMT, bool SUM>
   __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum, unsigned &least) const {
     const int rr = team_tid() >> 3;
+    if constexpr (FMT == kF32) {
+      float *q = lds + rr * Panel<ROWS, kF32>::kRowKStride + (team_tid() & 7) * 4;
+      if (r.fast) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i, q += 32 * Panel<ROWS, kF32>::kRowKStride) {
+          q[0] = r.v[i].x;
+          q[1] = r.v[i].y;
+          q[2] = r.v[i].z;
+          q[3] = r.v[i].w;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < NV; ++i, q += 32 * Panel<ROWS, kF32>::kRowKStride) {
+          const float t[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
+          const bool rv = (rowvalid >> i) & 1u;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q[e] = (((r.kmask >> e) & 1u) && rv) ? t[e] : 0.f;
+        }
+      }
+      return;
+    }
     char *p = reinterpret_cast<char *>(lds) + rr * Panel<ROWS, kSplit>::kRowBytes + (team_tid() & 1) * 8;
     const int chunk = panel_chunk(rr, (team_tid() & 7) >> 1);
 #pragma unroll
@@ -283,12 +304,6 @@ struct LoaderKC {
         const bool rv = (rowvalid >> i) & 1u;
 #pragma unroll
         for (int e = 0; e < 4; ++e) t[e] = (rv && ((r.kmask >> e) & 1u)) ? t[e] : 0.f;
-      }
-      if constexpr (FMT == kF32) {
-        float *q = lds + (rr + 32 * i) * Panel<ROWS, kF32>::kRowKStride + (team_tid() & 7) * 4;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) q[e] = t[e];
-        continue;
       }
       if (SUM) sum[i] += (t[0] + t[1]) + (t[2] + t[3]);
       // rows 32 apart: the chunk index differs in bit 1
@@ -310,7 +325,7 @@ struct LoaderKC<ROWS, false, F> {
   static constexpr int NR = ROWS / RPP;       // rows per thread
   struct Regs {
     float v[NR][E];
-    unsigned kvalid;   // bit e: k-value e of this thread is inside the range
+    bool kvalid[E];   // k-value e of this thread is inside the range
   };
   const float *base;
   unsigned sample_stride;
@@ -334,13 +349,11 @@ struct LoaderKC<ROWS, false, F> {
 
   __device__ __forceinline__ void load(Regs &r, int, long long k0, long long k_end) const {
     const long long kg = k0 + team_tid() % LPR * E;
-    const long long left = k_end - kg;
-    r.kvalid = left > 0 ? 1u : 0u;
-    if (E == 2 && left > 1) r.kvalid = 3u;
     unsigned koff[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const unsigned kc = ((r.kvalid >> e) & 1u) ? (unsigned)kg + e : 0u;
+      r.kvalid[e] = kg + e < k_end;
+      const unsigned kc = r.kvalid[e] ? (unsigned)kg + e : 0u;
       koff[e] = kc;
       if (L < (unsigned)k_end || line_len) {  // more than one sample, or subsampled rows
         const unsigned s = kc / L;
@@ -379,7 +392,7 @@ struct LoaderKC<ROWS, false, F> {
       const bool rv = first_row + RPP * i < rows_valid;
       float t[E];
 #pragma unroll
-      for (int e = 0; e < E; ++e) t[e] = (rv && ((r.kvalid >> e) & 1u)) ? r.v[i][e] : 0.f;
+      for (int e = 0; e < E; ++e) t[e] = (r.kvalid[e] && rv) ? r.v[i][e] : 0.f;
       store_row<ROWS, FMT, SUM, RPP>(lds, team_tid() / LPR, pr, i, t, sum, least);
     }
   }
@@ -465,19 +478,21 @@ struct LoaderKS {
   __device__ __forceinline__ void store(const Regs &r, float *lds, float *sum, unsigned &least) const {
     const int rq = team_tid() % RQ;
     if constexpr (FMT == kF32) {
+      float *q = lds + rq * 4;
+      if (r.fast) {
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        float t[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
-        if (!r.fast) {
+        for (int i = 0; i < NV; ++i)
+          *reinterpret_cast<float4 *>(q + k_of(i) * Panel<ROWS, kF32>::kKRowStride) = r.v[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+          const float t[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
           const bool kv = (r.kmask >> i) & 1u;
+          float o[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int re = row + e;
-            t[e] = kv && is_row(re) ? t[e] : 0.f;
-          }
+          for (int e = 0; e < 4; ++e) o[e] = kv && is_row(row + e) ? t[e] : 0.f;
+          *reinterpret_cast<float4 *>(q + k_of(i) * Panel<ROWS, kF32>::kKRowStride) = make_float4(o[0], o[1], o[2], o[3]);
         }
-        *reinterpret_cast<float4 *>(lds + k_of(i) * Panel<ROWS, kF32>::kKRowStride + rq * 4) =
-            make_float4(t[0], t[1], t[2], t[3]);
       }
       return;
     }
