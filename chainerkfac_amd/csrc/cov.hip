@@ -13,9 +13,9 @@
 // so C is exactly symmetric and every store is a contiguous row segment.
 // A bias ("ones") column is kept out of the tile grid: d = 9C + 1 would pay a
 // whole extra tile row for it.  Its row of C is the vector of row sums of the
-// operand, which the diagonal tiles' workgroups accumulate on the side from the
-// operand values they feed to the matrix cores anyway, and its corner entry is
-// the reduction length.
+// operand, which the diagonal tiles' workgroups accumulate on the side (from the
+// float32 values that they stage or, with the float32 instruction, feed to the
+// matrix cores), and its corner entry is the reduction length.
 //
 // Replaces the im2col + transpose + column_stack + GEMM + scale chain of
 // chainerkfac/optimizers/fisher_blocks/connections/{linear,convolution_2d}.py
@@ -68,7 +68,8 @@ long long max_splits(int ntile) {
 
 SyrkPlan plan_syrk_panels(int d, long long nk, int panel_len) {
   SyrkPlan p;
-  int bm64_max = 520;   // measured: 64-tiles win up to d = 512 (more workgroups, 4x smaller partial tiles)
+  // measured with the float32 instruction: 64-tiles win up to d = 512 (more workgroups, 4x smaller partial tiles)
+  int bm64_max = 520;
   bm64_max = kfac::option_int(kfac::kOptSyrkBm64Max, bm64_max);   // tuning override
   p.bm = d <= bm64_max ? 64 : 128;
   // A short reduction (batch-norm blocks: K = batch size) is all output traffic:
@@ -215,19 +216,18 @@ __device__ __forceinline__ void tri_decode(int t, int &I, int &J) {
 // direct: C[d-1, row] = C[row, d-1] = alpha * sum + beta * C[d-1, row], and the
 // first tile also writes the corner alpha * count + beta * C[d-1, d-1];
 // otherwise the sums go to the k-slice's row-sum slot.
-// rowmask: bit im set = row block im of this wave is its to write.
 template <int WM>
 __device__ __forceinline__ void write_rowsums(float (&rs)[WM], int I, int dt, int d, int direct,
                                               float count, float alpha, float beta,
                                               float *__restrict__ vec, float *__restrict__ C,
-                                              int wave = threadIdx.x >> 6, unsigned rowmask = 0xffffffffu) {
+                                              int wave = threadIdx.x >> 6) {
   constexpr int BM = 64 * WM;
   const int lane = threadIdx.x & 63;
   const int wm = wave >> 1, wn = wave & 1;
 #pragma unroll
   for (int im = 0; im < WM; ++im) {
     const float tot = rs[im] + __shfl_xor(rs[im], 32, 64);
-    if (wn != 0 || lane >= 32 || !((rowmask >> im) & 1u)) continue;
+    if (wn != 0 || lane >= 32) continue;
     const int row = I * BM + (wm * WM + im) * 32 + lane;
     if (!direct) {
       vec[row] = tot;
@@ -238,7 +238,7 @@ __device__ __forceinline__ void write_rowsums(float (&rs)[WM], int I, int dt, in
       C[(long long)row * d + d - 1] = v;
     }
   }
-  if (direct && I == 0 && wave == 0 && (rowmask & 1u) && lane == 0) {
+  if (direct && I == 0 && wave == 0 && lane == 0) {
     float v = alpha * count;
     if (beta != 0.f) v += beta * C[(long long)(d - 1) * d + d - 1];
     C[(long long)(d - 1) * d + d - 1] = v;

@@ -1,5 +1,5 @@
-// Gradient preconditioning  kf = (G^-1 . [dW | db]) . A^-1  as two FP32 MFMA
-// GEMMs, and the batch-norm block's  kf = F^-1 . [dgamma ; dbeta]  as a GEMV
+// Gradient preconditioning  kf = (G^-1 . [dW | db]) . A^-1  as two float32 GEMMs
+// on the matrix cores (mma_core.h), and the batch-norm block's  kf = F^-1 . [dgamma ; dbeta]  as a GEMV
 // with the NaN fallback.  The [dW | db] concatenation is folded into the
 // operand loader of the first product and the kfgrad split into the epilogue
 // of the second, so no concatenated or sliced copy is made.
