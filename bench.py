@@ -39,6 +39,7 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 FP32_MFMA_PEAK_TFLOPS = 157.3   # MI355X dense FP32 matrix peak
+SPLIT_PEAK_TFLOPS = 2516.6 / 6   # float32 products as six bfloat16 products: a sixth of the dense bfloat16 peak
 HBM_PEAK_GBPS = 8000.0           # MI355X HBM3E peak
 # HBM bytes per launch of the covariance SYRK family, written by
 # `bench.py --summarize-traffic` from two `rocprofv3 --pmc` runs (FETCH_SIZE, WRITE_SIZE)
@@ -189,15 +190,37 @@ def family_times(lib):
     return fam
 
 
-def family_roofline(label, kernels, flop, members, fam, empty, note, reference_flop=None):
+def takes_split_products(layer, i, batch):
+    """Whether factor i of a layer (0: input, 1: output gradient) is made of split products: linear layers and slabs
+    (every output gradient, the input of a 1x1 convolution) over more than 128 k-values.  The k x k convolutions of
+    the benchmark's networks have kernels of the float32 instruction."""
+    from chainerkfac_amd import workloads as W
+    if W.cov_rows(layer, batch) <= 128 or layer['kind'] == 'bn':
+        return False
+    return i == 1 or layer['kind'] == 'linear' or layer['k'] == 1
+
+
+def cov_peak(layers, batch):
+    """Matrix peak of the covariance work of a network: what its split products take at a sixth of the bfloat16 peak
+    and the rest at the float32 peak."""
+    from chainerkfac_amd import workloads as W
+    split = 0.0
+    for layer in layers:
+        m = W.cov_rows(layer, batch)
+        split += sum(m * d * (d + 1) for i, d in enumerate(W.factor_dims(layer)) if takes_split_products(layer, i, batch))
+    total = float(W.cov_flops_executed(layers, batch))
+    return total / (split / SPLIT_PEAK_TFLOPS + (total - split) / FP32_MFMA_PEAK_TFLOPS)
+
+
+def family_roofline(label, kernels, flop, members, fam, empty, note, reference_flop=None, peak=FP32_MFMA_PEAK_TFLOPS):
     """Roofline entry of one kernel family: `flop` is the work its kernels are given (issued
     multiply-adds x 2), the time is the sum of the event brackets of `members` (each bracket less
     what an empty bracket measures)."""
     n = sum(fam[m][0] for m in members)
     ms = sum(max(fam[m][1] - fam[m][0] * empty, 0.0) for m in members)
     rate = flop / (ms * 1e-3) / 1e12 if ms > 0 else 0.0
-    out = {'kernel': kernels, 'bound': 'mfma', 'achieved': round(rate, 2), 'peak': FP32_MFMA_PEAK_TFLOPS,
-           'unit': 'TFLOP/s', 'frac': round(rate / FP32_MFMA_PEAK_TFLOPS, 4),
+    out = {'kernel': kernels, 'bound': 'mfma', 'achieved': round(rate, 2), 'peak': round(peak, 1),
+           'unit': 'TFLOP/s', 'frac': round(rate / peak, 4),
            'gflop_per_step': round(flop / 1e9, 1), 'kernel_ms_per_step': round(ms, 4), 'brackets': n,
            'avg_bracket_ms': round(ms / max(n, 1), 4), 'timed': note}
     if reference_flop is not None and ms > 0:
@@ -485,7 +508,8 @@ def run_step_config(args, name, cfg, host=None):
         'cov_syrk': family_roofline(
             'cov_syrk', 'covariance SYRK family: shift::corr_kernel, syrk_rows_kernel, syrk_group_kernel, syrk_kernel, '
             'syrk_conv_kernel and the kernels around them (edge_sums, corr_finish, assemble, finish_group, finish, reduce)',
-            cov_executed, ('syrk', 'cov_aux'), fam, empty, one_stream, reference_flop=flops['cov']),
+            cov_executed, ('syrk', 'cov_aux'), fam, empty, one_stream, reference_flop=flops['cov'],
+            peak=cov_peak(layers, batch)),
         'inverse_tiles': family_roofline(
             'inverse_tiles', 'batched dense inverse: copy_in, diag, update, panel, border, lauum kernels',
             dense_inverse_flops, ('inv_call',), fam, empty,
@@ -495,9 +519,9 @@ def run_step_config(args, name, cfg, host=None):
         'precond_gemm': family_roofline(
             'precond_gemm', 'preconditioning GEMMs: gemm_group_kernel (both phases), gemm_group_finish_kernel, '
             'gemv_kernel + bn_select_kernel of the batch-norm blocks',
-            flops['precondition'], ('gemm', 'gemm_aux'), fam, empty, one_stream),
+            flops['precondition'], ('gemm', 'gemm_aux'), fam, empty, one_stream, peak=SPLIT_PEAK_TFLOPS),
     }
-    main_syrk = family_roofline('', '', cov_executed, ('syrk',), fam, empty, '')
+    main_syrk = family_roofline('', '', cov_executed, ('syrk',), fam, empty, '', peak=cov_peak(layers, batch))
     families['cov_syrk']['main_kernels_only'] = {
         'launches': main_syrk['brackets'], 'kernel_ms_per_step': main_syrk['kernel_ms_per_step'],
         'achieved': main_syrk['achieved'], 'frac': main_syrk['frac']}
@@ -771,7 +795,7 @@ def write_per_layer(path, layers, config='c3'):
     """Per-layer roofline table of the covariance kernels (markdown): every distinct
     convolution / linear shape of the workload, its A and G factor timed alone on one
     stream (HIP events inside the library around the SYRK launch, empty bracket
-    subtracted), against min(FP32 MFMA peak, arithmetic intensity x HBM peak)."""
+    subtracted), against min(matrix peak, arithmetic intensity x HBM peak)."""
     import torch
     from chainerkfac_amd import _lib, ops
     from chainerkfac_amd import workloads as W
@@ -829,7 +853,9 @@ def write_per_layer(path, layers, config='c3'):
             if fac == 'A' and W.takes_shift_route(layer):   # shifted correlations: fewer multiply-adds than M d (d+1)
                 issued = float(W.cov_flops_executed([layer], BATCH)) - float(M) * dG * (dG + 1)
             ai = flop / (in_bytes + 4.0 * d * d)
-            cap = min(FP32_MFMA_PEAK_TFLOPS, ai * HBM_PEAK_GBPS / 1e3)
+            matrix = SPLIT_PEAK_TFLOPS if takes_split_products(layer, 0 if fac == 'A' else 1, BATCH) else \
+                FP32_MFMA_PEAK_TFLOPS
+            cap = min(matrix, ai * HBM_PEAK_GBPS / 1e3)
             rows.append((desc, count, fac, d, M, flop / 1e9, issued / 1e9, t * 1e3, flop / t / 1e9, issued / t / 1e9,
                          ai, cap, issued / t / 1e9 / cap))
         del x, gy
@@ -846,7 +872,9 @@ def write_per_layer(path, layers, config='c3'):
                 'patch / activation product; "issued" is what the kernel gives the matrix cores, which is less for the A '
                 'factor of a 3x3 stride-1 convolution (29 shifted correlations of C x C instead of a 9C x 9C product); '
                 'flop/B = M d (d+1) over the bytes of the input tensor read once plus the factor written once; roofline '
-                'cap = min(157.3 TFLOP/s FP32 MFMA, flop/B x 8 TB/s); the last column is the issued rate over the cap.'
+                'cap = min(matrix peak, flop/B x 8 TB/s), the matrix peak being 157.3 TFLOP/s of the float32 instruction for the '
+                'k x k convolutions and for reductions of at most 128 rows, and 419.4 TFLOP/s (a sixth of the dense bfloat16 '
+                'peak) for the rest; the last column is the issued rate over the cap.'
                 '\n\n'.format(config, path, empty * 1e3))
         f.write('| layer (x count) | factor | d | rows M | GFLOP | GFLOP issued | SYRK kernel us | TFLOP/s (M d (d+1)) | '
                 'TFLOP/s issued | flop/B | roofline cap TFLOP/s | issued / cap |\n'
@@ -1097,14 +1125,16 @@ def summarize_mfma(pmc_dir, out_path, command):
         a[2] += d['GRBM_GUI_ACTIVE']
     if not agg:
         raise SystemExit('no SQ_VALU_MFMA_BUSY_CYCLES / GRBM_GUI_ACTIVE rows under ' + pmc_dir)
-    lines = ['# FP32 matrix-pipe utilisation by kernel: ' + os.path.basename(out_path)[:-3].replace('_', ' '), '',
+    lines = ['# Matrix-pipe utilisation by kernel: ' + os.path.basename(out_path)[:-3].replace('_', ' '), '',
              'Command (one MI355X, repository root; every kernel launched from the host on one stream so that each '
              'dispatch has its own counter record):', '', '```', command, '```', '',
              '`SQ_VALU_MFMA_BUSY_CYCLES` sums, over the 1024 SIMDs, the cycles in which a SIMD\'s matrix pipe was '
              'busy; `GRBM_GUI_ACTIVE` sums the active cycles of the 8 XCDs.  busy = MFMA_BUSY / (GUI_ACTIVE / 8 x '
              '1024): the share of all matrix-pipe cycles of the launch (ramp-up, tail and padding work included) '
-             'in which an MFMA was executing.  Only `v_mfma_f32_32x32x2_f32` is used, so busy x 157.3 TFLOP/s is '
-             'the rate of executed (padded) matrix work.', '',
+             'in which an MFMA was executing.  `syrk_group_kernel`, `syrk_kernel` and the GEMM kernels execute '
+             '`v_mfma_f32_32x32x16_bf16`, six per 16 k-values of a float32 block (reductions of at most 128 k-values: '
+             '`v_mfma_f32_32x32x2_f32`), so busy x 419.4 TFLOP/s is their rate of executed (padded) float32 work; the '
+             'other kernels execute `v_mfma_f32_32x32x2_f32`: busy x 157.3 TFLOP/s.', '',
              '| family | launches | matrix pipe busy |', '|---|---:|---:|']
     fam = {}
     for name, a in agg.items():
