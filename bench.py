@@ -511,7 +511,7 @@ def run_step_config(args, name, cfg, host=None):
             cov_executed, ('syrk', 'cov_aux'), fam, empty, one_stream, reference_flop=flops['cov'],
             peak=cov_peak(layers, batch)),
         'inverse_tiles': family_roofline(
-            'inverse_tiles', 'batched dense inverse: copy_in, diag, update, panel, border, lauum kernels',
+            'inverse_tiles', 'batched dense inverse: copy_in, sweep, border, lauum kernels',
             dense_inverse_flops, ('inv_call',), fam, empty,
             'd^3 flop of the densely inverted factors over the time between the first and the last launch of the '
             'batched call (its kernels overlap on three streams, so their durations do not add up)',
@@ -716,7 +716,7 @@ def run_inverse_config(args, name, cfg):
         'max_residual': worst,      # max over sizes of ||M M^-1 - I||_F / sqrt(d); the bound is 1e-3
         'roofline': {
             'family': 'inverse_tiles',
-            'kernel': 'batched dense inverse: copy_in, diag, update, panel, border, lauum kernels', 'bound': 'mfma',
+            'kernel': 'batched dense inverse: copy_in, sweep, border, lauum kernels', 'bound': 'mfma',
             'achieved': round(achieved, 2), 'peak': FP32_MFMA_PEAK_TFLOPS, 'unit': 'TFLOP/s',
             'frac': round(achieved / FP32_MFMA_PEAK_TFLOPS, 4),
             'timed': 'd^3 flop per matrix over the wall time of the whole batched call (its kernels overlap on two '
@@ -1020,8 +1020,7 @@ KERNEL_FAMILIES = (
     ('batch-norm rank-n inverses', ('lr_',)),
     ('split-K finish, edge sums and assembly of the covariances', ('finish_', 'reduce_kernel', 'shift::assemble',
                                                                   'shift::edge_sums')),
-    ('inverse tile kernels', ('diag_kernel', 'update_kernel', 'lauum_kernel', 'panel_kernel', 'copy_in', 'copy_out',
-                              'border_kernel', 'trtri', 'potrf', 'small_inverse')),
+    ('inverse tile kernels', ('sweep_kernel', 'lauum_kernel', 'copy_in', 'border_kernel')),
     ('damping', ('pi_damp', 'add_diag')),
     ('pack / unpack / copy', ('pack_kernel', 'unpack_kernel', 'stream_copy', 'stream_fanout')),
 )
@@ -1061,7 +1060,7 @@ def summarize_kernel_trace(trace_dir, out_path, command):
     for t0, t1, name in ordered:
         if 'copy_in_kernel' in name and begin is None:
             begin, inside = t0, 0
-        elif begin is not None and ('diag_kernel' in name or 'update_kernel' in name):
+        elif begin is not None and 'sweep_kernel' in name:
             inside += 1
         elif 'lauum_kernel' in name and begin is not None:
             spans.append((t1 - begin, inside))
@@ -1073,11 +1072,7 @@ def summarize_kernel_trace(trace_dir, out_path, command):
              command, '```', '',
              'All launches of the run are counted (warm-up, timed steps, the phase split and the pass that times '
              'every launch with HIP events), so "launches" is a multiple of the per-step count. Durations are '
-             'summed per kernel: the kernels of the batched inverse run side by side on three streams (diagonal '
-             'tiles and panels, column updates, trailing updates), so their sum is about 1.7 times the time the '
-             'inverse takes (what `roofline.families.inverse_tiles` of the bench line divides by is the time '
-             'between the first and the last launch of the call), and "share" is a share of summed kernel time, '
-             'not of elapsed time.', '',
+             'summed per kernel, and "share" is a share of summed kernel time, not of elapsed time.', '',
              '| family | launches | total ms | avg us / launch | share of summed kernel time |', '|---|---:|---:|---:|---:|']
     fam = {}
     for name, a in agg.items():
@@ -1162,8 +1157,7 @@ TRAFFIC_FAMILIES = (
     # family, kernels of the family, the kernel whose launches count the steps of the run
     ('cov_syrk', ('syrk_', 'shift::corr_kernel', 'finish_group_kernel', 'finish_kernel', 'reduce_kernel',
                   'shift::assemble', 'shift::edge_sums', 'shift::corr_finish'), 'finish_group_kernel'),
-    ('inverse_tiles', ('copy_in_kernel', 'diag_kernel', 'update_kernel', 'panel_kernel', 'border_kernel',
-                       'lauum_kernel'), 'lauum_kernel'),
+    ('inverse_tiles', ('copy_in_kernel', 'sweep_kernel', 'border_kernel', 'lauum_kernel'), 'lauum_kernel'),
     ('precond_gemm', ('gemm_group', 'gemv_', 'bn_select'), 'gemm_group_finish_kernel<1>'),
 )
 

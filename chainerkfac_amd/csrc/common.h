@@ -258,8 +258,8 @@ enum Option : int {
   kOptGroupSideStream,    // grouped covariances: 0 = every launch on the caller's stream
   kOptInverseGroup,       // inverse: block columns per trailing update
   kOptInverseBorder,      // inverse: 0 = matrices of 128 m + 1 rows are tiled whole
-  kOptInverseLookahead,   // inverse: 0 = everything on the caller's stream
-  kOptInverseRestLds,     // inverse: bytes of LDS the trailing update asks for
+  kOptInverseLookahead,   // inverse: 0 = a trailing update is one launch's work
+  kOptInverseRestLds,     // inverse: no effect (accepted as before)
   kOptInverseAlign,       // inverse: 0 = sweeps start together ... 100 = end together
   kOptPrecondTasks,       // grouped preconditioning: workgroups per launch
   kOptBnStatsLoop,        // 1: batch-norm statistics always by the looping kernel

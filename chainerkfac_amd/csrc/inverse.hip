@@ -1,50 +1,40 @@
 // Batched damped inverse of SPD Kronecker factors: blocked Cholesky (potrf)
-// followed by the triangular inverse and L^-T L^-1 (potri), FP32 MFMA.
+// followed by the triangular inverse and L^-T L^-1 (potri).
 //
-// All matrices of a batch advance together.  Each is copied (lower tiles
-// only) into a zero/identity padded workspace of NB x NB tiles (NB = 128),
-// stored tile by tile (tile (I,J) of a T x T grid is the contiguous 64 KB block
-// number I*T + J), so that every operand panel and every tile that is read and
-// written back is one dense block instead of 128 short rows a matrix row apart.
-// The strictly lower tiles end up holding L, the upper tiles U = L^-T (the
-// triangular inverse, stored transposed), the diagonal tiles U_kk = L_kk^-T.
-// With M(a,j) the tile in slot (a,j), every product of the sweep has one form,
+// All matrices of a batch advance together, in tiles of NB x NB (NB = 128) of a
+// zero/identity padded workspace.  The strictly lower tiles end up holding L, the
+// upper tiles U = L^-T (the triangular inverse, stored transposed), the diagonal
+// tiles U_kk = L_kk^-T.  With M(a,j) the tile in slot (a,j), every product of the
+// sweep has one form,
 //
 //     C(a,b) -= sum_{j = j_lo .. j_hi} M(a,j) M(b,j)^T                   (*)
 //
 //   a >= b   potrf:  A(a,b) -= sum_j L(a,j) L(b,j)^T                (j < b)
 //   a <  b   trtri:  X^T(a,b) = -sum_j U(a,j) L(b,j)^T         (a <= j < b)
-//            followed by U(a,b) = X^T(a,b) L_bb^-T once the sum is complete,
+//            followed by U(a,b) = X^T(a,b) L_bb^-T once the sum is complete.
 //
-// both k-contiguous "NT" tile GEMMs over row slabs of the workspace.  Block
-// columns are processed in groups of kGroup (2): inside a group the sweep is
-// left-looking (column k receives the products of the group's earlier columns
-// just before it is factored, K up to (kGroup-1)*NB), and after a group every
-// column to its right receives the whole group at once (K = kGroup*NB), which
-// reads and writes each trailing tile once per group instead of once per
-// column.  Per block column k, three launches:
+// Block columns are processed in groups of kGroup (2): inside a group the sweep is
+// left-looking, after a group every tile right of the next group receives the
+// whole group at once (K = kGroup * NB, "rest").  One launch per block column k:
 //
-//   diag(k)    one workgroup per matrix gives the diagonal tile the products it
-//              is still owed, then does its Cholesky and U_kk = L_kk^-T inside
-//              LDS on 32x32 MFMA blocks
-//   column(k)  beside diag(k), on a stream of its own: (*) for the rest of
-//              column k (inside a group: the group's earlier columns; on a
-//              group's first column: the previous group, for both columns of
-//              this group)
-//   panel(k)   after both: M(x,k) = M(x,k) U_kk for x != k  (L(x,k) below,
-//              U(x,k) above)
+//   column     M(x,k) = (M(x,k) - what (*) still owes it) U_kk for every x != k
+//   diagonal   one workgroup per matrix does that for the tile x = k + 1, then the
+//              tile (k+1,k+1) and its Cholesky and inverse: U_{k+1,k+1}, which the next
+//              launch multiplies by
+//   rest       a share of the trailing update of the previous group
 //
-// and after a group's last column, on a further stream beside the next group's
-// sweep, rest(g): (*) for all tiles right of the next group.  A final launch
+// so that everything a launch reads is final when it starts and the chain of
+// diagonal tiles costs one launch per column.  The items of a launch are dealt to
+// at most kSweepWorkgroups workgroups on the host (one per CU).  A final launch
 // forms  out(i,j) = sum_{k >= i} U(i,k) U(j,k)^T  (lauum) and writes the full
 // symmetric inverse.  Matrices of different sizes end their sweeps together (a
-// matrix of T tiles joins at step max_T - T).  The tiles of every launch are
-// listed in a task table built once per plan.
+// matrix of T tiles joins at step max_T - T).
 //
 // Replaces chainerkfac/optimizers/cholesky_inverse.py:16-102 (potrf + potrs
 // against the identity, one matrix at a time).
-#include <cstdlib>
 #include <algorithm>
+#include <cstdlib>
+#include <new>
 #include <numeric>
 
 #include "chol32.h"
@@ -57,14 +47,11 @@ using namespace kfac::mma;
 
 constexpr int NB = 128;
 constexpr int SB = 32;
-constexpr int LS = NB + 1;  // LDS row stride of the diagonal-tile kernel
+constexpr int LS = NB + 1;  // LDS row stride of the diagonal tile
 constexpr int PS = SB + 1;  // row stride of a wave's private 32x32 block
 
-// One tile product, resolved on the host when the plan is built: a workgroup
-// reads its record (one scalar load) and can issue its operand loads at once,
-// instead of walking the per-matrix tables first (three dependent round trips
-// of 1-2 us each on a busy GPU, on the critical path of every launch of the
-// sweep).  Offsets are float offsets into the workspace.
+// One tile product of the sweep as the planner lists it, launch by launch.  Offsets count
+// NB * NB per tile: offset / (NB * NB) is the number of a tile's slot in the workspace.
 struct TileTask {
   long long c_off;   // tile that is updated / written; lauum: the slot of the matrix
   long long a_off;   // first tile of the A operand's run
@@ -72,8 +59,24 @@ struct TileTask {
   int K;             // reduction length; 0: nothing to do (diagonal task: no products owed)
   int flags;         // update: kFirst | kSame; diagonal task: block column k; lauum: I | J << 16
 };
-constexpr int kFirst = 1;   // the accumulators start from zero (first product of an upper tile)
+constexpr int kFirst = 1;   // the sum starts from zero (first product of an upper tile)
 constexpr int kSame = 2;    // both operands are the same run
+
+// What a workgroup of the sweep does next: the tile products merged into the step they
+// belong to, resolved on the host (one scalar load per item).
+enum ItemKind { kItemUpdate = 0, kItemPanel = 1, kItemDiag = 2, kItemBorder = 3 };
+struct SweepItem {
+  int kind;
+  int c, a, b;   // slots: the tile, the first tiles of the operand runs
+  int blocks;    // tiles in either run; 0: nothing is owed
+  int first;     // the tile starts from zero
+  int ut;        // panel: slot of U_kk^T; diagonal: slot that U^T is written to
+  int col;       // diagonal: block column
+  int caller;    // diagonal: caller's index of the matrix
+  int core;      // diagonal: rows of the tiled part
+  int border;    // border: index of the vector task
+  int pad;
+};
 
 struct BorderTask;
 struct InvTables {
@@ -85,26 +88,16 @@ struct InvTables {
   const long long *vec_off;  // [count] bordered matrix: float offset of its vectors a | y | w (core floats
                              // each) and the scalars alpha, S, 1/S behind them; -1 otherwise
   const int *nt;             // [count] tiles per side
-  const long long *ws_off;   // [count] float offset of the padded matrix
-  const int *tile_cs;        // [count+1] cumulative lower-tile counts (copy-in)
-  const int2 *tile_owner;    // [tiles] copy-in: (slot, I | J << 16) of every lower tile, one load instead of a search
-  const TileTask *tasks;     // the tile tasks of all launches
+  const long long *ws_off;   // [count] offset of the padded matrix, NB * NB per tile
+  const int2 *tile_owner;    // [tiles] copy-in: (slot, I | J << 16) of every lower tile
+  const TileTask *tasks;     // the final products
+  const SweepItem *items;    // the items of all sweep launches
+  const int2 *ranges;        // per launch and workgroup: its items [x, y)
   const BorderTask *btasks;  // the vector tasks of the bordered matrices
-  float *ws;                 // padded matrices
+  int ut0;                   // first slot of the U_kk^T buffers, two per matrix
+  float *ws;                 // slots
   int *info;
 };
-
-__device__ __forceinline__ int find_slot(const int *__restrict__ cs, int n, int idx) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (cs[mid] <= idx)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
-}
 
 __device__ __forceinline__ void tri_decode(int t, int &I, int &J) {
   int r = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
@@ -114,286 +107,430 @@ __device__ __forceinline__ void tri_decode(int t, int &I, int &J) {
   J = t - r * (r + 1) / 2;
 }
 
-__device__ __forceinline__ float *tile_ptr(const InvTables &tb, int s, int I, int J) {
-  return tb.ws + tb.ws_off[s] + ((long long)I * tb.nt[s] + J) * (NB * NB);
+// ---------------------------------------------------------------------------
+// Tile slots
+// ---------------------------------------------------------------------------
+// A slot holds a tile in one of two forms.  While products are still owed to it, its negative as
+// float32 in the order of the accumulators below: block (ib, jb) of 32 x 32, then four groups g of
+// eight columns, then the lanes, four consecutive columns 32 jb + 8 g + 4 (lane / 32) .. + 3 of
+// row 32 ib + lane % 32 each (64 KB; a wave reads and writes 1 KB per instruction).  Once
+// final, as the three bfloat16 planes of the split (see mma_core.h) in the order in which
+// v_mfma_f32_32x32x16_bf16 takes them: for every 16 columns (ks), 32 rows (rb) and plane q 64 chunks
+// of 16 bytes, lane l's being columns 16 ks + 8 (l / 32) .. + 7 of row 32 rb + l % 32 (96
+// KB).  A tile is split once, where it becomes final, and multiplied many times; a run of tiles of a
+// tile row is one contiguous stream of panels, which go to LDS as they are and are read
+// from there without bank conflicts at constant offsets.
+//
+// The split is exact from 2^-110 up (mma_core.h); below that the planes drop parts under 2^-126,
+// far below the rounding of any sum they enter: the diagonal entries of L and U are at least 1e-20 in
+// magnitude (square roots of float32 numbers and their reciprocals), and every entry of a
+// product is rounded in proportion to the rows it comes from.  Entries of 3.39e38 and more, and
+// infinities, become NaN: only matrices that are not positive definite (reported in info)
+// or whose inverse overflows have them.
+constexpr int kSlotFloats = NB * NB * 3 / 2;
+constexpr int kStageFloats = kSlotFloats / 4;   // 32 columns of a final tile
+constexpr int kFragBytes = 1024;
+constexpr int kStageBytes = kStageFloats * (int)sizeof(float);
+constexpr int kTileLdsBytes = 4 * kStageBytes;  // two operands, double-buffered; also: the planes of a tile
+static_assert(kTileLdsBytes == kSlotFloats * (int)sizeof(float), "the planes of a tile fit the panels' LDS");
+
+typedef float vfloat4 __attribute__((ext_vector_type(4)));   // register arrays of HIP's float4 struct can end up in scratch
+typedef unsigned vuint4 __attribute__((ext_vector_type(4)));
+
+// byte offset of the fragment of columns 16 ks .., rows 32 rb .., plane q in a final tile
+__device__ __forceinline__ constexpr int frag_off(int ks, int rb, int q) { return ((ks * 4 + rb) * 3 + q) * kFragBytes; }
+
+__device__ __forceinline__ float *slot_ptr(const InvTables &tb, int slot) {
+  return tb.ws + (size_t)slot * kSlotFloats;
+}
+__device__ __forceinline__ int tile_slot(const InvTables &tb, int s, int I, int J) {
+  return (int)(tb.ws_off[s] / (NB * NB)) + I * tb.nt[s] + J;
 }
 
-// ---------------------------------------------------------------------------
-// The tile product  acc(128 x 128) += A(128 x K) B(128 x K)^T  of this file
-// ---------------------------------------------------------------------------
-// Operands are runs of consecutive workspace tiles (k-value k is column k % NB
-// of tile k / NB: 128 rows of 128 contiguous bytes per panel of KT k-values, no
-// edge masks, the workspace is padded) or one tile read as its transpose.
-//
-// Everything around the matrix instructions is kept off the vector ALU and
-// placed between them by hand: the products are short (K = 128 .. 512) and run
-// one or two workgroups per CU, so instructions that the compiler leaves in one
-// block (the LDS stores and the global loads of the next panels, 90 instructions
-// per pass with their address arithmetic) stall the matrix pipe with nothing
-// else to fill it.
-//   * global loads: wave-uniform base (scalar registers, advanced per pass) plus
-//     a per-lane 32-bit offset that never changes;
-//   * LDS: row-major panels with a row stride of KT + 4 floats, written and read
-//     16 bytes at a time.  v_mfma_f32_32x32x2_f32 takes two k-values per
-//     instruction, one from each half of the wave; which two does not matter as
-//     long as both operands agree, so the lanes of half h read the four k-values
-//     8g + 4h .. 8g + 4h + 3 of their row in one instruction and feed them to
-//     four consecutive MFMAs (k pairs {8g + j, 8g + 4 + j});
-//   * the LDS panels are double-buffered: one barrier per pass, and the stores
-//     and loads for the passes ahead are dealt out one per group of four MFMAs.
-// The global loads run PD passes ahead of the LDS stores (with less than two
-// passes of 64 k-values in flight, a third of the passes of a full GPU waited
-// 2-4 us for their operands, measured with time stamps).
-typedef float vfloat4 __attribute__((ext_vector_type(4)));   // register arrays of HIP's float4 struct can end up in scratch
-
-constexpr int RS = KT + 4;      // row stride of a row-major LDS panel (16-byte aligned rows; 8 lanes
-                                // of a 16-byte access then cover all 32 banks)
-constexpr int TS = NB + 4;      // k-row stride of a transposed LDS panel
-constexpr int PF = NB * RS;     // floats per LDS panel
-static_assert(KT * TS <= PF, "a transposed panel must fit the same buffer");
-constexpr int kTileLdsFloats = 4 * PF;   // A even / odd pass, B even / odd pass
-constexpr size_t kTileLdsBytes = kTileLdsFloats * sizeof(float);
-
-// States that a pointer is the same in every lane, so that it is kept in scalar
+// States that a value is the same in every lane, so that it is kept in scalar
 // registers (the compiler cannot always see this through the table lookups).
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ const float *wave_uniform(const float *p) {
   const unsigned long long v = reinterpret_cast<unsigned long long>(p);
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
   const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
   return reinterpret_cast<const float *>(((unsigned long long)hi << 32) | lo);
 }
-
 __device__ __forceinline__ vfloat4 gload16(const float *base, unsigned byte_off) {
   return *(const KFAC_GLOBAL_AS vfloat4 *)((const KFAC_GLOBAL_AS char *)base + byte_off);
 }
-
-__device__ __forceinline__ void gstore1(float *base, unsigned byte_off, float v) {
-  *(KFAC_GLOBAL_AS float *)((KFAC_GLOBAL_AS char *)base + byte_off) = v;
+template <class V>
+__device__ __forceinline__ void gstore16(float *base, unsigned byte_off, V v) {
+  *(KFAC_GLOBAL_AS V *)((KFAC_GLOBAL_AS char *)base + byte_off) = v;
 }
 
-// The accumulators <-> a row-major NB x NB tile at a wave-uniform address, as
-// scalar base + one lane offset per group of eight elements + immediates (no
-// 64-bit address per element).
-__device__ __forceinline__ unsigned acc_lane_offset() {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int row0 = (wave >> 1) * 64 + 4 * (lane >> 5), col0 = (wave & 1) * 64 + (lane & 31);
-  return (unsigned)((row0 * NB + col0) * sizeof(float));
+// ---------------------------------------------------------------------------
+// The tile product  sum(128 x 128) = A(128 x K) B(128 x K)^T
+// ---------------------------------------------------------------------------
+// 256 threads, wave (wi, wj) has rows 64 wi .. and columns 64 wj ..: acc[im][in] is the block of
+// columns 32 (2 wj + im) and rows 32 (2 wi + in).  The operands are passed to the matrix
+// instruction the other way round, so that a lane's sixteen values are four runs of four consecutive
+// columns of one row.  Six plane products, hi * hi in acc and the other five in low (mma_core.h).
+// In an update of (*) acc starts from -C: factors of rectified activations have one large eigenvalue,
+// which the first column's products take out of C, and the sums after that are small and rounded
+// as such.  (From zero, C subtracted at the end, every sum is rounded at the size of C: 1.3 to 2 times
+// the error of the float32 instruction for such matrices, where this form has 0.3 to 0.6 times; matrices without such an eigenvalue 0.2 to 0.5 and 0.3 to 0.5.)
+//
+// One workgroup per CU (96 KB of LDS, up to 512 registers per lane), so nothing else hides
+// its latencies and everything is placed by hand:
+//   * global loads run three stages of 32 k-values ahead of the matrix instructions,
+//     through two register sets, and across the end of a product into the next item's;
+//   * LDS is double-buffered (one barrier per stage); fragments are read one half stage
+//     ahead, the second half of a stage being multiplied after the barrier beside the reads of
+//     the next one;
+//   * LDS reads, LDS writes and global loads are dealt out one per matrix instruction.
+struct Frags {
+  bf16x8 a[2][3], b[2][3];
+};
+struct Panels {   // one stage of both operands in registers: 6 + 6 x 16 bytes
+  vfloat4 v[12];
+};
+// The loads ahead: the run that is being loaded and the one after it.
+struct Cursor {
+  const float *a, *b;
+  int left;
+  const float *next_a, *next_b;
+  int next_left;
+};
+
+__device__ __forceinline__ void cursor_turn(Cursor &cu) {
+  if (cu.left == 0 && cu.next_left > 0) {
+    cu.a = cu.next_a;
+    cu.b = cu.next_b;
+    cu.left = cu.next_left;
+    cu.next_left = 0;
+  }
 }
-// acc = -C
-__device__ __forceinline__ void load_neg_tile(const float *C, floatx16 (&acc)[2][2]) {
-  const unsigned lane_off = acc_lane_offset();
+__device__ __forceinline__ void cursor_step(Cursor &cu) {
+  if (cu.left > 0) {
+    cu.a += kStageFloats;
+    cu.b += kStageFloats;
+    --cu.left;
+  }
+}
+// The loads go through buffer descriptors, whose size is zero once there is nothing left to load: no
+// branch around the loads, no memory access.
+struct StageSource {
+  __amdgpu_buffer_rsrc_t a, b;
+};
+__device__ __forceinline__ StageSource stage_source(const Cursor &cu) {
+  const int bytes = cu.left > 0 ? kStageBytes : 0;
+  constexpr int kRawDwords = 0x00020000;
+  return StageSource{__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(cu.a), 0, bytes, kRawDwords),
+                     __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(cu.b), 0, bytes, kRawDwords)};
+}
+__device__ __forceinline__ void panel_load1(const StageSource &src, Panels &r, int i) {
+  r.v[i] = __builtin_bit_cast(vfloat4, __builtin_amdgcn_raw_buffer_load_b128(i < 6 ? src.a : src.b, threadIdx.x * 16,
+                                                                              (i % 6) * 4096, 0));
+}
+__device__ __forceinline__ void panel_write1(const Panels &r, char *buf, int i) {
+  *reinterpret_cast<vfloat4 *>(buf + threadIdx.x * 16 + i * 4096) = r.v[i];   // A stage, then B stage
+}
+__device__ __forceinline__ void frag_read1(Frags &f, const char *buf, int ks, int i) {
+  const int wave = threadIdx.x >> 6, wi = wave >> 1, wj = wave & 1;
+  const int lane16 = (threadIdx.x & 63) * 16;
+  const int blk = (i % 6) / 3, q = i % 3;
+  if (i < 6)
+    f.a[blk][q] = *reinterpret_cast<const bf16x8 *>(buf + lane16 + wi * (2 * 3 * kFragBytes) + frag_off(ks, blk, q));
+  else
+    f.b[blk][q] = *reinterpret_cast<const bf16x8 *>(buf + lane16 + kStageBytes + wj * (2 * 3 * kFragBytes) +
+                                                    frag_off(ks, blk, q));
+}
+__device__ __forceinline__ void frag_mma1(const Frags &f, floatx16 (&acc)[2][2], floatx16 (&low)[2][2], int i) {
+  const int t = i / 4, im = (i / 2) & 1, in = i & 1;
+  floatx16 &sum = t == kSplitTerms - 1 ? acc[im][in] : low[im][in];
+  sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[im][kSplitB[t]], f.a[in][kSplitA[t]], sum, 0, 0, 0);
+}
+
+// Stage of which LDS buffer `cur` holds the panels: multiplies the previous stage's second half
+// (f1; not when FIRST) and this stage's first half, leaves this stage's second half in f1.
+// Beside them `r`, the next stage, is written to `nxt` and refilled from the cursor.
+template <bool FIRST>
+__device__ __forceinline__ void product_stage(const char *cur, char *nxt, Panels &r, Cursor &cu, Frags &f1,
+                                              floatx16 (&acc)[2][2], floatx16 (&low)[2][2]) {
+  Frags f0;
+#pragma unroll
+  for (int i = 0; i < 24; ++i) {
+    if (!FIRST) frag_mma1(f1, acc, low, i);
+    if (i < 12)
+      frag_read1(f0, cur, 0, i);
+    else
+      panel_write1(r, nxt, i - 12);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  cursor_turn(cu);
+  const StageSource src = stage_source(cu);
+#pragma unroll
+  for (int i = 0; i < 24; ++i) {
+    frag_mma1(f0, acc, low, i);
+    if (i < 12)
+      frag_read1(f1, cur, 1, i);
+    else
+      panel_load1(src, r, i - 12);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  cursor_step(cu);
+  __syncthreads();
+}
+
+// Fills the pipeline: stage 0 in LDS buffer 0, stages 1 and 2 in flight.
+__device__ __forceinline__ void product_start(Cursor &cu, Panels (&r)[2], char *lds) {
+  // (a run has at least four stages)
+  StageSource src = stage_source(cu);
+#pragma unroll
+  for (int i = 0; i < 12; ++i) panel_load1(src, r[0], i);
+  cursor_step(cu);
+  src = stage_source(cu);
+#pragma unroll
+  for (int i = 0; i < 12; ++i) panel_load1(src, r[1], i);
+  cursor_step(cu);
+#pragma unroll
+  for (int i = 0; i < 12; ++i) panel_write1(r[0], lds, i);
+  src = stage_source(cu);
+#pragma unroll
+  for (int i = 0; i < 12; ++i) panel_load1(src, r[0], i);
+  cursor_step(cu);
+  __syncthreads();
+}
+
+// acc += sum over the `blocks` tiles of the runs; started by product_start or by the product before.
+// `before_last` is called two stages before the end.
+template <class F>
+__device__ __forceinline__ void product_run(int blocks, Cursor &cu, Panels (&r)[2], char *lds, floatx16 (&acc)[2][2],
+                                            F before_last) {
+  floatx16 low[2][2];
+  zero_acc<2, 2>(low);
+  Frags f1;
+  char *b0 = lds, *b1 = lds + 2 * kStageBytes;
+  product_stage<true>(b0, b1, r[1], cu, f1, acc, low);
+  product_stage<false>(b1, b0, r[0], cu, f1, acc, low);
+  for (int p = blocks * 2 - 2; p > 0; --p) {
+    product_stage<false>(b0, b1, r[1], cu, f1, acc, low);
+    product_stage<false>(b1, b0, r[0], cu, f1, acc, low);
+  }
+  before_last();
+  product_stage<false>(b0, b1, r[1], cu, f1, acc, low);
+  product_stage<false>(b1, b0, r[0], cu, f1, acc, low);
+#pragma unroll
+  for (int i = 0; i < 24; ++i) frag_mma1(f1, acc, low, i);
 #pragma unroll
   for (int im = 0; im < 2; ++im)
 #pragma unroll
-    for (int vq = 0; vq < 4; ++vq) {
-      const unsigned o = lane_off + (unsigned)((im * 32 + 8 * vq) * NB * sizeof(float));
-#pragma unroll
-      for (int vr = 0; vr < 4; ++vr)
-#pragma unroll
-        for (int in = 0; in < 2; ++in)
-          acc[im][in][vq * 4 + vr] = -gload1(C, o + (unsigned)((vr * NB + in * 32) * sizeof(float)));
-    }
+    for (int in = 0; in < 2; ++in) acc[im][in] += low[im][in];
 }
-// C = -acc
-__device__ __forceinline__ void store_neg_tile(float *C, const floatx16 (&acc)[2][2]) {
-  const unsigned lane_off = acc_lane_offset();
+
+// Byte offset of this lane's values of block (im, in), group 0, in a float32 tile; groups 1 KB apart.
+__device__ __forceinline__ unsigned acc_offset(int im, int in) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int ib = (wave >> 1) * 2 + in, jb = (wave & 1) * 2 + im;
+  return (unsigned)((ib * 4 + jb) * 4096 + lane * 16);
+}
+struct TileRegs {
+  vfloat4 v[2][2][4];
+};
+__device__ __forceinline__ void tile_load(const float *tile, TileRegs &c) {
 #pragma unroll
   for (int im = 0; im < 2; ++im)
 #pragma unroll
-    for (int vq = 0; vq < 4; ++vq) {
-      const unsigned o = lane_off + (unsigned)((im * 32 + 8 * vq) * NB * sizeof(float));
+    for (int in = 0; in < 2; ++in)
 #pragma unroll
-      for (int vr = 0; vr < 4; ++vr)
+      for (int g = 0; g < 4; ++g) c.v[im][in][g] = gload16(tile, acc_offset(im, in) + g * 1024u);
+}
+__device__ __forceinline__ void tile_zero(TileRegs &c) {
 #pragma unroll
-        for (int in = 0; in < 2; ++in)
-          gstore1(C, o + (unsigned)((vr * NB + in * 32) * sizeof(float)), -acc[im][in][vq * 4 + vr]);
-    }
+  for (int im = 0; im < 2; ++im)
+#pragma unroll
+    for (int in = 0; in < 2; ++in)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) c.v[im][in][g] = vfloat4{0.f, 0.f, 0.f, 0.f};
+}
+__device__ __forceinline__ void tile_store(float *tile, const TileRegs &c) {
+#pragma unroll
+  for (int im = 0; im < 2; ++im)
+#pragma unroll
+    for (int in = 0; in < 2; ++in)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) gstore16(tile, acc_offset(im, in) + g * 1024u, c.v[im][in][g]);
+}
+__device__ __forceinline__ void tile_to_acc(const TileRegs &c, floatx16 (&acc)[2][2]) {
+#pragma unroll
+  for (int im = 0; im < 2; ++im)
+#pragma unroll
+    for (int in = 0; in < 2; ++in)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[im][in][v] = c.v[im][in][v >> 2][v & 3];
+}
+__device__ __forceinline__ void tile_from_acc(TileRegs &c, const floatx16 (&acc)[2][2]) {
+#pragma unroll
+  for (int im = 0; im < 2; ++im)
+#pragma unroll
+    for (int in = 0; in < 2; ++in)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) c.v[im][in][v >> 2][v & 3] = acc[im][in][v];
 }
 
-// k along the rows of a run of consecutive tiles
-struct OperandRows {
-  const float *base;   // first tile of the run
-  __device__ __forceinline__ static unsigned lane_offset() {
-    return (unsigned)(((threadIdx.x >> 3) * NB + (threadIdx.x & 7) * 4) * sizeof(float));
-  }
-  __device__ __forceinline__ void load(vfloat4 (&r)[4], unsigned off, int pass) const {
-    const int k = pass * KT;
-    const float *b = wave_uniform(base + (size_t)(k / NB) * (NB * NB) + (k % NB));
+// The planes of columns 16 s .. of a block in accumulator order: lanes l and l + 32 hold four of
+// each other's eight columns and exchange them.
+__device__ __forceinline__ void block_frags(const vfloat4 (&v)[4], int s, vuint4 (&f)[3]) {
+  unsigned x[3][2], y[3][2];   // groups 2 s and 2 s + 1: planes of columns 0, 1 and 2, 3 of the lane's four
+  const vfloat4 lo = v[2 * s], hi = v[2 * s + 1];
+  split_pair(lo[0], lo[1], x[0][0], x[1][0], x[2][0]);
+  split_pair(lo[2], lo[3], x[0][1], x[1][1], x[2][1]);
+  split_pair(hi[0], hi[1], y[0][0], y[1][0], y[2][0]);
+  split_pair(hi[2], hi[3], y[0][1], y[1][1], y[2][1]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = gload16(b, off + i * (32 * NB * (unsigned)sizeof(float)));
+  for (int q = 0; q < 3; ++q) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const auto r = __builtin_amdgcn_permlane32_swap(x[q][e], y[q][e], false, false);
+      x[q][e] = r[0];
+      y[q][e] = r[1];
+    }
+    f[q] = vuint4{x[q][0], x[q][1], y[q][0], y[q][1]};
   }
-  __device__ __forceinline__ static void store1(const vfloat4 (&r)[4], int i, float *panel) {
-    float *p = panel + (threadIdx.x >> 3) * RS + (threadIdx.x & 7) * 4;
-    *reinterpret_cast<vfloat4 *>(p + 32 * i * RS) = r[i];
-  }
-  // the four k-values 8g + 4h .. + 3 of operand row `row`
-  __device__ __forceinline__ static vfloat4 fetch4(const float *panel, int row, int g, int h) {
-    return *reinterpret_cast<const vfloat4 *>(panel + row * RS + 8 * g + 4 * h);
-  }
-};
+}
 
-// one tile read as its transpose: operand row c, k-value q is element (q, c)
-struct OperandCols {
-  const float *base;
-  __device__ __forceinline__ static unsigned lane_offset() {
-    return (unsigned)(((threadIdx.x >> 5) * NB + (threadIdx.x & 31) * 4) * sizeof(float));
-  }
-  __device__ __forceinline__ void load(vfloat4 (&r)[4], unsigned off, int pass) const {
-    const float *b = wave_uniform(base + pass * (KT * NB));
+// M(x,k) = M(x,k) U_kk: the tile from registers, its planes shared through LDS; operand rows of
+// U_kk^T straight from memory (two waves read the same, once).  U_kk is upper triangular: column
+// block cb takes the blocks q <= cb, and the waves of a row half take the column blocks {0, 3} and
+// {1, 2}, five blocks each.  The result is final: stored as planes.
+template <int WJ>
+__device__ __forceinline__ void panel_columns(const char *lds, const vuint4 (&ut)[5][2][3], float *tile) {
+  constexpr int CB[2] = {WJ == 0 ? 0 : 1, WJ == 0 ? 3 : 2};
+  const int wi = threadIdx.x >> 7;
+  const int lane16 = (threadIdx.x & 63) * 16;
+  floatx16 acc[2][2], low[2][2];   // [column block][row block]
+  zero_acc<2, 2>(acc);
+  zero_acc<2, 2>(low);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = gload16(b, off + i * (8 * NB * (unsigned)sizeof(float)));
-  }
-  __device__ __forceinline__ static void store1(const vfloat4 (&r)[4], int i, float *panel) {
-    float *p = panel + (threadIdx.x >> 5) * TS + (threadIdx.x & 31) * 4;
-    *reinterpret_cast<vfloat4 *>(p + 8 * i * TS) = r[i];
-  }
-  __device__ __forceinline__ static vfloat4 fetch4(const float *panel, int row, int g, int h) {
-    const float *p = panel + (8 * g + 4 * h) * TS + row;
-    vfloat4 v;
-    v.x = p[0];
-    v.y = p[TS];
-    v.z = p[2 * TS];
-    v.w = p[3 * TS];
-    return v;
-  }
-};
-
-// One pass of KT k-values from the LDS panels `pa` / `pb` (both `pa` when SAME),
-// ending with a barrier.  Beside the MFMAs it writes the register set `ra` /
-// `rb` (the pass after this one) to the panels `na` / `nb`, then calls
-// `refill_a()` / `refill_b()`, which load that register set again.
-template <bool SAME, class LA, class LB, class FA, class FB>
-__device__ __forceinline__ void tile_pass(const float *pa, const float *pb, float *na, float *nb,
-                                          vfloat4 (&ra)[4], vfloat4 (&rb)[4],
-                                          floatx16 (&acc)[2][2], FA refill_a, FB refill_b) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int lrow = lane & 31, lk = lane >> 5;
-  vfloat4 fa[2], fb[2];
+  for (int qb = 0; qb < 4; ++qb) {
+    if (qb > CB[1]) break;
 #pragma unroll
-  for (int im = 0; im < 2; ++im) fa[im] = LA::fetch4(pa, (wm * 2 + im) * 32 + lrow, 0, lk);
-#pragma unroll
-  for (int in = 0; in < 2; ++in)
-    fb[in] = SAME ? LA::fetch4(pa, (wn * 2 + in) * 32 + lrow, 0, lk)
-                  : LB::fetch4(pb, (wn * 2 + in) * 32 + lrow, 0, lk);
-#pragma unroll
-  for (int g = 0; g < KT / 8; ++g) {
-    vfloat4 ga[2], gb[2];
-    if (g + 1 < KT / 8) {
-#pragma unroll
-      for (int im = 0; im < 2; ++im) ga[im] = LA::fetch4(pa, (wm * 2 + im) * 32 + lrow, g + 1, lk);
+    for (int s = 0; s < 2; ++s) {
+      bf16x8 m[2][3];
 #pragma unroll
       for (int in = 0; in < 2; ++in)
-        gb[in] = SAME ? LA::fetch4(pa, (wn * 2 + in) * 32 + lrow, g + 1, lk)
-                      : LB::fetch4(pb, (wn * 2 + in) * 32 + lrow, g + 1, lk);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          m[in][q] = *reinterpret_cast<const bf16x8 *>(lds + lane16 + wi * (2 * 3 * kFragBytes) + frag_off(2 * qb + s, in, q));
+#pragma unroll
+      for (int t = 0; t < kSplitTerms; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int in = 0; in < 2; ++in) {
+            if (qb > CB[c]) continue;
+            const int u = c == 0 ? qb : CB[0] + 1 + qb;
+            floatx16 &sum = t == kSplitTerms - 1 ? acc[c][in] : low[c][in];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ut[u][s][kSplitB[t]]),
+                                                          m[in][kSplitA[t]], sum, 0, 0, 0);
+          }
     }
+  }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      __builtin_amdgcn_sched_barrier(0);
+  for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int im = 0; im < 2; ++im)
+    for (int in = 0; in < 2; ++in) {
+      vfloat4 v[4];
 #pragma unroll
-        for (int in = 0; in < 2; ++in)
-          acc[im][in] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[im][j], fb[in][j], acc[im][in], 0, 0, 0);
-      // slot 4g + j of 16: one LDS store at most (the last pass of a product stores what it
-      // holds as well, into the buffer nobody reads any more: cheaper than a branch per store)
-      const int slot = 4 * g + j;
-      if (slot >= 1 && slot < 5) LA::store1(ra, slot - 1, na);
-      if (!SAME && slot >= 5 && slot < 9) LB::store1(rb, slot - 5, nb);
-    }
-    if (g == 1) refill_a();               // after its stores (slots 1 .. 4)
-    if (!SAME && g == 2) refill_b();      // slots 5 .. 8
-    if (g + 1 < KT / 8) {
+      for (int g = 0; g < 4; ++g)
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        fa[i] = ga[i];
-        fb[i] = gb[i];
+        for (int e = 0; e < 4; ++e) v[g][e] = acc[c][in][4 * g + e] + low[c][in][4 * g + e];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        vuint4 f[3];
+        block_frags(v, s, f);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          gstore16(tile, (unsigned)(lane16 + wi * (2 * 3 * kFragBytes) + frag_off(2 * CB[c] + s, in, q)), f[q]);
       }
     }
+}
+template <int WJ>
+__device__ __forceinline__ void panel_operand(const float *ut_tile, vuint4 (&ut)[5][2][3]) {
+  constexpr int CB[2] = {WJ == 0 ? 0 : 1, WJ == 0 ? 3 : 2};
+  const unsigned lane16 = (threadIdx.x & 63) * 16u;
+#pragma unroll
+  for (int u = 0; u < 5; ++u) {
+    const int c = u <= CB[0] ? 0 : 1, qb = c == 0 ? u : u - CB[0] - 1;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        ut[u][s][q] = __builtin_bit_cast(vuint4, gload16(ut_tile, lane16 + (unsigned)frag_off(2 * qb + s, CB[c], q)));
   }
+}
+// ends with a barrier
+__device__ __forceinline__ void panel_role(const InvTables &tb, const SweepItem &it, const TileRegs &c, char *lds) {
+  float *tile = const_cast<float *>(wave_uniform(slot_ptr(tb, it.c)));
+  const float *ut_tile = wave_uniform(slot_ptr(tb, it.ut));
+  const int wave = uniform(threadIdx.x >> 6), wi = wave >> 1, wj = wave & 1;
+  const int lane16 = (threadIdx.x & 63) * 16;
+#pragma unroll
+  for (int im = 0; im < 2; ++im)
+#pragma unroll
+    for (int in = 0; in < 2; ++in) {
+      vfloat4 m[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) m[g] = -c.v[im][in][g];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        vuint4 f[3];
+        block_frags(m, s, f);
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          *reinterpret_cast<vuint4 *>(lds + lane16 + frag_off(2 * (2 * wj + im) + s, 2 * wi + in, q)) = f[q];
+      }
+    }
+  vuint4 ut[5][2][3];
+  if (wj == 0)
+    panel_operand<0>(ut_tile, ut);
+  else
+    panel_operand<1>(ut_tile, ut);
+  __syncthreads();
+  if (wj == 0)
+    panel_columns<0>(lds, ut, tile);
+  else
+    panel_columns<1>(lds, ut, tile);
   __syncthreads();
 }
 
-// K must be a multiple of 4 * KT.  lds: kTileLdsFloats.  Ends with a barrier.
-template <bool SAME, int PD, class LA, class LB>
-__device__ __forceinline__ void tile_mainloop(const LA &la, const LB &lb, int K, float *lds,
-                                              floatx16 (&acc)[2][2]) {
-  constexpr int UNROLL = PD % 2 == 0 ? PD : 2 * PD;   // register set and LDS buffer of a pass are static
-  float *ldsA = lds, *ldsB = lds + 2 * PF;
-  const int P = K / KT;
-  const unsigned offA = LA::lane_offset(), offB = LB::lane_offset();
-  vfloat4 ra[PD][4];
-  vfloat4 rb[SAME ? 1 : PD][4];
-#pragma unroll
-  for (int q = 0; q < PD; ++q) {
-    if (q < P) {
-      la.load(ra[q], offA, q);
-      if (!SAME) lb.load(rb[q], offB, q);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    LA::store1(ra[0], i, ldsA);
-    if (!SAME) LB::store1(rb[0], i, ldsB);
-  }
-  if (PD < P) {
-    la.load(ra[0], offA, PD);
-    if (!SAME) lb.load(rb[0], offB, PD);
-  }
-  __syncthreads();
-  for (int pb = 0; pb < P; pb += UNROLL) {
-#pragma unroll
-    for (int u = 0; u < UNROLL; ++u) {
-      const int p = pb + u;
-      if (UNROLL > 4 && p >= P) break;   // P is a multiple of 4
-      const int r = (u + 1) % PD;            // register set of pass p + 1 (static once unrolled)
-      const bool ahead = p + 1 + PD < P;     // which then takes pass p + 1 + PD
-      tile_pass<SAME, LA, LB>(
-          ldsA + (u & 1) * PF, ldsB + (u & 1) * PF, ldsA + ((u + 1) & 1) * PF, ldsB + ((u + 1) & 1) * PF,
-          ra[r], rb[SAME ? 0 : r], acc,
-          [&]() { if (ahead) la.load(ra[r], offA, p + 1 + PD); },
-          [&]() { if (ahead) lb.load(rb[SAME ? 0 : r], offB, p + 1 + PD); });
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// copy-in: lower tiles of in -> padded workspace (identity on the padding)
+// copy-in: the negative of the lower tiles of in -> float32 slots (identity on the padding)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void copy_in_kernel(InvTables tb, int count, int tile0) {
-  const int2 owner = tb.tile_owner[(int)blockIdx.x + tile0];
+__global__ __launch_bounds__(256) void copy_in_kernel(InvTables tb) {
+  const int2 owner = tb.tile_owner[blockIdx.x];
   const int s = owner.x, I = owner.y & 0xffff, J = owner.y >> 16;
   const int d = tb.dim[s], dc = tb.core[s];
   const float *__restrict__ src = tb.in[s];
-  float *__restrict__ dst = tile_ptr(tb, s, I, J);
-  const int c4 = (threadIdx.x & 31) * 4;
-  const int r0 = threadIdx.x >> 5;
+  float *__restrict__ dst = slot_ptr(tb, tile_slot(tb, s, I, J));
+  const int lane = threadIdx.x & 63, ib = threadIdx.x >> 6;
+  const int r = I * NB + ib * 32 + (lane & 31);
   // 16-byte loads at float granularity (the rows of an odd-sized matrix do not start on
-  // 16-byte boundaries); the quads cut by the edge of the matrix go element by element
+  // 16-byte boundaries); the quads cut by the edge of the matrix go element by element.  Four
+  // consecutive loads of a lane cover a 128-byte piece of its row.
   typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
-#pragma unroll 8
-  for (int p = 0; p < NB / 8; ++p) {
-    const int rl = r0 + 8 * p;
-    const int r = I * NB + rl;
-    const int c = J * NB + c4;
-    float v[4];
+#pragma unroll
+  for (int p = 0; p < 16; ++p) {
+    const int c = J * NB + 8 * p + 4 * (lane >> 5);   // block p / 4, group p % 4
+    vfloat4 v;
     if (r < dc && c + 3 < dc) {
       const floatx4u x = *reinterpret_cast<const floatx4u *>(src + (long long)r * d + c);
-      v[0] = x.x;
-      v[1] = x.y;
-      v[2] = x.z;
-      v[3] = x.w;
+      v = vfloat4{x.x, x.y, x.z, x.w};
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int ce = c + e;
-        float x = (r == ce) ? 1.f : 0.f;
-        if (r < dc && ce < dc) x = src[(long long)r * d + ce];
+        float x = (r == c + e) ? 1.f : 0.f;
+        if (r < dc && c + e < dc) x = src[(long long)r * d + c + e];
         v[e] = x;
       }
     }
-    *reinterpret_cast<float4 *>(dst + rl * NB + c4) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<vfloat4 *>(dst + (ib * 16 + p) * 256 + lane * 4) = -v;
   }
   // a bordered matrix: its last column and corner go beside the tiles
   const long long vo = tb.vec_off[s];
@@ -430,36 +567,23 @@ __device__ __forceinline__ void wave_visit(const floatx16 &acc, F f) {
   for (int v = 0; v < 16; ++v) f(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3), lane & 31, acc[v]);
 }
 
-// Diagonal tile (k,k) of a matrix: first the products it is still owed,
-//   C(k,k) -= sum_{j = lo .. hi} M(k,j) M(k,j)^T        (nothing when K = 0),
-// through the shared main loop (the other tiles of the column receive theirs
-// from the update workgroups of the same launch), then the factorisation.
-__device__ __forceinline__ void diag_role(const InvTables &tb, const TileTask &t, float *smem) {
+// The diagonal tile (k,k) after its last products, its negative in registers: factored in LDS, U_kk written to
+// its slot and U_kk^T, which the next launch multiplies by, to the item's.  Ends with a barrier.
+__device__ __forceinline__ void diag_role(const InvTables &tb, const SweepItem &it, const TileRegs &tile, float *smem) {
   float *S = smem;                      // NB x LS working tile
   float *scratch = smem + NB * LS;      // 3 waves x SB x PS
-  const int d = (int)(t.b_off >> 32);
-  const int k = t.flags;
-  constexpr int ld = NB;
-  float *tile = tb.ws + t.c_off;
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  if (t.K > 0) {
-    floatx16 acc[2][2];
-    fill_acc<2, 2>(acc, [&](int rr, int cc) { return -tile[rr * NB + cc]; });
-    const OperandRows la{tb.ws + t.a_off};
-    tile_mainloop<true, 2>(la, la, t.K, smem, acc);   // ends with a barrier
-    for_each_acc<2, 2>(acc, [&](int rr, int cc, float v) { S[rr * LS + cc] = -v; });
-  } else {
-    const int c4 = (threadIdx.x & 31) * 4, r0 = threadIdx.x >> 5;
-#pragma unroll 4
-    for (int p = 0; p < NB / 8; ++p) {
-      const int r = r0 + 8 * p;
-      const float4 v = *reinterpret_cast<const float4 *>(tile + r * ld + c4);
-      S[r * LS + c4 + 0] = v.x;
-      S[r * LS + c4 + 1] = v.y;
-      S[r * LS + c4 + 2] = v.z;
-      S[r * LS + c4 + 3] = v.w;
-    }
+  {
+    float *p = S + ((wave >> 1) * 64 + (lane & 31)) * LS + (wave & 1) * 64 + 4 * (lane >> 5);
+#pragma unroll
+    for (int im = 0; im < 2; ++im)
+#pragma unroll
+      for (int in = 0; in < 2; ++in)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) p[in * 32 * LS + im * 32 + 8 * g + e] = -tile.v[im][in][g][e];
   }
   __syncthreads();
   floatx16 zero;
@@ -471,10 +595,10 @@ __device__ __forceinline__ void diag_role(const InvTables &tb, const TileTask &t
     if (wave == 0) {
       const int bad = kfac::chol_inv_32<LS>(S, jb * SB);
       if (lane == 0) {
-        int *pinfo = &tb.info[(int)(t.b_off & 0xffffffffLL)];
-        if (k == 0 && jb == 0) *pinfo = 0;
-        const int col = k * NB + jb * SB + bad - 1;
-        if (bad && col < d && *pinfo == 0) *pinfo = col + 1;
+        int *pinfo = &tb.info[it.caller];
+        if (it.col == 0 && jb == 0) *pinfo = 0;
+        const int col = it.col * NB + jb * SB + bad - 1;
+        if (bad && col < it.core && *pinfo == 0) *pinfo = col + 1;
       }
     }
     __syncthreads();
@@ -516,23 +640,27 @@ __device__ __forceinline__ void diag_role(const InvTables &tb, const TileTask &t
     __syncthreads();
   }
 
-  // ---- outputs
-  // U -> diagonal tile of the workspace, exact zeros below the diagonal
-  {
-    const int c4 = (threadIdx.x & 31) * 4, r0 = threadIdx.x >> 5;
-#pragma unroll 4
-    for (int p = 0; p < NB / 8; ++p) {
-      const int r = r0 + 8 * p;
-      float v[4];
+  // ---- U and U^T as final tiles, exact zeros on the other side of the diagonal
+  float *u_tile = slot_ptr(tb, it.c), *ut_tile = slot_ptr(tb, it.ut);
+#pragma unroll 2
+  for (int ks = 0; ks < NB / 16; ++ks) {
+    const int rb = wave, row = rb * 32 + (lane & 31), c0 = ks * 16 + 8 * (lane >> 5);
+    vuint4 u[3], t[3];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = c4 + e;
-        const bool up = (c / SB > r / SB) || (c / SB == r / SB && c >= r);
-        v[e] = up ? S[r * LS + c] : 0.f;
-      }
-      *reinterpret_cast<float4 *>(tile + r * ld + c4) = make_float4(v[0], v[1], v[2], v[3]);
+    for (int e = 0; e < 4; ++e) {
+      const int c = c0 + 2 * e;
+      split_pair(c >= row ? S[row * LS + c] : 0.f, c + 1 >= row ? S[row * LS + c + 1] : 0.f, *((unsigned *)&u[0] + e),
+                 *((unsigned *)&u[1] + e), *((unsigned *)&u[2] + e));
+      split_pair(c <= row ? S[c * LS + row] : 0.f, c + 1 <= row ? S[(c + 1) * LS + row] : 0.f, *((unsigned *)&t[0] + e),
+                 *((unsigned *)&t[1] + e), *((unsigned *)&t[2] + e));
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      gstore16(u_tile, (unsigned)(frag_off(ks, rb, q) + lane * 16), u[q]);
+      gstore16(ut_tile, (unsigned)(frag_off(ks, rb, q) + lane * 16), t[q]);
     }
   }
+  __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
@@ -548,31 +676,35 @@ __device__ __forceinline__ void diag_role(const InvTables &tb, const TileTask &t
 // as do the last column of the triangular inverse and the last pivot,
 //     w = U l = A^-1 a  (w_i = sum_{k >= i} U(i,k) l_k),   S = alpha - l^T l,
 //     M^-1 = [A^-1 + w w^T / S, -w / S; -w^T / S, 1 / S].
-// These are tile-by-vector products, a few workgroups per step that ride in the
-// launches of the sweep: beside the diagonal tiles of step k the partial sums of
-// sum_{j<k} L(k,j) l_j (chunks of kBorderChunk tiles) and w += U(.,k-1) l_{k-1},
-// beside the panel step l_k itself.  (Forming l = U^T a from the finished inverse
+// These are tile-by-vector products, a few items of the launches of the sweep: in the
+// launch of column k the partial sums of sum_{j<k} L(k+1,j) l_j (chunks of kBorderChunk
+// tiles), l_k itself, which takes the last of its terms, L(k,k-1) l_{k-1}, along, and
+// w += U(.,k-1) l_{k-1}.  (Forming l = U^T a from the finished inverse
 // instead loses a factor of cond(L) in accuracy against the substitution.)  The
 // rank-1 term is added to the accumulators of the final product.
 // ---------------------------------------------------------------------------
 constexpr int kBorderChunk = 6;
-constexpr int kBorderSum = 0;     // part[j] = sum_{c in chunk j} L(i,c) l_c          (i = k, j = chunk)
-constexpr int kBorderSolve = 1;   // l_i = U_ii^T (a_i - sum of the partial vectors)
+constexpr int kBorderSum = 0;     // part[j] = sum_{c in chunk j, c < i - 1} L(i,c) l_c
+constexpr int kBorderSolve = 1;   // l_i = U_ii^T (a_i - sum of the partial vectors - L(i,i-1) l_{i-1})
 constexpr int kBorderW = 2;       // w_i (+)= U(i,j) l_j, the first term (j = i) overwrites
 constexpr int kBorderPivot = 3;   // S = alpha - l^T l in float64, 1 / S, info
 struct BorderTask {
   int s, kind, i, j;
 };
-constexpr int kBorderLdsFloats = NB + NB * 33;
+// chunks of the sum that is owed to l_i (its last term is added where l_i is solved)
+__host__ __device__ constexpr int border_chunks(int i) { return i > 1 ? (i - 2) / kBorderChunk + 1 : 0; }
+constexpr int kBorderLdsFloats = kBorderChunk * NB + NB * 17;
 
-// vectors of a bordered matrix in the workspace: a | l | w | scalars (64) | partial vectors
+// vectors of a bordered matrix in the workspace: a | l | w | scalars (64) | partial vectors of
+// the even and of the odd rows
 struct BorderVecs {
   float *a, *y, *w, *scal, *part;
-  int dc;
+  int dc, nch;
 };
 __device__ __forceinline__ BorderVecs border_vecs(const InvTables &tb, int s) {
   BorderVecs v;
   v.dc = tb.core[s];
+  v.nch = border_chunks(tb.nt[s] - 1);
   v.a = tb.ws + tb.vec_off[s];
   v.y = v.a + v.dc;
   v.w = v.y + v.dc;
@@ -581,85 +713,79 @@ __device__ __forceinline__ BorderVecs border_vecs(const InvTables &tb, int s) {
   return v;
 }
 
-// p[r] += sum_{c in the thread's 4 columns} M[rg * 16 + r][c] x[c] for one NB x NB tile; x in LDS
-__device__ __forceinline__ void border_rows_acc(const float *tile, const float *xs, float (&p)[16]) {
-  const int c4 = (threadIdx.x & 31) * 4, rg = threadIdx.x >> 5;
-  const float4 x = *reinterpret_cast<const float4 *>(xs + c4);
-  const float *m = tile + (rg * 16) * NB + c4;
+// p[r] += sum_{c in the thread's 8 columns} M[rg * 8 + r][c] x[c] for one final tile; x in LDS
+__device__ __forceinline__ void border_rows_acc(const float *tile, const float *xs, float (&p)[8]) {
+  const int c8 = threadIdx.x & 15, rg = threadIdx.x >> 4;
+  float x[8];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const float4 u = *reinterpret_cast<const float4 *>(m + r * NB);
-    p[r] += u.x * x.x + u.y * x.y + u.z * x.z + u.w * x.w;
+  for (int e = 0; e < 8; ++e) x[e] = xs[c8 * 8 + e];
+  const char *m = reinterpret_cast<const char *>(tile) + frag_off(c8 >> 1, rg >> 2, 0) + ((rg & 3) * 8 + (c8 & 1) * 32) * 16;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    vuint4 f[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) f[q] = *reinterpret_cast<const vuint4 *>(m + r * 16 + q * kFragBytes);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      // lo + mid, then + hi: exactly the value that was split
+      const float u0 = (__uint_as_float(f[2][e] << 16) + __uint_as_float(f[1][e] << 16)) + __uint_as_float(f[0][e] << 16);
+      const float u1 = (__uint_as_float(f[2][e] & 0xffff0000u) + __uint_as_float(f[1][e] & 0xffff0000u)) +
+                       __uint_as_float(f[0][e] & 0xffff0000u);
+      p[r] += u0 * x[2 * e] + u1 * x[2 * e + 1];
+    }
   }
 }
-// the row sums of p over the 32 threads of a row group, in a fixed order; valid in threads < NB
-__device__ __forceinline__ float border_rows_reduce(const float (&p)[16], float *red) {
-  const int q = threadIdx.x & 31, rg = threadIdx.x >> 5;
+// the row sums of p over the 16 threads of a row group, in a fixed order; valid in threads < NB
+__device__ __forceinline__ float border_rows_reduce(const float (&p)[8], float *red) {
+  const int q = threadIdx.x & 15, rg = threadIdx.x >> 4;
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < 16; ++r) red[(rg * 16 + r) * 33 + q] = p[r];
+  for (int r = 0; r < 8; ++r) red[(rg * 8 + r) * 17 + q] = p[r];
   __syncthreads();
   float t = 0.f;
   if (threadIdx.x < NB) {
 #pragma unroll
-    for (int i = 0; i < 32; ++i) t += red[threadIdx.x * 33 + i];
+    for (int i = 0; i < 16; ++i) t += red[threadIdx.x * 17 + i];
   }
   return t;
 }
 
+// ends with a barrier
 __device__ __forceinline__ void border_role(const InvTables &tb, const BorderTask t, float *lds) {
-  float *xs = lds;         // NB floats
-  float *red = lds + NB;   // NB x 33
+  float *xs = lds;                        // kBorderChunk x NB
+  float *red = lds + kBorderChunk * NB;   // NB x 17
   const BorderVecs v = border_vecs(tb, t.s);
-  if (t.kind == kBorderSum) {
-    float p[16];
+  float p[8];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) p[r] = 0.f;
-    const int j_end = min((t.j + 1) * kBorderChunk, t.i);
-    for (int j = t.j * kBorderChunk; j < j_end; ++j) {
-      __syncthreads();
-      if (threadIdx.x < NB) xs[threadIdx.x] = v.y[j * NB + threadIdx.x];
-      __syncthreads();
-      border_rows_acc(tile_ptr(tb, t.s, t.i, j), xs, p);
-    }
+  for (int r = 0; r < 8; ++r) p[r] = 0.f;
+  // p += tiles (i, j0 .. j1 - 1) times l (no barrier between the tiles: their loads overlap)
+  auto add_tiles = [&](int i, int j0, int j1) {
+    for (int e = threadIdx.x; e < (j1 - j0) * NB; e += THREADS) xs[e] = v.y[j0 * NB + e];
+    __syncthreads();
+    const float *tile = slot_ptr(tb, tile_slot(tb, t.s, i, j0));
+    for (int j = 0; j < j1 - j0; ++j) border_rows_acc(tile + (size_t)j * kSlotFloats, xs + j * NB, p);
+  };
+  if (t.kind == kBorderSum) {
+    add_tiles(t.i, t.j * kBorderChunk, min((t.j + 1) * kBorderChunk, t.i - 1));
     const float sum = border_rows_reduce(p, red);
-    if (threadIdx.x < NB) v.part[t.j * NB + threadIdx.x] = sum;
+    if (threadIdx.x < NB) v.part[((t.i & 1) * v.nch + t.j) * NB + threadIdx.x] = sum;
   } else if (t.kind == kBorderSolve) {
+    if (t.i > 0) add_tiles(t.i, t.i - 1, t.i);
+    const float last = border_rows_reduce(p, red);
     if (threadIdx.x < NB) {
       float x = v.a[t.i * NB + threadIdx.x];
-      const int nch = (t.i + kBorderChunk - 1) / kBorderChunk;
-      for (int ch = 0; ch < nch; ++ch) x -= v.part[ch * NB + threadIdx.x];
-      xs[threadIdx.x] = x;
+      for (int ch = 0; ch < border_chunks(t.i); ++ch) x -= v.part[((t.i & 1) * v.nch + ch) * NB + threadIdx.x];
+      xs[threadIdx.x] = x - last;
     }
     __syncthreads();
-    // l_k[c] = sum_r U_kk[r][c] x[r]
-    const int c4 = (threadIdx.x & 31) * 4, rg = threadIdx.x >> 5;
-    const float *U = tile_ptr(tb, t.s, t.i, t.i) + (rg * 16) * NB + c4;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    // l_k[c] = sum_r U_kk[r][c] x[r]: rows of U_kk^T
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float4 u = *reinterpret_cast<const float4 *>(U + r * NB);
-      const float xv = xs[rg * 16 + r];
-      acc.x += u.x * xv;
-      acc.y += u.y * xv;
-      acc.z += u.z * xv;
-      acc.w += u.w * xv;
-    }
-    *reinterpret_cast<float4 *>(red + rg * NB + c4) = acc;
-    __syncthreads();
-    if (threadIdx.x < NB) {
-      float l = 0.f;
-#pragma unroll
-      for (int g = 0; g < 8; ++g) l += red[g * NB + threadIdx.x];
-      v.y[t.i * NB + threadIdx.x] = l;
-    }
+    for (int r = 0; r < 8; ++r) p[r] = 0.f;
+    border_rows_acc(slot_ptr(tb, tb.ut0 + 2 * t.s + (t.i & 1)), xs, p);
+    const float l = border_rows_reduce(p, red);
+    if (threadIdx.x < NB) v.y[t.i * NB + threadIdx.x] = l;
   } else if (t.kind == kBorderW) {
-    float p[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) p[r] = 0.f;
-    if (threadIdx.x < NB) xs[threadIdx.x] = v.y[t.j * NB + threadIdx.x];
-    __syncthreads();
-    border_rows_acc(tile_ptr(tb, t.s, t.i, t.j), xs, p);
+    add_tiles(t.i, t.j, t.j + 1);
     const float sum = border_rows_reduce(p, red);
     if (threadIdx.x < NB) {
       float *w = v.w + t.i * NB + threadIdx.x;
@@ -683,6 +809,7 @@ __device__ __forceinline__ void border_role(const InvTables &tb, const BorderTas
       if (!(S > 0.0) && *pinfo == 0) *pinfo = tb.dim[t.s];
     }
   }
+  __syncthreads();
 }
 
 // the border tasks that follow the last step of the sweep
@@ -692,106 +819,195 @@ __global__ __launch_bounds__(THREADS) void border_kernel(InvTables tb, int btask
 }
 
 // ---------------------------------------------------------------------------
-// panel and update: 128x128x128 tile products through the shared main loop
+// the launches
 // ---------------------------------------------------------------------------
-// M(x,k) = M(x,k) W^T = M(x,k) U_kk in place for every x != k; the operand
-// W^T is the diagonal tile itself, read transposed.
-__global__ __launch_bounds__(THREADS, 2) void panel_kernel(InvTables tb, int task0, int ntask, int btask0) {
-  extern __shared__ float lds[];
-  if ((int)blockIdx.x >= ntask) {   // bordered matrices: l_k of this step
-    border_role(tb, tb.btasks[btask0 + blockIdx.x - ntask], lds);
-    return;
+__device__ __forceinline__ SweepItem load_item(const SweepItem *p) {
+  SweepItem it;
+  it.kind = uniform(p->kind);
+  it.c = uniform(p->c);
+  it.a = uniform(p->a);
+  it.b = uniform(p->b);
+  it.blocks = uniform(p->blocks);
+  it.first = uniform(p->first);
+  it.ut = uniform(p->ut);
+  it.col = uniform(p->col);
+  it.caller = uniform(p->caller);
+  it.core = uniform(p->core);
+  it.border = uniform(p->border);
+  it.pad = 0;
+  return it;
+}
+
+// One step of the sweep: every workgroup runs its list of items.  Behind an update the loads
+// of the next item's first panels are already in flight.
+__global__ __launch_bounds__(THREADS, 1) void sweep_kernel(InvTables tb, int range0) {
+  extern __shared__ char lds[];
+  const int2 range = tb.ranges[range0 + blockIdx.x];
+  const int end = uniform(range.y);
+  for (int i = uniform(range.x); i < end; ++i) {
+    SweepItem it = load_item(tb.items + i);
+    if (it.kind == kItemBorder) {
+      border_role(tb, tb.btasks[it.border], reinterpret_cast<float *>(lds));
+      continue;
+    }
+    TileRegs c;
+    if (it.first)
+      tile_zero(c);
+    else
+      tile_load(wave_uniform(slot_ptr(tb, it.c)), c);
+    if (it.blocks > 0) {
+      Cursor cu;
+      cu.a = wave_uniform(slot_ptr(tb, it.a));
+      cu.b = wave_uniform(slot_ptr(tb, it.b));
+      cu.left = it.blocks * 4;
+      Panels r[2];
+      product_start(cu, r, lds);
+      for (;;) {   // this item and, as long as it is an update, those behind it
+        const SweepItem next = load_item(tb.items + (i + 1 < end ? i + 1 : i));
+        const bool ahead = it.kind == kItemUpdate && i + 1 < end && next.kind != kItemBorder && next.blocks > 0;
+        cu.next_a = wave_uniform(slot_ptr(tb, next.a));
+        cu.next_b = wave_uniform(slot_ptr(tb, next.b));
+        cu.next_left = ahead ? next.blocks * 4 : 0;
+        const float *next_tile = wave_uniform(slot_ptr(tb, next.c));
+        floatx16 acc[2][2];
+        tile_to_acc(c, acc);
+        product_run(it.blocks, cu, r, lds, acc, [&]() {
+          if (ahead) {
+            if (next.first)
+              tile_zero(c);
+            else
+              tile_load(next_tile, c);
+          }
+        });
+        if (it.kind != kItemUpdate) {
+          tile_from_acc(c, acc);
+          break;
+        }
+        TileRegs done;
+        tile_from_acc(done, acc);
+        tile_store(const_cast<float *>(wave_uniform(slot_ptr(tb, it.c))), done);
+        if (!ahead) break;
+        it = load_item(tb.items + ++i);
+      }
+    }
+    if (it.kind == kItemPanel)
+      panel_role(tb, it, c, lds);
+    else if (it.kind == kItemDiag)
+      diag_role(tb, it, c, reinterpret_cast<float *>(lds));
   }
-  const TileTask t = tb.tasks[task0 + blockIdx.x];
-  float *tile = tb.ws + t.c_off;
-  floatx16 acc[2][2];
-  zero_acc<2, 2>(acc);
-  tile_mainloop<false, 2>(OperandRows{tile}, OperandCols{tb.ws + t.b_off}, NB, lds, acc);
-  for_each_acc<2, 2>(acc, [&](int rr, int cc, float v) { tile[rr * NB + cc] = v; });
 }
 
-// One task of (*): tile (a,b) of a matrix, products over the block columns of
-// the launch clipped to the tile's own range (resolved in the task record).  The
-// accumulators start from -C, so the tile is read while the first operand panels
-// are in flight and the epilogue is a plain store.  An upper tile whose row lies
-// inside the source columns receives its first product here and is overwritten
-// (it holds stale data): kFirst.
-template <int D>
-__device__ __forceinline__ void update_role(const InvTables &tb, const TileTask &t, float *lds) {
-  float *C = const_cast<float *>(wave_uniform(tb.ws + t.c_off));
-  floatx16 acc[2][2];
-  if (t.flags & kFirst)
-    zero_acc<2, 2>(acc);
-  else
-    load_neg_tile(C, acc);
-  const OperandRows la{tb.ws + t.a_off}, lb{tb.ws + t.b_off};
-  if (t.flags & kSame)
-    tile_mainloop<true, D>(la, lb, t.K, lds, acc);
-  else
-    tile_mainloop<false, D>(la, lb, t.K, lds, acc);
-  store_neg_tile(C, acc);
-}
-
-// One workgroup per active matrix: the diagonal tile of sweep step `step`
-// (after it has received the products of columns [step0, step1]).  This is the
-// serial part of the sweep, and most of it is one wave's dependent chain of
-// vector instructions.  It runs at a third of its speed when its waves share
-// their SIMDs with those of a trailing update (measured: 20 us against 60-80 us
-// for the 128 x 128 factorisation), so the kernel asks for more LDS than fits
-// beside a workgroup of the trailing update (kDiagKernelLds): it waits for a CU
-// without one, at most the few microseconds until the next of them retires, and
-// keeps the following ones away from that CU while it runs.
-__global__ __launch_bounds__(THREADS, 2) void diag_kernel(InvTables tb, int task0, int ntask, int btask0) {
-  extern __shared__ float lds[];
-  if ((int)blockIdx.x >= ntask) {   // bordered matrices: the vector work this step can start with
-    border_role(tb, tb.btasks[btask0 + blockIdx.x - ntask], lds);
-    return;
+// The finished tile (I, J), I >= J, of the inverse and its mirror image written to C
+// (leading dimension d, rows and columns below dt): the whole tile is
+// laid out in LDS (128 x 129 floats), then every thread stores 16 bytes at
+// a time (at float granularity: rows of an odd-sized matrix do not start on
+// 16-byte boundaries), rows of the tile and rows of the mirrored tile alike.
+constexpr int kWholeTileLdsBytes = NB * LS * (int)sizeof(float);
+__device__ __forceinline__ void write_whole_tile(const floatx16 (&acc)[2][2], float *lds, int I, int J, int dt,
+                                                 int d, float *__restrict__ C) {
+  typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+  constexpr int LD = LS;
+  {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    float *p = lds + ((wave >> 1) * 64 + (lane & 31)) * LD + (wave & 1) * 64 + 4 * (lane >> 5);
+#pragma unroll
+    for (int im = 0; im < 2; ++im)
+#pragma unroll
+      for (int in = 0; in < 2; ++in)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) p[in * 32 * LD + im * 32 + 8 * (v >> 2) + (v & 3)] = acc[im][in][v];
   }
-  const TileTask t = tb.tasks[task0 + blockIdx.x];
-  diag_role(tb, t, lds);
-}
-
-// A list of tasks of (*): the column updates of a sweep step (the tiles the next
-// panel step reads; beside the diagonal kernel) or the part of a trailing update
-// that the next group's sweep does not read.
-__global__ __launch_bounds__(THREADS, 2) void update_kernel(InvTables tb, int task0) {
-  extern __shared__ float lds[];
-  const TileTask t = tb.tasks[task0 + blockIdx.x];
-  update_role<2>(tb, t, lds);
+  __syncthreads();
+  const int q = (threadIdx.x & 31) * 4;    // four columns
+  const int r0 = threadIdx.x >> 5;         // 8 rows per pass
+  const int row0 = I * 128, col0 = J * 128;
+  const bool diag = I == J;
+#pragma unroll 4
+  for (int p = 0; p < 16; ++p) {
+    const int lr = r0 + 8 * p;
+    const int r = row0 + lr, c = col0 + q;
+    if (r >= dt) continue;
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (!diag || q + e <= lr) ? lds[lr * LD + q + e] : lds[(q + e) * LD + lr];
+    float *dst = C + (long long)r * d + c;
+    if (c + 3 < dt) {
+      floatx4u o;
+      o.x = v[0];
+      o.y = v[1];
+      o.z = v[2];
+      o.w = v[3];
+      *reinterpret_cast<floatx4u *>(dst) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < dt) dst[e] = v[e];
+    }
+  }
+  if (diag) return;
+  // mirrored tile (J, I): its row lr is column lr of the tile
+#pragma unroll 4
+  for (int p = 0; p < 16; ++p) {
+    const int lr = r0 + 8 * p;
+    const int r = col0 + lr, c = row0 + q;
+    if (r >= dt) continue;
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = lds[(q + e) * LD + lr];
+    float *dst = C + (long long)r * d + c;
+    if (c + 3 < dt) {
+      floatx4u o;
+      o.x = v[0];
+      o.y = v[1];
+      o.z = v[2];
+      o.w = v[3];
+      *reinterpret_cast<floatx4u *>(dst) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (c + e < dt) dst[e] = v[e];
+    }
+  }
 }
 
 // out(i,j) = sum_{k >= i} U(i,k) U(j,k)^T for i >= j, written with its mirror.
 // One task per tile; the table deals whole tile rows to XCDs (see the plan).
-__global__ __launch_bounds__(THREADS, 2) void lauum_kernel(InvTables tb, int task0) {
-  extern __shared__ float lds[];
+__global__ __launch_bounds__(THREADS, 1) void lauum_kernel(InvTables tb, int task0) {
+  extern __shared__ char lds[];
   const TileTask t = tb.tasks[task0 + blockIdx.x];
   if (t.K == 0) return;   // padding of an XCD's shorter list
-  const int s = (int)t.c_off;
-  const int I = t.flags & 0xffff, J = t.flags >> 16;
+  const int s = uniform((int)t.c_off);
+  const int I = uniform(t.flags) & 0xffff, J = uniform(t.flags) >> 16;
   const int d = tb.dim[s], dc = tb.core[s];
   const long long vo = tb.vec_off[s];
   float *out = tb.out[s];
-  const OperandRows la{tb.ws + t.a_off}, lb{tb.ws + t.b_off};
   floatx16 acc[2][2];
-  zero_acc<2, 2>(acc);
-  if (I == J)
-    tile_mainloop<true, 4>(la, lb, t.K, lds, acc);
-  else
-    tile_mainloop<false, 4>(la, lb, t.K, lds, acc);
+  {
+    Cursor cu;
+    cu.a = wave_uniform(slot_ptr(tb, (int)(t.a_off / (NB * NB))));
+    cu.b = wave_uniform(slot_ptr(tb, (int)(t.b_off / (NB * NB))));
+    cu.left = uniform(t.K) / NB * 4;
+    cu.next_a = cu.next_b = nullptr;
+    cu.next_left = 0;
+    Panels r[2];
+    zero_acc<2, 2>(acc);
+    product_start(cu, r, lds);
+    product_run(uniform(t.K) / NB, cu, r, lds, acc, []() {});
+  }
   if (vo >= 0) {
     // bordered matrix: + w w^T / S on the leading block, -w / S in the last row and column
     const BorderVecs bv = border_vecs(tb, s);
     const float sigma = bv.scal[2];
     const float *wi = bv.w + I * NB, *wj = bv.w + J * NB;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int im = 0; im < 2; ++im)
 #pragma unroll
       for (int in = 0; in < 2; ++in)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-          const int row = ((wave >> 1) * 2 + im) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-          const int col = ((wave & 1) * 2 + in) * 32 + (lane & 31);
+          const int row = ((wave >> 1) * 2 + in) * 32 + (lane & 31);
+          const int col = ((wave & 1) * 2 + im) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
           acc[im][in][v] += sigma * wi[row] * wj[col];
         }
     if (I == J && threadIdx.x < NB) {
@@ -801,27 +1017,14 @@ __global__ __launch_bounds__(THREADS, 2) void lauum_kernel(InvTables tb, int tas
       if (I == 0 && threadIdx.x == 0) out[(long long)(d - 1) * d + d - 1] = sigma;
     }
   }
-  // through LDS, so that the mirror is written in row segments too
-  static_assert(kWholeTileLdsFloats <= kTileLdsFloats, "the tile must fit the panels' LDS");
-  write_whole_tile(acc, lds, I, J, dc, d, out);
+  static_assert(kWholeTileLdsBytes <= kTileLdsBytes, "the tile must fit the panels' LDS");
+  write_whole_tile(acc, reinterpret_cast<float *>(lds), I, J, dc, d, out);
 }
 
-// Dynamic LDS.  The trailing update ("rest") asks for 81 KB although it uses 74:
-// then one of its workgroups fits a CU, not two, and a column or panel workgroup
-// of the sweep (74 KB) always finds room beside it instead of queueing behind
-// the rest for a slot.  The diagonal kernel needs 77 KB (its working tile and
-// three private blocks: at most three waves are busy in a pass of the triangular
-// inverse) and asks for 80: two of its workgroups share a CU, but none shares
-// one with a workgroup of the rest.
-constexpr size_t kDiagLds = (size_t)(NB * LS + 3 * SB * PS) * sizeof(float);
-constexpr size_t kRestLdsBytes = 81 * 1024;
-constexpr size_t kDiagKernelLds = 80 * 1024;
-static_assert(kDiagLds <= kDiagKernelLds && kTileLdsBytes <= kDiagKernelLds, "diagonal role's LDS");
-static_assert(2 * kDiagKernelLds <= 160 * 1024 && kDiagKernelLds + kRestLdsBytes > 160 * 1024 &&
-                  kDiagKernelLds + kTileLdsBytes <= 160 * 1024,
-              "a diagonal workgroup shares a CU with another or with a column workgroup, not with the rest");
-static_assert(2 * kRestLdsBytes > 160 * 1024 && kRestLdsBytes + kTileLdsBytes <= 160 * 1024,
-              "one rest workgroup per CU, with room for a column or panel workgroup");
+constexpr int kDiagLdsBytes = (NB * LS + 3 * SB * PS) * (int)sizeof(float);
+static_assert(kDiagLdsBytes <= kTileLdsBytes && kBorderLdsFloats * (int)sizeof(float) <= kTileLdsBytes,
+              "the roles of a sweep workgroup share its LDS");
+static_assert(2 * kTileLdsBytes > 160 * 1024, "one workgroup per CU: the diagonal tiles have their SIMDs to themselves");
 
 }  // namespace
 
@@ -839,39 +1042,15 @@ struct kfac_inverse_plan {
   std::vector<int> nactive;        // per step
   std::vector<int> panel_total;    // per step
   std::vector<int> diag_task0, panel_task0;   // per step: first record of the launch
-  // per step: the update tasks that share the launch with the diagonal tiles:
-  // inside a group the left-looking update of column k, on a group's first
-  // column the previous group's trailing update of this group's columns
+  // per step: the products that column k is owed inside a group, and on a group's first
+  // column those of the previous group for all columns of this group
   std::vector<UpdateLaunch> with_diag;
   // per step, set on the last column of a group: its trailing update of
   // everything right of the next group
   std::vector<UpdateLaunch> rest;
-  // The rest of a trailing update touches nothing the next group's sweep needs,
-  // so it runs on a second stream beside that sweep.
-  bool lookahead = true;
-  // Under stream capture the fork onto `side` is only safe from the stream the
-  // capture began on (a fork of a forked stream has crashed the runtime), which
-  // the library cannot find out by itself: the caller says so.
+  // a captured graph holds one stream's launches whatever this says (kept for the ABI)
   bool capture_origin = false;
-  size_t rest_lds = 0;
-  hipStream_t side = nullptr;
-  // The column updates of a step are independent of its diagonal tiles: they run
-  // on a third stream beside the diagonal kernel.
-  hipStream_t col = nullptr;
-  std::vector<hipEvent_t> ev_main, ev_side, ev_fork, ev_col;   // per step
-  // The matrices that join the sweep at its first step are copied in on the caller's
-  // stream; the others (they join later) on the side stream, beside the first step.
-  int first_tiles = 0;
-  hipEvent_t ev_copy_fork = nullptr, ev_copy = nullptr;
-  ~kfac_inverse_plan() {
-    for (hipEvent_t e : {ev_copy_fork, ev_copy})
-      if (e) (void)hipEventDestroy(e);
-    for (auto *v : {&ev_main, &ev_side, &ev_fork, &ev_col})
-      for (hipEvent_t e : *v)
-        if (e) (void)hipEventDestroy(e);
-    if (side) (void)hipStreamDestroy(side);
-    if (col) (void)hipStreamDestroy(col);
-  }
+  int first_tiles = 0;             // copy-in: tiles of the matrices that join at the first step
   int total_tiles = 0;
   int lauum_task0 = 0, lauum_count = 0;
   // bordered matrices: their vector tasks per step (beside the diagonal tiles, beside the
@@ -880,9 +1059,14 @@ struct kfac_inverse_plan {
   std::vector<int> bdiag_task0, bdiag_count, bpanel_task0, bpanel_count;
   int bfinal_task0 = 0, bfinal_count = 0;
   kfac::DevTable d_core, d_orig, d_vec, d_btasks;
-  size_t ws_floats = 0;            // padded matrices
+  // the launches of the sweep (the first factors the first diagonal tiles): workgroups and
+  // their item ranges
+  std::vector<int> sweep_range0, sweep_count;
+  kfac::DevTable d_items, d_ranges;
+  int ut0 = 0;                     // first slot of the U_kk^T buffers
+  size_t ws_floats = 0;            // slots and border vectors
   std::vector<const void *> in_sorted, out_sorted;
-  kfac::DevTable d_in, d_out, d_dim, d_nt, d_off, d_tile, d_tile_owner, d_tasks;
+  kfac::DevTable d_in, d_out, d_dim, d_nt, d_off, d_tile_owner, d_tasks;
   bool attr_set = false;
 };
 
@@ -907,6 +1091,92 @@ void append_tasks(std::vector<T> &table, const std::vector<T> &natural) {
   table.insert(table.end(), dealt.begin(), dealt.end());
 }
 
+// The sweep as launches of items.  Costs are in units of one 128 x 128 x 128 product on a CU
+// (about 3 us); they only balance the workgroups' lists.
+constexpr int kSweepWorkgroups = 256;   // one per CU
+// Side of the blocks of tiles that are worked on together.  The 32 workgroups of an XCD read 12 operand
+// runs for 36 tiles instead of 33 for 32, through an L2 of 4 MB.
+constexpr int kBlock = 6;
+double item_cost(const SweepItem &it) {
+  switch (it.kind) {
+    case kItemUpdate: return 0.6 + it.blocks;
+    case kItemPanel: return 2.2 + it.blocks;
+    case kItemDiag: return 8.0 + it.blocks;
+    default: return it.blocks;   // about a third of a unit per tile and one for the rest
+  }
+}
+
+struct SweepBuilder {
+  std::vector<SweepItem> items;
+  std::vector<int2> ranges;
+
+  // One launch.  `chains`: items that one workgroup runs in order, the longest of the launch, each to a
+  // workgroup of its own as long as there are enough; `list`: independent items in their natural
+  // order, in which neighbours share operand runs.  Workgroup i runs on XCD i % 8: every XCD gets a
+  // contiguous run of the list, as much as its workgroups have room for, and inside an XCD the least
+  // loaded workgroup takes the next item.
+  // `vectors`: border items, few tiles to read and nothing to share.
+  void launch(const std::vector<std::vector<SweepItem>> &chains, const std::vector<SweepItem> &list,
+              const std::vector<SweepItem> &vectors, int *range0, int *count) {
+    const size_t total = chains.size() + list.size() + vectors.size();
+    const int n = (int)std::min<size_t>(kSweepWorkgroups, total);
+    *range0 = (int)ranges.size();
+    *count = n;
+    if (n == 0) return;
+    std::vector<std::vector<SweepItem>> mine(n);
+    std::vector<double> load(n, 0.0);
+    double sum = 0.0;
+    for (size_t i = 0; i < chains.size(); ++i) {
+      const int w = (int)(i % n);
+      for (const SweepItem &it : chains[i]) {
+        mine[w].push_back(it);
+        load[w] += item_cost(it);
+      }
+    }
+    for (size_t i = 0; i < vectors.size(); ++i) {
+      const int w = (int)((chains.size() + i) % n);
+      mine[w].push_back(vectors[i]);
+      load[w] += item_cost(vectors[i]);
+    }
+    for (const SweepItem &it : list) sum += item_cost(it);
+    for (int w = 0; w < n; ++w) sum += load[w];
+    if (total == (size_t)n) {   // one each
+      for (size_t i = 0; i < list.size(); ++i) mine[chains.size() + vectors.size() + i].push_back(list[i]);
+    } else {
+      deal(list, mine, load, sum);
+    }
+    for (int w = 0; w < n; ++w) {
+      const int first = (int)items.size();
+      items.insert(items.end(), mine[w].begin(), mine[w].end());
+      ranges.push_back(make_int2(first, (int)items.size()));
+    }
+  }
+
+  static void deal(const std::vector<SweepItem> &list, std::vector<std::vector<SweepItem>> &mine,
+                   std::vector<double> &load, double sum) {
+    const int n = (int)mine.size();
+    // what each XCD has room for below the common level
+    const int nx = std::min(8, n);
+    double room[8] = {0, 0, 0, 0, 0, 0, 0, 0}, all = 0.0, list_sum = 0.0;
+    for (const SweepItem &it : list) list_sum += item_cost(it);
+    for (int w = 0; w < n; ++w) room[w % 8] += std::max(0.0, sum / n - load[w]);
+    for (int x = 0; x < nx; ++x) all += room[x];
+    size_t at = 0;
+    double done = 0.0, upto = 0.0;
+    for (int x = 0; x < nx; ++x) {
+      upto += all > 0.0 ? list_sum * room[x] / all : list_sum / nx;
+      while (at < list.size() && (x == nx - 1 || done + 0.5 * item_cost(list[at]) <= upto)) {
+        int w = x;
+        for (int v = x; v < n; v += 8)
+          if (load[v] < load[w]) w = v;
+        mine[w].push_back(list[at]);
+        load[w] += item_cost(list[at]);
+        done += item_cost(list[at++]);
+      }
+    }
+  }
+};
+
 }  // namespace
 
 extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
@@ -929,6 +1199,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
   std::stable_sort(p->order.begin(), p->order.end(),
                    [&](int a, int b) { return dims[a] > dims[b]; });
   std::vector<int> dim(count), tile_cs(count + 1, 0), panel_cs(count + 1, 0);
+  size_t slots = 0;
   std::vector<long long> off(count);
   p->nt.resize(count);
   size_t total = 0;
@@ -945,18 +1216,25 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
     p->nt[s] = T;
     off[s] = (long long)total;
     total += (size_t)T * NB * T * NB;
+    slots += (size_t)T * T;
     tile_cs[s + 1] = tile_cs[s] + T * (T + 1) / 2;
     panel_cs[s + 1] = panel_cs[s] + (T - 1);
   }
+  if (slots + 2 * (size_t)count > 0x7fffffffu) {
+    delete p;
+    return kfac::fail(KFAC_EINVAL, "too many matrices: %zu tiles", slots);
+  }
+  p->ut0 = (int)slots;
+  slots += 2 * (size_t)count;
+  p->ws_floats = slots * kSlotFloats;
   for (int s = 0; s < count; ++s) {
     if (core[s] == dim[s]) continue;
-    vec_off[s] = (long long)total;
-    const int nch = (p->nt[s] - 1) / kBorderChunk + 1;
-    total += (size_t)3 * core[s] + 64 + (size_t)nch * NB;
+    vec_off[s] = (long long)p->ws_floats;
+    p->ws_floats += (size_t)3 * core[s] + 64 + (size_t)2 * border_chunks(p->nt[s] - 1) * NB;
+    p->ws_floats = (p->ws_floats + 63) / 64 * 64;
     border_slots.push_back(s);
   }
   p->nborder = (int)border_slots.size();
-  p->ws_floats = total;
   p->total_tiles = tile_cs[count];
   p->first_tiles = tile_cs[count];   // set once the steps are known
   // copy-in: the lower tiles of every matrix in row-major order, slot by slot
@@ -970,16 +1248,9 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
   std::vector<int2> natural;
   p->with_diag.resize(p->max_t);
   p->rest.resize(p->max_t);
-  p->lookahead = kfac::option_int(kfac::kOptInverseLookahead, 1) != 0;
-  // The rest asks for more LDS than it uses, 81 KB: then one of its workgroups
-  // fits a CU, not two, and a step or panel workgroup always finds room beside
-  // it instead of queueing behind the rest for a slot (measured: the rest alone
-  // loses 14 %, the sweep as a whole gains).  Option inverse_rest_lds overrides.
-  p->rest_lds = kRestLdsBytes;
-  {
-    const long v = (long)kfac::option_value(kfac::kOptInverseRestLds, 0.0);
-    if (v >= (long)kTileLdsBytes && v <= 160 * 1024) p->rest_lds = (size_t)v;
-  }
+  // option inverse_lookahead = 0: a trailing update is one launch's work instead of being spread over
+  // the next group's launches
+  const bool lookahead = kfac::option_int(kfac::kOptInverseLookahead, 1) != 0;
   auto pack = [](int s, int a, int b) { return make_int2(s, a | (b << 16)); };
   // Matrix s joins the sweep at step shift[s] and runs nt[s] steps.  Aligning
   // the ends (shift = max_t - nt) puts the short sweeps of the small matrices
@@ -993,16 +1264,15 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
   std::vector<int> shift(count);
   for (int s = 0; s < count; ++s) shift[s] = (p->max_t - p->nt[s]) * align / 100;
   std::vector<BorderTask> btasks;
-  // step g, bordered matrix s at its block column k = g - shift: beside the diagonal tiles the
-  // chunks of sum_{j<k} L(k,j) l_j and w_i (+)= U(i,k-1) l_{k-1} (k = nt: only the latter);
-  // beside the panel step l_k
+  // step g, bordered matrix s at its block column k = g - shift: the chunks of sum_{j<k} L(k+1,j) l_j
+  // for the next l, w_i (+)= U(i,k-1) l_{k-1} (k = nt: only that), and l_k itself
   for (int g = 0; g <= p->max_t; ++g) {
     const int first = (int)btasks.size();
     for (int s : border_slots) {
       const int k = g - shift[s], T = p->nt[s];
-      if (k < 1 || k > T) continue;
-      if (k < T)
-        for (int ch = 0; ch * kBorderChunk < k; ++ch) btasks.push_back(BorderTask{s, kBorderSum, k, ch});
+      if (k < 0 || k > T) continue;
+      if (k + 1 < T)
+        for (int ch = 0; ch < border_chunks(k + 1); ++ch) btasks.push_back(BorderTask{s, kBorderSum, k + 1, ch});
       for (int i = 0; i < k; ++i) btasks.push_back(BorderTask{s, kBorderW, i, k - 1});
     }
     if (g < p->max_t) {
@@ -1071,6 +1341,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
         for (int b = c_lo; b <= c_hi; ++b) tail.push_back(pack(s, a, b));
     }
   };
+  std::vector<std::vector<TileTask>> column_list(p->max_t), rest_list(p->max_t);   // natural order
   for (int g = 0; g < p->max_t; ++g) {
     // active matrices: shift <= g < shift + nt; a prefix of the sorted order
     // (shift grows and shift + nt shrinks with the slot number)
@@ -1103,8 +1374,13 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
     }
     w.task0 = (int)tasks.size();
     w.count = (int)(natural.size() + tail.size());
-    append_tasks(tasks, resolve(natural, w.k0, w.k1));
-    append_tasks(tasks, resolve(tail, w.k0, w.k1));
+    column_list[g] = resolve(natural, w.k0, w.k1);
+    append_tasks(tasks, column_list[g]);
+    {
+      const std::vector<TileTask> t = resolve(tail, w.k0, w.k1);
+      append_tasks(tasks, t);
+      column_list[g].insert(column_list[g].end(), t.begin(), t.end());
+    }
     // the diagonal tiles of the step, which take the same columns' products themselves
     p->diag_task0.push_back((int)tasks.size());
     for (int s = 0; s < na; ++s) {
@@ -1145,47 +1421,227 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       u.count = (int)(natural.size() + tail.size());
       u.k0 = g0;
       u.k1 = g1;
-      append_tasks(tasks, resolve(natural, u.k0, u.k1));
-      append_tasks(tasks, resolve(tail, u.k0, u.k1));
+      rest_list[g] = resolve(natural, u.k0, u.k1);
+      append_tasks(tasks, rest_list[g]);
+      const std::vector<TileTask> t = resolve(tail, u.k0, u.k1);
+      append_tasks(tasks, t);
+      rest_list[g].insert(rest_list[g].end(), t.begin(), t.end());
     }
   }
-  // Final products out(I,J) = sum_k U(I,k) U(J,k)^T: the I + 1 tiles of tile row I
-  // all read the row U(I, I..T-1).  A whole row goes to one XCD (workgroup i of a
-  // launch runs on XCD i % 8), so that the row stays in that XCD's L2 while its
-  // tiles stream the U(J, .) rows; rows are dealt longest first to the XCD with
-  // the least work, and each XCD runs its long-K rows first.
+  // The launches.  Launch g + 1 is step g: its panel tasks, each behind the column's product for the
+  // same tile; for every matrix the tile below the diagonal and the next diagonal tile as one
+  // workgroup's chain; the step's other column products, the vector tasks and a share of the trailing
+  // update before.  (Launch 0: the first diagonal tiles.)
+  SweepBuilder sweep;
   {
-    struct Row { int s, I; double cost; };
-    std::vector<Row> rows;
+    auto slot_of = [](long long o) { return (int)(o / (NB * NB)); };
+    auto update_item = [&](const TileTask &t) {
+      SweepItem it = {};
+      it.kind = kItemUpdate;
+      it.c = slot_of(t.c_off);
+      it.a = slot_of(t.a_off);
+      it.b = slot_of(t.b_off);
+      it.blocks = t.K / NB;
+      it.first = (t.flags & kFirst) != 0;
+      return it;
+    };
+    const int nslots = p->ut0;
+    auto slot_matrix = [&](int c) {   // a matrix's slots are contiguous
+      return (int)(std::upper_bound(off.begin(), off.end(), (long long)c * (NB * NB)) - off.begin()) - 1;
+    };
+    std::vector<int> owed(nslots, -1);               // slot -> index in the step's column list
+    std::vector<std::vector<SweepItem>> rest(p->max_t + 1);   // trailing updates by step
+    // trailing products that only the chain of a diagonal tile can apply (groups of one column)
+    std::vector<int> chain_rest(nslots, -1);
+    std::vector<TileTask> chain_rest_tasks;
+    std::vector<SweepItem> list, vectors;
+    std::vector<std::vector<SweepItem>> chains;
+    // tiles that share operand runs follow each other: blocks of kBlock x kBlock tiles of a matrix
+    auto sort_blocks = [&](std::vector<SweepItem> &v) {
+      std::vector<std::pair<unsigned long long, int>> key(v.size());
+      for (size_t i = 0; i < v.size(); ++i) {
+        const int s = slot_matrix(v[i].c), at = v[i].c - slot_of(off[s]), I = at / p->nt[s], J = at % p->nt[s];
+        key[i] = {((unsigned long long)s << 40) | ((unsigned long long)(I / kBlock) << 28) |
+                      ((unsigned long long)(J / kBlock) << 16) | (I % kBlock * kBlock + J % kBlock),
+                  (int)i};
+      }
+      std::sort(key.begin(), key.end());
+      std::vector<SweepItem> out;
+      out.reserve(v.size());
+      for (const auto &k : key) out.push_back(v[k.second]);
+      v.swap(out);
+    };
+    for (int g = -1; g < p->max_t; ++g) {
+      list.clear();
+      vectors.clear();
+      chains.clear();
+      std::vector<char> taken;
+      if (g >= 0) {
+        const std::vector<TileTask> &col = column_list[g];
+        taken.assign(col.size(), 0);
+        for (size_t i = 0; i < col.size(); ++i) owed[slot_of(col[i].c_off)] = (int)i;
+      }
+      auto take = [&](int slot) -> const TileTask * {
+        if (g < 0 || owed[slot] < 0) return nullptr;
+        taken[owed[slot]] = 1;
+        return &column_list[g][owed[slot]];
+      };
+      // the chains: matrices with a diagonal tile in step g + 1
+      std::vector<int> chain_of(count, -1);
+      if (g + 1 < p->max_t)
+        for (int i = 0; i < p->nactive[g + 1]; ++i) {
+          const TileTask &t = tasks[p->diag_task0[g + 1] + i];
+          SweepItem it = {};
+          it.kind = kItemDiag;
+          it.c = slot_of(t.c_off);
+          it.a = slot_of(t.a_off);
+          it.blocks = t.K / NB;
+          // products listed for this tile in this step: the same run, further left
+          const TileTask *pre = take(it.c);
+          if (pre) {
+            it.a = slot_of(pre->a_off);
+            it.blocks += pre->K / NB;
+          }
+          if (chain_rest[it.c] >= 0) {
+            const TileTask &r = chain_rest_tasks[chain_rest[it.c]];
+            it.a = slot_of(r.a_off);
+            it.blocks += r.K / NB;
+          }
+          it.b = it.a;
+          it.col = t.flags;
+          it.caller = (int)(t.b_off & 0xffffffffLL);
+          it.core = (int)(t.b_off >> 32);
+          it.ut = p->ut0 + 2 * i + (it.col & 1);
+          chain_of[i] = (int)chains.size();
+          chains.push_back({it});
+        }
+      if (g >= 0) {
+        const int na = p->nactive[g];
+        size_t at = p->panel_task0[g];
+        for (int s = 0; s < na; ++s) {
+          const int k = g - shift[s];
+          for (int x = 0; x < p->nt[s]; ++x) {
+            if (x == k) continue;
+            const TileTask &t = tasks[at++];
+            SweepItem it = {};
+            it.kind = kItemPanel;
+            it.c = it.a = it.b = slot_of(t.c_off);
+            it.ut = p->ut0 + 2 * s + (k & 1);
+            if (const TileTask *u = take(it.c)) {
+              it.a = slot_of(u->a_off);
+              it.b = slot_of(u->b_off);
+              it.blocks = u->K / NB;
+              it.first = (u->flags & kFirst) != 0;
+            }
+            if (x == k + 1)
+              chains[chain_of[s]].insert(chains[chain_of[s]].begin(), it);
+            else
+              list.push_back(it);
+          }
+        }
+        for (size_t i = 0; i < column_list[g].size(); ++i)
+          if (!taken[i]) list.push_back(update_item(column_list[g][i]));
+        for (const TileTask &t : column_list[g]) owed[slot_of(t.c_off)] = -1;
+        list.insert(list.end(), rest[g].begin(), rest[g].end());
+        rest[g].clear();
+        for (int pass = 0; pass < 2; ++pass) {
+          const int t0 = pass ? p->bpanel_task0[g] : p->bdiag_task0[g], n = pass ? p->bpanel_count[g] : p->bdiag_count[g];
+          for (int i = 0; i < n; ++i) {
+            SweepItem it = {};
+            it.kind = kItemBorder;
+            it.border = t0 + i;
+            // read by the cost alone: the tiles of the task
+            const BorderTask &b = btasks[t0 + i];
+            it.blocks = b.kind == kBorderSum ? 1 + std::min(kBorderChunk, b.i - 1 - b.j * kBorderChunk) / 2 : 1;
+            vectors.push_back(it);
+          }
+        }
+      }
+      int range0, n;
+      sort_blocks(list);
+      sweep.launch(chains, list, vectors, &range0, &n);
+      p->sweep_range0.push_back(range0);
+      p->sweep_count.push_back(n);
+      if (g < 0 || rest_list[g].empty()) continue;
+      // The trailing update of the group that ends with step g, over the next group's steps: as much
+      // to each as makes their products equal.  A diagonal tile whose chain runs in the last of them comes
+      // in the first, or, where the group is that one step, into the chain.
+      const int last = std::min(lookahead ? g + p->group : g + 1, p->max_t - 1);
+      std::vector<double> base(last - g, 0.0);
+      double sum = 0.0, part = 0.0;
+      for (int h = g + 1; h <= last; ++h) {
+        for (const TileTask &t : column_list[h]) base[h - g - 1] += 0.6 + t.K / NB;
+        base[h - g - 1] += 2.0 * p->panel_total[h];
+        sum += base[h - g - 1];
+      }
+      for (const TileTask &t : rest_list[g]) sum += 0.6 + t.K / NB;
+      int h = g + 1;
+      for (const TileTask &t : rest_list[g]) {
+        const int c = slot_of(t.c_off);
+        const int s = slot_matrix(c);
+        const int I = (c - slot_of(off[s])) / p->nt[s], J = (c - slot_of(off[s])) % p->nt[s];
+        if (I == J) {
+          const int chain_step = J + shift[s] - 1;
+          if (chain_step <= g + 1) {
+            chain_rest[c] = (int)chain_rest_tasks.size();
+            chain_rest_tasks.push_back(t);
+          } else {
+            rest[g + 1].push_back(update_item(t));
+          }
+          part += 0.6 + t.K / NB;
+          continue;
+        }
+        while (h < last && base[h - g - 1] + part >= sum / (last - g)) {
+          part -= sum / (last - g) - base[h - g - 1];
+          if (part < 0.0) part = 0.0;
+          ++h;
+        }
+        rest[h].push_back(update_item(t));
+        part += 0.6 + t.K / NB;
+      }
+    }
+  }
+  // Final products out(I,J) = sum_k U(I,k) U(J,k)^T, in blocks of kBlock x kBlock tiles whose operand
+  // rows stay in an XCD's L2 (workgroup i of a launch runs on XCD i % 8); blocks are dealt longest first to
+  // the XCD with the least work, and each XCD runs its long-K blocks first.
+  {
+    struct Block { int s, I, J; double cost; };
+    std::vector<Block> blocks;
     for (int s = 0; s < count; ++s)
-      for (int I = 0; I < p->nt[s]; ++I)
-        rows.push_back({s, I, (double)(I + 1) * (p->nt[s] - I) + 0.5 * (I + 1)});
-    std::stable_sort(rows.begin(), rows.end(), [](const Row &a, const Row &b) { return a.cost > b.cost; });
-    std::vector<Row> mine[8];
+      for (int I = 0; I < p->nt[s]; I += kBlock)
+        for (int J = 0; J <= I; J += kBlock) {
+          Block b{s, I, J, 0.0};
+          for (int i = I; i < std::min(I + kBlock, p->nt[s]); ++i)
+            b.cost += (std::min(i + 1, J + kBlock) - J) * (p->nt[s] - i + 1.0);
+          blocks.push_back(b);
+        }
+    std::stable_sort(blocks.begin(), blocks.end(), [](const Block &a, const Block &b) { return a.cost > b.cost; });
+    std::vector<Block> mine[8];
     double load[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (const Row &r : rows) {
+    for (const Block &b : blocks) {
       int x = 0;
       for (int i = 1; i < 8; ++i)
         if (load[i] < load[x]) x = i;
-      mine[x].push_back(r);
-      load[x] += r.cost;
+      mine[x].push_back(b);
+      load[x] += b.cost;
     }
     std::vector<TileTask> list[8];
     size_t longest = 0;
     for (int x = 0; x < 8; ++x) {
-      std::stable_sort(mine[x].begin(), mine[x].end(), [&](const Row &a, const Row &b) {
+      std::stable_sort(mine[x].begin(), mine[x].end(), [&](const Block &a, const Block &b) {
         return p->nt[a.s] - a.I > p->nt[b.s] - b.I;
       });
-      for (const Row &r : mine[x])
-        for (int J = 0; J <= r.I; ++J) {
-          TileTask t;
-          t.c_off = r.s;
-          t.a_off = tile_off(r.s, r.I, r.I);
-          t.b_off = tile_off(r.s, J, r.I);
-          t.K = (p->nt[r.s] - r.I) * NB;
-          t.flags = r.I | (J << 16);
-          list[x].push_back(t);
-        }
+      for (const Block &b : mine[x])
+        for (int I = b.I; I < std::min(b.I + kBlock, p->nt[b.s]); ++I)
+          for (int J = b.J; J < std::min(I + 1, b.J + kBlock); ++J) {
+            TileTask t;
+            t.c_off = b.s;
+            t.a_off = tile_off(b.s, I, I);
+            t.b_off = tile_off(b.s, J, I);
+            t.K = (p->nt[b.s] - I) * NB;
+            t.flags = I | (J << 16);
+            list[x].push_back(t);
+          }
       longest = std::max(longest, list[x].size());
     }
     p->lauum_task0 = (int)tasks.size();
@@ -1206,25 +1662,12 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
   up(p->d_btasks, btasks.data(), sizeof(BorderTask) * btasks.size());
   up(p->d_nt, p->nt.data(), sizeof(int) * count);
   up(p->d_off, off.data(), sizeof(long long) * count);
-  up(p->d_tile, tile_cs.data(), sizeof(int) * (count + 1));
   up(p->d_tile_owner, tile_owner.data(), sizeof(int2) * tile_owner.size());
   up(p->d_tasks, tasks.data(), sizeof(TileTask) * tasks.size());
-  if (rc == KFAC_OK && p->lookahead && p->max_t > p->group) {
-    const bool real = !kfac::host_only();   // host-only mode: null handles that nothing ever uses
-    bool ok = !real || (hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking) == hipSuccess &&
-                        hipStreamCreateWithFlags(&p->col, hipStreamNonBlocking) == hipSuccess);
-    for (int g = 0; ok && g < p->max_t; ++g)
-      for (auto *v : {&p->ev_main, &p->ev_side, &p->ev_fork, &p->ev_col}) {
-        hipEvent_t e = nullptr;
-        ok = ok && (!real || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
-        if (ok) v->push_back(e);
-      }
-    for (hipEvent_t *e : {&p->ev_copy_fork, &p->ev_copy})
-      ok = ok && (!real || hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess);
-    if (!ok) rc = kfac::fail(KFAC_EHIP, "cannot create the look-ahead stream or its events");
-  } else {
-    p->lookahead = false;
-  }
+  if (sweep.items.empty()) sweep.items.push_back(SweepItem{});
+  if (sweep.ranges.empty()) sweep.ranges.push_back(make_int2(0, 0));
+  up(p->d_items, sweep.items.data(), sizeof(SweepItem) * sweep.items.size());
+  up(p->d_ranges, sweep.ranges.data(), sizeof(int2) * sweep.ranges.size());
   if (rc != KFAC_OK) {
     delete p;
     return rc;
@@ -1261,19 +1704,6 @@ extern "C" int kfac_spd_inverse_batched_f32(kfac_inverse_plan_t plan,
     return kfac::fail(KFAC_ENOMEM, "inverse workspace too small: %zu < %zu bytes", ws_bytes,
                       kfac_inverse_plan_workspace_bytes(plan));
   hipStream_t s = kfac::as_stream(stream);
-  // The trailing updates fork onto the plan's own stream.  While `s` is being
-  // captured into a graph that is done only if the caller has declared `s` the
-  // capture's origin; otherwise everything stays on `s`, in program order.
-  bool lookahead = plan->lookahead;
-  if (lookahead && !plan->capture_origin && !kfac::host_only()) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
-      (void)hipGetLastError();   // e.g. the null stream beside a global-mode capture
-      lookahead = false;
-    } else if (cs != hipStreamCaptureStatusNone) {
-      lookahead = false;
-    }
-  }
   plan->in_sorted.resize(count);
   plan->out_sorted.resize(count);
   for (int i = 0; i < count; ++i) {
@@ -1289,15 +1719,8 @@ extern "C" int kfac_spd_inverse_batched_f32(kfac_inverse_plan_t plan,
   rc = plan->d_out.set(plan->out_sorted.data(), sizeof(void *) * count, s);
   if (rc != KFAC_OK) return rc;
   if (!plan->attr_set) {
-    KFAC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(diag_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)kDiagKernelLds));
-    for (const void *f : {reinterpret_cast<const void *>(panel_kernel),
-                          reinterpret_cast<const void *>(lauum_kernel)})
-      KFAC_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)kTileLdsBytes));
-    KFAC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(update_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    for (const void *f : {reinterpret_cast<const void *>(sweep_kernel), reinterpret_cast<const void *>(lauum_kernel)})
+      KFAC_HIP_CHECK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kTileLdsBytes));
     plan->attr_set = true;
   }
   InvTables tb;
@@ -1309,94 +1732,24 @@ extern "C" int kfac_spd_inverse_batched_f32(kfac_inverse_plan_t plan,
   tb.vec_off = plan->d_vec.as<const long long>();
   tb.nt = plan->d_nt.as<const int>();
   tb.ws_off = plan->d_off.as<const long long>();
-  tb.tile_cs = plan->d_tile.as<const int>();
   tb.tile_owner = plan->d_tile_owner.as<const int2>();
   tb.tasks = plan->d_tasks.as<const TileTask>();
+  tb.items = plan->d_items.as<const SweepItem>();
+  tb.ranges = plan->d_ranges.as<const int2>();
   tb.btasks = plan->d_btasks.as<const BorderTask>();
+  tb.ut0 = plan->ut0;
   uintptr_t base = (reinterpret_cast<uintptr_t>(ws) + 255) & ~(uintptr_t)255;
   tb.ws = reinterpret_cast<float *>(base);
   tb.info = info_dev;
 
-  kfac::TimedLaunch timed_call(KFAC_TIMED_INV_CALL, s);   // copy-in to the final product (the side streams rejoin `s`)
-  // copy-in: what the first step needs on `s`, the rest beside it on the side stream
-  const int late_tiles = lookahead ? plan->total_tiles - plan->first_tiles : 0;
-  if (late_tiles > 0) {
-    KFAC_HIP_CHECK(hipEventRecord(plan->ev_copy_fork, s));
-    KFAC_HIP_CHECK(hipStreamWaitEvent(plan->side, plan->ev_copy_fork, 0));
-    KFAC_LAUNCH(copy_in_kernel, dim3(late_tiles), dim3(256), 0, plan->side, tb, count, plan->first_tiles);
-    KFAC_HIP_CHECK(hipEventRecord(plan->ev_copy, plan->side));
-  }
-  if (plan->total_tiles - late_tiles > 0)
-    KFAC_LAUNCH(copy_in_kernel, dim3(plan->total_tiles - late_tiles), dim3(256), 0, s, tb, count, 0);
+  kfac::TimedLaunch timed_call(KFAC_TIMED_INV_CALL, s);   // copy-in to the final product
+  if (plan->total_tiles > 0) KFAC_LAUNCH(copy_in_kernel, dim3(plan->total_tiles), dim3(256), 0, s, tb);
   KFAC_HIP_CHECK(hipGetLastError());
-  // Side stream: after the last column of a group, the rest of its trailing
-  // update.  It is queued just after the next step's launch, so that the step's
-  // workgroups (the serial part of the sweep) are placed first and the rest
-  // fills the GPU around them.
-  int pending = -1;    // step of the latest work queued on the side stream
-  int deferred = -1;   // step whose rest is still to be queued
-  auto queue_rest = [&]() -> int {
-    if (deferred < 0) return KFAC_OK;
-    const UpdateLaunch &r = plan->rest[deferred];
-    hipStream_t st = s;
-    if (lookahead) {
-      KFAC_HIP_CHECK(hipStreamWaitEvent(plan->side, plan->ev_main[deferred], 0));
-      st = plan->side;
-    }
-    {
-      kfac::TimedLaunch timed(KFAC_TIMED_INV_UPDATE, st);
-      KFAC_LAUNCH(update_kernel, dim3(r.count), dim3(THREADS), plan->rest_lds, st, tb,
-                         r.task0);
-    }
-    if (lookahead) {
-      KFAC_HIP_CHECK(hipEventRecord(plan->ev_side[deferred], plan->side));
-      pending = deferred;
-    }
-    deferred = -1;
-    return KFAC_OK;
-  };
-  for (int k = 0; k < plan->max_t; ++k) {
-    const int na = plan->nactive[k];
-    const UpdateLaunch &w = plan->with_diag[k];
-    // the matrices that join from the second step on have been copied in by then
-    if (k == 1 && late_tiles > 0) KFAC_HIP_CHECK(hipStreamWaitEvent(s, plan->ev_copy, 0));
-    // A group's first step applies the previous group to this group's columns,
-    // tiles that the rest of the group before that one (two back) also updated.
-    // The rest of the previous group itself only touches columns further right
-    // and runs beside this group's sweep.
-    const int two_back = k - 1 - plan->group;
-    if (lookahead && k % plan->group == 0 && two_back >= 0 && plan->rest[two_back].count > 0)
-      KFAC_HIP_CHECK(hipStreamWaitEvent(s, plan->ev_side[two_back], 0));
-    if (!lookahead)
-      if (int rc2 = queue_rest()) return rc2;   // one stream: keep the program order
-    // the diagonal tiles on `s`, the column updates beside them
-    hipStream_t cs = s;
-    if (lookahead && w.count > 0) {
-      KFAC_HIP_CHECK(hipEventRecord(plan->ev_fork[k], s));
-      KFAC_HIP_CHECK(hipStreamWaitEvent(plan->col, plan->ev_fork[k], 0));
-      cs = plan->col;
-    }
-    KFAC_LAUNCH(diag_kernel, dim3(na + plan->bdiag_count[k]), dim3(THREADS), kDiagKernelLds, s, tb,
-                       plan->diag_task0[k], na, plan->bdiag_task0[k]);
-    if (w.count > 0) {
-      kfac::TimedLaunch timed(KFAC_TIMED_INV_UPDATE, cs);
-      KFAC_LAUNCH(update_kernel, dim3(w.count), dim3(THREADS), kTileLdsBytes, cs, tb, w.task0);
-    }
-    if (cs != s) {
-      KFAC_HIP_CHECK(hipEventRecord(plan->ev_col[k], cs));
-      KFAC_HIP_CHECK(hipStreamWaitEvent(s, plan->ev_col[k], 0));
-    }
-    if (int rc2 = queue_rest()) return rc2;
-    if (plan->panel_total[k] + plan->bpanel_count[k] > 0)
-      KFAC_LAUNCH(panel_kernel, dim3(plan->panel_total[k] + plan->bpanel_count[k]), dim3(THREADS),
-                         kTileLdsBytes, s, tb, plan->panel_task0[k], plan->panel_total[k],
-                         plan->bpanel_task0[k]);
-    if (plan->rest[k].count == 0) continue;
-    if (lookahead) KFAC_HIP_CHECK(hipEventRecord(plan->ev_main[k], s));
-    deferred = k;
+  for (size_t i = 0; i < plan->sweep_count.size(); ++i) {
+    if (plan->sweep_count[i] == 0) continue;
+    kfac::TimedLaunch timed(KFAC_TIMED_INV_UPDATE, s);
+    KFAC_LAUNCH(sweep_kernel, dim3(plan->sweep_count[i]), dim3(THREADS), kTileLdsBytes, s, tb, plan->sweep_range0[i]);
   }
-  if (int rc2 = queue_rest()) return rc2;
-  if (pending >= 0) KFAC_HIP_CHECK(hipStreamWaitEvent(s, plan->ev_side[pending], 0));
   KFAC_HIP_CHECK(hipGetLastError());
   if (plan->bfinal_count > 0) {
     KFAC_LAUNCH(border_kernel, dim3(plan->bfinal_count), dim3(THREADS), 0, s, tb, plan->bfinal_task0);

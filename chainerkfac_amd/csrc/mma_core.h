@@ -1,6 +1,6 @@
 // Float32 tile engine on the matrix cores, shared by the covariance (SYRK) and
-// preconditioning (GEMM) kernels; the convolution and inverse kernels use its tile
-// shapes, accumulator layout and epilogues with main loops of their own.
+// preconditioning (GEMM) kernels; the convolution kernels use its tile shapes, accumulator
+// layout and epilogues with main loops of their own, the inverse its split of operands.
 //
 // A workgroup of 256 threads (4 waves, 2 x 2) computes a (64*WM) x (64*WN)
 // tile of  D[i][j] = sum_k Aop(i, k) * Bop(j, k);  each wave owns WM x WN
@@ -894,24 +894,6 @@ __device__ __forceinline__ DiagRole diag_tile_role(int wave) {
   }
 }
 
-// Set every accumulator element of this lane to f(row, col), row / col relative
-// to the workgroup tile.
-template <int WM, int WN, class F>
-__device__ __forceinline__ void fill_acc(floatx16 (&acc)[WM][WN], F f, int wave = threadIdx.x >> 6) {
-  const int lane = threadIdx.x & 63;
-  const int wm = wave >> 1, wn = wave & 1;
-#pragma unroll
-  for (int im = 0; im < WM; ++im)
-#pragma unroll
-    for (int in = 0; in < WN; ++in)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = (wm * WM + im) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        const int col = (wn * WN + in) * 32 + (lane & 31);
-        acc[im][in][v] = f(row, col);
-      }
-}
-
 // Visit every accumulator element of this lane: f(row, col, value) with row /
 // col relative to the workgroup tile.
 template <int WM, int WN, class F>
@@ -1000,72 +982,6 @@ __device__ __forceinline__ void write_tile(floatx16 (&acc)[WM][WM], float *lds, 
         const int mr = c0 + lr, mc = r0 + lc;   // row of the mirrored quadrant = column here
         if (mr < dt && mc < dt) C[(long long)mr * d + mc] = v;
       }
-    }
-  }
-}
-
-// The finished 128 x 128 tile (I, J), I >= J, and its mirror image written to C
-// (leading dimension d, rows and columns below dt) in one go: the whole tile is
-// laid out in LDS (128 x 129 floats) once, then every thread stores 16 bytes at
-// a time (at float granularity: rows of an odd-sized matrix do not start on
-// 16-byte boundaries), rows of the tile and rows of the mirrored tile alike.
-// For C = acc (no scaling, no accumulation); ends without a barrier.
-constexpr int kWholeTileLdsFloats = 128 * 129;
-__device__ __forceinline__ void write_whole_tile(floatx16 (&acc)[2][2], float *lds, int I, int J, int dt,
-                                                 int d, float *__restrict__ C) {
-  typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
-  constexpr int LD = 129;
-  __syncthreads();   // the main loop's last LDS reads
-  for_each_acc<2, 2>(acc, [&](int r, int c, float v) { lds[r * LD + c] = v; });
-  __syncthreads();
-  const int q = (threadIdx.x & 31) * 4;    // four columns
-  const int r0 = threadIdx.x >> 5;         // 8 rows per pass
-  const int row0 = I * 128, col0 = J * 128;
-  const bool diag = I == J;
-#pragma unroll 4
-  for (int p = 0; p < 16; ++p) {
-    const int lr = r0 + 8 * p;
-    const int r = row0 + lr, c = col0 + q;
-    if (r >= dt) continue;
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (!diag || q + e <= lr) ? lds[lr * LD + q + e] : lds[(q + e) * LD + lr];
-    float *dst = C + (long long)r * d + c;
-    if (c + 3 < dt) {
-      floatx4u o;
-      o.x = v[0];
-      o.y = v[1];
-      o.z = v[2];
-      o.w = v[3];
-      *reinterpret_cast<floatx4u *>(dst) = o;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c + e < dt) dst[e] = v[e];
-    }
-  }
-  if (diag) return;
-  // mirrored tile (J, I): its row lr is column lr of the tile
-#pragma unroll 4
-  for (int p = 0; p < 16; ++p) {
-    const int lr = r0 + 8 * p;
-    const int r = col0 + lr, c = row0 + q;
-    if (r >= dt) continue;
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = lds[(q + e) * LD + lr];
-    float *dst = C + (long long)r * d + c;
-    if (c + 3 < dt) {
-      floatx4u o;
-      o.x = v[0];
-      o.y = v[1];
-      o.z = v[2];
-      o.w = v[3];
-      *reinterpret_cast<floatx4u *>(dst) = o;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c + e < dt) dst[e] = v[e];
     }
   }
 }

@@ -481,11 +481,6 @@ class InversePlan(object):
         if info is None:
             info = torch.empty(len(mats), dtype=torch.int32, device=dev)
         ws = _dev.workspace('inverse', self.workspace_bytes, dev)
-        # Under HIP-graph capture the plan may fork its trailing updates onto its
-        # own stream only from the stream the capture began on: torch's current
-        # stream when the call is not inside a lane (a lane is itself a fork).
-        origin = stream is None and _dev.current_lane() is None
-        _lib.check(_lib.load().kfac_inverse_plan_set_capture_origin(self._plan, int(origin)))
         _lib.check(_lib.load().kfac_spd_inverse_batched_f32(
             self._plan, _lib.ptr_array([m.data_ptr() for m in mats]),
             _lib.ptr_array([o.data_ptr() for o in outs]), info.data_ptr(), ws.data_ptr(),

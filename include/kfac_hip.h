@@ -284,14 +284,10 @@ int kfac_inverse_plan_create(int count, const int32_t *dims,
 size_t kfac_inverse_plan_workspace_bytes(kfac_inverse_plan_t plan);
 int kfac_inverse_plan_destroy(kfac_inverse_plan_t plan);
 
-/* kfac_spd_inverse_batched_f32 runs part of its trailing updates on a stream
- * of the plan's own, forked from and joined back into `stream` with events.
- * While `stream` is being captured into a HIP graph that fork is only taken
- * when the caller has declared, with is_origin != 0, that `stream` is the
- * stream the capture began on; on any other capturing stream (one that itself
- * was forked into the capture) the call keeps all launches on `stream`.  The
- * results are the same either way.  No counterpart in the reference (which has
- * no stream structure). */
+/* Accepted for callers that declare the stream a HIP-graph capture began on, as
+ * the calls with side streams need it.  kfac_spd_inverse_batched_f32 keeps all
+ * its launches on `stream`, captured or not, so it changes nothing.  No
+ * counterpart in the reference (which has no stream structure). */
 int kfac_inverse_plan_set_capture_origin(kfac_inverse_plan_t plan, int is_origin);
 
 /* out_i = in_i^-1 for SPD in_i (dims given at plan creation); the full

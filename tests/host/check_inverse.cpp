@@ -27,6 +27,116 @@ bool locate(const std::vector<long long> &off, const std::vector<int> &nt, long 
   return false;
 }
 
+// The launches that the tasks are merged into, replayed: every product once and from final tiles only,
+// nothing that a launch reads written by another workgroup of it, and every slot inside the workspace.
+void check_sweep(const kfac_inverse_plan *plan, const std::vector<long long> &offs, const char *what) {
+  const int count = plan->count, launches = (int)plan->sweep_count.size();
+  const SweepItem *items = reinterpret_cast<const SweepItem *>(plan->d_items.shadow().data());
+  const int2 *ranges = reinterpret_cast<const int2 *>(plan->d_ranges.shadow().data());
+  const BorderTask *bt = reinterpret_cast<const BorderTask *>(plan->d_btasks.shadow().data());
+  const int nitems = (int)(plan->d_items.shadow().size() / sizeof(SweepItem));
+  const int nranges = (int)(plan->d_ranges.shadow().size() / sizeof(int2));
+  EXPECT(launches == plan->max_t + 1 && plan->sweep_range0.size() == plan->sweep_count.size(), "%s: launches", what);
+  EXPECT(((size_t)plan->ut0 + 2 * count) * kSlotFloats <= plan->ws_floats, "%s: slots outside the workspace", what);
+  struct State {
+    int s, I, J;
+    int upto;        // columns below this one are applied
+    int final_in;    // launch that finished the tile, -1: none yet
+    int final_by;    // and its workgroup
+    int touched_in, touched_by;
+  };
+  std::vector<State> tile(plan->ut0);
+  for (int s = 0; s < count; ++s)
+    for (int I = 0; I < plan->nt[s]; ++I)
+      for (int J = 0; J < plan->nt[s]; ++J)
+        tile[offs[s] / (NB * NB) + I * plan->nt[s] + J] = State{s, I, J, I < J ? I : 0, -1, -1, -1, -1};
+  std::vector<int> ut_in(2 * count, -1), ut_col(2 * count, -1), solved(count, -1), solved_in(count, -1);
+  std::vector<int> sum_in(count * 512, -1), w_done(count, 0);
+  long long seen_items = 0;
+  for (int l = 0; l < launches; ++l) {
+    EXPECT(plan->sweep_count[l] >= 0 && plan->sweep_count[l] <= kSweepWorkgroups &&
+               plan->sweep_range0[l] + plan->sweep_count[l] <= nranges,
+           "%s: launch %d ranges", what, l);
+    std::vector<std::pair<int, int>> ut_written, solves, w_terms;
+    for (int w = 0; w < plan->sweep_count[l]; ++w) {
+      const int2 r = ranges[plan->sweep_range0[l] + w];
+      EXPECT(r.x >= 0 && r.x <= r.y && r.y <= nitems, "%s: launch %d workgroup %d items", what, l, w);
+      for (int i = r.x; i < r.y && i < nitems; ++i) {
+        ++seen_items;
+        const SweepItem &it = items[i];
+        auto final_for = [&](int slot) {
+          return slot >= 0 && slot < plan->ut0 && tile[slot].final_in >= 0 &&
+                 (tile[slot].final_in < l || tile[slot].final_by == w);
+        };
+        if (it.kind == kItemBorder) {
+          const BorderTask &b = bt[it.border];
+          const int at = (int)(offs[b.s] / (NB * NB)), T = plan->nt[b.s];
+          if (b.kind == kBorderSum) {
+            for (int j = b.j * kBorderChunk; j < std::min((b.j + 1) * kBorderChunk, b.i - 1); ++j)
+              EXPECT(final_for(at + b.i * T + j) && tile[at + b.i * T + j].final_in < l && solved[b.s] >= j &&
+                         (solved[b.s] > j || solved_in[b.s] < l),
+                     "%s: launch %d border sum", what, l);
+            EXPECT(b.j < border_chunks(b.i), "%s: launch %d border chunk", what, l);
+            sum_in[b.s * 512 + b.i] = l;
+          } else if (b.kind == kBorderSolve) {
+            EXPECT(ut_col[2 * b.s + (b.i & 1)] == b.i && ut_in[2 * b.s + (b.i & 1)] < l, "%s: launch %d border U^T", what, l);
+            if (b.i > 0) EXPECT(final_for(at + b.i * T + b.i - 1) && tile[at + b.i * T + b.i - 1].final_in < l, "%s: launch %d border term", what, l);
+            if (border_chunks(b.i) > 0) EXPECT(sum_in[b.s * 512 + b.i] >= 0 && sum_in[b.s * 512 + b.i] < l, "%s: launch %d border parts", what, l);
+            EXPECT(solved[b.s] == b.i - 1, "%s: launch %d border order", what, l);
+            solves.push_back({b.s, b.i});
+          } else {
+            EXPECT(b.kind == kBorderW && final_for(at + b.i * T + b.j) && tile[at + b.i * T + b.j].final_in < l && solved[b.s] >= b.j,
+                   "%s: launch %d border w", what, l);
+          }
+          continue;
+        }
+        EXPECT(it.c >= 0 && it.c < plan->ut0, "%s: launch %d item slot", what, l);
+        if (!(it.c >= 0 && it.c < plan->ut0)) continue;
+        State &t = tile[it.c];
+        const int at = (int)(offs[t.s] / (NB * NB)), T = plan->nt[t.s];
+        EXPECT(t.final_in < 0 && (t.touched_in < l || t.touched_by == w), "%s: launch %d tile (%d,%d) twice", what, l, t.I, t.J);
+        if (it.blocks > 0) {
+          EXPECT(it.a == at + t.I * T + t.upto && it.b == at + t.J * T + t.upto, "%s: launch %d tile (%d,%d): runs do not go on at column %d",
+                 what, l, t.I, t.J, t.upto);
+          EXPECT((it.first != 0) == (t.I < t.J && t.upto == t.I), "%s: launch %d tile (%d,%d) first", what, l, t.I, t.J);
+          for (int j = 0; j < it.blocks; ++j)
+            EXPECT(final_for(it.a + j) && final_for(it.b + j), "%s: launch %d tile (%d,%d) reads column %d too early", what, l, t.I,
+                   t.J, t.upto + j);
+          t.upto += it.blocks;
+        }
+        t.touched_in = l;
+        t.touched_by = w;
+        if (it.kind == kItemUpdate) {
+          EXPECT(it.blocks > 0 && t.upto <= t.J, "%s: launch %d update", what, l);
+          continue;
+        }
+        EXPECT(t.upto == t.J, "%s: launch %d tile (%d,%d) is final with %d of its columns", what, l, t.I, t.J, t.upto);
+        t.final_in = l;
+        t.final_by = w;
+        const int u = it.ut - plan->ut0;
+        EXPECT(u == 2 * t.s + (t.J & 1), "%s: launch %d U^T slot", what, l);
+        if (it.kind == kItemPanel) {
+          EXPECT(t.I != t.J && ut_col[u] == t.J && ut_in[u] < l, "%s: launch %d panel (%d,%d)", what, l, t.I, t.J);
+        } else {
+          EXPECT(it.kind == kItemDiag && t.I == t.J && it.col == t.J && it.caller == plan->order[t.s], "%s: launch %d diagonal", what, l);
+          ut_written.push_back({u, t.J});
+        }
+      }
+    }
+    for (auto &u : ut_written) {
+      // the buffer's readers (the panel step of two columns before) are done
+      ut_col[u.first] = u.second;
+      ut_in[u.first] = l;
+    }
+    for (auto &v : solves) {
+      solved[v.first] = v.second;
+      solved_in[v.first] = l;
+    }
+  }
+  EXPECT(seen_items == nitems || plan->max_t == 0, "%s: items outside the launches", what);
+  for (const State &t : tile) EXPECT(t.final_in >= 0, "%s: slot %d tile (%d,%d) never final", what, t.s, t.I, t.J);
+}
+
 void check_dims(const std::vector<int> &dims, const char *what) {
   const int count = (int)dims.size();
   kfac_inverse_plan_t plan = nullptr;
@@ -196,6 +306,8 @@ void check_dims(const std::vector<int> &dims, const char *what) {
   for (int s = 0; s < count; ++s)
     for (int I = 0; I < plan->nt[s]; ++I)
       for (int J = 0; J <= I; ++J) EXPECT(final_seen[s][std::make_pair(I, J)] == 1, "%s: slot %d final tile (%d,%d)", what, s, I, J);
+
+  check_sweep(plan, offs, what);
 
   // and one run through the entry point: argument checks, launch grids, event bookkeeping
   std::vector<const float *> in(count);

@@ -360,3 +360,33 @@ def test_inverse_error_of_well_conditioned_matrices(d):
     assert int(info.max()) == 0
     assert torch.equal(out, out.t())
     assert float((out.cpu().double() - want).norm() / want.norm()) <= 1.2 * 2.0 ** -24 * d ** 0.5
+
+
+@pytest.mark.parametrize('d', [97, 384, 513, 1100])
+@pytest.mark.parametrize('kind', ['rectified', 'banded', 'tiny', 'huge'])
+def test_inverse_error_of_other_matrices(kind, d):
+    """Factors with one large eigenvalue (rectified activations), a banded matrix, whose triangular factors and inverse
+    have entries down to the least float32 numbers and zero, and scales whose factors lie far from one.  The bound is that
+    of the test above, and at least 20 u for a single tile of a rectified matrix, which is rounded at the size of its
+    large eigenvalue (15 u were measured at 127 rows).  Rectified matrices of 1100 rows whose sums start from zero
+    instead of the matrix have 1.5 u sqrt(d)."""
+    from chainerkfac_amd import ops
+    gen = torch.Generator(device='cuda').manual_seed(d)
+    bound = 1.2 * 2.0 ** -24 * d ** 0.5
+    if kind == 'banded':
+        a = 2.5 * torch.eye(d, device='cuda')
+        a.diagonal(1).fill_(-0.02)
+        a.diagonal(-1).fill_(-0.02)
+    else:
+        x = torch.randn((4 * d, d), device='cuda', generator=gen)
+        if kind == 'rectified':
+            x.relu_()
+            bound = max(bound, 20 * 2.0 ** -24)
+        a = x.t() @ x / (4 * d)
+        a.diagonal().add_(1e-3)
+        a = (a + a.t()) / 2 * {'tiny': 1e-30, 'huge': 1e30}.get(kind, 1.0)
+    out, info = ops.spd_inverse_batched([a])
+    want = torch.linalg.inv(a.cpu().double())
+    assert int(info.max()) == 0
+    assert torch.equal(out[0], out[0].t())
+    assert float((out[0].cpu().double() - want).norm() / want.norm()) <= bound
