@@ -13,7 +13,7 @@
 //   a <  b   trtri:  X^T(a,b) = -sum_j U(a,j) L(b,j)^T         (a <= j < b)
 //            followed by U(a,b) = X^T(a,b) L_bb^-T once the sum is complete.
 //
-// Block columns are processed in groups of kGroup (2): inside a group the sweep is
+// Block columns are processed in groups of kGroup (3): inside a group the sweep is
 // left-looking, after a group every tile right of the next group receives the
 // whole group at once (K = kGroup * NB, "rest").  One launch per block column k:
 //
@@ -48,7 +48,6 @@ using namespace kfac::mma;
 constexpr int NB = 128;
 constexpr int SB = 32;
 constexpr int LS = NB + 1;  // LDS row stride of the diagonal tile
-constexpr int PS = SB + 1;  // row stride of a wave's private 32x32 block
 
 // One tile product of the sweep as the planner lists it, launch by launch.  Offsets count
 // NB * NB per tile: offset / (NB * NB) is the number of a tile's slot in the workspace.
@@ -98,14 +97,6 @@ struct InvTables {
   float *ws;                 // slots
   int *info;
 };
-
-__device__ __forceinline__ void tri_decode(int t, int &I, int &J) {
-  int r = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);
-  while (r * (r + 1) / 2 > t) --r;
-  while ((r + 1) * (r + 2) / 2 <= t) ++r;
-  I = r;
-  J = t - r * (r + 1) / 2;
-}
 
 // ---------------------------------------------------------------------------
 // Tile slots
@@ -183,7 +174,11 @@ __device__ __forceinline__ void gstore16(float *base, unsigned byte_off, V v) {
 //   * LDS is double-buffered (one barrier per stage); fragments are read one half stage
 //     ahead, the second half of a stage being multiplied after the barrier beside the reads of
 //     the next one;
-//   * LDS reads, LDS writes and global loads are dealt out one per matrix instruction.
+//   * LDS reads alternate with LDS writes in the first half of a stage and with global loads in the
+//     second, one per matrix instruction: 6630 cycles per tile of k-values, where the matrix
+//     instructions alone take 6144.  (Twelve writes or twelve loads one after the other, from four waves
+//     at once, stall the issue of what follows them: 8290 cycles.)  With all CUs at it the clock
+//     falls to 1.7 GHz: 3.9 us per tile of k-values, 275 TFLOP/s of float32 on the chip.
 struct Frags {
   bf16x8 a[2][3], b[2][3];
 };
@@ -231,15 +226,21 @@ __device__ __forceinline__ void panel_load1(const StageSource &src, Panels &r, i
 __device__ __forceinline__ void panel_write1(const Panels &r, char *buf, int i) {
   *reinterpret_cast<vfloat4 *>(buf + threadIdx.x * 16 + i * 4096) = r.v[i];   // A stage, then B stage
 }
+__device__ __forceinline__ void frag_read_plane(Frags &f, const char *buf, int ks, bool of_a, int blk, int q, int wi,
+                                                int wj) {
+  if (of_a)
+    f.a[blk][q] = *reinterpret_cast<const bf16x8 *>(buf + wi * (2 * 3 * kFragBytes) + frag_off(ks, blk, q));
+  else
+    f.b[blk][q] = *reinterpret_cast<const bf16x8 *>(buf + kStageBytes + wj * (2 * 3 * kFragBytes) + frag_off(ks, blk, q));
+}
 __device__ __forceinline__ void frag_read1(Frags &f, const char *buf, int ks, int i) {
   const int wave = threadIdx.x >> 6, wi = wave >> 1, wj = wave & 1;
   const int lane16 = (threadIdx.x & 63) * 16;
-  const int blk = (i % 6) / 3, q = i % 3;
-  if (i < 6)
-    f.a[blk][q] = *reinterpret_cast<const bf16x8 *>(buf + lane16 + wi * (2 * 3 * kFragBytes) + frag_off(ks, blk, q));
-  else
-    f.b[blk][q] = *reinterpret_cast<const bf16x8 *>(buf + lane16 + kStageBytes + wj * (2 * 3 * kFragBytes) +
-                                                    frag_off(ks, blk, q));
+  // in the order in which frag_mma1 needs them: planes hi of B and lo of A, lo and hi, mid and mid
+  const int q = i / 4, e = i % 4;
+  const bool of_a = e == 1 || e == 2;
+  constexpr int PA[3] = {2, 0, 1}, PB[3] = {0, 2, 1};
+  frag_read_plane(f, buf + lane16, ks, of_a, of_a ? e - 1 : e / 2, of_a ? PA[q] : PB[q], wi, wj);
 }
 __device__ __forceinline__ void frag_mma1(const Frags &f, floatx16 (&acc)[2][2], floatx16 (&low)[2][2], int i) {
   const int t = i / 4, im = (i / 2) & 1, in = i & 1;
@@ -257,10 +258,10 @@ __device__ __forceinline__ void product_stage(const char *cur, char *nxt, Panels
 #pragma unroll
   for (int i = 0; i < 24; ++i) {
     if (!FIRST) frag_mma1(f1, acc, low, i);
-    if (i < 12)
-      frag_read1(f0, cur, 0, i);
+    if (i % 2 == 0)
+      frag_read1(f0, cur, 0, i / 2);
     else
-      panel_write1(r, nxt, i - 12);
+      panel_write1(r, nxt, i / 2);
     __builtin_amdgcn_sched_barrier(0);
   }
   cursor_turn(cu);
@@ -268,10 +269,10 @@ __device__ __forceinline__ void product_stage(const char *cur, char *nxt, Panels
 #pragma unroll
   for (int i = 0; i < 24; ++i) {
     frag_mma1(f0, acc, low, i);
-    if (i < 12)
-      frag_read1(f1, cur, 1, i);
+    if (i % 2 == 0)
+      frag_read1(f1, cur, 1, i / 2);
     else
-      panel_load1(src, r, i - 12);
+      panel_load1(src, r, i / 2);
     __builtin_amdgcn_sched_barrier(0);
   }
   cursor_step(cu);
@@ -545,33 +546,143 @@ __global__ __launch_bounds__(256) void copy_in_kernel(InvTables tb) {
 // diagonal tile: Cholesky + triangular inverse inside LDS
 // ---------------------------------------------------------------------------
 
-// acc += A(32 x K) * B^T, A at a[row*AS + k]; B at b[row*LS + k] or, when BT,
-// at b[k*LS + row].
-template <bool BT, int AS = LS>
-__device__ __forceinline__ floatx16 wave_gemm(const float *a, const float *b, int K,
-                                              floatx16 acc) {
+// Products of 32 x 32 blocks of the tile by one wave: acc += A B^T, A at a[row * LS + k], B at
+// b[row * LS + k] or, when BT, at b[k * LS + row].
+template <bool BT>
+__device__ __forceinline__ floatx16 wave_gemm(const float *a, const float *b, floatx16 acc) {
   const int lane = threadIdx.x & 63;
   const int r = lane & 31, h = lane >> 5;
-  for (int k = 0; k < K; k += 2) {
-    const float av = a[r * AS + k + h];
+#pragma unroll
+  for (int k = 0; k < SB; k += 2) {
+    const float av = a[r * LS + k + h];
     const float bv = BT ? b[(k + h) * LS + r] : b[r * LS + k + h];
     acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
   }
   return acc;
 }
-
-template <class F>
-__device__ __forceinline__ void wave_visit(const floatx16 &acc, F f) {
+// blk = alpha * acc + beta * blk, by the wave that reads it next (its LDS accesses execute in order)
+__device__ __forceinline__ void wave_put(float *blk, const floatx16 &acc, float alpha, float beta) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int v = 0; v < 16; ++v) f(8 * (v >> 2) + 4 * (lane >> 5) + (v & 3), lane & 31, acc[v]);
+  for (int v = 0; v < 16; ++v) {
+    float *p = blk + (8 * (v >> 2) + 4 * (lane >> 5) + (v & 3)) * LS + (lane & 31);
+    *p = alpha * acc[v] + (beta != 0.f ? beta * *p : 0.f);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+// Quadrant (rows 16 qr .., columns 16 qc ..) of such a product, for the steps that all four waves share.
+typedef float floatx4q __attribute__((ext_vector_type(4)));
+template <bool BT>
+__device__ __forceinline__ floatx4q quad_gemm(const float *a, const float *b, int qr, int qc) {
+  const int lane = threadIdx.x & 63;
+  const int r = lane & 15, h = lane >> 4;
+  floatx4q acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < SB; k += 4) {
+    const float av = a[(16 * qr + r) * LS + k + h];
+    const float bv = BT ? b[(k + h) * LS + 16 * qc + r] : b[(16 * qc + r) * LS + k + h];
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc, 0, 0, 0);
+  }
+  return acc;
+}
+__device__ __forceinline__ float *quad_at(float *blk, int qr, int qc, int v) {
+  const int lane = threadIdx.x & 63;
+  return blk + (16 * qr + 4 * (lane >> 4) + v) * LS + 16 * qc + (lane & 15);
+}
+
+// Cholesky factor and triangular inverse of the tile S in 32 x 32 blocks: on return the upper block
+// triangle holds U = L^-T (the blocks on the diagonal with zeros below it).  Returns 0 or 1 + the first
+// non-positive pivot (in wave 0).
+//
+// The chain is the four diagonal blocks, each factored and inverted by wave 0 (2.5 us); between two
+// of them all waves form the next off-diagonal block L(j+1,j) and its product for the next diagonal
+// block, in quadrants.  Everything else, the other blocks of L, their products and the
+// sums P(j,i) = sum_k U(j,k) L(i,k)^T of U(j,i) = -P(j,i) U(i,i), belongs to waves 1 to 3 beside the
+// next diagonal block.  (One step after the other a launch of nothing but
+// this took 32 us, now 24.)
+__device__ __forceinline__ int factor_tile(float *S) {
+  const int wave = uniform(threadIdx.x >> 6);
+  const int qr = wave >> 1, qc = wave & 1;
+  floatx16 zero;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) zero[v] = 0.f;
+  auto at = [&](int i, int j) { return S + i * SB * LS + j * SB; };
+  auto solve = [&](int i, int j, float sign) {   // block (i, j) times U(j, j)
+    wave_put(at(i, j), wave_gemm<true>(at(i, j), at(j, j), zero), sign, 0.f);
+  };
+  auto update = [&](int i, int c, int j) {   // A(i, c) -= L(i, j) L(c, j)^T
+    wave_put(at(i, c), wave_gemm<false>(at(i, j), at(c, j), zero), -1.f, 1.f);
+  };
+  auto sum = [&](int j, int i) {   // P(j, i)
+    floatx16 p = zero;
+    for (int k = j; k < i; ++k) p = wave_gemm<false>(at(j, k), at(i, k), p);
+    wave_put(at(j, i), p, 1.f, 0.f);
+  };
+  int bad = 0;
+  for (int jb = 0; jb < NB / SB; ++jb) {
+    if (wave == 0) {
+      const int b = kfac::chol_inv_32<LS>(S, jb * SB);
+      if (b && !bad) bad = jb * SB + b;
+    } else if (jb == 1) {
+      if (wave < 3) {
+        const int i = wave + 1;
+        solve(i, 0, 1.f);
+        update(i, 1, 0);
+        update(i, i, 0);
+      } else {
+        sum(0, 1);
+      }
+    } else if (jb == 2) {
+      if (wave == 1) {
+        sum(1, 2);
+      } else if (wave == 2) {
+        solve(3, 1, 1.f);
+        update(3, 2, 0);
+        update(3, 2, 1);
+        update(3, 3, 1);
+      } else {
+        solve(0, 1, -1.f);
+        sum(0, 2);
+      }
+    } else if (jb == 3) {
+      if (wave < 3) {
+        solve(wave - 1, 2, -1.f);
+        sum(wave - 1, 3);
+      } else {
+        sum(2, 3);
+      }
+    }
+    __syncthreads();
+    if (jb == 3) break;
+    float *next = at(jb + 1, jb), *diag = at(jb + 1, jb + 1);
+    const floatx4q l = quad_gemm<true>(next, at(jb, jb), qr, qc);
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) *quad_at(next, qr, qc, v) = l[v];
+    __syncthreads();
+    if (qr >= qc) {
+      const floatx4q p = quad_gemm<false>(next, next, qr, qc);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) *quad_at(diag, qr, qc, v) -= p[v];
+    }
+    __syncthreads();
+  }
+  floatx4q u[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) u[j] = quad_gemm<true>(at(j, 3), at(3, 3), qr, qc);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) *quad_at(at(j, 3), qr, qc, v) = -u[j][v];
+  __syncthreads();
+  return bad;
 }
 
 // The diagonal tile (k,k) after its last products, its negative in registers: factored in LDS, U_kk written to
 // its slot and U_kk^T, which the next launch multiplies by, to the item's.  Ends with a barrier.
 __device__ __forceinline__ void diag_role(const InvTables &tb, const SweepItem &it, const TileRegs &tile, float *smem) {
   float *S = smem;                      // NB x LS working tile
-  float *scratch = smem + NB * LS;      // 3 waves x SB x PS
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   {
@@ -586,58 +697,12 @@ __device__ __forceinline__ void diag_role(const InvTables &tb, const SweepItem &
           for (int e = 0; e < 4; ++e) p[in * 32 * LS + im * 32 + 8 * g + e] = -tile.v[im][in][g][e];
   }
   __syncthreads();
-  floatx16 zero;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) zero[v] = 0.f;
-
-  // ---- potrf on 32x32 blocks
-  for (int jb = 0; jb < NB / SB; ++jb) {
-    if (wave == 0) {
-      const int bad = kfac::chol_inv_32<LS>(S, jb * SB);
-      if (lane == 0) {
-        int *pinfo = &tb.info[it.caller];
-        if (it.col == 0 && jb == 0) *pinfo = 0;
-        const int col = it.col * NB + jb * SB + bad - 1;
-        if (bad && col < it.core && *pinfo == 0) *pinfo = col + 1;
-      }
-    }
-    __syncthreads();
-    // panel: L(ib,jb) = A(ib,jb) U32(jb), one block per wave
-    for (int ib = jb + 1 + wave; ib < NB / SB; ib += 4) {
-      float *blk = S + (ib * SB) * LS + jb * SB;
-      const floatx16 acc = wave_gemm<true>(blk, S + (jb * SB) * LS + jb * SB, SB, zero);
-      wave_visit(acc, [&](int r, int c, float v) { blk[r * LS + c] = v; });
-    }
-    __syncthreads();
-    // trailing update: A(ib,cb) -= L(ib,jb) L(cb,jb)^T for jb < cb <= ib
-    const int rem = NB / SB - jb - 1;
-    for (int t = wave; t < rem * (rem + 1) / 2; t += 4) {
-      int a, b;
-      tri_decode(t, a, b);
-      const int ib = jb + 1 + a, cb = jb + 1 + b;
-      float *blk = S + (ib * SB) * LS + cb * SB;
-      const floatx16 acc = wave_gemm<false>(S + (ib * SB) * LS + jb * SB,
-                                            S + (cb * SB) * LS + jb * SB, SB, zero);
-      wave_visit(acc, [&](int r, int c, float v) { blk[r * LS + c] -= v; });
-    }
-    __syncthreads();
-  }
-
-  // ---- trtri: U(jb,ib) = -[sum_kb U(jb,kb) L(ib,kb)^T] U32(ib), by distance
-  float *P = scratch + wave * SB * PS;
-  for (int dd = 1; dd < NB / SB; ++dd) {
-    for (int jb = wave; jb + dd < NB / SB; jb += 4) {
-      const int ib = jb + dd;
-      const floatx16 p = wave_gemm<false>(S + (jb * SB) * LS + jb * SB,
-                                          S + (ib * SB) * LS + jb * SB, dd * SB, zero);
-      wave_visit(p, [&](int r, int c, float v) { P[r * PS + c] = v; });
-      // the same wave re-reads P: LDS accesses of one wave execute in order
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      const floatx16 u = wave_gemm<true, PS>(P, S + (ib * SB) * LS + ib * SB, SB, zero);
-      float *blk = S + (jb * SB) * LS + ib * SB;
-      wave_visit(u, [&](int r, int c, float v) { blk[r * LS + c] = -v; });
-    }
-    __syncthreads();
+  const int bad = factor_tile(S);
+  if (threadIdx.x == 0) {
+    int *pinfo = &tb.info[it.caller];
+    if (it.col == 0) *pinfo = 0;
+    const int col = it.col * NB + bad - 1;
+    if (bad && col < it.core && *pinfo == 0) *pinfo = col + 1;
   }
 
   // ---- U and U^T as final tiles, exact zeros on the other side of the diagonal
@@ -1021,7 +1086,7 @@ __global__ __launch_bounds__(THREADS, 1) void lauum_kernel(InvTables tb, int tas
   write_whole_tile(acc, reinterpret_cast<float *>(lds), I, J, dc, d, out);
 }
 
-constexpr int kDiagLdsBytes = (NB * LS + 3 * SB * PS) * (int)sizeof(float);
+constexpr int kDiagLdsBytes = NB * LS * (int)sizeof(float);
 static_assert(kDiagLdsBytes <= kTileLdsBytes && kBorderLdsFloats * (int)sizeof(float) <= kTileLdsBytes,
               "the roles of a sweep workgroup share its LDS");
 static_assert(2 * kTileLdsBytes > 160 * 1024, "one workgroup per CU: the diagonal tiles have their SIMDs to themselves");
@@ -1036,7 +1101,7 @@ struct UpdateLaunch {
 struct kfac_inverse_plan {
   int count = 0;
   int max_t = 0;
-  int group = 2;                   // block columns per trailing update (measured best of 1..8)
+  int group = 3;                   // block columns per trailing update (2 to 4 within 2 %)
   std::vector<int> order;          // slot -> caller index
   std::vector<int> nt;             // per slot
   std::vector<int> nactive;        // per step
@@ -1091,18 +1156,19 @@ void append_tasks(std::vector<T> &table, const std::vector<T> &natural) {
   table.insert(table.end(), dealt.begin(), dealt.end());
 }
 
-// The sweep as launches of items.  Costs are in units of one 128 x 128 x 128 product on a CU
-// (about 3 us); they only balance the workgroups' lists.
+// The sweep as launches of items.  Costs are in units of one 128 x 128 x 128 product on a busy GPU
+// (3.9 us, measured with time stamps like the others); they only balance the workgroups' lists.
 constexpr int kSweepWorkgroups = 256;   // one per CU
+constexpr double kUpdateCost = 0.7, kPanelCost = 2.4, kDiagCost = 7.2;
 // Side of the blocks of tiles that are worked on together.  The 32 workgroups of an XCD read 12 operand
 // runs for 36 tiles instead of 33 for 32, through an L2 of 4 MB.
 constexpr int kBlock = 6;
 double item_cost(const SweepItem &it) {
   switch (it.kind) {
-    case kItemUpdate: return 0.6 + it.blocks;
-    case kItemPanel: return 2.2 + it.blocks;
-    case kItemDiag: return 8.0 + it.blocks;
-    default: return it.blocks;   // about a third of a unit per tile and one for the rest
+    case kItemUpdate: return kUpdateCost + it.blocks;
+    case kItemPanel: return kPanelCost + it.blocks;
+    case kItemDiag: return kDiagCost + it.blocks;
+    default: return 1.5 + 0.5 * it.blocks;   // (of tiles read)
   }
 }
 
@@ -1428,10 +1494,10 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       rest_list[g].insert(rest_list[g].end(), t.begin(), t.end());
     }
   }
-  // The launches.  Launch g + 1 is step g: its panel tasks, each behind the column's product for the
-  // same tile; for every matrix the tile below the diagonal and the next diagonal tile as one
-  // workgroup's chain; the step's other column products, the vector tasks and a share of the trailing
-  // update before.  (Launch 0: the first diagonal tiles.)
+  // The launches.  Launch g + 1 is step g: its panel tasks, each behind the column products listed for
+  // the same tile so far (those of the previous group and of this one's columns in one run); for every matrix the
+  // tile below the diagonal and the next diagonal tile as one workgroup's chain; the vector tasks and a share of
+  // the trailing update before.  (Launch 0: the first diagonal tiles.)
   SweepBuilder sweep;
   {
     auto slot_of = [](long long o) { return (int)(o / (NB * NB)); };
@@ -1449,13 +1515,19 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
     auto slot_matrix = [&](int c) {   // a matrix's slots are contiguous
       return (int)(std::upper_bound(off.begin(), off.end(), (long long)c * (NB * NB)) - off.begin()) - 1;
     };
-    std::vector<int> owed(nslots, -1);               // slot -> index in the step's column list
+    struct Owed {
+      int a, b, blocks, first;
+    };
+    std::vector<Owed> owed(nslots, Owed{0, 0, 0, 0});   // column products listed so far, by slot
     std::vector<std::vector<SweepItem>> rest(p->max_t + 1);   // trailing updates by step
     // trailing products that only the chain of a diagonal tile can apply (groups of one column)
     std::vector<int> chain_rest(nslots, -1);
     std::vector<TileTask> chain_rest_tasks;
-    std::vector<SweepItem> list, vectors;
-    std::vector<std::vector<SweepItem>> chains;
+    struct Launch {
+      std::vector<SweepItem> list, vectors;
+      std::vector<std::vector<SweepItem>> chains;
+    };
+    std::vector<Launch> launches(p->max_t + 1);
     // tiles that share operand runs follow each other: blocks of kBlock x kBlock tiles of a matrix
     auto sort_blocks = [&](std::vector<SweepItem> &v) {
       std::vector<std::pair<unsigned long long, int>> key(v.size());
@@ -1472,20 +1544,14 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       v.swap(out);
     };
     for (int g = -1; g < p->max_t; ++g) {
-      list.clear();
-      vectors.clear();
-      chains.clear();
-      std::vector<char> taken;
-      if (g >= 0) {
-        const std::vector<TileTask> &col = column_list[g];
-        taken.assign(col.size(), 0);
-        for (size_t i = 0; i < col.size(); ++i) owed[slot_of(col[i].c_off)] = (int)i;
-      }
-      auto take = [&](int slot) -> const TileTask * {
-        if (g < 0 || owed[slot] < 0) return nullptr;
-        taken[owed[slot]] = 1;
-        return &column_list[g][owed[slot]];
-      };
+      std::vector<SweepItem> &list = launches[g + 1].list, &vectors = launches[g + 1].vectors;
+      std::vector<std::vector<SweepItem>> &chains = launches[g + 1].chains;
+      if (g >= 0)
+        for (const TileTask &t : column_list[g]) {
+          Owed &o = owed[slot_of(t.c_off)];
+          if (o.blocks == 0) o = Owed{slot_of(t.a_off), slot_of(t.b_off), 0, (t.flags & kFirst) != 0};
+          o.blocks += t.K / NB;
+        }
       // the chains: matrices with a diagonal tile in step g + 1
       std::vector<int> chain_of(count, -1);
       if (g + 1 < p->max_t)
@@ -1496,11 +1562,10 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
           it.c = slot_of(t.c_off);
           it.a = slot_of(t.a_off);
           it.blocks = t.K / NB;
-          // products listed for this tile in this step: the same run, further left
-          const TileTask *pre = take(it.c);
-          if (pre) {
-            it.a = slot_of(pre->a_off);
-            it.blocks += pre->K / NB;
+          // products listed for this tile before: the same run, further left
+          if (owed[it.c].blocks > 0) {
+            it.a = owed[it.c].a;
+            it.blocks += owed[it.c].blocks;
           }
           if (chain_rest[it.c] >= 0) {
             const TileTask &r = chain_rest_tasks[chain_rest[it.c]];
@@ -1527,11 +1592,12 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
             it.kind = kItemPanel;
             it.c = it.a = it.b = slot_of(t.c_off);
             it.ut = p->ut0 + 2 * s + (k & 1);
-            if (const TileTask *u = take(it.c)) {
-              it.a = slot_of(u->a_off);
-              it.b = slot_of(u->b_off);
-              it.blocks = u->K / NB;
-              it.first = (u->flags & kFirst) != 0;
+            const Owed &o = owed[it.c];
+            if (o.blocks > 0) {
+              it.a = o.a;
+              it.b = o.b;
+              it.blocks = o.blocks;
+              it.first = o.first;
             }
             if (x == k + 1)
               chains[chain_of[s]].insert(chains[chain_of[s]].begin(), it);
@@ -1539,9 +1605,6 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
               list.push_back(it);
           }
         }
-        for (size_t i = 0; i < column_list[g].size(); ++i)
-          if (!taken[i]) list.push_back(update_item(column_list[g][i]));
-        for (const TileTask &t : column_list[g]) owed[slot_of(t.c_off)] = -1;
         list.insert(list.end(), rest[g].begin(), rest[g].end());
         rest[g].clear();
         for (int pass = 0; pass < 2; ++pass) {
@@ -1552,16 +1615,11 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
             it.border = t0 + i;
             // read by the cost alone: the tiles of the task
             const BorderTask &b = btasks[t0 + i];
-            it.blocks = b.kind == kBorderSum ? 1 + std::min(kBorderChunk, b.i - 1 - b.j * kBorderChunk) / 2 : 1;
+            it.blocks = b.kind == kBorderSum ? std::min(kBorderChunk, b.i - 1 - b.j * kBorderChunk) : 1;
             vectors.push_back(it);
           }
         }
       }
-      int range0, n;
-      sort_blocks(list);
-      sweep.launch(chains, list, vectors, &range0, &n);
-      p->sweep_range0.push_back(range0);
-      p->sweep_count.push_back(n);
       if (g < 0 || rest_list[g].empty()) continue;
       // The trailing update of the group that ends with step g, over the next group's steps: as much
       // to each as makes their products equal.  A diagonal tile whose chain runs in the last of them comes
@@ -1570,11 +1628,11 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       std::vector<double> base(last - g, 0.0);
       double sum = 0.0, part = 0.0;
       for (int h = g + 1; h <= last; ++h) {
-        for (const TileTask &t : column_list[h]) base[h - g - 1] += 0.6 + t.K / NB;
-        base[h - g - 1] += 2.0 * p->panel_total[h];
+        // a panel item of step h: the source group's products and those of the group's own columns
+        base[h - g - 1] += (kPanelCost + p->group + (h - g - 1)) * p->panel_total[h];
         sum += base[h - g - 1];
       }
-      for (const TileTask &t : rest_list[g]) sum += 0.6 + t.K / NB;
+      for (const TileTask &t : rest_list[g]) sum += kUpdateCost + t.K / NB;
       int h = g + 1;
       for (const TileTask &t : rest_list[g]) {
         const int c = slot_of(t.c_off);
@@ -1588,7 +1646,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
           } else {
             rest[g + 1].push_back(update_item(t));
           }
-          part += 0.6 + t.K / NB;
+          part += kUpdateCost + t.K / NB;
           continue;
         }
         while (h < last && base[h - g - 1] + part >= sum / (last - g)) {
@@ -1597,8 +1655,43 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
           ++h;
         }
         rest[h].push_back(update_item(t));
-        part += 0.6 + t.K / NB;
+        part += kUpdateCost + t.K / NB;
       }
+    }
+    // What a chain's tiles are owed from columns that are final a launch earlier goes to that launch: the
+    // chain keeps one product for the tile below the diagonal and two for the diagonal tile.
+    std::vector<int> where(nslots, -1);   // slot -> index in a launch's list
+    for (int l = 1; l <= p->max_t; ++l) {
+      std::vector<SweepItem> &before = launches[l - 1].list;
+      for (size_t i = 0; i < before.size(); ++i)
+        if (before[i].kind == kItemUpdate) where[before[i].c] = (int)i;
+      for (std::vector<SweepItem> &chain : launches[l].chains)
+        for (SweepItem &it : chain) {
+          const int keep = it.kind == kItemDiag ? 2 : 1, move = it.blocks - keep;
+          if (move <= 0) continue;
+          if (where[it.c] >= 0) {
+            before[where[it.c]].blocks += move;
+          } else {
+            SweepItem u = {};
+            u.kind = kItemUpdate;
+            u.c = it.c;
+            u.a = it.a;
+            u.b = it.b;
+            u.blocks = move;
+            before.push_back(u);
+          }
+          it.a += move;
+          it.b += move;
+          it.blocks = keep;
+        }
+      for (const SweepItem &it : before) where[it.c] = -1;
+    }
+    for (Launch &l : launches) {
+      int range0, n;
+      sort_blocks(l.list);
+      sweep.launch(l.chains, l.list, l.vectors, &range0, &n);
+      p->sweep_range0.push_back(range0);
+      p->sweep_count.push_back(n);
     }
   }
   // Final products out(I,J) = sum_k U(I,k) U(J,k)^T, in blocks of kBlock x kBlock tiles whose operand
