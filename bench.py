@@ -511,7 +511,7 @@ def run_step_config(args, name, cfg, host=None):
             cov_executed, ('syrk', 'cov_aux'), fam, empty, one_stream, reference_flop=flops['cov'],
             peak=cov_peak(layers, batch)),
         'inverse_tiles': family_roofline(
-            'inverse_tiles', 'batched dense inverse: copy_in, sweep, border, lauum kernels',
+            'inverse_tiles', 'batched dense inverse: sweep, border, lauum kernels',
             dense_inverse_flops, ('inv_call',), fam, empty,
             'd^3 flop of the densely inverted factors over the time between the first and the last launch of the '
             'batched call (its kernels overlap on three streams, so their durations do not add up)',
@@ -716,7 +716,7 @@ def run_inverse_config(args, name, cfg):
         'max_residual': worst,      # max over sizes of ||M M^-1 - I||_F / sqrt(d); the bound is 1e-3
         'roofline': {
             'family': 'inverse_tiles',
-            'kernel': 'batched dense inverse: copy_in, sweep, border, lauum kernels', 'bound': 'mfma',
+            'kernel': 'batched dense inverse: sweep, border, lauum kernels', 'bound': 'mfma',
             'achieved': round(achieved, 2), 'peak': FP32_MFMA_PEAK_TFLOPS, 'unit': 'TFLOP/s',
             'frac': round(achieved / FP32_MFMA_PEAK_TFLOPS, 4),
             'timed': 'd^3 flop per matrix over the wall time of the whole batched call (its kernels overlap on two '
@@ -1020,7 +1020,7 @@ KERNEL_FAMILIES = (
     ('batch-norm rank-n inverses', ('lr_',)),
     ('split-K finish, edge sums and assembly of the covariances', ('finish_', 'reduce_kernel', 'shift::assemble',
                                                                   'shift::edge_sums')),
-    ('inverse tile kernels', ('sweep_kernel', 'lauum_kernel', 'copy_in', 'border_kernel')),
+    ('inverse tile kernels', ('sweep_kernel', 'lauum_kernel', 'border_kernel')),
     ('damping', ('pi_damp', 'add_diag')),
     ('pack / unpack / copy', ('pack_kernel', 'unpack_kernel', 'stream_copy', 'stream_fanout')),
 )
@@ -1052,15 +1052,15 @@ def summarize_kernel_trace(trace_dir, out_path, command):
     if not agg:
         raise SystemExit('no kernel_trace.csv under ' + trace_dir)
     total = float(sum(a[1] for a in agg.values()))
-    # elapsed time of every batched inverse: first copy_in after the previous call's lauum .. end of lauum
+    # elapsed time of every batched inverse: first sweep launch after the previous call's lauum .. end of lauum
     # (only calls with the whole sweep in between: the three-matrix inverses of other runs are left out)
     spans, begin, inside = [], None, 0
     ordered = sorted((int(r['Start_Timestamp']), int(r['End_Timestamp']), r['Kernel_Name'])
                      for r in _csv_rows(trace_dir, 'kernel_trace.csv'))
     for t0, t1, name in ordered:
-        if 'copy_in_kernel' in name and begin is None:
-            begin, inside = t0, 0
-        elif begin is not None and 'sweep_kernel' in name:
+        if 'sweep_kernel' in name:
+            if begin is None:
+                begin, inside = t0, 0
             inside += 1
         elif 'lauum_kernel' in name and begin is not None:
             spans.append((t1 - begin, inside))
@@ -1086,7 +1086,7 @@ def summarize_kernel_trace(trace_dir, out_path, command):
             n, t = fam[f]
             lines.append('| {} | {} | {:.3f} | {:.1f} | {:.1f} % |'.format(f, n, t / 1e6, t / n / 1e3, 100 * t / total))
     if spans:
-        lines += ['', 'Elapsed time of a batched inverse (start of its first `copy_in_kernel` to the end of its '
+        lines += ['', 'Elapsed time of a batched inverse (start of its first `sweep_kernel` to the end of its '
                   '`lauum_kernel`, {} calls with the full sweep): median {:.3f} ms, min {:.3f}, max {:.3f}.'.format(
                       len(spans), spans[len(spans) // 2] / 1e6, spans[0] / 1e6, spans[-1] / 1e6)]
     lines += ['', '| kernel | launches | total ms | avg us | min us | max us | share |', '|---|---:|---:|---:|---:|---:|---:|']
@@ -1157,7 +1157,7 @@ TRAFFIC_FAMILIES = (
     # family, kernels of the family, the kernel whose launches count the steps of the run
     ('cov_syrk', ('syrk_', 'shift::corr_kernel', 'finish_group_kernel', 'finish_kernel', 'reduce_kernel',
                   'shift::assemble', 'shift::edge_sums', 'shift::corr_finish'), 'finish_group_kernel'),
-    ('inverse_tiles', ('copy_in_kernel', 'sweep_kernel', 'border_kernel', 'lauum_kernel'), 'lauum_kernel'),
+    ('inverse_tiles', ('sweep_kernel', 'border_kernel', 'lauum_kernel'), 'lauum_kernel'),
     ('precond_gemm', ('gemm_group', 'gemv_', 'bn_select'), 'gemm_group_finish_kernel<1>'),
 )
 

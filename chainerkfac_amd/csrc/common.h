@@ -164,6 +164,11 @@ class DevTable {
     shadow_.assign(static_cast<const char *>(host), static_cast<const char *>(host) + bytes);
     return KFAC_OK;
   }
+  // The contents alone, for tables that only the host reads.
+  int keep(const void *host, size_t bytes) {
+    shadow_.assign(static_cast<const char *>(host), static_cast<const char *>(host) + bytes);
+    return KFAC_OK;
+  }
   template <typename T>
   T *as() const {
     return static_cast<T *>(dev_);

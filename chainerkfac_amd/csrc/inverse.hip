@@ -1,8 +1,8 @@
 // Batched damped inverse of SPD Kronecker factors: blocked Cholesky (potrf)
 // followed by the triangular inverse and L^-T L^-1 (potri).
 //
-// All matrices of a batch advance together, in tiles of NB x NB (NB = 128) of a
-// zero/identity padded workspace.  The strictly lower tiles end up holding L, the
+// All matrices of a batch advance together, in tiles of NB x NB (NB = 128); what lies past a
+// matrix in its last tiles is taken as the identity.  The strictly lower tiles end up holding L, the
 // upper tiles U = L^-T (the triangular inverse, stored transposed), the diagonal
 // tiles U_kk = L_kk^-T.  With M(a,j) the tile in slot (a,j), every product of the
 // sweep has one form,
@@ -13,7 +13,7 @@
 //   a <  b   trtri:  X^T(a,b) = -sum_j U(a,j) L(b,j)^T         (a <= j < b)
 //            followed by U(a,b) = X^T(a,b) L_bb^-T once the sum is complete.
 //
-// Block columns are processed in groups of kGroup (3): inside a group the sweep is
+// Block columns are processed in groups of kGroup (4): inside a group the sweep is
 // left-looking, after a group every tile right of the next group receives the
 // whole group at once (K = kGroup * NB, "rest").  One launch per block column k:
 //
@@ -63,18 +63,20 @@ constexpr int kSame = 2;    // both operands are the same run
 
 // What a workgroup of the sweep does next: the tile products merged into the step they
 // belong to, resolved on the host (one scalar load per item).
-enum ItemKind { kItemUpdate = 0, kItemPanel = 1, kItemDiag = 2, kItemBorder = 3 };
+enum ItemKind { kItemUpdate = 0, kItemPanel = 1, kItemDiag = 2, kItemBorder = 3, kItemOut = 4 };
+enum ItemStart { kFromSlot = 0, kFromZero = 1, kFromInput = 2 };
 struct SweepItem {
   int kind;
   int c, a, b;   // slots: the tile, the first tiles of the operand runs
   int blocks;    // tiles in either run; 0: nothing is owed
-  int first;     // the tile starts from zero
+  int start;     // what the tile is before: its slot, zero, or (the first time) the input's tile
   int ut;        // panel: slot of U_kk^T; diagonal: slot that U^T is written to
   int col;       // diagonal: block column
   int caller;    // diagonal: caller's index of the matrix
   int core;      // diagonal: rows of the tiled part
   int border;    // border: index of the vector task
-  int pad;
+  int matrix;    // input or output tile: sorted slot of the matrix
+  int at;        // and tile row | tile column << 16
 };
 
 struct BorderTask;
@@ -88,9 +90,7 @@ struct InvTables {
                              // each) and the scalars alpha, S, 1/S behind them; -1 otherwise
   const int *nt;             // [count] tiles per side
   const long long *ws_off;   // [count] offset of the padded matrix, NB * NB per tile
-  const int2 *tile_owner;    // [tiles] copy-in: (slot, I | J << 16) of every lower tile
-  const TileTask *tasks;     // the final products
-  const SweepItem *items;    // the items of all sweep launches
+  const SweepItem *items;    // the items of all launches
   const int2 *ranges;        // per launch and workgroup: its items [x, y)
   const BorderTask *btasks;  // the vector tasks of the bordered matrices
   int ut0;                   // first slot of the U_kk^T buffers, two per matrix
@@ -502,44 +502,66 @@ __device__ __forceinline__ void panel_role(const InvTables &tb, const SweepItem 
 }
 
 // ---------------------------------------------------------------------------
-// copy-in: the negative of the lower tiles of in -> float32 slots (identity on the padding)
+// input tiles: the negative of tile (I, J) of a matrix, identity on the padding
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void copy_in_kernel(InvTables tb) {
-  const int2 owner = tb.tile_owner[blockIdx.x];
-  const int s = owner.x, I = owner.y & 0xffff, J = owner.y >> 16;
-  const int d = tb.dim[s], dc = tb.core[s];
-  const float *__restrict__ src = tb.in[s];
-  float *__restrict__ dst = slot_ptr(tb, tile_slot(tb, s, I, J));
-  const int lane = threadIdx.x & 63, ib = threadIdx.x >> 6;
-  const int r = I * NB + ib * 32 + (lane & 31);
-  // 16-byte loads at float granularity (the rows of an odd-sized matrix do not start on
-  // 16-byte boundaries); the quads cut by the edge of the matrix go element by element.  Four
-  // consecutive loads of a lane cover a 128-byte piece of its row.
-  typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+// The item that touches a lower tile first reads it from the input.  16-byte loads at float
+// granularity (the rows of an odd-sized matrix do not start on 16-byte boundaries; four
+// consecutive loads of a lane cover a 128-byte piece of its row); the tiles at the edge of the
+// matrix are read by the element.
+__device__ __forceinline__ void input_load(const InvTables &tb, int s, int at, TileRegs &c) {
+  const int I = at & 0xffff, J = at >> 16;
+  const int d = uniform(tb.dim[s]), dc = uniform(tb.core[s]);
+  const float *src = wave_uniform(tb.in[s] + (long long)I * NB * d);   // offsets inside a tile row are below 2^25
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r0 = (wave >> 1) * 64 + (lane & 31), c0 = J * NB + (wave & 1) * 64 + 4 * (lane >> 5);
+  if ((I + 1) * NB <= dc && (J + 1) * NB <= dc) {
 #pragma unroll
-  for (int p = 0; p < 16; ++p) {
-    const int c = J * NB + 8 * p + 4 * (lane >> 5);   // block p / 4, group p % 4
-    vfloat4 v;
-    if (r < dc && c + 3 < dc) {
-      const floatx4u x = *reinterpret_cast<const floatx4u *>(src + (long long)r * d + c);
-      v = vfloat4{x.x, x.y, x.z, x.w};
-    } else {
+    for (int in = 0; in < 2; ++in) {
+      const unsigned o = (unsigned)(((r0 + 32 * in) * d + c0) * (int)sizeof(float));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float x = (r == c + e) ? 1.f : 0.f;
-        if (r < dc && c + e < dc) x = src[(long long)r * d + c + e];
-        v[e] = x;
-      }
+      for (int im = 0; im < 2; ++im)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 x = gload4(src, o + (unsigned)((32 * im + 8 * g) * sizeof(float)));
+          c.v[im][in][g] = vfloat4{-x.x, -x.y, -x.z, -x.w};
+        }
     }
-    *reinterpret_cast<vfloat4 *>(dst + (ib * 16 + p) * 256 + lane * 4) = -v;
+    return;
   }
-  // a bordered matrix: its last column and corner go beside the tiles
-  const long long vo = tb.vec_off[s];
-  if (vo >= 0 && I == J) {
-    float *vec = tb.ws + vo;
-    if (threadIdx.x < NB) vec[I * NB + threadIdx.x] = src[(long long)(I * NB + threadIdx.x) * d + d - 1];
-    if (I == 0 && threadIdx.x == 0) vec[3 * (long long)dc] = src[(long long)(d - 1) * d + d - 1];   // scal[0]
+  // clamped addresses, so that the loads are in flight together (behind tests they took 30 us)
+  const int rows = dc - I * NB;
+#pragma unroll
+  for (int in = 0; in < 2; ++in) {
+    const unsigned o = (unsigned)(min(r0 + 32 * in, rows - 1) * d * (int)sizeof(float));
+#pragma unroll
+    for (int im = 0; im < 2; ++im) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          c.v[im][in][g][e] = gload1(src, o + (unsigned)(min(c0 + 32 * im + 8 * g + e, dc - 1) * (int)sizeof(float)));
+    }
   }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int im = 0; im < 2; ++im)
+#pragma unroll
+    for (int in = 0; in < 2; ++in)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = r0 + 32 * in, k = c0 + 32 * im + 8 * g + e;
+          c.v[im][in][g][e] = r < rows && k < dc ? -c.v[im][in][g][e] : I * NB + r == k ? -1.f : 0.f;
+        }
+}
+__device__ __forceinline__ void start_tile(const InvTables &tb, const SweepItem &it, TileRegs &c) {
+  if (it.start == kFromSlot)
+    tile_load(wave_uniform(slot_ptr(tb, it.c)), c);
+  else if (it.start == kFromZero)
+    tile_zero(c);
+  else
+    input_load(tb, it.matrix, it.at, c);
 }
 
 // ---------------------------------------------------------------------------
@@ -748,11 +770,12 @@ __device__ __forceinline__ void diag_role(const InvTables &tb, const SweepItem &
 // instead loses a factor of cond(L) in accuracy against the substitution.)  The
 // rank-1 term is added to the accumulators of the final product.
 // ---------------------------------------------------------------------------
-constexpr int kBorderChunk = 6;
+constexpr int kBorderChunk = 4;
 constexpr int kBorderSum = 0;     // part[j] = sum_{c in chunk j, c < i - 1} L(i,c) l_c
 constexpr int kBorderSolve = 1;   // l_i = U_ii^T (a_i - sum of the partial vectors - L(i,i-1) l_{i-1})
 constexpr int kBorderW = 2;       // w_i (+)= U(i,j) l_j, the first term (j = i) overwrites
 constexpr int kBorderPivot = 3;   // S = alpha - l^T l in float64, 1 / S, info
+constexpr int kBorderCopy = 4;    // a and alpha from the input
 struct BorderTask {
   int s, kind, i, j;
 };
@@ -828,6 +851,7 @@ __device__ __forceinline__ void border_role(const InvTables &tb, const BorderTas
     for (int e = threadIdx.x; e < (j1 - j0) * NB; e += THREADS) xs[e] = v.y[j0 * NB + e];
     __syncthreads();
     const float *tile = slot_ptr(tb, tile_slot(tb, t.s, i, j0));
+#pragma unroll 2
     for (int j = 0; j < j1 - j0; ++j) border_rows_acc(tile + (size_t)j * kSlotFloats, xs + j * NB, p);
   };
   if (t.kind == kBorderSum) {
@@ -856,6 +880,11 @@ __device__ __forceinline__ void border_role(const InvTables &tb, const BorderTas
       float *w = v.w + t.i * NB + threadIdx.x;
       *w = t.j == t.i ? sum : *w + sum;
     }
+  } else if (t.kind == kBorderCopy) {
+    const long long d = tb.dim[t.s];
+    const float *src = tb.in[t.s] + d - 1;
+    for (int i = threadIdx.x; i < v.dc; i += THREADS) v.a[i] = src[i * d];
+    if (threadIdx.x == 0) v.scal[0] = src[(d - 1) * d];
   } else {
     double *dred = reinterpret_cast<double *>(lds);
     double sum = 0.0;
@@ -893,34 +922,100 @@ __device__ __forceinline__ SweepItem load_item(const SweepItem *p) {
   it.a = uniform(p->a);
   it.b = uniform(p->b);
   it.blocks = uniform(p->blocks);
-  it.first = uniform(p->first);
+  it.start = uniform(p->start);
   it.ut = uniform(p->ut);
   it.col = uniform(p->col);
   it.caller = uniform(p->caller);
   it.core = uniform(p->core);
   it.border = uniform(p->border);
-  it.pad = 0;
+  it.matrix = uniform(p->matrix);
+  it.at = uniform(p->at);
   return it;
 }
 
-// One step of the sweep: every workgroup runs its list of items.  Behind an update the loads
-// of the next item's first panels are already in flight.
-__global__ __launch_bounds__(THREADS, 1) void sweep_kernel(InvTables tb, int range0) {
-  extern __shared__ char lds[];
+// The finished tile (I, J), I >= J, of the inverse and its mirror image, straight from the
+// accumulators: 16 bytes of a row per lane (at float granularity: rows of an odd-sized matrix do not
+// start on 16-byte boundaries) and 32 consecutive floats of a mirrored row per half wave.  The stores drain
+// behind the next item's products; laid out in LDS first, for whole rows, they kept the workgroup for
+// a fifth of the launch.  On the diagonal the lower triangle is written both ways.
+__device__ __forceinline__ void output_store(const InvTables &tb, const SweepItem &it, floatx16 (&acc)[2][2]) {
+  typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+  const int s = it.matrix, I = it.at & 0xffff, J = it.at >> 16;
+  const int d = uniform(tb.dim[s]), dc = uniform(tb.core[s]);
+  const long long vo = tb.vec_off[s];
+  float *out = const_cast<float *>(wave_uniform(tb.out[s]));
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r0 = I * NB + (wave >> 1) * 64 + (lane & 31), c0 = J * NB + (wave & 1) * 64 + 4 * (lane >> 5);
+  if (vo >= 0) {
+    // bordered matrix: + w w^T / S on the leading block, -w / S in the last row and column
+    const BorderVecs bv = border_vecs(tb, s);
+    const float sigma = bv.scal[2];
+#pragma unroll
+    for (int in = 0; in < 2; ++in) {
+      const float wi = sigma * bv.w[r0 + 32 * in];
+#pragma unroll
+      for (int im = 0; im < 2; ++im)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[im][in][v] += wi * bv.w[c0 + 32 * im + 8 * (v >> 2) + (v & 3)];
+    }
+    if (I == J && threadIdx.x < NB) {
+      const float b = -sigma * bv.w[I * NB + threadIdx.x];
+      out[(long long)(d - 1) * d + I * NB + threadIdx.x] = b;
+      out[(long long)(I * NB + threadIdx.x) * d + d - 1] = b;
+      if (I == 0 && threadIdx.x == 0) out[(long long)(d - 1) * d + d - 1] = sigma;
+    }
+  }
+  if (I > J && (I + 1) * NB <= dc) {   // (columns are below the rows)
+#pragma unroll
+    for (int in = 0; in < 2; ++in) {
+      const int r = r0 + 32 * in;
+      KFAC_GLOBAL_AS float *row = (KFAC_GLOBAL_AS float *)out + (long long)r * d + c0;
+      KFAC_GLOBAL_AS float *mirror = (KFAC_GLOBAL_AS float *)out + (long long)c0 * d + r;
+#pragma unroll
+      for (int im = 0; im < 2; ++im)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          floatx4u o;
+          o.x = acc[im][in][4 * g];
+          o.y = acc[im][in][4 * g + 1];
+          o.z = acc[im][in][4 * g + 2];
+          o.w = acc[im][in][4 * g + 3];
+          *(KFAC_GLOBAL_AS floatx4u *)(row + 32 * im + 8 * g) = o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) mirror[(long long)(32 * im + 8 * g + e) * d] = acc[im][in][4 * g + e];
+        }
+    }
+    return;
+  }
+#pragma unroll
+  for (int im = 0; im < 2; ++im)
+#pragma unroll
+    for (int in = 0; in < 2; ++in)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int r = r0 + 32 * in, c = c0 + 32 * im + 8 * (v >> 2) + (v & 3);
+        if (r < dc && c <= r) {
+          out[(long long)r * d + c] = acc[im][in][v];
+          out[(long long)c * d + r] = acc[im][in][v];
+        }
+      }
+}
+
+// The items of one launch: every workgroup runs its list.  Behind an update or a final product the loads
+// of the next item's first panels (and its tile) are already in flight.
+template <bool OUT>
+__device__ __forceinline__ void run_items(const InvTables &tb, int range0, char *lds) {
   const int2 range = tb.ranges[range0 + blockIdx.x];
   const int end = uniform(range.y);
   for (int i = uniform(range.x); i < end; ++i) {
     SweepItem it = load_item(tb.items + i);
-    if (it.kind == kItemBorder) {
+    if (!OUT && it.kind == kItemBorder) {
       border_role(tb, tb.btasks[it.border], reinterpret_cast<float *>(lds));
       continue;
     }
     TileRegs c;
-    if (it.first)
-      tile_zero(c);
-    else
-      tile_load(wave_uniform(slot_ptr(tb, it.c)), c);
-    if (it.blocks > 0) {
+    if (!OUT) start_tile(tb, it, c);
+    if (OUT || it.blocks > 0) {
       Cursor cu;
       cu.a = wave_uniform(slot_ptr(tb, it.a));
       cu.b = wave_uniform(slot_ptr(tb, it.b));
@@ -929,161 +1024,52 @@ __global__ __launch_bounds__(THREADS, 1) void sweep_kernel(InvTables tb, int ran
       product_start(cu, r, lds);
       for (;;) {   // this item and, as long as it is an update, those behind it
         const SweepItem next = load_item(tb.items + (i + 1 < end ? i + 1 : i));
-        const bool ahead = it.kind == kItemUpdate && i + 1 < end && next.kind != kItemBorder && next.blocks > 0;
+        const bool ahead =
+            i + 1 < end && (OUT || (it.kind == kItemUpdate && next.kind != kItemBorder && next.blocks > 0));
         cu.next_a = wave_uniform(slot_ptr(tb, next.a));
         cu.next_b = wave_uniform(slot_ptr(tb, next.b));
         cu.next_left = ahead ? next.blocks * 4 : 0;
-        const float *next_tile = wave_uniform(slot_ptr(tb, next.c));
         floatx16 acc[2][2];
-        tile_to_acc(c, acc);
+        if (OUT)
+          zero_acc<2, 2>(acc);
+        else
+          tile_to_acc(c, acc);
         product_run(it.blocks, cu, r, lds, acc, [&]() {
-          if (ahead) {
-            if (next.first)
-              tile_zero(c);
-            else
-              tile_load(next_tile, c);
-          }
+          if (!OUT && ahead) start_tile(tb, next, c);
         });
-        if (it.kind != kItemUpdate) {
-          tile_from_acc(c, acc);
-          break;
+        if (OUT) {
+          output_store(tb, it, acc);
+        } else {
+          if (it.kind != kItemUpdate) {
+            tile_from_acc(c, acc);
+            break;
+          }
+          TileRegs done;
+          tile_from_acc(done, acc);
+          tile_store(const_cast<float *>(wave_uniform(slot_ptr(tb, it.c))), done);
         }
-        TileRegs done;
-        tile_from_acc(done, acc);
-        tile_store(const_cast<float *>(wave_uniform(slot_ptr(tb, it.c))), done);
         if (!ahead) break;
         it = load_item(tb.items + ++i);
       }
     }
-    if (it.kind == kItemPanel)
-      panel_role(tb, it, c, lds);
-    else if (it.kind == kItemDiag)
-      diag_role(tb, it, c, reinterpret_cast<float *>(lds));
-  }
-}
-
-// The finished tile (I, J), I >= J, of the inverse and its mirror image written to C
-// (leading dimension d, rows and columns below dt): the whole tile is
-// laid out in LDS (128 x 129 floats), then every thread stores 16 bytes at
-// a time (at float granularity: rows of an odd-sized matrix do not start on
-// 16-byte boundaries), rows of the tile and rows of the mirrored tile alike.
-constexpr int kWholeTileLdsBytes = NB * LS * (int)sizeof(float);
-__device__ __forceinline__ void write_whole_tile(const floatx16 (&acc)[2][2], float *lds, int I, int J, int dt,
-                                                 int d, float *__restrict__ C) {
-  typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
-  constexpr int LD = LS;
-  {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    float *p = lds + ((wave >> 1) * 64 + (lane & 31)) * LD + (wave & 1) * 64 + 4 * (lane >> 5);
-#pragma unroll
-    for (int im = 0; im < 2; ++im)
-#pragma unroll
-      for (int in = 0; in < 2; ++in)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) p[in * 32 * LD + im * 32 + 8 * (v >> 2) + (v & 3)] = acc[im][in][v];
-  }
-  __syncthreads();
-  const int q = (threadIdx.x & 31) * 4;    // four columns
-  const int r0 = threadIdx.x >> 5;         // 8 rows per pass
-  const int row0 = I * 128, col0 = J * 128;
-  const bool diag = I == J;
-#pragma unroll 4
-  for (int p = 0; p < 16; ++p) {
-    const int lr = r0 + 8 * p;
-    const int r = row0 + lr, c = col0 + q;
-    if (r >= dt) continue;
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (!diag || q + e <= lr) ? lds[lr * LD + q + e] : lds[(q + e) * LD + lr];
-    float *dst = C + (long long)r * d + c;
-    if (c + 3 < dt) {
-      floatx4u o;
-      o.x = v[0];
-      o.y = v[1];
-      o.z = v[2];
-      o.w = v[3];
-      *reinterpret_cast<floatx4u *>(dst) = o;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c + e < dt) dst[e] = v[e];
-    }
-  }
-  if (diag) return;
-  // mirrored tile (J, I): its row lr is column lr of the tile
-#pragma unroll 4
-  for (int p = 0; p < 16; ++p) {
-    const int lr = r0 + 8 * p;
-    const int r = col0 + lr, c = row0 + q;
-    if (r >= dt) continue;
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = lds[(q + e) * LD + lr];
-    float *dst = C + (long long)r * d + c;
-    if (c + 3 < dt) {
-      floatx4u o;
-      o.x = v[0];
-      o.y = v[1];
-      o.z = v[2];
-      o.w = v[3];
-      *reinterpret_cast<floatx4u *>(dst) = o;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c + e < dt) dst[e] = v[e];
+    if (!OUT) {
+      if (it.kind == kItemPanel)
+        panel_role(tb, it, c, lds);
+      else if (it.kind == kItemDiag)
+        diag_role(tb, it, c, reinterpret_cast<float *>(lds));
     }
   }
 }
 
-// out(i,j) = sum_{k >= i} U(i,k) U(j,k)^T for i >= j, written with its mirror.
-// One task per tile; the table deals whole tile rows to XCDs (see the plan).
-__global__ __launch_bounds__(THREADS, 1) void lauum_kernel(InvTables tb, int task0) {
+// one step of the sweep
+__global__ __launch_bounds__(THREADS, 1) void sweep_kernel(InvTables tb, int range0) {
   extern __shared__ char lds[];
-  const TileTask t = tb.tasks[task0 + blockIdx.x];
-  if (t.K == 0) return;   // padding of an XCD's shorter list
-  const int s = uniform((int)t.c_off);
-  const int I = uniform(t.flags) & 0xffff, J = uniform(t.flags) >> 16;
-  const int d = tb.dim[s], dc = tb.core[s];
-  const long long vo = tb.vec_off[s];
-  float *out = tb.out[s];
-  floatx16 acc[2][2];
-  {
-    Cursor cu;
-    cu.a = wave_uniform(slot_ptr(tb, (int)(t.a_off / (NB * NB))));
-    cu.b = wave_uniform(slot_ptr(tb, (int)(t.b_off / (NB * NB))));
-    cu.left = uniform(t.K) / NB * 4;
-    cu.next_a = cu.next_b = nullptr;
-    cu.next_left = 0;
-    Panels r[2];
-    zero_acc<2, 2>(acc);
-    product_start(cu, r, lds);
-    product_run(uniform(t.K) / NB, cu, r, lds, acc, []() {});
-  }
-  if (vo >= 0) {
-    // bordered matrix: + w w^T / S on the leading block, -w / S in the last row and column
-    const BorderVecs bv = border_vecs(tb, s);
-    const float sigma = bv.scal[2];
-    const float *wi = bv.w + I * NB, *wj = bv.w + J * NB;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int im = 0; im < 2; ++im)
-#pragma unroll
-      for (int in = 0; in < 2; ++in)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = ((wave >> 1) * 2 + in) * 32 + (lane & 31);
-          const int col = ((wave & 1) * 2 + im) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-          acc[im][in][v] += sigma * wi[row] * wj[col];
-        }
-    if (I == J && threadIdx.x < NB) {
-      const float b = -sigma * wi[threadIdx.x];
-      out[(long long)(d - 1) * d + I * NB + threadIdx.x] = b;
-      out[(long long)(I * NB + threadIdx.x) * d + d - 1] = b;
-      if (I == 0 && threadIdx.x == 0) out[(long long)(d - 1) * d + d - 1] = sigma;
-    }
-  }
-  static_assert(kWholeTileLdsBytes <= kTileLdsBytes, "the tile must fit the panels' LDS");
-  write_whole_tile(acc, reinterpret_cast<float *>(lds), I, J, dc, d, out);
+  run_items<false>(tb, range0, lds);
+}
+// out(i,j) = sum_{k >= i} U(i,k) U(j,k)^T for i >= j, written with its mirror
+__global__ __launch_bounds__(THREADS, 1) void lauum_kernel(InvTables tb, int range0) {
+  extern __shared__ char lds[];
+  run_items<true>(tb, range0, lds);
 }
 
 constexpr int kDiagLdsBytes = NB * LS * (int)sizeof(float);
@@ -1101,7 +1087,7 @@ struct UpdateLaunch {
 struct kfac_inverse_plan {
   int count = 0;
   int max_t = 0;
-  int group = 3;                   // block columns per trailing update (2 to 4 within 2 %)
+  int group = 4;                   // block columns per trailing update (3 to 5 within 2 %)
   std::vector<int> order;          // slot -> caller index
   std::vector<int> nt;             // per slot
   std::vector<int> nactive;        // per step
@@ -1115,7 +1101,7 @@ struct kfac_inverse_plan {
   std::vector<UpdateLaunch> rest;
   // a captured graph holds one stream's launches whatever this says (kept for the ABI)
   bool capture_origin = false;
-  int first_tiles = 0;             // copy-in: tiles of the matrices that join at the first step
+  int first_tiles = 0;             // lower tiles of the matrices that join at the first step
   int total_tiles = 0;
   int lauum_task0 = 0, lauum_count = 0;
   // bordered matrices: their vector tasks per step (beside the diagonal tiles, beside the
@@ -1127,6 +1113,7 @@ struct kfac_inverse_plan {
   // the launches of the sweep (the first factors the first diagonal tiles): workgroups and
   // their item ranges
   std::vector<int> sweep_range0, sweep_count;
+  int out_range0 = 0, out_count = 0;   // the final products
   kfac::DevTable d_items, d_ranges;
   int ut0 = 0;                     // first slot of the U_kk^T buffers
   size_t ws_floats = 0;            // slots and border vectors
@@ -1165,10 +1152,11 @@ constexpr double kUpdateCost = 0.7, kPanelCost = 2.4, kDiagCost = 7.2;
 constexpr int kBlock = 6;
 double item_cost(const SweepItem &it) {
   switch (it.kind) {
-    case kItemUpdate: return kUpdateCost + it.blocks;
+    case kItemUpdate:
+    case kItemOut: return kUpdateCost + it.blocks;
     case kItemPanel: return kPanelCost + it.blocks;
     case kItemDiag: return kDiagCost + it.blocks;
-    default: return 1.5 + 0.5 * it.blocks;   // (of tiles read)
+    default: return 1.2 + 0.8 * it.blocks;   // (of tiles read)
   }
 }
 
@@ -1303,7 +1291,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
   p->nborder = (int)border_slots.size();
   p->total_tiles = tile_cs[count];
   p->first_tiles = tile_cs[count];   // set once the steps are known
-  // copy-in: the lower tiles of every matrix in row-major order, slot by slot
+  // the lower tiles of every matrix in row-major order, slot by slot
   std::vector<int2> tile_owner;
   tile_owner.reserve((size_t)p->total_tiles);
   for (int s = 0; s < count; ++s)
@@ -1358,6 +1346,8 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       p->bfinal_count = (int)btasks.size() - first;
     }
   }
+  const int bcopy_task0 = (int)btasks.size();   // before the first step
+  for (int s : border_slots) btasks.push_back(BorderTask{s, kBorderCopy, 0, 0});
   if (btasks.empty()) btasks.push_back(BorderTask{0, 0, 0, 0});
   auto tile_off = [&](int s, int I, int J) {
     return off[s] + ((long long)I * p->nt[s] + J) * (long long)(NB * NB);
@@ -1508,7 +1498,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       it.a = slot_of(t.a_off);
       it.b = slot_of(t.b_off);
       it.blocks = t.K / NB;
-      it.first = (t.flags & kFirst) != 0;
+      it.start = t.flags & kFirst ? kFromZero : kFromSlot;
       return it;
     };
     const int nslots = p->ut0;
@@ -1516,7 +1506,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       return (int)(std::upper_bound(off.begin(), off.end(), (long long)c * (NB * NB)) - off.begin()) - 1;
     };
     struct Owed {
-      int a, b, blocks, first;
+      int a, b, blocks, start;
     };
     std::vector<Owed> owed(nslots, Owed{0, 0, 0, 0});   // column products listed so far, by slot
     std::vector<std::vector<SweepItem>> rest(p->max_t + 1);   // trailing updates by step
@@ -1549,7 +1539,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       if (g >= 0)
         for (const TileTask &t : column_list[g]) {
           Owed &o = owed[slot_of(t.c_off)];
-          if (o.blocks == 0) o = Owed{slot_of(t.a_off), slot_of(t.b_off), 0, (t.flags & kFirst) != 0};
+          if (o.blocks == 0) o = Owed{slot_of(t.a_off), slot_of(t.b_off), 0, t.flags & kFirst ? kFromZero : kFromSlot};
           o.blocks += t.K / NB;
         }
       // the chains: matrices with a diagonal tile in step g + 1
@@ -1597,7 +1587,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
               it.a = o.a;
               it.b = o.b;
               it.blocks = o.blocks;
-              it.first = o.first;
+              it.start = o.start;
             }
             if (x == k + 1)
               chains[chain_of[s]].insert(chains[chain_of[s]].begin(), it);
@@ -1607,7 +1597,7 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
         }
         list.insert(list.end(), rest[g].begin(), rest[g].end());
         rest[g].clear();
-        for (int pass = 0; pass < 2; ++pass) {
+        for (int pass = 0; pass < 2; ++pass) {   // vector tasks
           const int t0 = pass ? p->bpanel_task0[g] : p->bdiag_task0[g], n = pass ? p->bpanel_count[g] : p->bdiag_count[g];
           for (int i = 0; i < n; ++i) {
             SweepItem it = {};
@@ -1615,11 +1605,19 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
             it.border = t0 + i;
             // read by the cost alone: the tiles of the task
             const BorderTask &b = btasks[t0 + i];
-            it.blocks = b.kind == kBorderSum ? std::min(kBorderChunk, b.i - 1 - b.j * kBorderChunk) : 1;
+            it.blocks = b.kind == kBorderSum ? std::min(kBorderChunk, b.i - 1 - b.j * kBorderChunk) : b.kind == kBorderSolve ? 2 : 1;
             vectors.push_back(it);
           }
         }
       }
+      if (g < 0)
+        for (int i = 0; i < (int)border_slots.size(); ++i) {
+          SweepItem it = {};
+          it.kind = kItemBorder;
+          it.border = bcopy_task0 + i;
+          it.blocks = 1;
+          vectors.push_back(it);
+        }
       if (g < 0 || rest_list[g].empty()) continue;
       // The trailing update of the group that ends with step g, over the next group's steps: as much
       // to each as makes their products equal.  A diagonal tile whose chain runs in the last of them comes
@@ -1686,6 +1684,22 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
         }
       for (const SweepItem &it : before) where[it.c] = -1;
     }
+    // the item that comes to a lower tile first reads it from the input
+    std::vector<char> seen(nslots, 0);
+    auto mark = [&](SweepItem &it) {
+      if (it.kind == kItemBorder || seen[it.c]) return;
+      seen[it.c] = 1;
+      const int s = slot_matrix(it.c), t = it.c - slot_of(off[s]), I = t / p->nt[s], J = t % p->nt[s];
+      if (I < J) return;
+      it.start = kFromInput;
+      it.matrix = s;
+      it.at = I | (J << 16);
+    };
+    for (Launch &l : launches) {
+      for (std::vector<SweepItem> &chain : l.chains)
+        for (SweepItem &it : chain) mark(it);
+      for (SweepItem &it : l.list) mark(it);
+    }
     for (Launch &l : launches) {
       int range0, n;
       sort_blocks(l.list);
@@ -1694,54 +1708,34 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
       p->sweep_count.push_back(n);
     }
   }
-  // Final products out(I,J) = sum_k U(I,k) U(J,k)^T, in blocks of kBlock x kBlock tiles whose operand
-  // rows stay in an XCD's L2 (workgroup i of a launch runs on XCD i % 8); blocks are dealt longest first to
-  // the XCD with the least work, and each XCD runs its long-K blocks first.
+  // Final products out(I,J) = sum_k U(I,k) U(J,k)^T, one task per lower tile, long sums first
   {
-    struct Block { int s, I, J; double cost; };
-    std::vector<Block> blocks;
-    for (int s = 0; s < count; ++s)
-      for (int I = 0; I < p->nt[s]; I += kBlock)
-        for (int J = 0; J <= I; J += kBlock) {
-          Block b{s, I, J, 0.0};
-          for (int i = I; i < std::min(I + kBlock, p->nt[s]); ++i)
-            b.cost += (std::min(i + 1, J + kBlock) - J) * (p->nt[s] - i + 1.0);
-          blocks.push_back(b);
-        }
-    std::stable_sort(blocks.begin(), blocks.end(), [](const Block &a, const Block &b) { return a.cost > b.cost; });
-    std::vector<Block> mine[8];
-    double load[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (const Block &b : blocks) {
-      int x = 0;
-      for (int i = 1; i < 8; ++i)
-        if (load[i] < load[x]) x = i;
-      mine[x].push_back(b);
-      load[x] += b.cost;
-    }
-    std::vector<TileTask> list[8];
-    size_t longest = 0;
-    for (int x = 0; x < 8; ++x) {
-      std::stable_sort(mine[x].begin(), mine[x].end(), [&](const Block &a, const Block &b) {
-        return p->nt[a.s] - a.I > p->nt[b.s] - b.I;
-      });
-      for (const Block &b : mine[x])
-        for (int I = b.I; I < std::min(b.I + kBlock, p->nt[b.s]); ++I)
-          for (int J = b.J; J < std::min(I + 1, b.J + kBlock); ++J) {
-            TileTask t;
-            t.c_off = b.s;
-            t.a_off = tile_off(b.s, I, I);
-            t.b_off = tile_off(b.s, J, I);
-            t.K = (p->nt[b.s] - I) * NB;
-            t.flags = I | (J << 16);
-            list[x].push_back(t);
-          }
-      longest = std::max(longest, list[x].size());
-    }
     p->lauum_task0 = (int)tasks.size();
-    for (size_t i = 0; i < longest; ++i)
-      for (int x = 0; x < 8; ++x)
-        tasks.push_back(i < list[x].size() ? list[x][i] : TileTask{0, 0, 0, 0, 0});
-    p->lauum_count = (int)(longest * 8);
+    std::vector<SweepItem> list;
+    for (int s = 0; s < count; ++s)
+      for (int I0 = 0; I0 < p->nt[s]; I0 += kBlock)
+        for (int J0 = 0; J0 <= I0; J0 += kBlock)
+          for (int I = I0; I < std::min(I0 + kBlock, p->nt[s]); ++I)
+            for (int J = J0; J < std::min(I + 1, J0 + kBlock); ++J) {
+              TileTask t;
+              t.c_off = s;
+              t.a_off = tile_off(s, I, I);
+              t.b_off = tile_off(s, J, I);
+              t.K = (p->nt[s] - I) * NB;
+              t.flags = I | (J << 16);
+              tasks.push_back(t);
+              SweepItem it = {};
+              it.kind = kItemOut;
+              it.a = (int)(t.a_off / (NB * NB));
+              it.b = (int)(t.b_off / (NB * NB));
+              it.blocks = t.K / NB;
+              it.start = kFromZero;
+              it.matrix = s;
+              it.at = t.flags;
+              list.push_back(it);
+            }
+    p->lauum_count = (int)tasks.size() - p->lauum_task0;
+    sweep.launch({}, list, {}, &p->out_range0, &p->out_count);
   }
   if (tasks.empty()) tasks.push_back(TileTask{0, 0, 0, 0, 0});
   int rc = KFAC_OK;
@@ -1755,8 +1749,8 @@ extern "C" int kfac_inverse_plan_create(int count, const int32_t *dims,
   up(p->d_btasks, btasks.data(), sizeof(BorderTask) * btasks.size());
   up(p->d_nt, p->nt.data(), sizeof(int) * count);
   up(p->d_off, off.data(), sizeof(long long) * count);
-  up(p->d_tile_owner, tile_owner.data(), sizeof(int2) * tile_owner.size());
-  up(p->d_tasks, tasks.data(), sizeof(TileTask) * tasks.size());
+  p->d_tile_owner.keep(tile_owner.data(), sizeof(int2) * tile_owner.size());   // for checks on the host
+  p->d_tasks.keep(tasks.data(), sizeof(TileTask) * tasks.size());
   if (sweep.items.empty()) sweep.items.push_back(SweepItem{});
   if (sweep.ranges.empty()) sweep.ranges.push_back(make_int2(0, 0));
   up(p->d_items, sweep.items.data(), sizeof(SweepItem) * sweep.items.size());
@@ -1825,8 +1819,6 @@ extern "C" int kfac_spd_inverse_batched_f32(kfac_inverse_plan_t plan,
   tb.vec_off = plan->d_vec.as<const long long>();
   tb.nt = plan->d_nt.as<const int>();
   tb.ws_off = plan->d_off.as<const long long>();
-  tb.tile_owner = plan->d_tile_owner.as<const int2>();
-  tb.tasks = plan->d_tasks.as<const TileTask>();
   tb.items = plan->d_items.as<const SweepItem>();
   tb.ranges = plan->d_ranges.as<const int2>();
   tb.btasks = plan->d_btasks.as<const BorderTask>();
@@ -1835,9 +1827,7 @@ extern "C" int kfac_spd_inverse_batched_f32(kfac_inverse_plan_t plan,
   tb.ws = reinterpret_cast<float *>(base);
   tb.info = info_dev;
 
-  kfac::TimedLaunch timed_call(KFAC_TIMED_INV_CALL, s);   // copy-in to the final product
-  if (plan->total_tiles > 0) KFAC_LAUNCH(copy_in_kernel, dim3(plan->total_tiles), dim3(256), 0, s, tb);
-  KFAC_HIP_CHECK(hipGetLastError());
+  kfac::TimedLaunch timed_call(KFAC_TIMED_INV_CALL, s);   // first launch to the final product
   for (size_t i = 0; i < plan->sweep_count.size(); ++i) {
     if (plan->sweep_count[i] == 0) continue;
     kfac::TimedLaunch timed(KFAC_TIMED_INV_UPDATE, s);
@@ -1850,8 +1840,7 @@ extern "C" int kfac_spd_inverse_batched_f32(kfac_inverse_plan_t plan,
   }
   {
     kfac::TimedLaunch timed(KFAC_TIMED_INV_LAUUM, s);
-    KFAC_LAUNCH(lauum_kernel, dim3(plan->lauum_count), dim3(THREADS), kTileLdsBytes, s, tb,
-                       plan->lauum_task0);
+    KFAC_LAUNCH(lauum_kernel, dim3(plan->out_count), dim3(THREADS), kTileLdsBytes, s, tb, plan->out_range0);
   }
   KFAC_HIP_CHECK(hipGetLastError());
   return KFAC_OK;

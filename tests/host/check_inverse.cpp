@@ -71,7 +71,9 @@ void check_sweep(const kfac_inverse_plan *plan, const std::vector<long long> &of
         if (it.kind == kItemBorder) {
           const BorderTask &b = bt[it.border];
           const int at = (int)(offs[b.s] / (NB * NB)), T = plan->nt[b.s];
-          if (b.kind == kBorderSum) {
+          if (b.kind == kBorderCopy) {
+            EXPECT(l == 0, "%s: launch %d border copy", what, l);
+          } else if (b.kind == kBorderSum) {
             for (int j = b.j * kBorderChunk; j < std::min((b.j + 1) * kBorderChunk, b.i - 1); ++j)
               EXPECT(final_for(at + b.i * T + j) && tile[at + b.i * T + j].final_in < l && solved[b.s] >= j &&
                          (solved[b.s] > j || solved_in[b.s] < l),
@@ -95,10 +97,13 @@ void check_sweep(const kfac_inverse_plan *plan, const std::vector<long long> &of
         State &t = tile[it.c];
         const int at = (int)(offs[t.s] / (NB * NB)), T = plan->nt[t.s];
         EXPECT(t.final_in < 0 && (t.touched_in < l || t.touched_by == w), "%s: launch %d tile (%d,%d) twice", what, l, t.I, t.J);
+        const int start = t.touched_in >= 0 ? kFromSlot : t.I < t.J ? kFromZero : kFromInput;
+        EXPECT(it.start == start && (start != kFromInput || (it.matrix == t.s && it.at == (t.I | (t.J << 16)))),
+               "%s: launch %d tile (%d,%d) starts from %d", what, l, t.I, t.J, it.start);
         if (it.blocks > 0) {
           EXPECT(it.a == at + t.I * T + t.upto && it.b == at + t.J * T + t.upto, "%s: launch %d tile (%d,%d): runs do not go on at column %d",
                  what, l, t.I, t.J, t.upto);
-          EXPECT((it.first != 0) == (t.I < t.J && t.upto == t.I), "%s: launch %d tile (%d,%d) first", what, l, t.I, t.J);
+          
           for (int j = 0; j < it.blocks; ++j)
             EXPECT(final_for(it.a + j) && final_for(it.b + j), "%s: launch %d tile (%d,%d) reads column %d too early", what, l, t.I,
                    t.J, t.upto + j);
@@ -133,6 +138,25 @@ void check_sweep(const kfac_inverse_plan *plan, const std::vector<long long> &of
       solved_in[v.first] = l;
     }
   }
+  // the final products
+  EXPECT(plan->out_count >= 0 && plan->out_count <= kSweepWorkgroups && plan->out_range0 + plan->out_count <= nranges, "%s: final ranges", what);
+  std::map<std::pair<int, int>, int> written;
+  for (int w = 0; w < plan->out_count; ++w) {
+    const int2 r = ranges[plan->out_range0 + w];
+    EXPECT(r.x >= 0 && r.x <= r.y && r.y <= nitems, "%s: final workgroup %d items", what, w);
+    for (int i = r.x; i < r.y && i < nitems; ++i, ++seen_items) {
+      const SweepItem &it = items[i];
+      const int s = it.matrix, I = it.at & 0xffff, J = it.at >> 16;
+      EXPECT(it.kind == kItemOut && s >= 0 && s < count && J <= I && I < plan->nt[s], "%s: final item", what);
+      if (!(s >= 0 && s < count)) continue;
+      const int at = (int)(offs[s] / (NB * NB)), T = plan->nt[s];
+      EXPECT(it.a == at + I * T + I && it.b == at + J * T + I && it.blocks == T - I, "%s: final item (%d,%d) operands", what, I, J);
+      ++written[{s, it.at}];
+    }
+  }
+  for (int s = 0; s < count; ++s)
+    for (int I = 0; I < plan->nt[s]; ++I)
+      for (int J = 0; J <= I; ++J) EXPECT((written[{s, I | (J << 16)}] == 1), "%s: slot %d output tile (%d,%d)", what, s, I, J);
   EXPECT(seen_items == nitems || plan->max_t == 0, "%s: items outside the launches", what);
   for (const State &t : tile) EXPECT(t.final_in >= 0, "%s: slot %d tile (%d,%d) never final", what, t.s, t.I, t.J);
 }
