@@ -507,7 +507,7 @@ def run_step_config(args, name, cfg, host=None):
     families = {
         'cov_syrk': family_roofline(
             'cov_syrk', 'covariance SYRK family: shift::corr_kernel, syrk_rows_kernel, syrk_group_kernel, syrk_kernel, '
-            'syrk_conv_kernel and the kernels around them (edge_sums, corr_finish, assemble, finish_group, finish, reduce)',
+            'syrk_conv_kernel and the kernels around them (split_input, corr_finish, assemble, finish_group, finish, reduce)',
             cov_executed, ('syrk', 'cov_aux'), fam, empty, one_stream, reference_flop=flops['cov'],
             peak=cov_peak(layers, batch)),
         'inverse_tiles': family_roofline(
@@ -1018,8 +1018,8 @@ KERNEL_FAMILIES = (
     ('preconditioning GEMMs (with their split-K finish and the batch-norm GEMV)', ('gemm_', 'gemv_', 'bn_select')),
     ('batch-norm statistics and finish', ('bn_',)),
     ('batch-norm rank-n inverses', ('lr_',)),
-    ('split-K finish, edge sums and assembly of the covariances', ('finish_', 'reduce_kernel', 'shift::assemble',
-                                                                  'shift::edge_sums')),
+    ('split-K finish, input planes and assembly of the covariances', ('finish_', 'reduce_kernel', 'shift::assemble',
+                                                                  'shift::split_input')),
     ('inverse tile kernels', ('sweep_kernel', 'lauum_kernel', 'border_kernel')),
     ('damping', ('pi_damp', 'add_diag')),
     ('pack / unpack / copy', ('pack_kernel', 'unpack_kernel', 'stream_copy', 'stream_fanout')),
@@ -1156,7 +1156,7 @@ def summarize_mfma(pmc_dir, out_path, command):
 TRAFFIC_FAMILIES = (
     # family, kernels of the family, the kernel whose launches count the steps of the run
     ('cov_syrk', ('syrk_', 'shift::corr_kernel', 'finish_group_kernel', 'finish_kernel', 'reduce_kernel',
-                  'shift::assemble', 'shift::edge_sums', 'shift::corr_finish'), 'finish_group_kernel'),
+                  'shift::assemble', 'shift::split_input', 'shift::corr_finish'), 'finish_group_kernel'),
     ('inverse_tiles', ('sweep_kernel', 'border_kernel', 'lauum_kernel'), 'lauum_kernel'),
     ('precond_gemm', ('gemm_group', 'gemv_', 'bn_select'), 'gemm_group_finish_kernel<1>'),
 )

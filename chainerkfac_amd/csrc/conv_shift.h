@@ -24,69 +24,9 @@
 // (im2col, A = col^T col / n, the ones column of _bias).
 #pragma once
 
+#include <type_traits>
+
 #include "mma_core.h"
-
-namespace kfac {
-namespace mma {
-
-constexpr int kRowStride = KT + 1;   // floats from row to row of the first operand's LDS panel
-
-// First operand of a group of products: rows = channels, k = (sample, p), p < L
-// running over the group's domain (a whole image, one image row, one border column
-// or one pixel):
-//   element = base[sample * sample_stride + row * row_stride + (p / line_len) * line_stride + p % line_len],
-// 0 for rows >= rows_valid and k past the end of the slice.  Dword loads, the 32
-// lanes of a half-wave on 32 consecutive k of one row (the layout of LoaderKC's
-// scalar variant).
-template <int ROWS>
-struct LoaderDomain {
-  static constexpr int NR = ROWS / 8;   // rows per thread
-  struct Regs {
-    float v[NR];
-    bool kvalid;
-  };
-  const float *base;
-  unsigned sample_stride, row_stride;
-  unsigned L, line_len, line_stride;
-  int rows_valid;
-  int first_row;
-  unsigned last_off;
-
-  __device__ __forceinline__ void init(int row0) {
-    first_row = row0 + (team_tid() >> 5);
-    last_off = (unsigned)(rows_valid > 0 ? rows_valid - 1 : 0) * row_stride;
-  }
-
-  __device__ __forceinline__ void load(Regs &r, long long k0, long long k_end) const {
-    const long long kg = k0 + (team_tid() & 31);
-    r.kvalid = kg < k_end;
-    const unsigned kc = r.kvalid ? (unsigned)kg : 0u;
-    const unsigned s = kc / L;
-    const unsigned p = kc - s * L;
-    const unsigned a = p / line_len;
-    const unsigned koff = s * sample_stride + a * line_stride + (p - a * line_len);
-    int fr = first_row;
-    asm volatile("" : "+v"(fr));   // keep the NR row offsets out of registers (see LoaderKC)
-    const unsigned off0 = (unsigned)fr * row_stride;
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const unsigned off = off0 + (unsigned)(8 * i) * row_stride;
-      r.v[i] = gload1(base, (koff + (off < last_off ? off : last_off)) * 4u);
-    }
-  }
-
-  __device__ __forceinline__ void store(const Regs &r, float *lds) const {
-    float *p = lds + (team_tid() >> 5) * kRowStride + (team_tid() & 31);
-#pragma unroll
-    for (int i = 0; i < NR; ++i) {
-      const int row = first_row + 8 * i;
-      p[8 * i * kRowStride] = (r.kvalid && row < rows_valid) ? r.v[i] : 0.f;
-    }
-  }
-};
-
-}  // namespace mma
-}  // namespace kfac
 
 namespace kfac {
 namespace shift {
@@ -105,37 +45,42 @@ constexpr int kProducts = 29;
 constexpr int kGroups = 11;
 constexpr int kChannelSums = 9;   // whole image, first / last row, first / last column, 4 corners
 
+// Pixels per sample and channel, as planes in the workspace: the whole image (0), and its first and
+// last column (1, 2), in which a column is a line.  Pixel (u, v), u < h lines of v < w, of sample s and
+// channel c is the input's
+//   x[s * C * H * W + c * H * W + org + u * su + v * sv]
+// and lies at  base + (s * C + c) * pitch + u * pw + v  of every plane.  Lines are padded with
+// two zeros and followed by zeros up to pitch, so a pixel up to two columns or lines outside
+// the image is read as zero without a test; `guard` zeros precede the first row.
+struct Source {
+  unsigned base, pitch, guard;   // elements
+  int h, w, pw, org, su, sv;
+};
+constexpr int kSources = 3;
+
 // Products that share their first operand and differ in the second operand's
-// shift along the domain are computed together, ns (3 or 5) at a time.  A domain
-// is a set of pixels per sample, numbered p < L: the whole image (three groups,
-// one per row shift di: column shifts 0..2 for di = 0, whose negative ones are
-// transposes, and -2..2 for di = 1, 2), the first or last image row (column shifts
-// 0..2), the first or last image column (row shifts 0..2, which move along the
-// column) or one corner pixel.
-//   memory:  pixel p of sample s, channel c at
-//            base[s * sample_stride + c * row_stride + (p / mem_line) * line_stride + p % mem_line]
-//   shift e (= dj0 + 0 .. ns - 1) of row shift di:  p -> p + di * vline + e, inside the
-//   domain if  p / vline + di < amax  and  0 <= p % vline + e < vline
-// The whole image and its first / last row are read from the input tensor; the
-// first / last column and the corners from a compact copy of the two border columns
-// ([2][n][C][H], written by edge_sums_kernel), where a column is contiguous.
+// shift along the line are computed together, ns (3 or 5) at a time: of the whole image three groups,
+// one per row shift di (column shifts 0..2 for di = 0, whose negative ones are
+// transposes, and -2..2 for di = 1, 2), of a row or column shifts 0..2, of a corner pixel one.
 // Layers of at most 32 channels would fill a quarter of a 64 x 64 tile.  Their
 // whole-image groups are `stacked`: the 64 first-operand rows are the channels at
 // row shift 0 and, 32 rows on, the same channels one image row up (X(c, u - 1, v):
 // against a second operand at row shift di that is the product of row shift di + 1),
-// the 64 second-operand rows the channels and, 32 rows on, the same channels three
-// columns on -- so the four 32 x 32 blocks of a tile and its three column offsets
-// are the products of row shifts di, di + 1 and column shifts dj0 .. dj0 + 5.
+// the 64 second-operand rows the channels twice, the waves of the second 32 taking the column shifts
+// three further on -- so the four 32 x 32 blocks of a tile and its three column offsets
+// are the products of row shifts di, di + 1 and column shifts dj0 .. dj0 + 4.
 // stacked = 2: both first-operand halves; 1: only the first (the waves of the
 // second issue no matrix instructions); 0: plain rows = channels.
 struct ShiftGroup {
-  const float *base;
-  unsigned sample_stride, row_stride, line_stride;
-  unsigned L, mem_line, vline;
-  short di, dj0, ns, amax;
-  int stacked;
+  int source;
+  int org;             // first position of the domain: an image row or the last pixel of a column
+  int valid, L;        // positions of a sample: those of the domain (of an image: all), and with two more, at
+                       // which the first operand is zero, to a multiple of 8
+  int offset;          // second operand this many elements on: di * pw
+  short dj0, ns, stacked;
   int K;               // reduction length: samples * L
   int klen, nsplit;    // k-values per slice (a multiple of KT), slices
+  int r32, step32;     // a panel of 32 k-values on: this far inside a sample, this far in memory
   int task0;           // first work item of the group
   unsigned part_off;   // its partial tiles: [item][shift][rows of the A tile][64]
 };
@@ -156,6 +101,11 @@ struct Plan {
   int C, H, W, n;
   int tiles_a, tiles_b;     // tile grid: 64 * WM first-operand channels x 64 second-operand channels
   int nsmall, total;        // work items of the groups 3.. (strips and corners), and of all groups
+  int nchunk;               // chunks of samples of the pass over the input
+  unsigned short *planes;
+  unsigned plane_stride;    // elements
+  int *odd;                 // [chunk][channel]: has values outside the split's range
+  Source src[kSources];
   ShiftGroup grp[kGroups];
   Product prod[kProducts];
 };
@@ -169,200 +119,398 @@ __device__ __forceinline__ int item_of_block(int bid, int total) {
   return xcd * base + (xcd < rem ? xcd : rem) + idx;
 }
 
-// k runs over (sample, pixel of the domain).  The workgroup stages 32 k-values of
-// its 64 * WM first-operand channels and the 36 values from di * vline - 2 places on
-// of its 64 second-operand channels; the NS shifts read the latter at NS
-// consecutive offsets.  Where a shifted pixel falls outside the domain is the same
-// for all channels: one 32-bit mask per shift and panel, applied to the operand
-// values as they are read (as 64-bit lane masks in scalar registers: one select
-// per value).  Per panel a wave issues 16 * WM * NS matrix instructions for
-// (8 * WM + 9) global loads of its lanes; one product at a time (WM * WM
-// instructions for 16 * WM loads per step) is bound by the loads.
-constexpr int kShiftCols = 36;
-constexpr int kShiftStride = 37;   // odd: the 32 rows of an operand read on 32 banks
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
-template <int WM, int NS, bool STACKED = false>
-__device__ __forceinline__ void corr_shifts_body(const Plan &pl, const ShiftGroup &g, int q, float *lds,
+// One pass over the input before the products: channel blockIdx.x of the samples of chunk
+// blockIdx.y (a contiguous range).  Writes the planes of all sources, padding included; the
+// per-channel sums that make the ones column,
+//   sums[chunk][c][0..8] = whole image, first row, last row, first column, last
+//   column, corners (first,first) (first,last) (last,first) (last,last);
+// and whether a value is outside the split's range (mma_core.h).  A thread takes eight positions
+// at a time.  The products read every value five to ten times per tile: split here once, their staging
+// is a copy (splitting while staging made them issue-bound: 63 to 74 cycles per matrix
+// instruction of 32).
+__global__ __launch_bounds__(256) void split_input_kernel(Plan pl, float *__restrict__ sums) {
+  __shared__ float red[4][kChannelSums];
+  const int c = blockIdx.x, chunk = blockIdx.y;
+  const int per = (pl.n + pl.nchunk - 1) / pl.nchunk;
+  const int s0 = chunk * per, s1 = s0 + per < pl.n ? s0 + per : pl.n;
+  float acc[kChannelSums];
+#pragma unroll
+  for (int e = 0; e < kChannelSums; ++e) acc[e] = 0.f;
+  unsigned least = kNothingSplit;
+  float largest = 0.f;
+  for (int i = 0; i < kSources; ++i) {
+    const Source &src = pl.src[i];
+    const int Q = (int)src.pitch / 8;
+    for (int e = (int)threadIdx.x; e < (s1 - s0) * Q; e += 256) {
+      const int s = s0 + e / Q, pp = (e % Q) * 8;
+      const float *from = pl.x + (size_t)s * pl.sample_stride + (size_t)c * pl.row_stride + src.org;
+      int u = pp / src.pw, v = pp - u * src.pw;
+      float t[8];
+      int at[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        at[k] = u < src.h && v < src.w ? (u << 16) | v : -1;
+        t[k] = from[at[k] >= 0 ? u * src.su + v * src.sv : 0];
+        if (++v == src.pw) {
+          v = 0;
+          ++u;
+        }
+      }
+      unsigned h[4], m[4], l[4];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) t[k] = at[k] >= 0 ? t[k] : 0.f;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        note_least(t[2 * k], t[2 * k + 1], least);
+        split_pair(t[2 * k], t[2 * k + 1], h[k], m[k], l[k]);
+      }
+      float all = 0.f, head = 0.f, tail = 0.f;   // everything; first and last line, or first and last pixel of a column
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int line = i == 0 ? at[k] >> 16 : at[k];   // (padding: -1)
+        largest = fmaxf(largest, fabsf(t[k]));
+        all += t[k];
+        head += line == 0 ? t[k] : 0.f;
+        tail += line == pl.H - 1 ? t[k] : 0.f;
+      }
+      if (i == 0) {
+        acc[0] += all;
+        acc[1] += head;
+        acc[2] += tail;
+      } else if (i == 1) {
+        acc[3] += all;
+        acc[5] += head;
+        acc[7] += tail;
+      } else {
+        acc[4] += all;
+        acc[6] += head;
+        acc[8] += tail;
+      }
+      unsigned short *to = pl.planes + src.base + ((size_t)s * pl.C + c) * src.pitch + pp;
+      *reinterpret_cast<uintx4 *>(to) = uintx4{h[0], h[1], h[2], h[3]};
+      *reinterpret_cast<uintx4 *>(to + pl.plane_stride) = uintx4{m[0], m[1], m[2], m[3]};
+      *reinterpret_cast<uintx4 *>(to + 2 * (size_t)pl.plane_stride) = uintx4{l[0], l[1], l[2], l[3]};
+    }
+    if (c == 0 && chunk == 0)   // the zeros before the first row
+      for (int e = (int)threadIdx.x; e < 3 * (int)(src.guard / 8); e += 256) {
+        const int q = e % 3, k = e / 3;
+        *reinterpret_cast<uintx4 *>(pl.planes + (size_t)q * pl.plane_stride + src.base - src.guard + k * 8) = uintx4{0, 0, 0, 0};
+      }
+  }
+#pragma unroll
+  for (int e = 0; e < kChannelSums; ++e) {
+    float v = acc[e];
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][e] = v;
+  }
+  // (an infinity or NaN shows in the sum, what would round to infinity in the largest magnitude)
+  const int odd = __syncthreads_or(least < kLeastSplit || largest >= 0x1.fep127f || !(acc[0] * 0.f == 0.f));
+  if (threadIdx.x < kChannelSums)
+    sums[((long long)chunk * pl.C + c) * kChannelSums + threadIdx.x] =
+        red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+  if (threadIdx.x == 0) pl.odd[chunk * pl.C + c] = odd != 0;
+}
+
+// k runs over (sample, position of the source).  A workgroup of 256 * WM threads stages 32 k-values of
+// its 64 * WM first-operand channels and, from the row shift on, of its 64 second-operand channels with two
+// more on either side; a wave has 32 x 32 channels of all NS products (acc and low: 160
+// registers for NS = 5, two waves per SIMD: one workgroup with WM = 2, two with WM = 1 per CU).  Panels are
+// copies of the planes.  A lane's operand of the matrix instruction is eight consecutive k-values of a
+// row; of the second operand it reads the two before and after as well, and forms the shifted ones by
+// v_alignbit (odd shifts) and moves: 48 vector instructions for 30 matrix instructions.
+// Items with channels that leave the split's range, and groups of at most kShiftF32K k-values
+// (kShiftF32K / 8 corner pixels), take the float32 instruction and the input itself.
+// corr_kernel alone, with the float32 instruction (one dword load, LDS word and select per value) and now, n = 32:
+// 64 channels of 56 x 56 128 and 85 us, 128 of 28 x 28 123 and 77, 256 of 14 x 14 123 and 85, 512 of 7 x 7
+// 145 and 112 (9 for 7 positions of a padded line), 32 of 112 x 112 235 and 110; a factor with its other
+// launches 157 -> 115 to 130, 150 -> 105, 152 -> 120, 199 -> 178 and 255 -> 163.  A slice's
+// last quarter of the launch and 6 to 8 us of prologue and partial tiles per item are what is left, besides
+// 56 % of the matrix rate, at the clock that the chip keeps (2.0 GHz), in the loop.
+constexpr int kShiftF32K = 128;
+constexpr int kPlaneA = KT * 2, kRowA = 3 * kPlaneA + 16;   // bytes; rows 13 x 16 apart: all banks
+constexpr int kPlaneB = 96, kRowB = 3 * kPlaneB + 16;       // 14 values, 2 before, 32, 2 after; rows 19 x 16 apart
+constexpr int kRowF32A = KT + 1, kRowF32B = 37;             // floats, odd
+template <int WM>
+struct ShiftLds {
+  static constexpr int kBuffer = 64 * WM * kRowA + 64 * kRowB;
+  static constexpr int kBytes = 2 * kBuffer;
+  static_assert(64 * WM * kRowF32A * 4 <= 64 * WM * kRowA && 64 * kRowF32B * 4 <= 64 * kRowB, "float32 panels fit");
+};
+
+// Position of a k-value: sample * C * pitch + p in memory.
+struct PanelPos {
+  int p;
+  unsigned off;
+  __device__ __forceinline__ void init(const Source &src, int C, const ShiftGroup &g, int k) {
+    const int s = k / g.L;
+    p = k - s * g.L;
+    off = (unsigned)s * (unsigned)C * src.pitch + (unsigned)p;
+  }
+  __device__ __forceinline__ void next(const Source &src, int C, const ShiftGroup &g) {
+    p += g.r32;
+    off += (unsigned)g.step32;
+    const bool over = p >= g.L;
+    p -= over ? g.L : 0;
+    off += over ? (unsigned)C * src.pitch - (unsigned)g.L : 0u;
+  }
+};
+
+template <int WM, int NS, bool STACKED, int DJ0>
+__device__ __forceinline__ bool corr_split(const Plan &pl, const ShiftGroup &g, int I, int J, int kbeg, int kend, char *lds,
+                                           floatx16 (&acc)[NS]) {
+  typedef uintx4 uintx4u __attribute__((aligned(2)));
+  typedef unsigned unsignedu __attribute__((aligned(2)));
+  constexpr int BMA = 64 * WM;
+  const Source &src = pl.src[g.source];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const unsigned short *base = pl.planes + (src.base - src.guard);   // offsets from here: none is negative
+  const size_t ps = pl.plane_stride;
+  auto from = [&](int q, unsigned element) {
+    return (const KFAC_GLOBAL_AS char *)(base + q * ps) + element * 2u;
+  };
+  // a chunk of eight k-values of a first-operand row, and (the first 256 threads) of a second-operand row
+  const int cq = tid & 3, ra = tid >> 2, rb = (tid & 255) >> 2;
+  const int ca = STACKED ? ra & 31 : min(I * BMA + ra, pl.C - 1);
+  const int cb = STACKED ? rb & 31 : min(J * 64 + rb, pl.C - 1);
+  const unsigned row_a = src.guard + (unsigned)g.org + (unsigned)min(ca, pl.C - 1) * src.pitch - (STACKED && ra >= 32 ? (unsigned)src.pw : 0u);
+  const unsigned row_b = src.guard + (unsigned)g.org + (unsigned)min(cb, pl.C - 1) * src.pitch + (unsigned)g.offset;
+  // two values before (side 0) or behind (side 1) a second-operand row's 32, of one plane: 384 in all
+  const int xt = WM == 2 ? tid & 255 : tid;
+  unsigned row_x[2];
+  int lds_x[2], side[2], plane_x[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int t = min(xt + 256 * i, 383), r = t & 63;
+    side[i] = (t >> 6) & 1;
+    plane_x[i] = t >> 7;
+    const int cx = STACKED ? r & 31 : min(J * 64 + r, pl.C - 1);
+    row_x[i] = src.guard + (unsigned)g.org + (unsigned)min(cx, pl.C - 1) * src.pitch + (unsigned)g.offset + (side[i] ? 8u : 0u) -
+               (side[i] ? 0u : 2u);
+    lds_x[i] = BMA * kRowA + r * kRowB + plane_x[i] * kPlaneB + (side[i] ? 32 + 64 - 16 : 12);
+  }
+  const bool loads_b = WM == 1 || wave < 4, loads_x = WM == 1 || wave >= 4;
+  PanelPos at, first, last;   // the thread's chunk; the panel's first and last chunk
+  at.init(src, pl.C, g, kbeg + 8 * cq);
+  first.init(src, pl.C, g, kbeg);
+  last.init(src, pl.C, g, kbeg + 24);
+  int k_load = kbeg + 8 * cq;
+  bool inside = true;   // the loaded chunk is part of the reduction
+  int beyond = 0;       // of its eight values, those from this one on are outside the domain
+  const bool masked = g.valid < g.L;
+  uintx4 va[3], vb[3];
+  unsigned vx[2];
+  auto load = [&]() {
+    inside = k_load < kend;
+    beyond = g.valid - at.p;
+    const unsigned o = inside ? at.off : 0u;   // (past the end: any place, stored as zeros)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) va[q] = *(const KFAC_GLOBAL_AS uintx4u *)from(q, o + row_a);
+    if (loads_b) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) vb[q] = *(const KFAC_GLOBAL_AS uintx4u *)from(q, o + row_b);
+    }
+    if (loads_x) {
+      const bool whole = k_load - 8 * cq + KT <= kend;   // (else chunks past the end meet zeros)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const unsigned ox = side[i] ? (whole ? last.off : 0u) : first.off;
+        vx[i] = *(const KFAC_GLOBAL_AS unsignedu *)((const KFAC_GLOBAL_AS char *)base +
+                                                    (size_t)(plane_x[i] * ps + (k_load - 8 * cq < kend ? ox : 2u) + row_x[i]) * 2);
+      }
+    }
+    k_load += KT;
+    at.next(src, pl.C, g);
+    first.next(src, pl.C, g);
+    last.next(src, pl.C, g);
+  };
+  auto store = [&](char *buf) {
+    if (masked) {   // strips and corners
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const unsigned keep = (beyond > 2 * i ? 0xffffu : 0u) | (beyond > 2 * i + 1 ? 0xffff0000u : 0u);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) va[q][i] &= keep;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      *reinterpret_cast<uintx4 *>(buf + ra * kRowA + q * kPlaneA + cq * 16) = inside ? va[q] : uintx4{0, 0, 0, 0};
+    if (loads_b) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        *reinterpret_cast<uintx4 *>(buf + BMA * kRowA + rb * kRowB + q * kPlaneB + 16 + cq * 16) = inside ? vb[q] : uintx4{0, 0, 0, 0};
+    }
+    if (loads_x) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) *reinterpret_cast<unsigned *>(buf + lds_x[i]) = vx[i];
+    }
+  };
+  floatx16 low[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[s][e] = low[s][e] = 0.f;
+  const bool active = !STACKED || wm < g.stacked;
+  const int lrow = lane & 31, lk = lane >> 5;
+  // the products of a panel: shift e from place PLACE + e of the window on (a stacked group's last
+  // column offset is not needed)
+  auto multiply = [&](const char *a0, const char *b0, auto place) {
+    constexpr int PLACE = decltype(place)::value;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      bf16x8 a[3];
+      unsigned w[3][6];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        a[q] = *reinterpret_cast<const bf16x8 *>(a0 + q * kPlaneA + s * 32);
+        const char *p = b0 + q * kPlaneB + s * 32;
+        w[q][0] = *reinterpret_cast<const unsigned *>(p + 12);
+        const uintx4 mid = *reinterpret_cast<const uintx4 *>(p + 16);
+        w[q][1] = mid[0];
+        w[q][2] = mid[1];
+        w[q][3] = mid[2];
+        w[q][4] = mid[3];
+        w[q][5] = *reinterpret_cast<const unsigned *>(p + 32);
+      }
+      auto shifted = [&](bf16x8 (&o)[3], int to) {
+        const int d = to >> 1;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          uintx4 t;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            t[i] = to & 1 ? __builtin_amdgcn_alignbit(w[q][d + i + 1 < 6 ? d + i + 1 : 5], w[q][d + i], 16) : w[q][d + i];
+          o[q] = __builtin_bit_cast(bf16x8, t);
+        }
+      };
+      // two shifts at a time, so that no instruction adds to the sum of the one before it
+#pragma unroll
+      for (int e = 0; e < NS; e += 2) {
+        bf16x8 b[2][3];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (e + i < NS && PLACE + e + i <= 4) shifted(b[i], PLACE + e + i);
+#pragma unroll
+        for (int t = 0; t < kSplitTerms; ++t)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            if (e + i >= NS || PLACE + e + i > 4) continue;
+            floatx16 &sum = t == kSplitTerms - 1 ? acc[e + i] : low[e + i];
+            sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kSplitA[t]], b[i][kSplitB[t]], sum, 0, 0, 0);
+          }
+      }
+    }
+  };
+  load();
+  store(lds);
+  load();
+  __syncthreads();
+  int buffer = 0;
+  for (int k0 = kbeg; k0 < kend; k0 += KT) {
+    char *cur = lds + buffer * ShiftLds<WM>::kBuffer, *nxt = lds + (buffer ^ 1) * ShiftLds<WM>::kBuffer;
+    store(nxt);
+    load();
+    const char *a0 = cur + (wm * 32 + lrow) * kRowA + lk * 16;
+    const char *b0 = cur + BMA * kRowA + (wn * 32 + lrow) * kRowB + lk * 16;
+    if (active) {
+      if (STACKED && wn)
+        multiply(a0, b0, std::integral_constant<int, 3>());
+      else
+        multiply(a0, b0, std::integral_constant<int, 2 + DJ0>());
+    }
+    buffer ^= 1;
+    __syncthreads();
+  }
+  float nonfinite = 0.f;   // NaN as soon as a sum is infinite or NaN
+#pragma unroll
+  for (int e = 0; e < NS; ++e) {
+    acc[e] += low[e];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) nonfinite = __builtin_fmaf(acc[e][i], 0.f, nonfinite);
+  }
+  return nonfinite != 0.f;
+}
+
+// The same sums with the float32 instruction, from the input.
+template <int WM, int NS, bool STACKED, int DJ0>
+__device__ __forceinline__ void corr_f32(const Plan &pl, const ShiftGroup &g, int I, int J, int kbeg, int kend, char *lds,
+                                         floatx16 (&acc)[NS]) {
+  constexpr int BMA = 64 * WM, T = 256 * WM;
+  const Source &src = pl.src[g.source];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+  float *la = reinterpret_cast<float *>(lds), *lb = la + BMA * kRowF32A;
+  // the value `on` elements on from k-value k of a channel
+  auto value = [&](int c, int k, int on, bool of_a) {
+    const int s = k / g.L, p = k - s * g.L, pp = g.org + p + on;
+    const int u = pp >= 0 ? pp / src.pw : -1, v = pp - u * src.pw;
+    const bool in = k < kend && c < pl.C && u >= 0 && u < src.h && v < src.w && (!of_a || p < g.valid);
+    return in ? pl.x[(size_t)s * pl.sample_stride + (size_t)c * pl.row_stride + src.org + u * src.su + v * src.sv] : 0.f;
+  };
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[s][e] = 0.f;
+  for (int k0 = kbeg; k0 < kend; k0 += KT) {
+    __syncthreads();
+    for (int e = tid; e < BMA * KT; e += T) {
+      const int r = e / KT, k = e % KT;
+      la[r * kRowF32A + k] = value(STACKED ? r & 31 : I * BMA + r, k0 + k, STACKED && r >= 32 ? -src.pw : 0, true);
+    }
+    for (int e = tid; e < 64 * 36; e += T) {
+      // place j: what is read for k-value k0 + j - 2 unshifted; at the panel's sides, on from its ends
+      const int r = e / 36, j = e % 36, k = k0 + min(max(j - 2, 0), KT - 1);
+      lb[r * kRowF32B + j] = value(STACKED ? r & 31 : J * 64 + r, k,
+                                   g.offset + (j - 2 - (k - k0)), false);
+    }
+    __syncthreads();
+    for (int kk = 0; kk < KT / 2; ++kk) {
+      const float a = la[(wm * 32 + (lane & 31)) * kRowF32A + 2 * kk + (lane >> 5)];
+#pragma unroll
+      for (int e = 0; e < NS; ++e)
+        acc[e] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+            a, lb[(wn * 32 + (lane & 31)) * kRowF32B + 2 * kk + (lane >> 5) + min(2 + DJ0 + (STACKED ? 3 * wn : 0) + e, 4)],
+            acc[e], 0, 0, 0);
+    }
+  }
+}
+
+template <int WM, int NS, bool STACKED, int DJ0>
+__device__ __forceinline__ void corr_shifts_body(const Plan &pl, const ShiftGroup &g, int q, char *lds,
                                                  float *__restrict__ partial) {
   static_assert(!STACKED || WM == 1, "stacked groups use 64-row tiles");
   constexpr int BMA = 64 * WM;
-  float *ldsA = lds, *ldsB = lds + BMA * kRowStride;
   const int ntile = pl.tiles_a * pl.tiles_b;
   const int split = q / ntile, tile = q - split * ntile;
   const int I = tile / pl.tiles_b, J = tile - I * pl.tiles_b;
-  const unsigned L = g.L, mem_line = g.mem_line, vline = g.vline;
-  const int K = g.K;
-  LoaderDomain<BMA> la;
-  la.base = g.base;
-  la.sample_stride = g.sample_stride;
-  la.row_stride = g.row_stride;
-  la.L = L;
-  la.line_len = mem_line;
-  la.line_stride = g.line_stride;
-  la.rows_valid = pl.C;
-  la.init(I * BMA);
-  if (STACKED) {   // all of a thread's rows are rows of one half: channel = row % 32
-    la.first_row = team_tid() >> 5;
-    la.rows_valid = pl.C;
+  const int kbeg = split * g.klen, kend = min(kbeg + g.klen, g.K);
+  int odd = 0;
+  for (int e = threadIdx.x; e < (BMA + 64) * pl.nchunk; e += 256 * WM) {
+    const int r = e % (BMA + 64), c = r < BMA ? I * BMA + r : J * 64 + r - BMA;
+    if (c < pl.C) odd |= pl.odd[e / (BMA + 64) * pl.C + c];
   }
-  const int tid = team_tid();
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int lrow = lane & 31, lk = lane >> 5;
-  // second operand: 32 columns x 8 row passes, then 4 columns x 64 rows
-  const int jm = tid & 31, rm = tid >> 5;
-  const int je = 32 + (tid & 3), re = tid >> 2;
-  const int shift = g.di * (int)vline - 2;
-  unsigned rowoff[8];
-  unsigned rowok = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int row = STACKED ? (rm + 8 * i) & 31 : J * 64 + rm + 8 * i;
-    rowoff[i] = (unsigned)(row < pl.C ? row : pl.C - 1) * g.row_stride;
-    if (row < pl.C) rowok |= 1u << i;
-  }
-  const int rowe = STACKED ? re & 31 : J * 64 + re;
-  const unsigned rowoff_e = (unsigned)(rowe < pl.C ? rowe : pl.C - 1) * g.row_stride;
-  const long long kbeg = (long long)split * g.klen;
-  long long kend = kbeg + g.klen;
-  if (kend > K) kend = K;
-  floatx16 acc[NS][WM];
-#pragma unroll
-  for (int s = 0; s < NS; ++s)
-#pragma unroll
-    for (int im = 0; im < WM; ++im)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[s][im][v] = 0.f;
-  typename LoaderDomain<BMA>::Regs ra;
-  float rb[9];
-  auto load_b = [&](long long k0) {
-    auto offset_of = [&](int j) {
-      long long kk = k0 + shift + j;
-      kk = kk < 0 ? 0 : (kk >= K ? K - 1 : kk);   // any element of the tensor will do: masked when read
-      const unsigned ku = (unsigned)kk, s = ku / L, p = ku - s * L;
-      const unsigned line = p / mem_line;
-      return s * g.sample_stride + line * g.line_stride + (p - line * mem_line);
-    };
-    const unsigned om = offset_of(jm), oe = offset_of(je + (STACKED && re >= 32 ? 3 : 0));
-    const unsigned om1 = STACKED ? offset_of(jm + 3) : om;   // rows 32..: three columns on
-#pragma unroll
-    for (int i = 0; i < 8; ++i) rb[i] = gload1(g.base, ((STACKED && i >= 4 ? om1 : om) + rowoff[i]) * 4u);
-    rb[8] = gload1(g.base, (oe + rowoff_e) * 4u);
-  };
-  // first operand of a stacked group: rows 32.. are the channels one image row up
-  auto load_a = [&](long long k0) {
-    if (!STACKED) {
-      la.load(ra, k0, kend);
-      return;
-    }
-    const long long kg = k0 + jm;
-    ra.kvalid = kg < kend;
-    const long long kc = ra.kvalid ? kg : 0;
-    auto offset_at = [&](long long kk) {
-      const unsigned ku = (unsigned)(kk < 0 ? 0 : kk), s = ku / L, p = ku - s * L;
-      return s * g.sample_stride + p;   // whole images: pixels are contiguous
-    };
-    const unsigned o0 = offset_at(kc), o1 = offset_at(kc - (long long)vline);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int row = (rm + 8 * i) & 31;
-      ra.v[i] = gload1(g.base, ((i >= 4 ? o1 : o0) + (unsigned)(row < pl.C ? row : pl.C - 1) * g.row_stride) * 4u);
-    }
-  };
-  auto store_a = [&]() {
-    if (!STACKED) {
-      la.store(ra, ldsA);
-      return;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      ldsA[(rm + 8 * i) * kRowStride + jm] = (ra.kvalid && ((rm + 8 * i) & 31) < pl.C) ? ra.v[i] : 0.f;
-  };
-  if (kbeg < kend) {
-    load_a(kbeg);
-    load_b(kbeg);
-  }
-  for (long long k0 = kbeg; k0 < kend; k0 += KT) {
-    store_a();
-#pragma unroll
-    for (int i = 0; i < 8; ++i) ldsB[(rm + 8 * i) * kShiftStride + jm] = ((rowok >> i) & 1u) ? rb[i] : 0.f;
-    ldsB[re * kShiftStride + je] = rowe < pl.C ? rb[8] : 0.f;
-    __syncthreads();
-    if (k0 + KT < kend) {
-      load_a(k0 + KT);
-      load_b(k0 + KT);
-    }
-    // validity of the NS shifted pixels of this panel's 32 k-values: bit k of m[s]
-    unsigned m[NS];
-    {
-      const long long kg = k0 + (lane & 31);
-      const unsigned kc = kg < kend ? (unsigned)kg : 0u;
-      const unsigned pix = kc % L;
-      const unsigned a = pix / vline, b = pix - a * vline;
-      // stacked: this wave's blocks are row shift di + wm (first operand one row up:
-      // not for the first image row) and column shifts dj0 + 3 wn + s
-      const bool row_in = kg < kend && (int)a + g.di < g.amax && (!STACKED || (int)a >= wm);
-      const int dj_first = g.dj0 + (STACKED ? 3 * wn : 0);
-#pragma unroll
-      for (int s = 0; s < NS; ++s)
-        m[s] = __builtin_amdgcn_readfirstlane(
-            (unsigned)__ballot(row_in && (unsigned)((int)b + dj_first + s) < vline));
-    }
-    const bool active = !STACKED || wm < g.stacked;
-    const float *pa = ldsA + (wm * WM * 32 + lrow) * kRowStride + lk;
-    const float *pb = ldsB + (wn * 32 + lrow) * kShiftStride + lk + 2 + g.dj0;
-    // operands of step kk + 1 are read from LDS before the matrix instructions of
-    // step kk issue (the scheduling barriers keep the compiler from sinking the
-    // reads to their first use, which would expose the LDS latency in every step)
-    float a[2][WM], b[2][NS];
-#pragma unroll
-    for (int im = 0; im < WM; ++im) a[0][im] = pa[im * 32 * kRowStride];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) b[0][s] = pb[s];
-    if (active) {
-#pragma unroll
-    for (int kk = 0; kk < KT / 2; ++kk) {
-      const int cur = kk & 1, nxt = cur ^ 1;
-      if (kk + 1 < KT / 2) {
-#pragma unroll
-        for (int im = 0; im < WM; ++im) a[nxt][im] = pa[im * 32 * kRowStride + 2 * kk + 2];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) b[nxt][s] = pb[2 * kk + 2 + s];
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        // lanes 0..31 hold k = 2 kk, lanes 32..63 k = 2 kk + 1: the lane mask of the
-        // valid ones, built from two bits of the panel's mask in scalar registers
-        const unsigned lo = 0u - ((m[s] >> (2 * kk)) & 1u), hi = 0u - ((m[s] >> (2 * kk + 1)) & 1u);
-        const unsigned long long lanes = ((unsigned long long)hi << 32) | lo;
-        const float v = __builtin_amdgcn_inverse_ballot_w64(lanes) ? b[cur][s] : 0.f;
-#pragma unroll
-        for (int im = 0; im < WM; ++im)
-          acc[s][im] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[cur][im], v, acc[s][im], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    }
-    __syncthreads();
-  }
+  floatx16 acc[NS];
+  bool f32 = __syncthreads_or(odd) || g.K <= kShiftF32K;
+  if (!f32) f32 = __syncthreads_or(corr_split<WM, NS, STACKED, DJ0>(pl, g, I, J, kbeg, kend, lds, acc));
+  if (__builtin_expect(f32, 0)) corr_f32<WM, NS, STACKED, DJ0>(pl, g, I, J, kbeg, kend, lds, acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
   float *out = partial + g.part_off + (long long)q * (NS * BMA * 64);
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
+  for (int e = 0; e < NS; ++e)
 #pragma unroll
-    for (int im = 0; im < WM; ++im)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = (wm * WM + im) * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        out[(s * BMA + row) * 64 + wn * 32 + (lane & 31)] = acc[s][im][v];
-      }
+    for (int v = 0; v < 16; ++v) {
+      const int row = wm * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+      out[(e * BMA + row) * 64 + wn * 32 + (lane & 31)] = acc[e][v];
+    }
 }
 
 // The strips and corners first (few items, bound by latency: they start early and
 // run beside the rest), then the whole-image groups.
 template <int WM>
-__global__ __launch_bounds__(THREADS, 2) void corr_kernel(Plan pl, float *__restrict__ partial) {
-  __shared__ float lds[64 * WM * kRowStride + 64 * kShiftStride];
+__global__ __launch_bounds__(256 * WM, 2) void corr_kernel(Plan pl, float *__restrict__ partial) {
+  extern __shared__ __align__(16) char lds[];
   int w = blockIdx.x;
   if (w >= pl.nsmall) w = pl.nsmall + item_of_block(w - pl.nsmall, pl.total - pl.nsmall);
   int gi = 0;
@@ -375,91 +523,14 @@ __global__ __launch_bounds__(THREADS, 2) void corr_kernel(Plan pl, float *__rest
   const ShiftGroup &g = pl.grp[gi];
   if constexpr (WM == 1) {
     if (g.stacked) {
-      corr_shifts_body<1, 3, true>(pl, g, w - g.task0, lds, partial);
+      corr_shifts_body<1, 3, true, -2>(pl, g, w - g.task0, lds, partial);
       return;
     }
   }
   if (g.ns == 3)
-    corr_shifts_body<WM, 3>(pl, g, w - g.task0, lds, partial);
+    corr_shifts_body<WM, 3, false, 0>(pl, g, w - g.task0, lds, partial);
   else
-    corr_shifts_body<WM, 5>(pl, g, w - g.task0, lds, partial);
-}
-
-// One pass over the input before the products: the per-channel sums that make the
-// ones column, over the samples of chunk blockIdx.y (a contiguous range),
-//   sums[chunk][c][0..8] = whole image, first row, last row, first column, last
-//   column, corners (first,first) (first,last) (last,first) (last,last),
-// and the compact copy of the first and last image column, edges[last][s][c][u].
-__global__ __launch_bounds__(256) void edge_sums_kernel(Plan pl, float *__restrict__ sums,
-                                                        float *__restrict__ edges) {
-  __shared__ float red[4][kChannelSums];
-  const int c = blockIdx.x, chunk = blockIdx.y, nchunk = gridDim.y;
-  const int H = pl.H, W = pl.W, HW = H * W;
-  const int per = (pl.n + nchunk - 1) / nchunk;
-  const int s0 = chunk * per, s1 = s0 + per < pl.n ? s0 + per : pl.n;
-  float acc[kChannelSums];
-#pragma unroll
-  for (int e = 0; e < kChannelSums; ++e) acc[e] = 0.f;
-  const float *base = pl.x + (long long)c * pl.row_stride;
-  float *e0 = edges + (long long)c * H, *e1 = e0 + (long long)pl.n * pl.C * H;
-  if (W % 4 == 0 && (reinterpret_cast<uintptr_t>(pl.x) & 15) == 0) {
-    // four pixels of one image row at a time
-    const int Q = HW / 4;
-    for (int e = s0 * Q + (int)threadIdx.x; e < s1 * Q; e += 256) {
-      const int s = e / Q, p = (e - s * Q) * 4;
-      const float4 v = *reinterpret_cast<const float4 *>(base + (long long)s * pl.sample_stride + p);
-      const int u = p / W, q = p - u * W;
-      const bool r0 = u == 0, r1 = u == H - 1, c0 = q == 0, c1 = q + 4 == W;
-      const float t = (v.x + v.y) + (v.z + v.w);
-      acc[0] += t;
-      if (r0) acc[1] += t;
-      if (r1) acc[2] += t;
-      if (c0) {
-        acc[3] += v.x;
-        e0[(long long)s * pl.C * H + u] = v.x;
-        if (r0) acc[5] += v.x;
-        if (r1) acc[7] += v.x;
-      }
-      if (c1) {
-        acc[4] += v.w;
-        e1[(long long)s * pl.C * H + u] = v.w;
-        if (r0) acc[6] += v.w;
-        if (r1) acc[8] += v.w;
-      }
-    }
-  } else {
-    for (int e = s0 * HW + (int)threadIdx.x; e < s1 * HW; e += 256) {
-      const int s = e / HW, p = e - s * HW;
-      const float v = base[(long long)s * pl.sample_stride + p];
-      const int u = p / W, q = p - u * W;
-      const bool r0 = u == 0, r1 = u == H - 1, c0 = q == 0, c1 = q == W - 1;
-      acc[0] += v;
-      if (r0) acc[1] += v;
-      if (r1) acc[2] += v;
-      if (c0) {
-        acc[3] += v;
-        e0[(long long)s * pl.C * H + u] = v;
-      }
-      if (c1) {
-        acc[4] += v;
-        e1[(long long)s * pl.C * H + u] = v;
-      }
-      if (r0 && c0) acc[5] += v;
-      if (r0 && c1) acc[6] += v;
-      if (r1 && c0) acc[7] += v;
-      if (r1 && c1) acc[8] += v;
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < kChannelSums; ++e) {
-    float v = acc[e];
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][e] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < kChannelSums)
-    sums[((long long)chunk * pl.C + c) * kChannelSums + threadIdx.x] =
-        red[0][threadIdx.x] + red[1][threadIdx.x] + red[2][threadIdx.x] + red[3][threadIdx.x];
+    corr_shifts_body<WM, 5, false, -2>(pl, g, w - g.task0, lds, partial);
 }
 
 // Sums the slices of one block of one product and writes it to the product's
@@ -496,13 +567,20 @@ __global__ __launch_bounds__(256) void corr_finish_kernel(Plan pl, const float *
     float4 v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = src[(s + e * G) * step4];
+    // (as a tree: the sums of short slices are rounded here more than in the products)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      a.x += v[e].x;
-      a.y += v[e].y;
-      a.z += v[e].z;
-      a.w += v[e].w;
-    }
+    for (int step = 1; step < 8; step *= 2)
+#pragma unroll
+      for (int e = 0; e < 8; e += 2 * step) {
+        v[e].x += v[e + step].x;
+        v[e].y += v[e + step].y;
+        v[e].z += v[e + step].z;
+        v[e].w += v[e + step].w;
+      }
+    a.x += v[0].x;
+    a.y += v[0].y;
+    a.z += v[0].z;
+    a.w += v[0].w;
   }
   for (; s < pr.nsplit; s += G) {
     const float4 v = src[s * step4];

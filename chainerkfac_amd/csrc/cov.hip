@@ -881,19 +881,24 @@ int try_conv_rows(const float *x, int n, int c, int h, int w, int kh, int kw, in
 }
 
 // Slices of the whole-image groups of the shifted-correlation route: the workgroups
-// of a launch run two to a CU, 512 at a time (three with 64 first-operand channels),
+// of a launch run one to a CU (two with 64 first-operand channels),
 // and a group of ns shifts does ns tile products per panel.  Among the slice counts
 // (s5 for the two groups of five shifts, s3 for the group of three) the pair with
 // the least rounds x longest item, plus what an item costs besides its panels
 // (prologue, partial tiles written and summed).  ntab: tile pairs per product, nk:
-// panels of the whole reduction.
+// panels of the whole reduction, strip: panels of a row, a column and a corner.
 struct ShiftSlices {
   long long s5, s3;
   double longest;   // shift-panels of the longest item
 };
-constexpr long long kShiftMaxItems = 1024;
+constexpr long long kShiftMaxItems = 512;
 
-ShiftSlices plan_shift_slices(int wm, int ntab, long long nk) {
+// Slices of a strip or corner group of gk panels: items about as long as the others'.
+long long shift_strip_slices(long long gk, double longest) {
+  return kfac::ceil_div<long long>(3 * gk, std::max<long long>(3, (long long)longest));
+}
+
+ShiftSlices plan_shift_slices(int wm, int ntab, long long nk, const long long (&strip)[3]) {
   long long best_s5 = 1, best_s3 = 1;
   double best_cost = 0.0, best_longest = (double)(5 * nk);
   for (long long s5 = 1; s5 <= nk && ntab * (2 * s5 + 1) <= kShiftMaxItems; ++s5) {
@@ -906,9 +911,11 @@ ShiftSlices plan_shift_slices(int wm, int ntab, long long nk) {
     const long long items = ntab * (2 * s5 + s3);
     if (items > kShiftMaxItems) continue;
     const double longest = (double)std::max(5 * len5, 3 * len3);
-    const double rounds = (double)kfac::ceil_div<long long>(items, wm == 1 ? 768 : 512);
+    const long long strips = ntab * (2 * shift_strip_slices(strip[0], longest) + 2 * shift_strip_slices(strip[1], longest) +
+                                     4 * shift_strip_slices(strip[2], longest));
+    const double rounds = (double)kfac::ceil_div<long long>(items + strips, wm == 1 ? 512 : 256);
     // an item's fixed cost in units of one shift-panel
-    const double cost = rounds * (longest + 6.0) + 0.004 * (double)items;
+    const double cost = rounds * (longest + 12.0) + 0.004 * (double)items;
     if (best_cost == 0.0 || cost < best_cost) {
       best_cost = cost;
       best_s5 = s5;
@@ -929,17 +936,12 @@ ShiftSlices plan_shift_slices(int wm, int ntab, long long nk) {
 }
 
 // Stacked groups (one tile pair, two groups of three column offsets): equal slices,
-// about 720 items in all for the 768 slots of three workgroups per CU.
+// about 490 items in all for the 512 slots of two workgroups per CU.
 ShiftSlices plan_stacked_slices(long long nk) {
-  const long long want = std::max<long long>(1, std::min<long long>(360, nk / 8));
+  const long long want = std::max<long long>(1, std::min<long long>(245, nk / 8));
   const long long len = kfac::ceil_div(nk, want);
   const long long ns = kfac::ceil_div(nk, len);
   return ShiftSlices{ns, ns, (double)(3 * len)};
-}
-
-// Slices of a strip or corner group of gk panels: items about as long as the others'.
-long long shift_strip_slices(long long gk, double longest) {
-  return kfac::ceil_div<long long>(3 * gk, std::max<long long>(3, (long long)longest));
 }
 
 // 64-row first-operand tiles unless 128 rows waste no more on the channel count
@@ -962,23 +964,38 @@ bool shift_route_takes(int c, int h, int w) {
   return (c >= min_c || (stacked_on && shift_stacked(c))) && h >= 4 && w >= 4 && h <= 32767 && w <= 32767;
 }
 
+// The sources of the products (conv_shift.h) of an n x c x h x w input, one after the other in a plane:
+// the elements of a plane.
+unsigned long long shift_sources(int n, int c, int h, int w, kfac::shift::Source *src) {
+  unsigned long long at = 0;
+  auto add = [&](int i, int sh, int sw, int org, int su, int sv) {
+    kfac::shift::Source &s = src[i];
+    s.h = sh; s.w = sw; s.pw = sw + 2; s.org = org; s.su = su; s.sv = sv;
+    // the last chunk of eight, two lines (of an image) and the widest shift further on: zeros
+    s.pitch = (unsigned)(((sh * s.pw + 7) / 8 * 8 + (sh > 1 ? 2 * s.pw : 0) + 5 + 7) / 8 * 8);
+    s.guard = (unsigned)((s.pw + 8 + 7) / 8 * 8);
+    s.base = (unsigned)(at + s.guard);
+    at += s.guard + (unsigned long long)n * c * s.pitch;
+  };
+  add(0, h, w, 0, w, 1);
+  for (int last = 0; last < 2; ++last) add(1 + last, 1, h, last * (w - 1), 0, w);
+  return (at + 7 + 16) / 8 * 8;   // (a corner's chunk reads past its column)
+}
+
 // Upper bound of the workspace floats the route takes for c channels and `rows` =
 // samples x pixels (the image's sides are not known here: at least 4 each).
 size_t shift_ws_floats_bound(int c, long long rows) {
   const int wm = shift_wm(c), bm = 64 * wm;
   const int ntab = kfac::ceil_div(c, bm) * kfac::ceil_div(c, 64);
-  const long long nk = kfac::ceil_div<long long>(rows, KT);
-  const bool stacked = shift_stacked(c);
-  const ShiftSlices sl = stacked ? plan_stacked_slices(nk) : plan_shift_slices(wm, ntab, nk);
-  size_t floats = stacked ? (size_t)(sl.s5 + sl.s3) * 3 * bm * 64
-                          : (size_t)ntab * (size_t)(2 * sl.s5 * 5 + sl.s3 * 3) * bm * 64;
-  // 8 strip / corner groups of three shifts; a strip has at most rows / 4 k-values
-  const long long strip =
-      shift_strip_slices(kfac::ceil_div<long long>(kfac::ceil_div<long long>(rows, 4), KT), sl.longest);
-  floats += (size_t)8 * ntab * (size_t)std::max(1ll, strip) * 3 * bm * 64;
+  // a group's items are at most kShiftMaxItems or one per tile; strips and corners add one per tile and
+  // group, or as many as make them no longer than the others
+  const size_t items = (size_t)2 * kShiftMaxItems + (size_t)11 * ntab;
+  size_t floats = items * 5 * bm * 64;
   floats += (size_t)kfac::shift::kArrays * c * c;
-  floats += (size_t)1024 * kfac::shift::kChannelSums + (size_t)c * 16;   // sums: at most 1024 (chunk, channel) pairs
-  floats += (size_t)c * (size_t)kfac::ceil_div<long long>(rows, 2);      // border columns: 2 n c h, h <= rows / (4 n)
+  floats += (size_t)1024 * (kfac::shift::kChannelSums + 1) + (size_t)c * 16;   // sums: at most 1024 (chunk, channel) pairs
+  // planes: an image of h x w pixels, both at least 4, takes h w + 2 h + 2 w + 30 elements at most and its two
+  // columns h + 21 each, together less than 6.5 h w; 3 planes of 2 bytes
+  floats += (size_t)((double)c * (double)rows * (6.5 * 6.0 / 4.0)) + 4096;
   return floats + 256;
 }
 
@@ -994,13 +1011,16 @@ int run_conv_shift(kfac::shift::Plan &pl, int d, int ones, float alpha, float be
   pl.tiles_a = kfac::ceil_div(c, BM);
   pl.tiles_b = kfac::ceil_div(c, 64);
   const int ntab = pl.tiles_a * pl.tiles_b;
-  // workspace: [partial tiles | arrays | channel sums | border columns]; the last two
+  // workspace: [partial tiles | arrays | channel sums | flags | planes]; all but the first
   // have sizes known up front and are placed from the end
-  const int nchunk = std::max(1, std::min(n, 1024 / c));
+  pl.nchunk = std::max(1, std::min(n, 1024 / c));
   const size_t array_floats = (size_t)kArrays * c * c;
-  const size_t sums_floats = (size_t)nchunk * c * kChannelSums;
-  const size_t edge_floats = (size_t)2 * n * c * h;
-  const size_t tail_floats = array_floats + sums_floats + edge_floats + 64;
+  const size_t sums_floats = (size_t)pl.nchunk * c * kChannelSums;
+  const size_t odd_floats = (size_t)pl.nchunk * c;
+  const unsigned long long plane = shift_sources(n, c, h, w, pl.src);
+  if (plane >= 1ull << 31) return 1;   // offsets inside a plane are 32 bits of bytes
+  const size_t plane_floats = (size_t)(plane * 3 / 2 + 8);
+  const size_t tail_floats = array_floats + sums_floats + odd_floats + plane_floats + 64;
   // a workspace smaller than the route needs sends the factor to the patch-product
   // kernels (option conv_shift_strict: an error instead, for the test of the workspace query)
   auto too_small = [&](size_t need_floats) {
@@ -1013,43 +1033,51 @@ int run_conv_shift(kfac::shift::Plan &pl, int d, int ones, float alpha, float be
   float *partial = static_cast<float *>(ws);
   float *arrays = partial + (ws_bytes / sizeof(float) - tail_floats) / 4 * 4;
   float *sums = arrays + array_floats;
-  float *edges = sums + sums_floats;
+  pl.odd = reinterpret_cast<int *>(sums + sums_floats);
+  pl.planes = reinterpret_cast<unsigned short *>(
+      (reinterpret_cast<uintptr_t>(pl.odd + odd_floats) + 15) / 16 * 16);
+  pl.plane_stride = (unsigned)plane;   // a multiple of 8
   // groups: whole image (di = 0, 1, 2), first / last row, first / last column, corners
-  auto group = [&](int gi, const float *base, long long sample_stride, int row_stride, int line_stride, int L,
-                   int mem_line, int vline, int di, int dj0, int ns, int amax) {
+  auto group = [&](int gi, int source, int org, int valid, int di, int dj0, int ns) {
     ShiftGroup &g = pl.grp[gi];
-    g.base = base;
-    g.sample_stride = (unsigned)sample_stride; g.row_stride = (unsigned)row_stride;
-    g.line_stride = (unsigned)line_stride;
-    g.L = (unsigned)L; g.mem_line = (unsigned)mem_line; g.vline = (unsigned)vline;
-    g.di = (short)di; g.dj0 = (short)dj0; g.ns = (short)ns; g.amax = (short)amax;
+    const Source &src = pl.src[source];
+    g.source = source;
+    g.org = org;
+    // at least two positions past the domain, where the first operand is zero: what is read on from
+    // there belongs to another sample
+    const bool whole = source == 0 && valid == src.h * src.pw;   // (an image ends with padding)
+    g.L = (valid + (whole ? 0 : 2) + 7) / 8 * 8;
+    g.valid = whole && !shift_stacked(c) ? g.L : valid;   // (stacked: one line up it is not)
+    g.offset = di * src.pw;
+    g.dj0 = (short)dj0; g.ns = (short)ns;
     g.stacked = 0;
-    g.K = n * L;
+    g.K = n * g.L;
+    g.r32 = KT % g.L;
+    g.step32 = (int)((unsigned)(KT / g.L) * (unsigned)c * src.pitch + (unsigned)(KT % g.L));
   };
-  const long long xs = (long long)c * h * w, es = (long long)c * h;
   const bool stacked = shift_stacked(c);
+  const int image = h * pl.src[0].pw;
   if (stacked) {
     // row shifts 0 and 1 from one group (both halves of the first operand), row shift 2 from another
-    group(0, pl.x, xs, h * w, w, h * w, h * w, w, 0, -2, 3, h);
-    group(1, pl.x, xs, h * w, w, h * w, h * w, w, 2, -2, 3, h);
-    group(2, pl.x, xs, h * w, w, h * w, h * w, w, 2, -2, 3, h);   // no items
+    group(0, 0, 0, image, 0, -2, 3);
+    group(1, 0, 0, image, 2, -2, 3);
+    group(2, 0, 0, image, 2, -2, 3);   // no items
     pl.grp[0].stacked = 2;
     pl.grp[1].stacked = 1;
   } else {
-    group(0, pl.x, xs, h * w, w, h * w, h * w, w, 0, 0, 3, h);
-    group(1, pl.x, xs, h * w, w, h * w, h * w, w, 1, -2, 5, h);
-    group(2, pl.x, xs, h * w, w, h * w, h * w, w, 2, -2, 5, h);
+    group(0, 0, 0, image, 0, 0, 3);
+    group(1, 0, 0, image, 1, -2, 5);
+    group(2, 0, 0, image, 2, -2, 5);
   }
   for (int last = 0; last < 2; ++last) {
-    group(3 + last, pl.x + (last ? (h - 1) * w : 0), xs, h * w, w, w, w, w, 0, 0, 3, 1);
-    const float *col = edges + (size_t)last * n * c * h;
-    group(5 + last, col, es, h, h, h, h, h, 0, 0, 3, 1);
+    group(3 + last, 0, last * (h - 1) * pl.src[0].pw, w, 0, 0, 3);
+    group(5 + last, 1 + last, 0, h, 0, 0, 3);
   }
   for (int lr = 0; lr < 2; ++lr)
-    for (int lc = 0; lc < 2; ++lc)
-      group(7 + 2 * lr + lc, edges + (size_t)lc * n * c * h + (lr ? h - 1 : 0), es, h, h, 1, 1, 1, 0, 0, 3, 1);
-  const long long nk = kfac::ceil_div(n * h * w, KT);
-  const ShiftSlices sl = stacked ? plan_stacked_slices(nk) : plan_shift_slices(WM, ntab, nk);
+    for (int lc = 0; lc < 2; ++lc) group(7 + 2 * lr + lc, 1 + lc, lr * (h - 1), 1, 0, 0, 3);
+  const long long nk = kfac::ceil_div(pl.grp[0].K, KT);
+  const long long strip[3] = {kfac::ceil_div(pl.grp[3].K, KT), kfac::ceil_div(pl.grp[5].K, KT), kfac::ceil_div(pl.grp[7].K, KT)};
+  const ShiftSlices sl = stacked ? plan_stacked_slices(nk) : plan_shift_slices(WM, ntab, nk, strip);
   const long long best_s5 = sl.s5, best_s3 = sl.s3;
   const double best_longest = sl.longest;
   // items: strips and corners first (block order), then the whole-image groups
@@ -1117,12 +1145,14 @@ int run_conv_shift(kfac::shift::Plan &pl, int d, int ones, float alpha, float be
   if (partial + partial_floats > arrays) return too_small(partial_floats + tail_floats + 4);
   {
     kfac::TimedLaunch timed(KFAC_TIMED_COV_AUX, stream);
-    KFAC_LAUNCH(edge_sums_kernel, dim3(c, nchunk), dim3(256), 0, stream, pl, sums, edges);
+    KFAC_LAUNCH(split_input_kernel, dim3(c, pl.nchunk), dim3(256), 0, stream, pl, sums);
   }
   KFAC_HIP_CHECK(hipGetLastError());
   {
     kfac::TimedLaunch timed(KFAC_TIMED_SYRK, stream);
-    KFAC_LAUNCH((corr_kernel<WM>), dim3(pl.total), dim3(THREADS), 0, stream, pl, partial);
+    KFAC_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(corr_kernel<WM>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, ShiftLds<WM>::kBytes));
+    KFAC_LAUNCH((corr_kernel<WM>), dim3(pl.total), dim3(256 * WM), ShiftLds<WM>::kBytes, stream, pl, partial);
   }
   KFAC_HIP_CHECK(hipGetLastError());
   int max_split = 1;
@@ -1139,7 +1169,7 @@ int run_conv_shift(kfac::shift::Plan &pl, int d, int ones, float alpha, float be
   }
   KFAC_HIP_CHECK(hipGetLastError());
   KFAC_LAUNCH(assemble_kernel, dim3(c, kfac::ceil_div(c, 64), c <= 128 ? 3 : 1), dim3(256), 0, stream, pl, arrays, sums,
-                     nchunk, d, ones, (float)((long long)n * h * w), alpha, beta, C);
+                     pl.nchunk, d, ones, (float)((long long)n * h * w), alpha, beta, C);
   KFAC_HIP_CHECK(hipGetLastError());
   return KFAC_OK;
 }

@@ -564,3 +564,30 @@ def test_resnet_3x3_shapes_take_the_shift_route(n, c, h, w):
     ops.cov_conv_a(torch.randn(2, 16, 9, 9, device='cuda'), 1, 1, 0, True, 0.5)
     assert lib.kfac_cov_conv_a_last_route() == 0      # KFAC_CONV_ROUTE_SLAB
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize('n,c,h,w', [(4, 64, 9, 12), (3, 32, 7, 10), (2, 130, 16, 5)])
+@pytest.mark.parametrize('kind', ['tiny', 'infinite', 'nan'])
+def test_shift_route_outside_the_range_of_the_split(kind, n, c, h, w):
+    """Values below 2^-110 keep their precision in products with large ones (three bfloat16 planes hold fewer than 24 bits
+    of them: about 1e-4 of the product), and an infinity or NaN in one channel leaves the entries of all others alone."""
+    import torch.nn.functional as TF
+    from chainerkfac_amd import ops
+    x = torch.randn((n, c, h, w), generator=torch.Generator().manual_seed(c))
+    if kind == 'tiny':
+        x[:, 3] *= 1e-36
+        x[:, 5] *= 1e30
+    else:
+        x[n - 1, 3, h // 2, w // 2] = float('inf') if kind == 'infinite' else float('nan')
+    out = ops.cov_conv_a(x.cuda(), 3, 1, 1, False, 1.0 / n).cpu().double()
+    p = TF.unfold(x.double(), 3, padding=1).transpose(1, 2).reshape(-1, 9 * c)
+    if kind == 'tiny':
+        got, want = out[27:36, 45:54], (p[:, 27:36].t() @ p[:, 45:54]) / n
+        scale = (p[:, 27:36].norm(dim=0)[:, None] * p[:, 45:54].norm(dim=0)[None, :]) / n
+        assert float(((got - want).abs() / scale).max()) < 2e-6
+    else:
+        others = [i for i in range(9 * c) if not 27 <= i < 36]
+        p = p[:, others]
+        assert bool(torch.isfinite(out[others][:, others]).all())
+        assert rel_err(out[others][:, others].numpy(), (p.t() @ p / n).numpy()) < RTOL
+        assert not bool(torch.isfinite(out[31, 31]))
