@@ -192,12 +192,12 @@ def family_times(lib):
 
 def takes_split_products(layer, i, batch):
     """Whether factor i of a layer (0: input, 1: output gradient) is made of split products: linear layers and slabs
-    (every output gradient, the input of a 1x1 convolution) over more than 128 k-values.  The k x k convolutions of
-    the benchmark's networks have kernels of the float32 instruction."""
+    (every output gradient, the input of a 1x1 convolution) over more than 128 k-values, and shifted correlations.  The
+    other k x k convolutions of the benchmark's networks have kernels of the float32 instruction."""
     from chainerkfac_amd import workloads as W
     if W.cov_rows(layer, batch) <= 128 or layer['kind'] == 'bn':
         return False
-    return i == 1 or layer['kind'] == 'linear' or layer['k'] == 1
+    return i == 1 or layer['kind'] == 'linear' or layer['k'] == 1 or W.takes_shift_route(layer)
 
 
 def cov_peak(layers, batch):
@@ -206,8 +206,12 @@ def cov_peak(layers, batch):
     from chainerkfac_amd import workloads as W
     split = 0.0
     for layer in layers:
-        m = W.cov_rows(layer, batch)
-        split += sum(m * d * (d + 1) for i, d in enumerate(W.factor_dims(layer)) if takes_split_products(layer, i, batch))
+        m, dims = W.cov_rows(layer, batch), W.factor_dims(layer)
+        gradient = m * dims[-1] * (dims[-1] + 1) if len(dims) > 1 else 0
+        if takes_split_products(layer, 0, batch):
+            split += W.cov_flops_executed([layer], batch) - gradient
+        if len(dims) > 1 and takes_split_products(layer, 1, batch):
+            split += gradient
     total = float(W.cov_flops_executed(layers, batch))
     return total / (split / SPLIT_PEAK_TFLOPS + (total - split) / FP32_MFMA_PEAK_TFLOPS)
 
@@ -514,8 +518,7 @@ def run_step_config(args, name, cfg, host=None):
             'inverse_tiles', 'batched dense inverse: sweep, border, lauum kernels',
             dense_inverse_flops, ('inv_call',), fam, empty,
             'd^3 flop of the densely inverted factors over the time between the first and the last launch of the '
-            'batched call (its kernels overlap on three streams, so their durations do not add up)',
-            reference_flop=flops['inverse']),
+            'batched call', reference_flop=flops['inverse'], peak=SPLIT_PEAK_TFLOPS),
         'precond_gemm': family_roofline(
             'precond_gemm', 'preconditioning GEMMs: gemm_group_kernel (both phases), gemm_group_finish_kernel, '
             'gemv_kernel + bn_select_kernel of the batch-norm blocks',
@@ -717,10 +720,9 @@ def run_inverse_config(args, name, cfg):
         'roofline': {
             'family': 'inverse_tiles',
             'kernel': 'batched dense inverse: sweep, border, lauum kernels', 'bound': 'mfma',
-            'achieved': round(achieved, 2), 'peak': FP32_MFMA_PEAK_TFLOPS, 'unit': 'TFLOP/s',
-            'frac': round(achieved / FP32_MFMA_PEAK_TFLOPS, 4),
-            'timed': 'd^3 flop per matrix over the wall time of the whole batched call (its kernels overlap on two '
-                     'streams, so their durations do not add up)',
+            'achieved': round(achieved, 2), 'peak': round(SPLIT_PEAK_TFLOPS, 1), 'unit': 'TFLOP/s',
+            'frac': round(achieved / SPLIT_PEAK_TFLOPS, 4),
+            'timed': 'd^3 flop per matrix over the wall time of the whole batched call',
             'traffic': None},
     }, dims
 
@@ -873,7 +875,7 @@ def write_per_layer(path, layers, config='c3'):
                 'factor of a 3x3 stride-1 convolution (29 shifted correlations of C x C instead of a 9C x 9C product); '
                 'flop/B = M d (d+1) over the bytes of the input tensor read once plus the factor written once; roofline '
                 'cap = min(matrix peak, flop/B x 8 TB/s), the matrix peak being 157.3 TFLOP/s of the float32 instruction for the '
-                'k x k convolutions and for reductions of at most 128 rows, and 419.4 TFLOP/s (a sixth of the dense bfloat16 '
+                'k x k convolutions that are not shifted correlations and for reductions of at most 128 rows, and 419.4 TFLOP/s (a sixth of the dense bfloat16 '
                 'peak) for the rest; the last column is the issued rate over the cap.'
                 '\n\n'.format(config, path, empty * 1e3))
         f.write('| layer (x count) | factor | d | rows M | GFLOP | GFLOP issued | SYRK kernel us | TFLOP/s (M d (d+1)) | '
@@ -1126,8 +1128,8 @@ def summarize_mfma(pmc_dir, out_path, command):
              '`SQ_VALU_MFMA_BUSY_CYCLES` sums, over the 1024 SIMDs, the cycles in which a SIMD\'s matrix pipe was '
              'busy; `GRBM_GUI_ACTIVE` sums the active cycles of the 8 XCDs.  busy = MFMA_BUSY / (GUI_ACTIVE / 8 x '
              '1024): the share of all matrix-pipe cycles of the launch (ramp-up, tail and padding work included) '
-             'in which an MFMA was executing.  `syrk_group_kernel`, `syrk_kernel` and the GEMM kernels execute '
-             '`v_mfma_f32_32x32x16_bf16`, six per 16 k-values of a float32 block (reductions of at most 128 k-values: '
+             'in which an MFMA was executing.  `syrk_group_kernel`, `syrk_kernel`, `shift::corr_kernel`, the GEMM '
+             'kernels, `sweep_kernel` and `lauum_kernel` execute `v_mfma_f32_32x32x16_bf16`, six per 16 k-values of a float32 block (reductions of at most 128 k-values: '
              '`v_mfma_f32_32x32x2_f32`), so busy x 419.4 TFLOP/s is their rate of executed (padded) float32 work; the '
              'other kernels execute `v_mfma_f32_32x32x2_f32`: busy x 157.3 TFLOP/s.', '',
              '| family | launches | matrix pipe busy |', '|---|---:|---:|']
