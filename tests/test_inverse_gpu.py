@@ -390,3 +390,15 @@ def test_inverse_error_of_other_matrices(kind, d):
     assert int(info.max()) == 0
     assert torch.equal(out[0], out[0].t())
     assert float((out[0].cpu().double() - want).norm() / want.norm()) <= bound
+
+
+def test_output_may_be_another_matrix():
+    """The sweep reads the inputs tile by tile while it runs and writes the outputs after it: a matrix that is the
+    output of another one changes nothing (its own output it may not be)."""
+    from chainerkfac_amd import ops
+    mats = [torch.from_numpy(spd(d, 500 + d)).cuda() * f for d in (513, 1025) for f in (1.0, 2.0)]
+    want, _ = ops.spd_inverse_batched(mats)
+    outs = [mats[1], mats[0], mats[3], mats[2]]
+    ops.spd_inverse_batched(mats, outs=outs)
+    for w, o in zip(want, outs):
+        assert torch.equal(w, o)
